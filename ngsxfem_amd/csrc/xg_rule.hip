@@ -5,11 +5,10 @@
 //            cutint/python_cutint.cpp:66-98 (IntegrateX sums).
 //
 // count: one thread per element (topology only, integer work).
-// fill : one wavefront per element, lanes = quadrature points; each lane
+// fill : a wavefront per run of elements, lanes = quadrature points; each lane
 //        writes one double4 (x, y, z, w), so a wave stores 2 KB contiguously.
-//        The decomposition is wave-uniform and recomputed by every lane
-//        (a few dozen FP64 operations) instead of being staged through HBM.
 #include "xg_device.hpp"
+#include "xg_elmat_core.hpp"
 #include "xg_internal.hpp"
 
 using namespace xg;
@@ -29,6 +28,15 @@ __device__ __forceinline__ void load_elem(const int32_t *__restrict__ el2v, cons
       for (int d = 0; d < 3; ++d) V[k][d] = d < D ? coords[(size_t)v * D + d] : 0.0;
     }
   }
+}
+
+// q / d for 0 <= q < 2^24, d >= 1 (float estimate, one correction step)
+__device__ __forceinline__ int small_div(int q, int d, float rd) {
+  int c = (int)((float)q * rd);
+  const int t = q - c * d;
+  if (t >= d) ++c;
+  else if (t < 0) --c;
+  return c;
 }
 
 template <int D>
@@ -57,114 +65,204 @@ __global__ void k_rule_count(int nel, const int32_t *__restrict__ elems, const i
   if (nsub) nsub[i] = (uint8_t)ns;
 }
 
+// One wave takes epw (a power of two, <= 64) consecutive elements.
+//  A. lane = element: the gathers, the class of the element and, for a cut
+//     one, its sign mask, cut parameters and interface factor;
+//  B. the uncut elements with points: lanes over (element, base point) pairs,
+//     so every lane stores whatever the rule's length;
+//  C. the cut elements in turn: the vertices and volumes of the sub-simplices
+//     are computed by a few lanes into LDS, then lanes = points.
+// Bound: the stores (32 B a point).  With one wave per element every element
+// without points cost a wave its whole chain of dependent gathers, an uncut
+// one filled 27 of 64 lanes at order 4, and the decomposition's indexed
+// private arrays lived in scratch memory (rule, coefficient, matrices and
+// vectors on 40^3 cells, order 6: 856 -> 728 us).
 template <int D>
 __global__ __launch_bounds__(256) void k_rule_fill(int nel, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
                                                    const double *__restrict__ coords,
-                                                   const double *__restrict__ lset, int dt, int order,
+                                                   const double *__restrict__ lset, int dt, int order, int epw,
                                                    const int32_t *__restrict__ offsets,
                                                    double4 *__restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int nwaves = (gridDim.x * blockDim.x) >> 6;
-  for (int i = wid; i < nel; i += nwaves) {
-    const int e = elems ? elems[i] : i;
-    double l[D + 1], V[D + 1][3];
-    load_elem<D>(el2v, lset, coords, e, l, V);
-    const int base = offsets[i];
-    const int npts = offsets[i + 1] - base;
-    if (npts == 0) continue;
-    const int eldom = check_if_straight_cut<D>(l);
-    if (eldom != IF) {
-      const int off = rule_off(D, order);
-      for (int q = lane; q < npts; q += 64) {
-        const double *r = xg_rule_data_d[off + q];
-        out[base + q] = make_double4(r[0], D > 1 ? r[1] : 0.0, D > 2 ? r[2] : 0.0, r[3]);
+  __shared__ int32_t s_base[4][64];
+  __shared__ double s_V[4][3][4][3];  // sub-simplex vertices (mapping order)
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const long long wid = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
+  const long long nwaves = (long long)gridDim.x * 4;
+  const int voff = rule_off(D, order), vcnt = rule_cnt(D, order);
+  const float rcnt = 1.0f / (float)vcnt;
+  const int Ds = dt == IF ? D - 1 : D, off = rule_off(Ds, order), nq = rule_cnt(Ds, order);
+  const float rnq = 1.0f / (float)nq;
+  for (long long i0 = wid * epw; i0 < nel; i0 += nwaves * epw) {
+    int base = 0, npts = 0, msk = 0;
+    bool uncut = false, cut = false;
+    double t[4] = {0.0, 0.0, 0.0, 0.0}, ifac = 1.0;
+    if (lane < epw && i0 + lane < nel) {
+      const int i = (int)i0 + lane;
+      base = offsets[i];
+      npts = offsets[i + 1] - base;
+      if (npts > 0) {
+        const int e = elems ? elems[i] : i;
+        double l[D + 1];
+        load_elem<D>(el2v, lset, nullptr, e, l, nullptr);
+        cut = check_if_straight_cut<D>(l) == IF;
+        uncut = !cut && npts >= vcnt;
+        if (cut) {
+          msk = sign_mask<D>(l);
+          // the cut points of the sign-changing edges in lexicographic order
+          // (p_i + (l_i / (l_i - l_j)) (p_j - p_i), straightcutrule.cpp:50)
+          int c = 0;
+#pragma unroll
+          for (int a = 0; a <= D; ++a)
+#pragma unroll
+            for (int b = a + 1; b <= D; ++b)
+              if (((msk >> a) & 1) != ((msk >> b) & 1)) {
+                const double q = l[a] / (l[a] - l[b]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) t[k] = c == k ? q : t[k];
+                ++c;
+              }
+          if (dt == IF) {
+            double ll[D + 1], V[D + 1][3], F[D * D], Finv[D * D], absdet;
+            load_elem<D>(el2v, lset, coords, e, ll, V);
+            jacobian<D>(V, F, Finv, absdet);
+            ifac = interface_factor<D>(l, Finv);
+          }
+        }
       }
-      continue;
     }
-    Decomp dc;
-    decompose<D>(l, dt, dc);
-    double P[D + 1 + 4][3];
-    cut_point_array<D>(l, dc, P);
-    const int Ds = dc.nv - 1;
-    const int nq = rule_cnt(Ds, order), off = rule_off(Ds, order);
-    double ifac = 1.0;
-    if (dt == IF) {
-      double F[D * D], Finv[D * D], absdet;
-      jacobian<D>(V, F, Finv, absdet);
-      ifac = interface_factor<D>(l, Finv);
+    const unsigned long long mu = __ballot(uncut), mc = __ballot(cut);
+    if (mu) {
+      if (uncut) s_base[wv][__popcll(mu & ((1ull << lane) - 1ull))] = base;
+      ecore::wave_sync();
+      const int total = __popcll(mu) * vcnt;
+      for (int g = lane; g < total; g += 64) {
+        const int s = small_div(g, vcnt, rcnt), k = g - s * vcnt;
+        const double *r = xg_rule_data_d[voff + k];
+        out[s_base[wv][s] + k] = make_double4(r[0], D > 1 ? r[1] : 0.0, D > 2 ? r[2] : 0.0, r[3]);
+      }
+      ecore::wave_sync();
     }
-    for (int g = lane; g < npts; g += 64) {
-      const int s = g / nq, k = g - s * nq;
-      const int8_t *idx = dc.v[s];
-      const double tf = simplex_volume(dc.nv, idx, P);
-      const double *r = xg_rule_data_d[off + k];
-      double ow = 1.0;
-      for (int m = 0; m < Ds; ++m) ow -= r[m];
-      double x[3];
+    for (unsigned long long m = mc; m; m &= m - 1) {
+      const int src = __builtin_ctzll(m);
+      const DecompEntry &E = xg_decomp_d.e[D - 1][dt][__builtin_amdgcn_readlane(msk, src)];
+      const int nv = E.nv, ns = E.ns;
+      const int cbase = __builtin_amdgcn_readlane(base, src), cnp = min(__builtin_amdgcn_readlane(npts, src), ns * nq);
+      const double t0 = __shfl(t[0], src, 64), t1 = __shfl(t[1], src, 64), t2 = __shfl(t[2], src, 64),
+                   t3 = __shfl(t[3], src, 64), cif = __shfl(ifac, src, 64);
+      if (lane < ns * nv) {
+        const int s = lane / nv, q = lane - s * nv;
+        const int code = E.v[s][q], c = code - (D + 1);
+        const int a = c >= 0 ? E.ce[c][0] : code, b = c >= 0 ? E.ce[c][1] : code;
+        const double tc = c == 1 ? t1 : (c == 2 ? t2 : (c == 3 ? t3 : t0));
 #pragma unroll
-      for (int d = 0; d < 3; ++d) x[d] = ow * P[idx[0]][d];
-      for (int m = 0; m < Ds; ++m)
+        for (int d = 0; d < 3; ++d) {
+          const double pa = (d == a && a < D) ? 1.0 : 0.0, pb = (d == b && b < D) ? 1.0 : 0.0;
+          s_V[wv][s][q][d] = c >= 0 ? pa + tc * (pb - pa) : pa;
+        }
+      }
+      ecore::wave_sync();
+      double tf[3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) x[d] += r[m] * P[idx[m + 1]][d];
-      double w = r[3] * tf;
-      if (dt == IF) w = w * ifac;
-      out[base + g] = make_double4(x[0], x[1], x[2], w);
+      for (int s = 0; s < 3; ++s) tf[s] = s < ns ? simplex_measure(nv - 1, s_V[wv][s]) : 0.0;
+      for (int g = lane; g < cnp; g += 64) {
+        const int s = small_div(g, nq, rnq), k = g - s * nq;
+        const double *r = xg_rule_data_d[off + k];
+        const double(*W)[3] = s_V[wv][s];
+        double ow = 1.0;
+#pragma unroll
+        for (int q = 0; q < D; ++q)
+          if (q < Ds) ow -= r[q];
+        double x[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) x[d] = ow * W[0][d];
+#pragma unroll
+        for (int q = 0; q < D; ++q)
+          if (q < Ds)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) x[d] += r[q] * W[q + 1][d];
+        double w = r[3] * (s == 0 ? tf[0] : (s == 1 ? tf[1] : tf[2]));
+        if (dt == IF) w = w * cif;
+        out[cbase + g] = make_double4(x[0], x[1], x[2], w);
+      }
+      ecore::wave_sync();
     }
   }
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void k_integrate(int nel, const int32_t *__restrict__ elems,
+// G lanes per element.  A wave per element ran most of its lanes on nothing
+// (27 points in 64 lanes, no points at all in the elements outside), and its
+// one atomic add per wave queued up on the single address of the total:
+// 262,144 adds took 3.16 ms at 64^3 cells, order 4.  Here a block adds its
+// waves' sums in LDS and at most 1024 blocks run, so the adds are few (count,
+// fill and integral together 3547 -> 340 us).
+template <int D, int G>
+__global__ __launch_bounds__(512) void k_integrate(int nel, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
                                                    const double *__restrict__ coords,
                                                    const int32_t *__restrict__ offsets,
                                                    const double4 *__restrict__ pts, Poly f,
                                                    double *__restrict__ per_elem, double *total) {
-  const int lane = threadIdx.x & 63;
-  const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int nwaves = (gridDim.x * blockDim.x) >> 6;
+  __shared__ double s_sum[8];
+  const int sub = threadIdx.x & (G - 1);
+  const long long ngrp = (long long)gridDim.x * (512 / G);
   double acc_all = 0.0;
-  for (int i = wid; i < nel; i += nwaves) {
-    const int e = elems ? elems[i] : i;
-    double V[D + 1][3];
-#pragma unroll
-    for (int k = 0; k <= D; ++k) {
-      const int v = el2v[(size_t)e * (D + 1) + k];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) V[k][d] = d < D ? coords[(size_t)v * D + d] : 0.0;
-    }
-    double F[D * D], Finv[D * D], absdet;
-    jacobian<D>(V, F, Finv, absdet);
+  for (long long i = ((long long)blockIdx.x * 512 + threadIdx.x) / G; i < nel; i += ngrp) {
+    const int q0 = offsets[i], q1 = offsets[i + 1];
     double s = 0.0;
-    for (int q = offsets[i] + lane; q < offsets[i + 1]; q += 64) {
-      const double4 p = pts[q];
-      const double xi[3] = {p.x, p.y, p.z};
-      double x[3] = {0.0, 0.0, 0.0};
+    if (q1 > q0) {
+      const int e = elems ? elems[i] : (int)i;
+      double V[D + 1][3];
 #pragma unroll
-      for (int r = 0; r < D; ++r) {
-        double a = V[D][r];
+      for (int k = 0; k <= D; ++k) {
+        const int v = el2v[(size_t)e * (D + 1) + k];
 #pragma unroll
-        for (int c = 0; c < D; ++c) a += F[r * D + c] * xi[c];
-        x[r] = a;
+        for (int d = 0; d < 3; ++d) V[k][d] = d < D ? coords[(size_t)v * D + d] : 0.0;
       }
-      double fv = 0.0;
-      for (int t = 0; t < f.n; ++t) {
-        double m = f.c[t];
-        for (int d = 0; d < 3; ++d)
-          for (int k = 0; k < f.ex[t][d]; ++k) m *= x[d];
-        fv += m;
+      double F[D * D], Finv[D * D], absdet;
+      jacobian<D>(V, F, Finv, absdet);
+      for (int q = q0 + sub; q < q1; q += G) {
+        const double4 p = pts[q];
+        const double xi[3] = {p.x, p.y, p.z};
+        double x[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int r = 0; r < D; ++r) {
+          double a = V[D][r];
+#pragma unroll
+          for (int c = 0; c < D; ++c) a += F[r * D + c] * xi[c];
+          x[r] = a;
+        }
+        double fv = 0.0;
+        for (int t = 0; t < f.n; ++t) {
+          double m = f.c[t];
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+            for (int k = 0; k < f.ex[t][d]; ++k) m *= x[d];
+          fv += m;
+        }
+        s += absdet * p.w * fv;
       }
-      s += absdet * p.w * fv;
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0 && per_elem) per_elem[i] = s;
-    acc_all += s;
+    for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (sub == 0) {
+      if (per_elem) per_elem[i] = s;
+      acc_all += s;
+    }
   }
-  if (lane == 0 && total) atomicAdd(total, acc_all);
+  if (!total) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) acc_all += __shfl_xor(acc_all, o, 64);
+  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = acc_all;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 8; ++w) acc_all += s_sum[w];
+    atomicAdd(total, acc_all);
+  }
 }
+
+__global__ void k_zero_f64(double *p) { *p = 0.0; }
 
 // integrals on fixed-node rules: W (nel x N) weights at the N nodes of the
 // degree-Q Lagrange lattice of the reference tetrahedron (xg_subdiv_weights);
@@ -215,11 +313,20 @@ __global__ __launch_bounds__(256) void k_integrate_nodes(int nel, const int32_t 
   if ((threadIdx.x & 63) == 0 && total) atomicAdd(total, s);
 }
 
-int grid_for_waves(int nel) {
-  long long blocks = ((long long)nel * 64 + 255) / 256;
-  if (blocks > 65536) blocks = 65536;
-  if (blocks < 1) blocks = 1;
-  return (int)blocks;
+// elements per wave of k_rule_fill: one while the waves would not fill the
+// device (8192 wave slots), then doubling up to a lane each
+int fill_epw(int nel) {
+  int epw = 1;
+  while (epw < 64 && nel / epw > 16384) epw *= 2;
+  return epw;
+}
+
+template <int D, int G>
+void launch_integrate(xg_ctx *ctx, int nel, const int32_t *elems, const int32_t *el2v, const double *coords,
+                      const int32_t *offsets, const double4 *pts, const Poly &f, double *per_elem, double *total) {
+  const long long want = ((long long)nel * G + 511) / 512;
+  const int grid = (int)(want < 1024 ? want : 1024);
+  k_integrate<D, G><<<grid, 512, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, pts, f, per_elem, total);
 }
 
 }  // namespace
@@ -257,12 +364,14 @@ extern "C" int xg_cut_rule_fill(xg_ctx *ctx, int D, int nel, const int32_t *elem
     return set_error(XG_ERR_ARG, "xg_cut_rule_fill: bad argument");
   if (nel == 0) return XG_OK;
   if (!el2v || !lset_v || !coords || !pts) return set_error(XG_ERR_ARG, "xg_cut_rule_fill: null pointer");
-  const int grid = grid_for_waves(nel);
+  const int epw = fill_epw(nel);
+  const long long want = ((long long)nel + 4LL * epw - 1) / (4LL * epw);
+  const int grid = (int)(want < 65536 ? want : 65536);
   double4 *o = reinterpret_cast<double4 *>(pts);
   switch (D) {
-    case 1: k_rule_fill<1><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, offsets, o); break;
-    case 2: k_rule_fill<2><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, offsets, o); break;
-    default: k_rule_fill<3><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, offsets, o); break;
+    case 1: k_rule_fill<1><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, epw, offsets, o); break;
+    case 2: k_rule_fill<2><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, epw, offsets, o); break;
+    default: k_rule_fill<3><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, epw, offsets, o); break;
   }
   XG_LAUNCH_CHECK();
   return XG_OK;
@@ -273,7 +382,8 @@ extern "C" int xg_integrate(xg_ctx *ctx, int D, int nel, const int32_t *elems, c
                             const double *coef, const int32_t *expo, double *per_elem, double *total) {
   if (!ctx || D < 1 || D > 3 || nel < 0 || nterms < 0 || nterms > 32 || (nterms > 0 && (!coef || !expo)))
     return set_error(XG_ERR_ARG, "xg_integrate: bad argument");
-  if (total) XG_CHECK(hipMemsetAsync(total, 0, sizeof(double), ctx->stream));
+  if (total) k_zero_f64<<<1, 1, 0, ctx->stream>>>(total);
+  XG_LAUNCH_CHECK();
   if (nel == 0) return XG_OK;
   if (!el2v || !coords || !offsets || !pts) return set_error(XG_ERR_ARG, "xg_integrate: null pointer");
   Poly f;
@@ -285,12 +395,13 @@ extern "C" int xg_integrate(xg_ctx *ctx, int D, int nel, const int32_t *elems, c
       f.ex[t][d] = expo[3 * t + d];
     }
   }
-  const int grid = grid_for_waves(nel);
+  // lanes per element: the fewest points that a rule of use has (order 2: 8
+  // on a tetrahedron, 4 on a triangle)
   const double4 *p = reinterpret_cast<const double4 *>(pts);
   switch (D) {
-    case 1: k_integrate<1><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
-    case 2: k_integrate<2><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
-    default: k_integrate<3><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
+    case 1: launch_integrate<1, 2>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
+    case 2: launch_integrate<2, 4>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
+    default: launch_integrate<3, 8>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
   }
   XG_LAUNCH_CHECK();
   return XG_OK;
