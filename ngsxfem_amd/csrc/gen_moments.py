@@ -425,6 +425,63 @@ def gen_affine(D, P, L, idx2):
     L.append("  }")
 
 
+def gen_series(D, P, L, idx2):
+    """aser_first / aser_step: the truncated power series of
+
+        prod_v 1 / (1 - <z, y_v>) = sum_beta h_beta z^beta,  |beta| <= 2P,
+
+    one vertex y_v of a simplex at a time (h in the slots of accum_aff).  The
+    integral of y^beta over a simplex of dimension k with vertices y_v is
+    |T| k! beta! / (|beta| + k)! h_beta (Dirichlet's integral), so a piece's
+    moments cost 3 FMAs per monomial of degree < 2P and vertex, whatever the
+    degree's quadrature rule: multiplying by 1 / (1 - l) is the in-place
+    recursion h_beta += sum_i l_i h_(beta - e_i) in ascending degree."""
+    n2 = 2 * P
+
+    def slot(b):
+        return idx2[tuple(b) + (n2 - sum(b),)]
+    for first in (True, False):
+        if first:
+            L.append("  // h = w / (1 - <z, y>), truncated at degree 2P")
+            L.append("  XG_DEV static void aser_first(const double *y, double w, double *h) {")
+            L.append("    h[%d] = w;" % slot([0] * D))
+        else:
+            L.append("  // h <- h / (1 - <z, y>), truncated at degree 2P")
+            L.append("  XG_DEV static void aser_step(const double *y, double *h) {")
+        for b in affine_monomials(D, n2):
+            if sum(b) == 0:
+                continue
+            e = None if first else "h[%d]" % slot(b)
+            for i in range(D):
+                if b[i] == 0:
+                    continue
+                c = list(b)
+                c[i] -= 1
+                src = "h[%d]" % slot(c)
+                e = "y[%d] * %s" % (i, src) if e is None else "fma(y[%d], %s, %s)" % (i, src, e)
+            L.append("    h[%d] = %s;" % (slot(b), e))
+        L.append("  }")
+
+
+def gen_series_table(D, P):
+    """beta! / (|beta| + k)! by slot, k = D (volume pieces, whose weight is
+    D! |T|) and k = D - 1 (interface pieces, weight (D - 1)! |T| times the
+    interface factor)"""
+    n2 = 2 * P
+    idx2 = {a: i for i, a in enumerate(monomials(D, n2))}
+    rows = [None] * len(idx2)
+    for b in affine_monomials(D, n2):
+        f = 1
+        for x in b:
+            f *= math.factorial(x)
+        rows[idx2[tuple(b) + (n2 - sum(b),)]] = [Fraction(f, math.factorial(sum(b) + k)) for k in (D, D - 1)]
+    L = ["// beta! / (|beta| + k)! of Moments<%d,%d>::aser_*, k = %d and %d" % (D, P, D, D - 1)]
+    L.append("XG_AFF_STORAGE const double xg_aser%d%d[%d][2] = {" % (D, P, len(rows)))
+    L += ["    {%r, %r}," % (float(a), float(b)) for a, b in rows]
+    L.append("};")
+    return "\n".join(L)
+
+
 def affine_monomials(D, n):
     """exponent tuples of length D with |beta| <= n, ascending degree"""
     res = []
@@ -543,6 +600,7 @@ def gen(D, P):
     L.append("  }")
     if D == 3:
         gen_affine(D, P, L, idx2)
+        gen_series(D, P, L, idx2)
     # ---- complement: m <- (moments of the whole reference simplex) - m.
     # int_T lam^alpha = |T| D! alpha! / (|alpha| + D)! with |T| = 1/D! (the
     # rule weights of the reference simplex sum to its volume)
@@ -667,7 +725,9 @@ def main():
     for D in (1, 2, 3):
         for P in (1, 2, 3):
             out.append(gen(D, P))
-    out.append(gen_affine_table(3, 3))
+    for P in (1, 2, 3):
+        out.append(gen_affine_table(3, P))
+        out.append(gen_series_table(3, P))
     out.append("#ifndef XG_MOM_NO_NODAL  // host builds of the identities leave the device table out")
     out.append(gen_nodal(3, 4))
     out.append("#endif")

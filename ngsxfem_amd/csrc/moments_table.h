@@ -1271,6 +1271,31 @@ struct Moments<3, 1> {
       m[7] = fma(wb, x[2], m[7]);
     }
   }
+  // h = w / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_first(const double *y, double w, double *h) {
+    h[9] = w;
+    h[3] = y[0] * h[9];
+    h[6] = y[1] * h[9];
+    h[8] = y[2] * h[9];
+    h[0] = y[0] * h[3];
+    h[1] = fma(y[1], h[3], y[0] * h[6]);
+    h[2] = fma(y[2], h[3], y[0] * h[8]);
+    h[4] = y[1] * h[6];
+    h[5] = fma(y[2], h[6], y[1] * h[8]);
+    h[7] = y[2] * h[8];
+  }
+  // h <- h / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_step(const double *y, double *h) {
+    h[3] = fma(y[0], h[9], h[3]);
+    h[6] = fma(y[1], h[9], h[6]);
+    h[8] = fma(y[2], h[9], h[8]);
+    h[0] = fma(y[0], h[3], h[0]);
+    h[1] = fma(y[1], h[3], fma(y[0], h[6], h[1]));
+    h[2] = fma(y[2], h[3], fma(y[0], h[8], h[2]));
+    h[4] = fma(y[1], h[6], h[4]);
+    h[5] = fma(y[2], h[6], fma(y[1], h[8], h[5]));
+    h[7] = fma(y[2], h[8], h[7]);
+  }
   // m_alpha <- int_T lam^alpha - m_alpha over the whole reference simplex T
   XG_DEV static void complement(double *m) {
     m[0] = 0.016666666666666666 - m[0];
@@ -1547,6 +1572,81 @@ struct Moments<3, 2> {
       m[31] = fma(wb, x[2], m[31]);
       m[30] = fma(wb, t5, m[30]);
     }
+  }
+  // h = w / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_first(const double *y, double w, double *h) {
+    h[34] = w;
+    h[19] = y[0] * h[34];
+    h[29] = y[1] * h[34];
+    h[33] = y[2] * h[34];
+    h[9] = y[0] * h[19];
+    h[15] = fma(y[1], h[19], y[0] * h[29]);
+    h[18] = fma(y[2], h[19], y[0] * h[33]);
+    h[25] = y[1] * h[29];
+    h[28] = fma(y[2], h[29], y[1] * h[33]);
+    h[32] = y[2] * h[33];
+    h[3] = y[0] * h[9];
+    h[6] = fma(y[1], h[9], y[0] * h[15]);
+    h[8] = fma(y[2], h[9], y[0] * h[18]);
+    h[12] = fma(y[1], h[15], y[0] * h[25]);
+    h[14] = fma(y[2], h[15], fma(y[1], h[18], y[0] * h[28]));
+    h[17] = fma(y[2], h[18], y[0] * h[32]);
+    h[22] = y[1] * h[25];
+    h[24] = fma(y[2], h[25], y[1] * h[28]);
+    h[27] = fma(y[2], h[28], y[1] * h[32]);
+    h[31] = y[2] * h[32];
+    h[0] = y[0] * h[3];
+    h[1] = fma(y[1], h[3], y[0] * h[6]);
+    h[2] = fma(y[2], h[3], y[0] * h[8]);
+    h[4] = fma(y[1], h[6], y[0] * h[12]);
+    h[5] = fma(y[2], h[6], fma(y[1], h[8], y[0] * h[14]));
+    h[7] = fma(y[2], h[8], y[0] * h[17]);
+    h[10] = fma(y[1], h[12], y[0] * h[22]);
+    h[11] = fma(y[2], h[12], fma(y[1], h[14], y[0] * h[24]));
+    h[13] = fma(y[2], h[14], fma(y[1], h[17], y[0] * h[27]));
+    h[16] = fma(y[2], h[17], y[0] * h[31]);
+    h[20] = y[1] * h[22];
+    h[21] = fma(y[2], h[22], y[1] * h[24]);
+    h[23] = fma(y[2], h[24], y[1] * h[27]);
+    h[26] = fma(y[2], h[27], y[1] * h[31]);
+    h[30] = y[2] * h[31];
+  }
+  // h <- h / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_step(const double *y, double *h) {
+    h[19] = fma(y[0], h[34], h[19]);
+    h[29] = fma(y[1], h[34], h[29]);
+    h[33] = fma(y[2], h[34], h[33]);
+    h[9] = fma(y[0], h[19], h[9]);
+    h[15] = fma(y[1], h[19], fma(y[0], h[29], h[15]));
+    h[18] = fma(y[2], h[19], fma(y[0], h[33], h[18]));
+    h[25] = fma(y[1], h[29], h[25]);
+    h[28] = fma(y[2], h[29], fma(y[1], h[33], h[28]));
+    h[32] = fma(y[2], h[33], h[32]);
+    h[3] = fma(y[0], h[9], h[3]);
+    h[6] = fma(y[1], h[9], fma(y[0], h[15], h[6]));
+    h[8] = fma(y[2], h[9], fma(y[0], h[18], h[8]));
+    h[12] = fma(y[1], h[15], fma(y[0], h[25], h[12]));
+    h[14] = fma(y[2], h[15], fma(y[1], h[18], fma(y[0], h[28], h[14])));
+    h[17] = fma(y[2], h[18], fma(y[0], h[32], h[17]));
+    h[22] = fma(y[1], h[25], h[22]);
+    h[24] = fma(y[2], h[25], fma(y[1], h[28], h[24]));
+    h[27] = fma(y[2], h[28], fma(y[1], h[32], h[27]));
+    h[31] = fma(y[2], h[32], h[31]);
+    h[0] = fma(y[0], h[3], h[0]);
+    h[1] = fma(y[1], h[3], fma(y[0], h[6], h[1]));
+    h[2] = fma(y[2], h[3], fma(y[0], h[8], h[2]));
+    h[4] = fma(y[1], h[6], fma(y[0], h[12], h[4]));
+    h[5] = fma(y[2], h[6], fma(y[1], h[8], fma(y[0], h[14], h[5])));
+    h[7] = fma(y[2], h[8], fma(y[0], h[17], h[7]));
+    h[10] = fma(y[1], h[12], fma(y[0], h[22], h[10]));
+    h[11] = fma(y[2], h[12], fma(y[1], h[14], fma(y[0], h[24], h[11])));
+    h[13] = fma(y[2], h[14], fma(y[1], h[17], fma(y[0], h[27], h[13])));
+    h[16] = fma(y[2], h[17], fma(y[0], h[31], h[16]));
+    h[20] = fma(y[1], h[22], h[20]);
+    h[21] = fma(y[2], h[22], fma(y[1], h[24], h[21]));
+    h[23] = fma(y[2], h[24], fma(y[1], h[27], h[23]));
+    h[26] = fma(y[2], h[27], fma(y[1], h[31], h[26]));
+    h[30] = fma(y[2], h[31], h[30]);
   }
   // m_alpha <- int_T lam^alpha - m_alpha over the whole reference simplex T
   XG_DEV static void complement(double *m) {
@@ -2353,6 +2453,179 @@ struct Moments<3, 3> {
       m[78] = fma(wb, t5, m[78]);
       m[77] = fma(wb, t15, m[77]);
     }
+  }
+  // h = w / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_first(const double *y, double w, double *h) {
+    h[83] = w;
+    h[55] = y[0] * h[83];
+    h[76] = y[1] * h[83];
+    h[82] = y[2] * h[83];
+    h[34] = y[0] * h[55];
+    h[49] = fma(y[1], h[55], y[0] * h[76]);
+    h[54] = fma(y[2], h[55], y[0] * h[82]);
+    h[70] = y[1] * h[76];
+    h[75] = fma(y[2], h[76], y[1] * h[82]);
+    h[81] = y[2] * h[82];
+    h[19] = y[0] * h[34];
+    h[29] = fma(y[1], h[34], y[0] * h[49]);
+    h[33] = fma(y[2], h[34], y[0] * h[54]);
+    h[44] = fma(y[1], h[49], y[0] * h[70]);
+    h[48] = fma(y[2], h[49], fma(y[1], h[54], y[0] * h[75]));
+    h[53] = fma(y[2], h[54], y[0] * h[81]);
+    h[65] = y[1] * h[70];
+    h[69] = fma(y[2], h[70], y[1] * h[75]);
+    h[74] = fma(y[2], h[75], y[1] * h[81]);
+    h[80] = y[2] * h[81];
+    h[9] = y[0] * h[19];
+    h[15] = fma(y[1], h[19], y[0] * h[29]);
+    h[18] = fma(y[2], h[19], y[0] * h[33]);
+    h[25] = fma(y[1], h[29], y[0] * h[44]);
+    h[28] = fma(y[2], h[29], fma(y[1], h[33], y[0] * h[48]));
+    h[32] = fma(y[2], h[33], y[0] * h[53]);
+    h[40] = fma(y[1], h[44], y[0] * h[65]);
+    h[43] = fma(y[2], h[44], fma(y[1], h[48], y[0] * h[69]));
+    h[47] = fma(y[2], h[48], fma(y[1], h[53], y[0] * h[74]));
+    h[52] = fma(y[2], h[53], y[0] * h[80]);
+    h[61] = y[1] * h[65];
+    h[64] = fma(y[2], h[65], y[1] * h[69]);
+    h[68] = fma(y[2], h[69], y[1] * h[74]);
+    h[73] = fma(y[2], h[74], y[1] * h[80]);
+    h[79] = y[2] * h[80];
+    h[3] = y[0] * h[9];
+    h[6] = fma(y[1], h[9], y[0] * h[15]);
+    h[8] = fma(y[2], h[9], y[0] * h[18]);
+    h[12] = fma(y[1], h[15], y[0] * h[25]);
+    h[14] = fma(y[2], h[15], fma(y[1], h[18], y[0] * h[28]));
+    h[17] = fma(y[2], h[18], y[0] * h[32]);
+    h[22] = fma(y[1], h[25], y[0] * h[40]);
+    h[24] = fma(y[2], h[25], fma(y[1], h[28], y[0] * h[43]));
+    h[27] = fma(y[2], h[28], fma(y[1], h[32], y[0] * h[47]));
+    h[31] = fma(y[2], h[32], y[0] * h[52]);
+    h[37] = fma(y[1], h[40], y[0] * h[61]);
+    h[39] = fma(y[2], h[40], fma(y[1], h[43], y[0] * h[64]));
+    h[42] = fma(y[2], h[43], fma(y[1], h[47], y[0] * h[68]));
+    h[46] = fma(y[2], h[47], fma(y[1], h[52], y[0] * h[73]));
+    h[51] = fma(y[2], h[52], y[0] * h[79]);
+    h[58] = y[1] * h[61];
+    h[60] = fma(y[2], h[61], y[1] * h[64]);
+    h[63] = fma(y[2], h[64], y[1] * h[68]);
+    h[67] = fma(y[2], h[68], y[1] * h[73]);
+    h[72] = fma(y[2], h[73], y[1] * h[79]);
+    h[78] = y[2] * h[79];
+    h[0] = y[0] * h[3];
+    h[1] = fma(y[1], h[3], y[0] * h[6]);
+    h[2] = fma(y[2], h[3], y[0] * h[8]);
+    h[4] = fma(y[1], h[6], y[0] * h[12]);
+    h[5] = fma(y[2], h[6], fma(y[1], h[8], y[0] * h[14]));
+    h[7] = fma(y[2], h[8], y[0] * h[17]);
+    h[10] = fma(y[1], h[12], y[0] * h[22]);
+    h[11] = fma(y[2], h[12], fma(y[1], h[14], y[0] * h[24]));
+    h[13] = fma(y[2], h[14], fma(y[1], h[17], y[0] * h[27]));
+    h[16] = fma(y[2], h[17], y[0] * h[31]);
+    h[20] = fma(y[1], h[22], y[0] * h[37]);
+    h[21] = fma(y[2], h[22], fma(y[1], h[24], y[0] * h[39]));
+    h[23] = fma(y[2], h[24], fma(y[1], h[27], y[0] * h[42]));
+    h[26] = fma(y[2], h[27], fma(y[1], h[31], y[0] * h[46]));
+    h[30] = fma(y[2], h[31], y[0] * h[51]);
+    h[35] = fma(y[1], h[37], y[0] * h[58]);
+    h[36] = fma(y[2], h[37], fma(y[1], h[39], y[0] * h[60]));
+    h[38] = fma(y[2], h[39], fma(y[1], h[42], y[0] * h[63]));
+    h[41] = fma(y[2], h[42], fma(y[1], h[46], y[0] * h[67]));
+    h[45] = fma(y[2], h[46], fma(y[1], h[51], y[0] * h[72]));
+    h[50] = fma(y[2], h[51], y[0] * h[78]);
+    h[56] = y[1] * h[58];
+    h[57] = fma(y[2], h[58], y[1] * h[60]);
+    h[59] = fma(y[2], h[60], y[1] * h[63]);
+    h[62] = fma(y[2], h[63], y[1] * h[67]);
+    h[66] = fma(y[2], h[67], y[1] * h[72]);
+    h[71] = fma(y[2], h[72], y[1] * h[78]);
+    h[77] = y[2] * h[78];
+  }
+  // h <- h / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_step(const double *y, double *h) {
+    h[55] = fma(y[0], h[83], h[55]);
+    h[76] = fma(y[1], h[83], h[76]);
+    h[82] = fma(y[2], h[83], h[82]);
+    h[34] = fma(y[0], h[55], h[34]);
+    h[49] = fma(y[1], h[55], fma(y[0], h[76], h[49]));
+    h[54] = fma(y[2], h[55], fma(y[0], h[82], h[54]));
+    h[70] = fma(y[1], h[76], h[70]);
+    h[75] = fma(y[2], h[76], fma(y[1], h[82], h[75]));
+    h[81] = fma(y[2], h[82], h[81]);
+    h[19] = fma(y[0], h[34], h[19]);
+    h[29] = fma(y[1], h[34], fma(y[0], h[49], h[29]));
+    h[33] = fma(y[2], h[34], fma(y[0], h[54], h[33]));
+    h[44] = fma(y[1], h[49], fma(y[0], h[70], h[44]));
+    h[48] = fma(y[2], h[49], fma(y[1], h[54], fma(y[0], h[75], h[48])));
+    h[53] = fma(y[2], h[54], fma(y[0], h[81], h[53]));
+    h[65] = fma(y[1], h[70], h[65]);
+    h[69] = fma(y[2], h[70], fma(y[1], h[75], h[69]));
+    h[74] = fma(y[2], h[75], fma(y[1], h[81], h[74]));
+    h[80] = fma(y[2], h[81], h[80]);
+    h[9] = fma(y[0], h[19], h[9]);
+    h[15] = fma(y[1], h[19], fma(y[0], h[29], h[15]));
+    h[18] = fma(y[2], h[19], fma(y[0], h[33], h[18]));
+    h[25] = fma(y[1], h[29], fma(y[0], h[44], h[25]));
+    h[28] = fma(y[2], h[29], fma(y[1], h[33], fma(y[0], h[48], h[28])));
+    h[32] = fma(y[2], h[33], fma(y[0], h[53], h[32]));
+    h[40] = fma(y[1], h[44], fma(y[0], h[65], h[40]));
+    h[43] = fma(y[2], h[44], fma(y[1], h[48], fma(y[0], h[69], h[43])));
+    h[47] = fma(y[2], h[48], fma(y[1], h[53], fma(y[0], h[74], h[47])));
+    h[52] = fma(y[2], h[53], fma(y[0], h[80], h[52]));
+    h[61] = fma(y[1], h[65], h[61]);
+    h[64] = fma(y[2], h[65], fma(y[1], h[69], h[64]));
+    h[68] = fma(y[2], h[69], fma(y[1], h[74], h[68]));
+    h[73] = fma(y[2], h[74], fma(y[1], h[80], h[73]));
+    h[79] = fma(y[2], h[80], h[79]);
+    h[3] = fma(y[0], h[9], h[3]);
+    h[6] = fma(y[1], h[9], fma(y[0], h[15], h[6]));
+    h[8] = fma(y[2], h[9], fma(y[0], h[18], h[8]));
+    h[12] = fma(y[1], h[15], fma(y[0], h[25], h[12]));
+    h[14] = fma(y[2], h[15], fma(y[1], h[18], fma(y[0], h[28], h[14])));
+    h[17] = fma(y[2], h[18], fma(y[0], h[32], h[17]));
+    h[22] = fma(y[1], h[25], fma(y[0], h[40], h[22]));
+    h[24] = fma(y[2], h[25], fma(y[1], h[28], fma(y[0], h[43], h[24])));
+    h[27] = fma(y[2], h[28], fma(y[1], h[32], fma(y[0], h[47], h[27])));
+    h[31] = fma(y[2], h[32], fma(y[0], h[52], h[31]));
+    h[37] = fma(y[1], h[40], fma(y[0], h[61], h[37]));
+    h[39] = fma(y[2], h[40], fma(y[1], h[43], fma(y[0], h[64], h[39])));
+    h[42] = fma(y[2], h[43], fma(y[1], h[47], fma(y[0], h[68], h[42])));
+    h[46] = fma(y[2], h[47], fma(y[1], h[52], fma(y[0], h[73], h[46])));
+    h[51] = fma(y[2], h[52], fma(y[0], h[79], h[51]));
+    h[58] = fma(y[1], h[61], h[58]);
+    h[60] = fma(y[2], h[61], fma(y[1], h[64], h[60]));
+    h[63] = fma(y[2], h[64], fma(y[1], h[68], h[63]));
+    h[67] = fma(y[2], h[68], fma(y[1], h[73], h[67]));
+    h[72] = fma(y[2], h[73], fma(y[1], h[79], h[72]));
+    h[78] = fma(y[2], h[79], h[78]);
+    h[0] = fma(y[0], h[3], h[0]);
+    h[1] = fma(y[1], h[3], fma(y[0], h[6], h[1]));
+    h[2] = fma(y[2], h[3], fma(y[0], h[8], h[2]));
+    h[4] = fma(y[1], h[6], fma(y[0], h[12], h[4]));
+    h[5] = fma(y[2], h[6], fma(y[1], h[8], fma(y[0], h[14], h[5])));
+    h[7] = fma(y[2], h[8], fma(y[0], h[17], h[7]));
+    h[10] = fma(y[1], h[12], fma(y[0], h[22], h[10]));
+    h[11] = fma(y[2], h[12], fma(y[1], h[14], fma(y[0], h[24], h[11])));
+    h[13] = fma(y[2], h[14], fma(y[1], h[17], fma(y[0], h[27], h[13])));
+    h[16] = fma(y[2], h[17], fma(y[0], h[31], h[16]));
+    h[20] = fma(y[1], h[22], fma(y[0], h[37], h[20]));
+    h[21] = fma(y[2], h[22], fma(y[1], h[24], fma(y[0], h[39], h[21])));
+    h[23] = fma(y[2], h[24], fma(y[1], h[27], fma(y[0], h[42], h[23])));
+    h[26] = fma(y[2], h[27], fma(y[1], h[31], fma(y[0], h[46], h[26])));
+    h[30] = fma(y[2], h[31], fma(y[0], h[51], h[30]));
+    h[35] = fma(y[1], h[37], fma(y[0], h[58], h[35]));
+    h[36] = fma(y[2], h[37], fma(y[1], h[39], fma(y[0], h[60], h[36])));
+    h[38] = fma(y[2], h[39], fma(y[1], h[42], fma(y[0], h[63], h[38])));
+    h[41] = fma(y[2], h[42], fma(y[1], h[46], fma(y[0], h[67], h[41])));
+    h[45] = fma(y[2], h[46], fma(y[1], h[51], fma(y[0], h[72], h[45])));
+    h[50] = fma(y[2], h[51], fma(y[0], h[78], h[50]));
+    h[56] = fma(y[1], h[58], h[56]);
+    h[57] = fma(y[2], h[58], fma(y[1], h[60], h[57]));
+    h[59] = fma(y[2], h[60], fma(y[1], h[63], h[59]));
+    h[62] = fma(y[2], h[63], fma(y[1], h[67], h[62]));
+    h[66] = fma(y[2], h[67], fma(y[1], h[72], h[66]));
+    h[71] = fma(y[2], h[72], fma(y[1], h[78], h[71]));
+    h[77] = fma(y[2], h[78], h[77]);
   }
   // m_alpha <- int_T lam^alpha - m_alpha over the whole reference simplex T
   XG_DEV static void complement(double *m) {
@@ -3959,6 +4232,116 @@ struct Moments<3, 3> {
     out[19] = (T)(s * (27.0 * m[14] + 81.0 * m[24] + 81.0 * m[27] + 81.0 * m[28] + 81.0 * m[39] + 162.0 * m[42] + 162.0 * m[43] + 81.0 * m[46] + 162.0 * m[47] + 81.0 * m[48] + 27.0 * m[60] + 81.0 * m[63] + 81.0 * m[64] + 81.0 * m[67] + 162.0 * m[68] + 81.0 * m[69] + 27.0 * m[72] + 81.0 * m[73] + 81.0 * m[74] + 27.0 * m[75]));
   }
 };  // 9054 coefficient terms
+// centred affine moments (y = lam - 1/4) -> homogeneous degree-2 moments, D = 3:
+// m[alpha] = sum_slot xg_aff31[slot][alpha % 64][alpha / 64] n[slot]
+#ifndef XG_AFF_STORAGE
+#define XG_AFF_STORAGE static __device__
+#endif
+XG_AFF_STORAGE const float xg_aff31[10][64][2] __attribute__((aligned(16))) = {
+    {{1.0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0.5, 0}, {0.25, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {0, 0}, {-0.25, 0}, {-0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0.25, 0}, {0, 0}, {-0.25, 0}, {0.5, 0}, {0.25, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {-0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0.5, 0}, {0, 0}, {-0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0.0625, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+};
+// beta! / (|beta| + k)! of Moments<3,1>::aser_*, k = 3 and 2
+XG_AFF_STORAGE const double xg_aser31[10][2] = {
+    {0.016666666666666666, 0.08333333333333333},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.16666666666666666, 0.5},
+};
+// centred affine moments (y = lam - 1/4) -> homogeneous degree-4 moments, D = 3:
+// m[alpha] = sum_slot xg_aff32[slot][alpha % 64][alpha / 64] n[slot]
+#ifndef XG_AFF_STORAGE
+#define XG_AFF_STORAGE static __device__
+#endif
+XG_AFF_STORAGE const float xg_aff32[35][64][2] __attribute__((aligned(16))) = {
+    {{1.0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {4.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {4.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{1.0, 0}, {0.25, 0}, {0.25, 0}, {-0.5, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {0, 0}, {-0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0.25, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {6.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {2.0, 0}, {-6.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-3.0, 0}, {12.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0.75, 0}, {0, 0}, {-0.75, 0}, {0.5, 0}, {0.25, 0}, {-0.5, 0}, {0, 0}, {-0.25, 0}, {0.5, 0}, {0, 0}, {0, 0}, {-0.5, 0}, {0, 0}, {-0.25, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0.5, 0}, {0.75, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.75, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-3.0, 0}, {6.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0.75, 0}, {-0.75, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0.5, 0}, {-0.5, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {0.5, 0}, {0, 0}, {-0.5, 0}, {0.25, 0}, {0.75, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {-0.75, 0}, {0, 0}, {0, 0}, {0.5, 0}, {0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0.375, 0}, {0.1875, 0}, {0.1875, 0}, {0, 0}, {0.0625, 0}, {0.0625, 0}, {-0.0625, 0}, {0.0625, 0}, {-0.0625, 0}, {-0.125, 0}, {0, 0}, {0, 0}, {-0.0625, 0}, {0, 0}, {-0.0625, 0}, {-0.0625, 0}, {0, 0}, {-0.0625, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {0.1875, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {0.1875, 0}, {0.375, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {4.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {2.0, 0}, {-6.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-3.0, 0}, {12.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.5, 0}, {0, 0}, {-0.5, 0}, {0, 0}, {0, 0}, {0.5, 0}, {0.75, 0}, {0.25, 0}, {-0.5, 0}, {0, 0}, {-0.25, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.75, 0}, {0, 0}, {-0.25, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0.5, 0}, {0.75, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.75, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {2.0, 0}, {-6.0, 0}, {12.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.5, 0}, {-0.5, 0}, {0, 0}, {-0.5, 0}, {1.0, 0}, {0, 0}, {0.5, 0}, {-0.5, 0}, {0.5, 0}, {-0.5, 0}, {0.5, 0}, {0, 0}, {-0.5, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.5, 0}, {1.0, 0}, {0, 0}, {-0.5, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {-6.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0.1875, 0}, {0, 0}, {-0.1875, 0}, {0.25, 0}, {0.125, 0}, {-0.0625, 0}, {0, 0}, {-0.125, 0}, {-0.125, 0}, {0.1875, 0}, {0.125, 0}, {-0.0625, 0}, {0.0625, 0}, {-0.0625, 0}, {-0.0625, 0}, {0, 0}, {-0.0625, 0}, {0, 0}, {0.1875, 0}, {0, 0}, {0, 0}, {-0.1875, 0}, {0, 0}, {-0.125, 0}, {-0.125, 0}, {0, 0}, {-0.0625, 0}, {0, 0}, {0.1875, 0}, {0, 0}, {0, 0}, {0.125, 0}, {0.375, 0}, {0.75, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {-3.0, 0}, {4.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.5, 0}, {-0.5, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0.25, 0}, {0.75, 0}, {-0.5, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {0.5, 0}, {-0.75, 0}, {0, 0}, {-0.75, 0}, {0.5, 0}, {0.75, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0.1875, 0}, {-0.1875, 0}, {0, 0}, {0.125, 0}, {-0.125, 0}, {0.25, 0}, {-0.0625, 0}, {-0.125, 0}, {0, 0}, {0.0625, 0}, {-0.0625, 0}, {0.125, 0}, {-0.0625, 0}, {0, 0}, {0.1875, 0}, {-0.0625, 0}, {-0.0625, 0}, {0.1875, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.0625, 0}, {0.125, 0}, {0, 0}, {-0.125, 0}, {0, 0}, {0.375, 0}, {0, 0}, {-0.1875, 0}, {-0.125, 0}, {0.1875, 0}, {0.75, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0.0625, 0}, {0.046875, 0}, {0.046875, 0}, {0.03125, 0}, {0.03125, 0}, {0.03125, 0}, {0.015625, 0}, {0.03125, 0}, {0.015625, 0}, {0, 0}, {0.015625, 0}, {0.015625, 0}, {0, 0}, {0.015625, 0}, {0, 0}, {-0.015625, 0}, {0.015625, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {0, 0}, {0, 0}, {-0.015625, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {-0.046875, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {-0.046875, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {-1.0, 0}, {4.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {0, 0}, {-0.25, 0}, {0, 0}, {0, 0}, {0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {1.0, 0}, {0.25, 0}, {-0.5, 0}, {0, 0}, {-0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0, 0}, {-0.25, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-3.0, 0}, {6.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0, 0}, {-0.25, 0}, {0.5, 0}, {0, 0}, {0, 0}, {0.25, 0}, {-0.75, 0}, {0, 0}, {0.75, 0}, {-0.75, 0}, {0.5, 0}, {-0.5, 0}, {0.5, 0}, {0, 0}, {-0.5, 0}, {0.25, 0}, {0.75, 0}, {0, 0}, {0, 0}, {0.5, 0}, {0, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {0, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {0.1875, 0}, {0.0625, 0}, {-0.0625, 0}, {0, 0}, {-0.0625, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {0.1875, 0}, {0.375, 0}, {0.1875, 0}, {0, 0}, {0.0625, 0}, {-0.0625, 0}, {-0.125, 0}, {0, 0}, {-0.0625, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {0.1875, 0}, {0.375, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {-1.0, 0}, {0, 0}, {-1.0, 0}, {2.0, 0}, {-3.0, 0}, {4.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0.25, 0}, {0, 0}, {-0.25, 0}, {0.5, 0}, {-0.75, 0}, {0, 0}, {0, 0}, {0, 0}, {0.5, 0}, {-0.5, 0}, {0.5, 0}, {0.75, 0}, {-0.5, 0}, {0.25, 0}, {0, 0}, {0, 0}, {-0.75, 0}, {0.5, 0}, {0.75, 0}, {-3.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {-0.0625, 0}, {0, 0}, {-0.0625, 0}, {0.125, 0}, {0, 0}, {0.125, 0}, {-0.125, 0}, {0.125, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {-0.125, 0}, {0, 0}, {0.375, 0}, {0, 0}, {0.1875, 0}, {-0.1875, 0}, {0.25, 0}, {-0.0625, 0}, {-0.125, 0}, {0.1875, 0}, {-0.0625, 0}, {-0.0625, 0}, {0.1875, 0}, {0, 0}, {-0.1875, 0}, {-0.125, 0}, {0.1875, 0}, {0.75, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0.015625, 0}, {0, 0}, {-0.015625, 0}, {0.03125, 0}, {0.015625, 0}, {0, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {0.046875, 0}, {0.03125, 0}, {0.015625, 0}, {0.015625, 0}, {0, 0}, {-0.015625, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {-0.046875, 0}, {0.0625, 0}, {0.046875, 0}, {0.03125, 0}, {0.03125, 0}, {0.015625, 0}, {0, 0}, {0.015625, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {0, 0}, {-0.015625, 0}, {-0.03125, 0}, {-0.046875, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {-1.0, 0}, {1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0.25, 0}, {-0.25, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.25, 0}, {-0.25, 0}, {0.25, 0}, {-0.25, 0}, {1.0, 0}, {-0.5, 0}, {0, 0}, {0.5, 0}, {-1.0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {-0.0625, 0}, {0.0625, 0}, {0, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {-0.0625, 0}, {0.0625, 0}, {0.1875, 0}, {-0.0625, 0}, {-0.0625, 0}, {0.1875, 0}, {0, 0}, {0, 0}, {0, 0}, {0.0625, 0}, {-0.0625, 0}, {0.0625, 0}, {0.1875, 0}, {-0.0625, 0}, {-0.0625, 0}, {0.1875, 0}, {0.375, 0}, {0, 0}, {-0.125, 0}, {0, 0}, {0.375, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0, 0}, {0, 0}, {0.015625, 0}, {-0.015625, 0}, {0, 0}, {0.015625, 0}, {-0.015625, 0}, {0.03125, 0}, {0, 0}, {-0.03125, 0}, {0, 0}, {0.015625, 0}, {-0.015625, 0}, {0.03125, 0}, {0, 0}, {-0.03125, 0}, {0.046875, 0}, {0.015625, 0}, {-0.015625, 0}, {-0.046875, 0}, {0, 0}, {0.015625, 0}, {-0.015625, 0}, {0.03125, 0}, {0, 0}, {-0.03125, 0}, {0.046875, 0}, {0.015625, 0}, {-0.015625, 0}, {-0.046875, 0}, {0.0625, 0}, {0.03125, 0}, {0, 0}, {-0.03125, 0}, {-0.0625, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+    {{0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0.00390625, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}},
+};
+// beta! / (|beta| + k)! of Moments<3,2>::aser_*, k = 3 and 2
+XG_AFF_STORAGE const double xg_aser32[35][2] = {
+    {0.004761904761904762, 0.03333333333333333},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.008333333333333333, 0.05},
+    {0.0007936507936507937, 0.005555555555555556},
+    {0.0003968253968253968, 0.002777777777777778},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.0007936507936507937, 0.005555555555555556},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.0003968253968253968, 0.002777777777777778},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.0003968253968253968, 0.002777777777777778},
+    {0.001388888888888889, 0.008333333333333333},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.004761904761904762, 0.03333333333333333},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.008333333333333333, 0.05},
+    {0.0007936507936507937, 0.005555555555555556},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.004761904761904762, 0.03333333333333333},
+    {0.008333333333333333, 0.05},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.16666666666666666, 0.5},
+};
 // centred affine moments (y = lam - 1/4) -> homogeneous degree-6 moments, D = 3:
 // m[alpha] = sum_slot xg_aff33[slot][alpha % 64][alpha / 64] n[slot]
 #ifndef XG_AFF_STORAGE
@@ -4049,6 +4432,93 @@ XG_AFF_STORAGE const float xg_aff33[84][64][2] __attribute__((aligned(16))) = {
     {{0, -0.00390625}, {0, 0.01171875}, {0, 0.0234375}, {0, 0}, {0, -0.0078125}, {0, 0}, {0, 0.0234375}, {0.00390625, 0.0390625}, {-0.00390625, 0.0078125}, {0.00390625, -0.0078125}, {0, -0.0078125}, {0, 0.0078125}, {0, 0.0390625}, {0.00390625, 0.05859375}, {-0.00390625, 0.01953125}, {0.00390625, -0.00390625}, {0.01171875, -0.01171875}, {-0.00390625, -0.00390625}, {-0.00390625, 0.01953125}, {0.01171875, 0.05859375}, {0, 0}, {0, 0}, {0, 0}, {0.00390625, 0}, {-0.00390625, 0}, {0.00390625, 0}, {0.01171875, 0}, {-0.00390625, 0}, {-0.00390625, 0}, {0.01171875, 0}, {0.0234375, 0}, {0, 0}, {-0.0078125, 0}, {0, 0}, {0.0234375, 0}, {0, 0}, {0, 0}, {0, 0}, {0.00390625, 0}, {-0.00390625, 0}, {0.00390625, 0}, {0.01171875, 0}, {-0.00390625, 0}, {-0.00390625, 0}, {0.01171875, 0}, {0.0234375, 0}, {0, 0}, {-0.0078125, 0}, {0, 0}, {0.0234375, 0}, {0.0390625, 0}, {0.0078125, 0}, {-0.0078125, 0}, {-0.0078125, 0}, {0.0078125, 0}, {0.0390625, 0}, {0, 0}, {0, 0}, {0, 0}, {0.00390625, 0}, {-0.00390625, 0}, {0.00390625, 0}, {0.01171875, 0}, {-0.00390625, 0}},
     {{0, -0.0009765625}, {0, -0.0029296875}, {0.0009765625, 0.00390625}, {-0.0009765625, 0.001953125}, {0, 0}, {0.0009765625, -0.001953125}, {-0.0009765625, -0.00390625}, {0.001953125, 0.0048828125}, {0, 0.0029296875}, {-0.001953125, 0.0009765625}, {0, -0.0009765625}, {0.0009765625, -0.0029296875}, {-0.0009765625, -0.0048828125}, {0.001953125, 0.005859375}, {0, 0.00390625}, {-0.001953125, 0.001953125}, {0.0029296875, 0}, {0.0009765625, -0.001953125}, {-0.0009765625, -0.00390625}, {-0.0029296875, -0.005859375}, {0, 0}, {0.0009765625, 0}, {-0.0009765625, 0}, {0.001953125, 0}, {0, 0}, {-0.001953125, 0}, {0.0029296875, 0}, {0.0009765625, 0}, {-0.0009765625, 0}, {-0.0029296875, 0}, {0.00390625, 0}, {0.001953125, 0}, {0, 0}, {-0.001953125, 0}, {-0.00390625, 0}, {0, 0}, {0.0009765625, 0}, {-0.0009765625, 0}, {0.001953125, 0}, {0, 0}, {-0.001953125, 0}, {0.0029296875, 0}, {0.0009765625, 0}, {-0.0009765625, 0}, {-0.0029296875, 0}, {0.00390625, 0}, {0.001953125, 0}, {0, 0}, {-0.001953125, 0}, {-0.00390625, 0}, {0.0048828125, 0}, {0.0029296875, 0}, {0.0009765625, 0}, {-0.0009765625, 0}, {-0.0029296875, 0}, {-0.0048828125, 0}, {0, 0}, {0.0009765625, 0}, {-0.0009765625, 0}, {0.001953125, 0}, {0, 0}, {-0.001953125, 0}, {0.0029296875, 0}, {0.0009765625, 0}},
     {{0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0.000244140625}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}, {0.000244140625, 0}},
+};
+// beta! / (|beta| + k)! of Moments<3,3>::aser_*, k = 3 and 2
+XG_AFF_STORAGE const double xg_aser33[84][2] = {
+    {0.001984126984126984, 0.017857142857142856},
+    {0.00033068783068783067, 0.002976190476190476},
+    {0.00033068783068783067, 0.002976190476190476},
+    {0.002976190476190476, 0.023809523809523808},
+    {0.00013227513227513228, 0.0011904761904761906},
+    {6.613756613756614e-05, 0.0005952380952380953},
+    {0.0005952380952380953, 0.004761904761904762},
+    {0.00013227513227513228, 0.0011904761904761906},
+    {0.0005952380952380953, 0.004761904761904762},
+    {0.004761904761904762, 0.03333333333333333},
+    {9.92063492063492e-05, 0.0008928571428571428},
+    {3.306878306878307e-05, 0.00029761904761904765},
+    {0.00029761904761904765, 0.002380952380952381},
+    {3.306878306878307e-05, 0.00029761904761904765},
+    {0.00014880952380952382, 0.0011904761904761906},
+    {0.0011904761904761906, 0.008333333333333333},
+    {9.92063492063492e-05, 0.0008928571428571428},
+    {0.00029761904761904765, 0.002380952380952381},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.008333333333333333, 0.05},
+    {0.00013227513227513228, 0.0011904761904761906},
+    {3.306878306878307e-05, 0.00029761904761904765},
+    {0.00029761904761904765, 0.002380952380952381},
+    {2.2045855379188714e-05, 0.0001984126984126984},
+    {9.92063492063492e-05, 0.0007936507936507937},
+    {0.0007936507936507937, 0.005555555555555556},
+    {3.306878306878307e-05, 0.00029761904761904765},
+    {9.92063492063492e-05, 0.0007936507936507937},
+    {0.0003968253968253968, 0.002777777777777778},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.00013227513227513228, 0.0011904761904761906},
+    {0.00029761904761904765, 0.002380952380952381},
+    {0.0007936507936507937, 0.005555555555555556},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.00033068783068783067, 0.002976190476190476},
+    {6.613756613756614e-05, 0.0005952380952380953},
+    {0.0005952380952380953, 0.004761904761904762},
+    {3.306878306878307e-05, 0.00029761904761904765},
+    {0.00014880952380952382, 0.0011904761904761906},
+    {0.0011904761904761906, 0.008333333333333333},
+    {3.306878306878307e-05, 0.00029761904761904765},
+    {9.92063492063492e-05, 0.0007936507936507937},
+    {0.0003968253968253968, 0.002777777777777778},
+    {0.002777777777777778, 0.016666666666666666},
+    {6.613756613756614e-05, 0.0005952380952380953},
+    {0.00014880952380952382, 0.0011904761904761906},
+    {0.0003968253968253968, 0.002777777777777778},
+    {0.001388888888888889, 0.008333333333333333},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.00033068783068783067, 0.002976190476190476},
+    {0.0005952380952380953, 0.004761904761904762},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.001984126984126984, 0.017857142857142856},
+    {0.00033068783068783067, 0.002976190476190476},
+    {0.002976190476190476, 0.023809523809523808},
+    {0.00013227513227513228, 0.0011904761904761906},
+    {0.0005952380952380953, 0.004761904761904762},
+    {0.004761904761904762, 0.03333333333333333},
+    {9.92063492063492e-05, 0.0008928571428571428},
+    {0.00029761904761904765, 0.002380952380952381},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.008333333333333333, 0.05},
+    {0.00013227513227513228, 0.0011904761904761906},
+    {0.00029761904761904765, 0.002380952380952381},
+    {0.0007936507936507937, 0.005555555555555556},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.00033068783068783067, 0.002976190476190476},
+    {0.0005952380952380953, 0.004761904761904762},
+    {0.0011904761904761906, 0.008333333333333333},
+    {0.002777777777777778, 0.016666666666666666},
+    {0.008333333333333333, 0.041666666666666664},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.001984126984126984, 0.017857142857142856},
+    {0.002976190476190476, 0.023809523809523808},
+    {0.004761904761904762, 0.03333333333333333},
+    {0.008333333333333333, 0.05},
+    {0.016666666666666666, 0.08333333333333333},
+    {0.041666666666666664, 0.16666666666666666},
+    {0.16666666666666666, 0.5},
 };
 #ifndef XG_MOM_NO_NODAL  // host builds of the identities leave the device table out
 // degree-4 Lagrange basis of the reference simplex (D = 3) in homogeneous

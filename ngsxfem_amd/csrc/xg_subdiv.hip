@@ -216,39 +216,6 @@ __device__ __forceinline__ void accum_tet(double *m, const double *p0, const dou
   Moments<3, PM>::accum(lam, rr[3] * tf, m);
 }
 
-constexpr double sd_inv_factorial(int n) { return n <= 1 ? 1.0 : sd_inv_factorial(n - 1) / n; }
-
-// exact moments of one tet from its vertices (p <= 2: Moments::hstep, the
-// complete homogeneous recursion over the 4 vertices' barycentrics) added
-// with the signed weight factor tf = +-6|T| (negative: a complemented
-// leaf's piece is subtracted, by negating the sums around the update); the
-// barycentrics are scaled by (|tf| / (2p + 3)!)^(1/2p) so the recursion's
-// top degree lands in m weighted, and the alpha! factors are applied once
-// per element (Moments::hfinish).  4 x 140 FMAs for a degree-4 tet against
-// 14 points x 73 operations with the base rule; the result is that rule's
-// point sum to rounding.
-template <int PM>
-__device__ __forceinline__ void htet(double *m, const double *p0, const double *p1, const double *p2,
-                                     const double *p3, double tf) {
-  using MM = Moments<3, PM>;
-  double h[MM::NH];
-#pragma unroll
-  for (int k = 0; k < MM::NH; ++k) h[k] = 0.0;
-  double c = sqrt(fabs(tf) * sd_inv_factorial(2 * PM + 3));
-  if constexpr (PM == 2) c = sqrt(c);
-  const double sg = tf < 0.0 ? -1.0 : 1.0;
-#pragma unroll
-  for (int k = 0; k < MM::NM; ++k) m[k] *= sg;
-  const double *P[4] = {p0, p1, p2, p3};
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const double l[4] = {c * P[v][0], c * P[v][1], c * P[v][2], c * (1.0 - P[v][0] - P[v][1] - P[v][2])};
-    MM::hstep(l, h, m);
-  }
-#pragma unroll
-  for (int k = 0; k < MM::NM; ++k) m[k] *= sg;
-}
-
 __device__ __forceinline__ double tet_tf(const double *p0, const double *p1, const double *p2, const double *p3,
                                          bool measure6) {
   double a[3], b[3], c[3];
@@ -935,42 +902,136 @@ __host__ __device__ inline size_t sdx_bytes(int L, int nq_vol, int nq_if, int NM
   return o;
 }
 
-// LDS of k_sdx_leaves alone: the arrays it uses (the walk's candidate and
-// lattice arrays left out), about 19 KB at p = 3, so 8 one-wave blocks fit
-// in a CU's 160 KB (2 waves on every SIMD; the whole SdxLds, 26 KB, allowed
-// 6)
-__host__ __device__ inline size_t sdx_leaf_bytes(int nq_vol, int nq_if, int NM, SdxLds *s, char *base) {
+// LDS of k_sdx_leaves: the vertices, sign and cut parameters of CAP cut leaves
+// (a chunk of the element's list) and the records of their pieces.  p = 3:
+// 19.4 KB, so that the 8 one-wave blocks that its registers allow (2 waves per
+// SIMD) fit in a CU's 160 KB; p <= 2: registers for 4 waves per SIMD and more,
+// so half the leaves.
+template <int PM>
+struct SdlCap {
+  static constexpr int CAP = PM == 3 ? 256 : 128;  // multiples of 64
+};
+// rows of the reduction scratch are 17 doubles (16 columns), so that lanes
+// reading consecutive rows hit distinct banks; it overlays the leaves
+constexpr int SDL_ROW = 17;
+struct SdlLds {
+  uint32_t *vert;      // CAP x 4: lattice vertices (level-5 units); top byte of the first: complemented
+  double *t;           // 4 x CAP: parameter of cut point c on its edge
+  double *scr;         // NG * 4 x SDL_ROW (over vert and t)
+  uint32_t *vol, *itf; // 3 CAP / 2 CAP piece records: leaf | corner codes << 8
+  uint32_t *tab;       // 16 x 6 words: the pieces of every sign pattern
+  double *red;         // 2 NM
+  double *cl;          // 20: the element's level-set nodal values
+  double *fi;          // 10: F^{-1} (row major) and |det F|
+};
+
+template <int PM>
+__host__ __device__ inline size_t sdl_bytes(SdlLds *s, char *base) {
+  constexpr int CAP = SdlCap<PM>::CAP, NM = Moments<3, PM>::NM, NG = (NM + 3) / 4;
   size_t o = 0;
   auto take = [&](size_t bytes) {
     const size_t at = o;
     o = sd_align(o + bytes);
     return at;
   };
+  const size_t leaf = (sizeof(uint32_t) * 4 + sizeof(double) * 4) * CAP, scr = sizeof(double) * NG * 4 * SDL_ROW;
+  const size_t a_leaf = take(leaf > scr ? leaf : scr);
+  const size_t a_vol = take(sizeof(uint32_t) * 3 * CAP);
+  const size_t a_itf = take(sizeof(uint32_t) * 2 * CAP);
+  const size_t a_tab = take(sizeof(uint32_t) * 16 * 6);
   const size_t a_red = take(sizeof(double) * 2 * NM);
-  const size_t a_rv = take(sizeof(double) * 4 * nq_vol);
-  const size_t a_ri = take(sizeof(double) * 4 * nq_if);
-  const size_t a_cp = take(sizeof(double) * 64 * 8 * 3);
-  const size_t a_vtf = take(sizeof(double) * 192);
-  const size_t a_ifw = take(sizeof(double) * 128);
-  const size_t a_vrec = take(sizeof(uint32_t) * 192);
-  const size_t a_irec = take(sizeof(uint32_t) * 128);
   const size_t a_cl = take(sizeof(double) * 20);
   const size_t a_fi = take(sizeof(double) * 10);
   if (s) {
-    *s = SdxLds{};
+    s->scr = (double *)(base + a_leaf);
+    s->t = (double *)(base + a_leaf);
+    s->vert = (uint32_t *)(base + a_leaf + sizeof(double) * 4 * CAP);
+    s->vol = (uint32_t *)(base + a_vol);
+    s->itf = (uint32_t *)(base + a_itf);
+    s->tab = (uint32_t *)(base + a_tab);
     s->red = (double *)(base + a_red);
-    s->rule_vol = (double(*)[4])(base + a_rv);
-    s->rule_if = (double(*)[4])(base + a_ri);
-    s->pool = (double(*)[8][3])(base + a_cp);
-    s->voltf = (double *)(base + a_vtf);
-    s->ifw = (double *)(base + a_ifw);
-    s->volrec = (uint32_t *)(base + a_vrec);
-    s->ifrec = (uint32_t *)(base + a_irec);
     s->cl = (double *)(base + a_cl);
     s->fi = (double *)(base + a_fi);
   }
   return o;
 }
+
+// The pieces of a cut leaf by its sign pattern (bit j: vertex j is POS, zero
+// included, xintegration.cpp:1159-1164): CutSimplex<3>::MakeQuad's split
+// (xintegration.cpp:1084-1388) as leaf_pieces gives it for the kept side, the
+// corner of a piece as lv | rv << 2 | c << 4: vertex lv (lv == rv) or cut point
+// c on the edge lv < rv.  meta: volume tets | triangles << 2 | complemented << 4
+// | cuts << 5 | edges (lv | rv << 2) << 8, 12, 16, 20; 0 where the reference
+// throws.
+struct LeafTab {
+  uint32_t w[2][16][6];  // [side][pattern]: vol[3], itf[2], meta
+  static constexpr int kth(int m, int k) {
+    for (int j = 0; j < 4; ++j)
+      if ((m >> j) & 1) {
+        if (k == 0) return j;
+        --k;
+      }
+    return 0;
+  }
+  constexpr LeafTab() : w{} {
+    constexpr int edge[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
+    for (int side = 0; side < 2; ++side)
+      for (int posm = 1; posm < 15; ++posm) {
+        const int negm = 15 & ~posm;
+        int npos = 0;
+        for (int j = 0; j < 4; ++j) npos += (posm >> j) & 1;
+        int ce[4] = {}, c1[4] = {15, 15, 15, 15}, c2[4] = {15, 15, 15, 15}, nc = 0;
+        uint32_t edges = 0;
+        for (int e = 0; e < 6; ++e) {
+          const int l = edge[e][0], r = edge[e][1];
+          if (((posm >> l) & 1) == ((posm >> r) & 1)) continue;
+          ce[nc] = l | (r << 2);
+          edges |= (uint32_t)ce[nc] << (4 * nc);
+          (c1[l] == 15 ? c1[l] : c2[l]) = nc;
+          (c1[r] == 15 ? c1[r] : c2[r]) = nc;
+          ++nc;
+        }
+        auto vx = [&](int j) { return (uint32_t)(j | (j << 2)); };
+        auto cp = [&](int c) { return (uint32_t)(ce[c] | (c << 4)); };
+        auto pk = [&](uint32_t a, uint32_t b, uint32_t c, uint32_t d) { return a | (b << 6) | (c << 12) | (d << 18); };
+        uint32_t *o = w[side][posm];
+        if (npos != 2) {
+          // the one-vertex corner tet is the minor side, the major side is
+          // the leaf minus the corner
+          const bool minor_pos = npos == 1;
+          const int mn = kth(minor_pos ? posm : negm, 0);
+          const bool comp = side == POS ? !minor_pos : minor_pos;
+          o[0] = pk(vx(mn), cp(0), cp(1), cp(2));
+          o[3] = pk(cp(0), cp(1), cp(2), 0);
+          o[5] = 1u | (1u << 2) | (comp ? 16u : 0u) | (3u << 5) | (edges << 8);
+          continue;
+        }
+        const int ownm = side == POS ? posm : negm, othm = side == POS ? negm : posm;
+        const int o0 = kth(ownm, 0), o1 = kth(ownm, 1), t0 = kth(othm, 0);
+        const int q1 = c1[o0], q2 = c2[o0];
+        int q3 = -1;
+        for (int l = 0; l < 4; ++l)
+          if (q1 != l && q2 != l) q3 = l;
+        int q4 = 6 - q3 - q2 - q1;
+        if ((c1[t0] == q1 && c2[t0] == q4) || (c1[t0] == q2 && c2[t0] == q3)) {
+          const int tt = q3;
+          q3 = q4;
+          q4 = tt;
+        }
+        o[0] = pk(vx(o0), cp(q1), cp(q2), vx(o1));
+        o[1] = pk(cp(q1), cp(q2), vx(o1), cp(q3));
+        o[2] = pk(cp(q2), vx(o1), cp(q3), cp(q4));
+        const int n0 = kth(negm, 0), n1 = kth(negm, 1), p0 = kth(posm, 0), p1 = kth(posm, 1);
+        const bool f1 = c1[n0] == c1[p0] || c2[n0] == c1[p0], f2 = c1[n1] == c1[p1] || c2[n1] == c1[p1];
+        const int d1 = f1 ? c1[p0] : c2[p0], e1 = f1 ? c2[p0] : c1[p0];
+        const int d2 = f2 ? c1[p1] : c2[p1], e2 = f2 ? c2[p1] : c1[p1];
+        o[3] = pk(cp(d1), cp(e1), cp(d2), 0);
+        o[4] = pk(cp(d2), cp(e2), cp(d1), 0);
+        o[5] = 3u | (2u << 2) | (4u << 5) | (edges << 8);
+      }
+  }
+};
+static __device__ const LeafTab xg_leaf_tab_d{};
 
 // The pieces of a cut leaf for the kept volume side SIDE (CutSimplex<3>::
 // MakeQuad, xintegration.cpp:1084-1388), as index lists into
@@ -1110,8 +1171,7 @@ __device__ __forceinline__ bool lat_bit(const uint32_t *bits, int idx) { return 
 // hit distinct banks).  Cheaper than 6 shuffle steps per entry.  Every lane
 // of the wave calls it; it ends with dst written and visible to the wave.
 template <int NM>
-__device__ __forceinline__ void wave_sum_lds(const double *m, double *scr, double *dst, int lane,
-                                             double *dst_hi = nullptr, int split = 64) {
+__device__ __forceinline__ void wave_sum_lds(const double *m, double *scr, double *dst, int lane) {
   constexpr int RB = 23;
 #pragma unroll
   for (int k0 = 0; k0 < NM; k0 += RB) {
@@ -1120,55 +1180,57 @@ __device__ __forceinline__ void wave_sum_lds(const double *m, double *scr, doubl
       if (k0 + kk < NM) scr[kk * 65 + lane] = m[k0 + kk < NM ? k0 + kk : 0];
     wave_sync();
     if (lane < RB && k0 + lane < NM) {
-      if (!dst_hi) {
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-        for (int j = 0; j < 64; j += 4) {
-          s0 += scr[lane * 65 + j];
-          s1 += scr[lane * 65 + j + 1];
-          s2 += scr[lane * 65 + j + 2];
-          s3 += scr[lane * 65 + j + 3];
-        }
-        dst[k0 + lane] = (s0 + s1) + (s2 + s3);
-      } else {
-        // two sums: lanes below `split` into dst, the others into dst_hi
-        double s0 = 0.0, s1 = 0.0, h0 = 0.0, h1 = 0.0;
-        for (int j = 0; j < 64; j += 2) {
-          const double v0 = scr[lane * 65 + j], v1 = scr[lane * 65 + j + 1];
-          if (j < split) s0 += v0; else h0 += v0;
-          if (j + 1 < split) s1 += v1; else h1 += v1;
-        }
-        dst[k0 + lane] = s0 + s1;
-        dst_hi[k0 + lane] = h0 + h1;
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+      for (int j = 0; j < 64; j += 4) {
+        s0 += scr[lane * 65 + j];
+        s1 += scr[lane * 65 + j + 1];
+        s2 += scr[lane * 65 + j + 2];
+        s3 += scr[lane * 65 + j + 3];
       }
+      dst[k0 + lane] = (s0 + s1) + (s2 + s3);
     }
     wave_sync();
   }
 }
 
-// centred affine degree-6 sums (Moments<3,3>::accum_aff of y = lam - 1/4,
-// NS sets of 84 in red) -> homogeneous moments in place: lane computes the
-// columns lane and lane + 64 of the dense FP32-exact map xg_aff33
-template <int NS>
-__device__ __forceinline__ void aff33_to_hom(double *red, int lane) {
-  constexpr int NM = Moments<3, 3>::NM;
+template <int PM>
+__device__ __forceinline__ float2 aff_entry(int r, int lane) {
+  if constexpr (PM == 1) return *reinterpret_cast<const float2 *>(&xg_aff31[r][lane][0]);
+  else if constexpr (PM == 2) return *reinterpret_cast<const float2 *>(&xg_aff32[r][lane][0]);
+  else return *reinterpret_cast<const float2 *>(&xg_aff33[r][lane][0]);
+}
+// beta! / (|beta| + 3)! or (wh = 1) / (|beta| + 2)! of a slot
+template <int PM>
+__device__ __forceinline__ double aser_scale(int slot, int wh) {
+  if constexpr (PM == 1) return xg_aser31[slot][wh];
+  else if constexpr (PM == 2) return xg_aser32[slot][wh];
+  else return xg_aser33[slot][wh];
+}
+
+// centred affine degree-2p sums (of y = lam - 1/4, NS sets of NM in red) ->
+// homogeneous moments in place: lane computes the columns lane and lane + 64
+// of the dense FP32-exact map xg_aff3p
+template <int PM, int NS>
+__device__ __forceinline__ void aff_to_hom(double *red, int lane) {
+  constexpr int NM = Moments<3, PM>::NM;
   double lo[NS], hi[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) lo[s] = hi[s] = 0.0;
 #pragma unroll 4
   for (int r = 0; r < NM; ++r) {
-    const float2 c = *reinterpret_cast<const float2 *>(&xg_aff33[r][lane][0]);
+    const float2 c = aff_entry<PM>(r, lane);
     const double c0 = c.x, c1 = c.y;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const double n = red[s * NM + r];
       lo[s] = fma(c0, n, lo[s]);
-      hi[s] = fma(c1, n, hi[s]);
+      if constexpr (NM > 64) hi[s] = fma(c1, n, hi[s]);
     }
   }
   wave_sync();
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    red[s * NM + lane] = lo[s];
+    if (lane < NM) red[s * NM + lane] = lo[s];
     if (lane + 64 < NM) red[s * NM + lane + 64] = hi[s];
   }
   wave_sync();
@@ -1651,10 +1713,10 @@ int subdiv_exact_pass(xg_ctx *ctx, int nel, const int32_t *elems, const double *
 //   1. k_sdx_tree: the walk (lattice sign checks, classification) at high
 //      occupancy; writes the cut leaves from the front of the element's list
 //      and the uncut nodes of the kept side (table rows) from the back
-//   2. k_sdx_leaves: the cut leaves' pieces and their base-rule points
-//      (the register-heavy part), once per requested part (volume side or
-//      interface) on the same lists; appends the complemented leaves after
-//      the cut leaves
+//   2. k_sdx_leaves: the cut leaves' pieces and their moments (the
+//      register-heavy part), the volume side and the interface in one launch
+//      where both are asked for; appends the complemented leaves after the
+//      cut leaves
 //   3. k_sdx_rows: the table rows (uncut nodes + complemented leaves),
 //      added to the moments
 // An element whose lists do not fit (2 cut leaves + rows > cap) is queued
@@ -2028,9 +2090,27 @@ __global__ __launch_bounds__(64) void k_sdx_tree(int nel, const int32_t *__restr
   }
 }
 
-// the cut leaves of each listed element: pieces and base-rule points (as in
-// k_subdiv_exact), moments written (not added); the complemented leaves of a
-// volume pass are appended after the cut leaves (cnt.z)
+// The cut leaves of each listed element, their pieces' moments added (volume,
+// to the walk's row sums) or written (interface); the complemented leaves of a
+// volume pass are appended after the cut leaves (cnt.z).
+//
+// Bound: FP64 issue at two waves per SIMD (p = 3).  A piece is one lane's: its
+// moments come from its vertices through the truncated series of
+// Moments::aser_step, 3 FMAs per monomial of degree < 2p and vertex (p = 3:
+// 4 x 168 for a tetrahedron, 3 x 168 for a triangle, against 24 and 12 points of
+// about 160 operations).  The 84 coefficients of a piece and 84 sums would
+// need 336 registers; so the sums are not a lane's: v_mfma_f64_4x4x4 with a
+// selection matrix (row r of ones) adds the coefficient 4 g + r of the lanes x,
+// x + 16, x + 32, x + 48 into accumulator row r of column x, 16 sums of every
+// coefficient in (NM + 3) / 4 registers (19 cycles each for 64 lanes, measured;
+// the probe's A index is lane % 4, its K index lane / 16).  Both parts in one
+// launch: the lanes of columns x < nc take volume pieces, the others triangles
+// (a tet with a zero fourth step).
+// A chunk of leaves is prepared first (lane = leaf: vertex values, sign pattern,
+// cut parameters; the pieces by pattern from a table), then its pieces run;
+// so the piece phase holds no sums and a piece reads its four corners only.
+// 128^3 cells, 405,341 elements, p = 3, L = 4, NEG + IF: the whole step 51.6 ->
+// 27.0 ms; 20^3, p = 2, L = 3: 400 -> 245 us.
 template <int LO, int PM, int SIDE, int WHICH>
 __global__ __launch_bounds__(64, 2) void k_sdx_leaves(int nel, const int32_t *__restrict__ elems,
                                                      const double *__restrict__ lset_nodal,
@@ -2043,43 +2123,20 @@ __global__ __launch_bounds__(64, 2) void k_sdx_leaves(int nel, const int32_t *__
                                                      double *__restrict__ out_if, int out_stride,
                                                      int32_t *__restrict__ stats, int stats_stride, int32_t *err,
                                                      int32_t *__restrict__ queue, int32_t *__restrict__ stats_if) {
+  using MM = Moments<3, PM>;
   constexpr int NL = ndof(3, LO);
-  constexpr int NM = Moments<3, PM>::NM;
-  // WHICH == 3 (both parts in one launch, p = 3): lanes [0, nn) integrate the
-  // volume pieces and lanes [nn, 64) the interface pieces, each lane into
-  // one set of 84 sums, with one task loop (blocks of 4 points, a triangle
-  // being a tet whose fourth rule coordinate is 0); nn follows the element's
-  // expected point split
-  static_assert(WHICH != 3 || PM == 3, "both parts in one launch: p = 3");
-  // p = 3: the task loops accumulate centred affine moments (accum_aff of
-  // y = lam - 1/4, 135 instead of 153 operations per point); the pool holds
-  // the leaf points shifted by -1/4 (weights and normals use differences)
-  // and the wave's sums are mapped to the homogeneous moments at the end
-  constexpr bool AFF = PM == 3;
-  constexpr double SHIFT = AFF ? 0.25 : 0.0;
-  constexpr int SDX_VB = PM == 1 ? 4 : (PM == 2 ? 7 : 8), SDX_NVB = PM == 1 ? 1 : (PM == 2 ? 2 : 3);
-  constexpr int SDX_IB = PM == 1 ? 3 : (PM == 2 ? 6 : 4), SDX_NIB = PM == 1 ? 1 : (PM == 2 ? 1 : 3);
+  constexpr int NM = MM::NM, NG = (NM + 3) / 4;
+  constexpr int CAP = SdlCap<PM>::CAP;
   extern __shared__ char smem[];
-  SdxLds S;
-  const int vol_nq = xg_minrule_cnt_d[3][PM];
-  const int if_nq = xg_minrule_cnt_d[2][PM];
-  sdx_leaf_bytes(vol_nq, if_nq, NM, &S, smem);
-  // leaf points lane-minor: (point j, coordinate d, leaf lane l)
-  double *pool = &S.pool[0][0][0];
+  SdlLds S;
+  sdl_bytes<PM>(&S, smem);
   const int lane = threadIdx.x & 63;
-  const int n = 1 << L;
-  const int shift = SDX_DMAX - L;
-  {
-    const double(*src_v)[4] = &xg_minrule_data_d[xg_minrule_off_d[3][PM]];
-    const double(*src_i)[4] = &xg_minrule_data_d[xg_minrule_off_d[2][PM]];
-    for (int k = lane; k < 4 * (vol_nq + if_nq); k += 64) {
-      const int q = k >> 2, c = k & 3;
-      if (q < vol_nq) S.rule_vol[q][c] = src_v[q][c];
-      else S.rule_if[q - vol_nq][c] = src_i[q - vol_nq][c];
-    }
-    wave_sync();
-  }
-  const double inv_n = 1.0 / n;
+  const int col = lane & 15, row = lane >> 4;
+  for (int k = lane; k < 16 * 6; k += 64) S.tab[k] = (&xg_leaf_tab_d.w[SIDE == POS ? 1 : 0][0][0])[k];
+  double sel[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) sel[r] = (lane & 3) == r ? 1.0 : 0.0;
+  constexpr double inv = 1.0 / (1 << SDX_DMAX);
   // elements from the work counter (persistent waves, the heavy elements do
   // not wait behind a fixed stride) or strided by the grid
   for (int i = queue ? next_item(queue, lane) : blockIdx.x; i < nel;
@@ -2103,278 +2160,205 @@ __global__ __launch_bounds__(64, 2) void k_sdx_leaves(int nel, const int32_t *__
           jacobian<3>(V, F, Fi, ad);
 #pragma unroll
           for (int k = 0; k < 9; ++k) S.fi[k] = Fi[k];
-          S.fi[9] = ad;
         }
       } else if (finv_all) {
         have_geo = true;
-        if (lane == 0) {
-          double Fi[9];
-#pragma unroll
-          for (int k = 0; k < 9; ++k) Fi[k] = finv_all[(size_t)i * 9 + k];
-          const double dinv = Fi[0] * (Fi[4] * Fi[8] - Fi[5] * Fi[7]) - Fi[1] * (Fi[3] * Fi[8] - Fi[5] * Fi[6]) +
-                              Fi[2] * (Fi[3] * Fi[7] - Fi[4] * Fi[6]);
-#pragma unroll
-          for (int k = 0; k < 9; ++k) S.fi[k] = Fi[k];
-          S.fi[9] = 1.0 / fabs(dinv);
-        }
+        if (lane < 9) S.fi[lane] = finv_all[(size_t)i * 9 + lane];
+      } else if (lane < 9) {
+        S.fi[lane] = lane % 4 == 0 ? 1.0 : 0.0;
       }
     }
     wave_sync();
     const double *cl = S.cl;
-    double mvol[(WHICH & 1) ? NM : 1], mif[(WHICH == 2) ? NM : 1];
+    double D[NG];
 #pragma unroll
-    for (int k = 0; k < ((WHICH & 1) ? NM : 1); ++k) mvol[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < ((WHICH == 2) ? NM : 1); ++k) mif[k] = 0.0;
+    for (int g = 0; g < NG; ++g) D[g] = 0.0;
     const int nleaf = c4.x;
-    int nn = 64;  // lanes of the volume role (WHICH == 3)
+    // columns of the volume role: the split with the fewest rounds (a 1-3 cut
+    // leaf has 1 tet and 1 triangle, a 2-2 one 3 and 2; c4.y: the walk's count
+    // of 2-2 leaves)
+    int nc = WHICH == 1 ? 16 : 0;
     if constexpr (WHICH == 3) {
-      // points: 24 per volume tet, 12 per triangle; a 1-3 cut leaf has 1
-      // tet and 1 triangle, a 2-2 cut leaf 3 tets and 2 triangles (c4.y:
-      // the walk's count of 2-2 leaves)
-      const int n22 = c4.y, n13 = nleaf - n22;
-      const double vp = 24.0 * (n13 + 3 * n22), ip = 12.0 * (n13 + 2 * n22);
-      nn = (vp + ip > 0.0) ? (int)(64.0 * vp / (vp + ip) + 0.5) : 44;
-      nn = nn < 16 ? 16 : (nn > 56 ? 56 : nn);
+      const int nv = nleaf + 2 * c4.y, ni = nleaf + c4.y;
+      int best = 1 << 30;
+      for (int c = 6; c <= 11; ++c) {
+        const int r = max((nv + 4 * c - 1) / (4 * c), (ni + 63 - 4 * c) / (64 - 4 * c));
+        if (r < best) {
+          best = r;
+          nc = c;
+        }
+      }
     }
+    const bool isv = col < nc;
+    const int wr = isv ? 4 * nc : 64 - 4 * nc, rank = isv ? row * nc + col : row * (16 - nc) + col - nc;
     uint16_t *lst = lists + (size_t)i * cap;
     int ncomp = 0, st_vol = 0, st_if = 0;
     bool ok = true;
-    for (int l0 = 0; l0 < nleaf; l0 += 64) {
-      const int l = l0 + lane;
-      LeafPieces2 PC;
-      PC.nvol = 0;
-      PC.nif = 0;
-      PC.comp = false;
-      int id = 0;
-      if (l < nleaf) {
-        id = lst[l];
-        int W[4][3];
-        unpack_uint4(nverts[id], shift, W);
-        double V[4][3], vv[4], cpt[4][3];
+    const int nchunk = (nleaf + CAP - 1) / CAP;
+    const int chunk = nchunk > 0 ? ((nleaf + nchunk - 1) / nchunk + 63) & ~63 : 64;
+    for (int k0 = 0; k0 < nleaf; k0 += chunk) {
+      const int kend = min(nleaf, k0 + chunk);
+      int tot_vol = 0, tot_if = 0;
+      for (int l0 = k0; l0 < kend; l0 += 64) {
+        const int l = l0 + lane, s = l - k0;
+        uint32_t meta = 0u, tb = 0u;
+        int id = 0;
+        if (l < kend) {
+          id = lst[l];
+          uint4 pv = nverts[id];
+          const uint32_t pk[4] = {pv.x, pv.y, pv.z, pv.w};
+          double vv[4];
+          int posm = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-          for (int d = 0; d < 3; ++d) V[j][d] = W[j][d] * inv_n;
-          vv[j] = lagrange_eval3<LO>(cl, V[j]);
-        }
-        if (!leaf_pieces<SIDE>(V, vv, cpt, PC)) {
-          ok = false;
-          PC.nvol = 0;
-          PC.nif = 0;
-          PC.comp = false;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            pool[(j * 3 + d) * 64 + lane] = V[j][d] - SHIFT;
-            pool[((4 + j) * 3 + d) * 64 + lane] = cpt[j][d] - SHIFT;
+          for (int j = 0; j < 4; ++j) {
+            int w[3];
+            unpack3(pk[j], w);
+            const double x[3] = {w[0] * inv, w[1] * inv, w[2] * inv};
+            vv[j] = lagrange_eval3<LO>(cl, x);
+            posm |= (vv[j] < 0.0 ? 0 : 1) << j;
           }
-      }
-      if (!(WHICH & 1)) {
-        PC.nvol = 0;
-        PC.comp = false;
-      }
-      if (!(WHICH & 2)) PC.nif = 0;
-      {
-        int cc;
-        const int sc = wave_slot(PC.comp, ncomp, lane, cc);
-        if (PC.comp) lst[nleaf + sc] = (uint16_t)id;
-        ncomp += cc;
-      }
-      int tot_vol, tot_if;
-      const int bvol = wave_excl_scan(PC.nvol, lane, tot_vol);
-      const int bif = wave_excl_scan(PC.nif, lane, tot_if);
+          tb = posm * 6;
+          meta = S.tab[tb + 5];
+          ok = ok && meta != 0u;
+          if (meta & 16u) pv.x |= 0x80000000u;
+          *reinterpret_cast<uint4 *>(&S.vert[4 * s]) = pv;
+          const int ncut = (int)((meta >> 5) & 7u);
 #pragma unroll
-      for (int q = 0; q < 3; ++q)
-        if (q < PC.nvol) S.volrec[bvol + q] = (uint32_t)lane | (PC.vol[q] << 8) | (PC.comp ? 0x80u : 0u);
+          for (int c = 0; c < 4; ++c) {
+            double t = 0.0;
+            if (c < ncut) {
+              const int lv = (int)((meta >> (8 + 4 * c)) & 3u), rv = (int)((meta >> (10 + 4 * c)) & 3u);
+              const double vl = lv == 0 ? vv[0] : (lv == 1 ? vv[1] : vv[2]);
+              const double vr = rv == 1 ? vv[1] : (rv == 2 ? vv[2] : vv[3]);
+              // a cut between two nonzero values whose product underflows is
+              // none to the reference, which then throws
+              ok = ok && (vl * vr < 0.0 || !(vl != 0.0) || !(vr != 0.0) || vl != vl || vr != vr);
+              t = vl / (vl - vr);
+            }
+            S.t[c * CAP + s] = t;
+          }
+        }
+        const int nv = (WHICH & 1) ? (int)(meta & 3u) : 0, ni = (WHICH & 2) ? (int)((meta >> 2) & 3u) : 0;
+        if (WHICH & 1) {
+          const bool comp = (meta & 16u) != 0u;
+          int cc;
+          const int sc = wave_slot(comp, ncomp, lane, cc);
+          if (comp) lst[nleaf + sc] = (uint16_t)id;
+          ncomp += cc;
+          // (1 or 3 tets, 1 or 2 triangles: prefix sums by ballots)
+          const unsigned long long b1 = __ballot(nv >= 1), b3 = __ballot(nv == 3), lt = (1ull << lane) - 1ull;
+          const int base = tot_vol + __popcll(b1 & lt) + 2 * __popcll(b3 & lt);
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
-        if (q < PC.nif) S.ifrec[bif + q] = (uint32_t)lane | (PC.itf[q] << 8);
+          for (int q = 0; q < 3; ++q)
+            if (q < nv) S.vol[base + q] = (uint32_t)s | (S.tab[tb + q] << 8);
+          tot_vol += __popcll(b1) + 2 * __popcll(b3);
+        }
+        if (WHICH & 2) {
+          const unsigned long long b1 = __ballot(ni >= 1), b2 = __ballot(ni == 2), lt = (1ull << lane) - 1ull;
+          const int base = tot_if + __popcll(b1 & lt) + __popcll(b2 & lt);
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            if (q < ni) S.itf[base + q] = (uint32_t)s | (S.tab[tb + 3 + q] << 8);
+          tot_if += __popcll(b1) + __popcll(b2);
+        }
+      }
       st_vol += tot_vol;
       st_if += tot_if;
       wave_sync();
-      // weight factors (as in k_subdiv_exact)
-      for (int q = lane; q < tot_vol; q += 64) {
-        const uint32_t rec = S.volrec[q];
-        const int ll = rec & 63;
-        double P4[4][3];
+      const int mine = isv ? tot_vol : tot_if;
+      int rounds = 0;
+      if (WHICH & 1) rounds = (tot_vol + 4 * nc - 1) / (4 * nc);
+      if (WHICH & 2) rounds = max(rounds, (tot_if + 63 - 4 * nc) / (64 - 4 * nc));
+      for (int rd = 0; rd < rounds; ++rd) {
+        const int q = rd * wr + rank;
+        double y[4][3], wgt = 0.0;
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          const int j = (rec >> (8 + 3 * m)) & 7;
+        for (int m = 0; m < 4; ++m)
 #pragma unroll
-          for (int d = 0; d < 3; ++d) P4[m][d] = pool[(j * 3 + d) * 64 + ll];
-        }
-        const double tf = tet_tf(P4[0], P4[1], P4[2], P4[3], true);
-        S.voltf[q] = (rec & 0x80u) ? -tf : tf;
-      }
-      for (int q = lane; q < tot_if; q += 64) {
-        const uint32_t rec = S.ifrec[q];
-        const int ll = rec & 63;
-        double s0[3], s1[3], s2[3], pp[3];
+          for (int d = 0; d < 3; ++d) y[m][d] = 0.0;
+        if (q < mine) {
+          const uint32_t rec = isv ? S.vol[q] : S.itf[q];
+          const int s = rec & 255u;
+          const uint32_t *vx = &S.vert[4 * s];
+          const bool comp = (vx[0] >> 31) != 0u;
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          s0[d] = pool[(((rec >> 8) & 7) * 3 + d) * 64 + ll];
-          s1[d] = pool[(((rec >> 11) & 7) * 3 + d) * 64 + ll];
-          s2[d] = pool[(((rec >> 14) & 7) * 3 + d) * 64 + ll];
-          pp[d] = pool[(((rec >> 17) & 7) * 3 + d) * 64 + ll];
-        }
-        double a[3], b[3], cc[3];
+          for (int m = 0; m < (WHICH == 2 ? 3 : 4); ++m) {
+            if (m == 3 && !isv) break;
+            const int code = (int)(rec >> (8 + 6 * m));
+            const uint32_t pl = vx[code & 3], pr = vx[(code >> 2) & 3];
+            const double t = S.t[((code >> 4) & 3) * CAP + s];
+            int a[3], b[3];
+            unpack3(pl, a);
+            unpack3(pr, b);
+            // (a lattice vertex has lv == rv: its coordinates, exactly)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          a[d] = s1[d] - s0[d];
-          b[d] = s2[d] - s0[d];
-        }
-        cc[0] = a[1] * b[2] - a[2] * b[1];
-        cc[1] = a[2] * b[0] - a[0] * b[2];
-        cc[2] = a[0] * b[1] - a[1] * b[0];
-        const double tf = norm3(cc);
-        const double na = norm3(a), nb = norm3(b);
-        const double rel = na > nb ? na : nb;
-        double wf = 0.0;
-        if (!(tf < 1e-14 * rel)) {
+            for (int d = 0; d < 3; ++d) y[m][d] = fma(t, (double)(b[d] - a[d]) * inv, (double)a[d] * inv - 0.25);
+          }
+          double a[3], b[3], cr[3];
 #pragma unroll
-          for (int d = 0; d < 3; ++d) cc[d] /= tf;
-          const double dd0 = pp[0] - s0[0], dd1 = pp[1] - s0[1], dd2 = pp[2] - s0[2];
-          if (dd0 * cc[0] + dd1 * cc[1] + dd2 * cc[2] >= 0)
+          for (int d = 0; d < 3; ++d) {
+            a[d] = y[1][d] - y[0][d];
+            b[d] = y[2][d] - y[0][d];
+          }
+          cr[0] = a[1] * b[2] - a[2] * b[1];
+          cr[1] = a[2] * b[0] - a[0] * b[2];
+          cr[2] = a[0] * b[1] - a[1] * b[0];
+          if (isv) {
+            double tf = 0.0;
 #pragma unroll
-            for (int d = 0; d < 3; ++d) cc[d] *= -1.0;
-          Geo geo;
-          geo.Finv = have_geo ? S.fi : nullptr;
-          geo.absdet = have_geo ? S.fi[9] : 1.0;
-          wf = tf * geo.if_factor(cc);
-        }
-        S.ifw[q] = wf;
-      }
-      wave_sync();
-      if constexpr (WHICH == 3) {
-        // one task loop for both roles: (piece, block of 4 points) tasks
-        const int ni = 64 - nn;
-        const int nvt = tot_vol * 6, nit = tot_if * 3;
-        const int rounds = max((nvt + nn - 1) / nn, (nit + ni - 1) / ni);
-        const bool isv = lane < nn;
-        const int rl = isv ? lane : lane - nn, rs = isv ? nn : ni;
-        for (int rd = 0; rd < rounds; ++rd) {
-          const int q = rd * rs + rl;
-          if (isv ? (q < nvt) : (q < nit)) {
-            const int pc = isv ? q / 6 : q / 3;
-            const int t0 = 4 * (isv ? q - pc * 6 : q - pc * 3);
-            const uint32_t rec = isv ? S.volrec[pc] : S.ifrec[pc];
-            const double wf = isv ? S.voltf[pc] : S.ifw[pc];
-            const double(*rule)[4] = isv ? S.rule_vol : S.rule_if;
-            const int ll = rec & 63;
-            double p0[3], p1[3], p2[3], p3[3];
+            for (int d = 0; d < 3; ++d) tf += cr[d] * (y[3][d] - y[0][d]);
+            tf = fabs(tf);
+            wgt = comp ? -tf : tf;
+          } else {
+            // |absdet F^{-T} n| / absdet times the triangle's measure; a
+            // degenerate one has no normal and no weight
+            const double tf = norm3(cr), na = norm3(a), nb = norm3(b);
+            if (!(tf < 1e-14 * (na > nb ? na : nb))) {
+              wgt = tf;
+              if (have_geo) {
+                double v[3];
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-              p0[d] = pool[(((rec >> 8) & 7) * 3 + d) * 64 + ll];
-              p1[d] = pool[(((rec >> 11) & 7) * 3 + d) * 64 + ll];
-              p2[d] = pool[(((rec >> 14) & 7) * 3 + d) * 64 + ll];
-              p3[d] = pool[(((rec >> 17) & 7) * 3 + d) * 64 + ll];
-            }
-            for (int t = t0; t < t0 + 4; ++t) {
-              const double r0 = rule[t][0], r1 = rule[t][1], r2 = rule[t][2], rw = rule[t][3];
-              const double ow = 1.0 - r0 - r1 - r2;
-              double y[3];
-#pragma unroll
-              for (int d = 0; d < 3; ++d) y[d] = ow * p0[d] + r0 * p1[d] + r1 * p2[d] + r2 * p3[d];
-              Moments<3, PM>::accum_aff(y, rw * wf, mvol);
+                for (int r = 0; r < 3; ++r) v[r] = S.fi[r] * cr[0] + S.fi[3 + r] * cr[1] + S.fi[6 + r] * cr[2];
+                wgt = norm3(v);
+              }
             }
           }
         }
-      }
-      if constexpr (WHICH == 1 && PM <= 2) {
-        // p <= 2: one task per piece, its moments from its vertices
-        for (int q = lane; q < tot_vol; q += 64) {
-          const uint32_t rec = S.volrec[q];
-          const int ll = rec & 63;
-          double p0[3], p1[3], p2[3], p3[3];
+        double h[NG * 4];
+        MM::aser_first(y[0], wgt, h);
+        MM::aser_step(y[1], h);
+        MM::aser_step(y[2], h);
+        if (WHICH & 1) MM::aser_step(y[3], h);
 #pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            p0[d] = pool[(((rec >> 8) & 7) * 3 + d) * 64 + ll];
-            p1[d] = pool[(((rec >> 11) & 7) * 3 + d) * 64 + ll];
-            p2[d] = pool[(((rec >> 14) & 7) * 3 + d) * 64 + ll];
-            p3[d] = pool[(((rec >> 17) & 7) * 3 + d) * 64 + ll];
-          }
-          htet<PM>(mvol, p0, p1, p2, p3, S.voltf[q]);
-        }
-      } else if (WHICH == 1) {
-        for (int q = lane; q < tot_vol * SDX_NVB; q += 64) {
-          const int pc = q / SDX_NVB, t0 = (q - pc * SDX_NVB) * SDX_VB;
-          const uint32_t rec = S.volrec[pc];
-          const int ll = rec & 63;
-          double p0[3], p1[3], p2[3], p3[3];
+        for (int k = NM; k < NG * 4; ++k) h[k] = 0.0;
 #pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            p0[d] = pool[(((rec >> 8) & 7) * 3 + d) * 64 + ll];
-            p1[d] = pool[(((rec >> 11) & 7) * 3 + d) * 64 + ll];
-            p2[d] = pool[(((rec >> 14) & 7) * 3 + d) * 64 + ll];
-            p3[d] = pool[(((rec >> 17) & 7) * 3 + d) * 64 + ll];
-          }
-          const double tf = S.voltf[pc];
-          // the next point's rule entry is read while this one accumulates
-          double nr[4];
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) nr[c] = S.rule_vol[t0][c];
-          for (int t = t0; t < t0 + SDX_VB; ++t) {
-            const double r0 = nr[0], r1 = nr[1], r2 = nr[2], rw = nr[3];
-            const int tn = t + 1 < t0 + SDX_VB ? t + 1 : t;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) nr[c] = S.rule_vol[tn][c];
-            const double ow = 1.0 - r0 - r1 - r2;
-            double y[3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) y[d] = ow * p0[d] + r0 * p1[d] + r1 * p2[d] + r2 * p3[d];
-            Moments<3, PM>::accum_aff(y, rw * tf, mvol);
-          }
-        }
-      }
-      if constexpr (WHICH == 2) {
-        for (int q = lane; q < tot_if * SDX_NIB; q += 64) {
-          const int pc = q / SDX_NIB, t0 = (q - pc * SDX_NIB) * SDX_IB;
-          const uint32_t rec = S.ifrec[pc];
-          const int ll = rec & 63;
-          double s0[3], s1[3], s2[3];
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            s0[d] = pool[(((rec >> 8) & 7) * 3 + d) * 64 + ll];
-            s1[d] = pool[(((rec >> 11) & 7) * 3 + d) * 64 + ll];
-            s2[d] = pool[(((rec >> 14) & 7) * 3 + d) * 64 + ll];
-          }
-          const double wf = S.ifw[pc];
-          double nr[3] = {S.rule_if[t0][0], S.rule_if[t0][1], S.rule_if[t0][3]};
-          for (int t = t0; t < t0 + SDX_IB; ++t) {
-            const double r0 = nr[0], r1 = nr[1], rw = nr[2];
-            const int tn = t + 1 < t0 + SDX_IB ? t + 1 : t;
-            nr[0] = S.rule_if[tn][0];
-            nr[1] = S.rule_if[tn][1];
-            nr[2] = S.rule_if[tn][3];
-            const double ow = 1.0 - r0 - r1;
-            double lam[4];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) lam[d] = ow * s0[d] + r0 * s1[d] + r1 * s2[d];
-            if constexpr (AFF) {
-              Moments<3, PM>::accum_aff(lam, rw * wf, mif);
-            } else {
-              lam[3] = 1.0 - lam[0] - lam[1] - lam[2];
-              Moments<3, PM>::accum(lam, rw * wf, mif);
-            }
-          }
-        }
+          for (int g = 0; g < NG; ++g)
+            D[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(sel[r], h[4 * g + r], D[g], 0, 0, 0);
       }
       wave_sync();
     }
-    // wave reduction of the per-lane moments through LDS (the point pool is
-    // free now)
-    if constexpr (WHICH == 1 && PM <= 2) Moments<3, PM>::hfinish(mvol);
-    if constexpr (WHICH == 3) wave_sum_lds<NM>(mvol, pool, S.red, lane, S.red + NM, nn);
-    else if constexpr (WHICH == 1) wave_sum_lds<NM>(mvol, pool, S.red, lane);
-    else wave_sum_lds<NM>(mif, pool, S.red + NM, lane);
-    if constexpr (AFF) {
-      if constexpr (WHICH == 3) aff33_to_hom<2>(S.red, lane);
-      else if constexpr (WHICH == 1) aff33_to_hom<1>(S.red, lane);
-      else aff33_to_hom<1>(S.red + NM, lane);
+    // the 16 column sums of every coefficient, by role, and the factors that
+    // depend on the coefficient only
+#pragma unroll
+    for (int g = 0; g < NG; ++g) S.scr[(4 * g + row) * SDL_ROW + col] = D[g];
+    wave_sync();
+    for (int k = lane; k < NM; k += 64) {
+      double sv = 0.0, si = 0.0;
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        const double v = S.scr[k * SDL_ROW + x];
+        if (x < nc) sv += v;
+        else si += v;
+      }
+      if (WHICH & 1) S.red[k] = sv * aser_scale<PM>(k, 0);
+      if (WHICH & 2) S.red[NM + k] = si * aser_scale<PM>(k, 1);
     }
+    wave_sync();
+    if constexpr (WHICH == 3) aff_to_hom<PM, 2>(S.red, lane);
+    else if constexpr (WHICH == 1) aff_to_hom<PM, 1>(S.red, lane);
+    else aff_to_hom<PM, 1>(S.red + NM, lane);
     for (int k = lane; k < NM; k += 64) {
       // (the volume side adds to the walk's table-row sums)
       if ((WHICH & 1) && out_vol) out_vol[(size_t)i * out_stride + k] += S.red[k];
@@ -2523,7 +2507,7 @@ int launch_sdx_leaves(xg_ctx *ctx, int nel, const int32_t *elems, const double *
                       int32_t *queue, int32_t *stats_if = nullptr) {
   constexpr int NM = Moments<3, PM>::NM;
   const void *kern = (const void *)k_sdx_leaves<LO, PM, SIDE, WHICH>;
-  const size_t lds = sdx_leaf_bytes(xg_minrule_cnt[3][PM], xg_minrule_cnt[2][PM], NM, nullptr, nullptr);
+  const size_t lds = sdl_bytes<PM>(nullptr, nullptr);
   if (lds > 65536) XG_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   int blocks = nel < (1 << 22) ? nel : (1 << 22);
   if (queue) {
@@ -2621,14 +2605,14 @@ int subdiv_staged(xg_ctx *ctx, int nel, const int32_t *elems, const double *lset
       // the overflowed elements (count in device memory) go through the
       // one-kernel path below; its launch strides over the count, so no
       // host round trip is needed
-      // p = 3 with the volume side and the interface both requested: one
-      // launch for both (lane roles), then the rows, then the overflow path
+      // the volume side and the interface both requested: one launch for
+      // both (lane roles), then the rows, then the overflow path
       int u_vol = -1, u_if = -1;
       for (int u = 0; u < ndt; ++u) {
         if (dts[u] == side) u_vol = u;
         if (dts[u] == IF && !if_done) u_if = u;
       }
-      if constexpr (PM == 3) {
+      {
         if (u_vol >= 0 && u_if >= 0 && !getenv("XG_SDX_NOFUSE")) {
           double *ov = o_u[u_vol], *oi = o_u[u_if];
           int32_t *sv = s_u[u_vol], *si = s_u[u_if];

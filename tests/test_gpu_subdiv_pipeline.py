@@ -103,6 +103,25 @@ def test_pipeline_uncut_and_fp32(orc, dev, p):
     assert np.all(g32[~nz] == 0)
 
 
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("dts", [[NEG], [POS], [IF], [NEG, IF], [IF, POS], [POS, IF, NEG]])
+def test_pipeline_leaf_chunks(orc, dev, p, dts):
+    """every combination of parts on elements with few and with many cut
+    leaves: the leaf kernel prepares them 128 (p <= 2) or 256 (p = 3) at a
+    time, 64 per pass (level 5, which the oracle holds for p = 1, has four
+    times the leaves of level 4)"""
+    torch, _abi, ctx = dev
+    mesh = MakeStructured3DMesh(nx=2)
+    vals = W.random_quadric_p2(mesh.ne, seed=5)
+    elems = np.array([0, 11, 12, 30, 47], np.int32)
+    for L in (1, 3, 4, 5) if p == 1 else (1, 3, 4):
+        got, st = run_pipeline(dev, p, L, elems, mesh, vals, dts, _abi.XG_PREC_FP64, stats=True)
+        ref = orc.subdiv_pipeline(p, L, 2 * p, elems, mesh.el2v, mesh.coords, vals, dts, 3, nthreads=8)
+        ref = np.asarray(ref).reshape(got.shape)
+        scale = np.abs(ref).max(axis=(-2, -1), keepdims=True)
+        assert np.all(np.abs(got - ref) <= 1e-12 * scale), (L, dts)
+
+
 def test_pipeline_zero_lattice_values(orc, dev):
     """a P2 level set that vanishes on whole lattice planes of a cut element
     (x * (y - h) with h = 2^-L on the reference tet): zero values count as

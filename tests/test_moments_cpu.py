@@ -5,6 +5,7 @@ random elements and random (inexact) point sets, for D = 1..3, p = 1..3 and
 the three form masks.  The identities hold point by point, so the agreement
 is to rounding (1e-12), whatever the points."""
 import ctypes
+import math
 import os
 import shutil
 import subprocess
@@ -144,6 +145,29 @@ extern "C" int mom_accum_aff(const double *pts, const double *w, int n, double *
   }
   return M::NM;
 }
+// the truncated series of a simplex (Moments<3, P>::aser_*) of k + 1 vertices
+// y - 1/4, scaled and mapped as the subdivision kernel does it: moments of the
+// weight w = k! |T| on the tetrahedron (k = 3) or the triangle (k = 2)
+extern "C" int mom_series(int P, const double *verts, int k, double w, double *m) {
+#define SCASE(PP)                                                                             \
+  if (P == PP) {                                                                              \
+    using M = xg::Moments<3, PP>;                                                             \
+    double h[M::NM], y[4][3] = {};                                                            \
+    for (int v = 0; v <= k; ++v)                                                              \
+      for (int d = 0; d < 3; ++d) y[v][d] = verts[3 * v + d] - 0.25;                          \
+    M::aser_first(y[0], w, h);                                                                \
+    for (int v = 1; v < 4; ++v) M::aser_step(y[v], h); /* a zero step changes nothing */      \
+    for (int r = 0; r < M::NM; ++r) h[r] *= xg::xg_aser3##PP[r][k == 3 ? 0 : 1];              \
+    for (int a = 0; a < M::NM; ++a) {                                                         \
+      double s = 0;                                                                           \
+      for (int r = 0; r < M::NM; ++r) s += (double)xg::xg_aff3##PP[r][a % 64][a / 64] * h[r]; \
+      m[a] = s;                                                                               \
+    }                                                                                         \
+    return M::NM;                                                                             \
+  }
+  SCASE(1) SCASE(2) SCASE(3)
+  return -1;
+}
 """
 
 
@@ -160,6 +184,7 @@ def momlib(tmp_path_factory):
                    check=True, capture_output=True)
     lib = ctypes.CDLL(str(so))
     lib.mom_elmat.restype = ctypes.c_int
+    lib.mom_series.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_void_p]
     lib.mom_hsimplex.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_double,
                                  ctypes.c_void_p]
     return lib
@@ -266,6 +291,35 @@ def test_affine_accumulation_equals_homogeneous(momlib):
     full = np.zeros(128)
     momlib.mom_complement(3, 3, _p(full))
     assert np.abs(got[:nm] - full[:nm]).max() <= 1e-14 * np.abs(full[:nm]).max()
+
+
+@pytest.mark.parametrize("P", [1, 2, 3])
+@pytest.mark.parametrize("k", [2, 3])
+def test_series_moments_of_simplices(momlib, P, k):
+    """aser_first / aser_step with the tables xg_aser3P and xg_aff3P give the
+    degree-2P moments of a tetrahedron and of a triangle (with a zero fourth
+    step): against a Grundmann-Moeller rule on random pieces of the reference
+    tetrahedron, thin ones, and small ones at each of its vertices, where the
+    centred map cancels most.  Bar: as for the point sums of that map."""
+    import sys
+    sys.path.insert(0, HERE)
+    from test_oracle_invariants import gm_rule
+    rng = np.random.default_rng(10 * P + k)
+    corners = np.vstack([np.eye(3), np.zeros(3)])
+    b, w = gm_rule(k, 3)  # degree 7
+    w = np.ascontiguousarray(w / w.sum())
+    for trial in range(24):
+        V = rng.dirichlet(np.ones(4), k + 1)[:, :3]
+        if trial % 3 == 1:
+            V[1:] = V[0] + 1e-5 * (V[1:] - V[0])
+        if trial % 3 == 2:
+            V = corners[trial % 4] + 0.02 * (V - corners[trial % 4])
+        V = np.ascontiguousarray(V)
+        pts = np.ascontiguousarray(b @ V)
+        ref, got = np.zeros(128), np.zeros(128)
+        nm = momlib.mom_accum(3, P, _p(pts), _p(w), len(w), _p(ref))
+        assert momlib.mom_series(P, _p(V), k, float(math.factorial(k)), _p(got)) == nm
+        assert np.abs(got[:nm] - ref[:nm]).max() <= 1e-14 * np.abs(ref[:nm]).max(), trial
 
 
 def test_moment_table_is_current():
