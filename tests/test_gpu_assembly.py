@@ -147,6 +147,43 @@ def test_csr_pattern_device_matches_numpy(dev_abi):
         ctx.sync()
 
 
+@pytest.mark.parametrize("ndof,deg,n", [(1, 1, 1), (3, 21, 50), (3, 22, 50), (4, 32, 9), (8, 33, 700), (10, 25, 900),
+                                        (10, 52, 40), (20, 51, 3000), (20, 52, 3000), (64, 90, 4000), (64, 300, 700)])
+def test_csr_pattern_row_lengths(dev_abi, ndof, deg, n):
+    """rows of every length that changes how they are sorted (64, 128, .. 1024
+    candidates per row, longer ones, and the radix sort of dense tables), with
+    skipped dofs, repeated dofs in an element and empty rows; a column list
+    that is too short is an error"""
+    torch, _abi, ctx = dev_abi
+    rng = np.random.default_rng(ndof * deg + n)
+    nel = max(1, deg * max(n // 3, 1) // ndof)
+    # the first two dofs of an element are in few rows: those get `deg` and more elements
+    dofs = rng.integers(0, n, (nel, ndof)).astype(np.int32)
+    dofs[:, 0] = rng.integers(0, max(1, nel // deg), nel) % n
+    if ndof > 2:
+        dofs[::5, 2] = -1
+        dofs[::3, 1] = dofs[::3, 0]
+    dofs[dofs == n - 1] = -1  # an empty last row
+    rows = np.repeat(dofs, ndof, axis=1).ravel().astype(np.int64)
+    cols = np.tile(dofs, (1, ndof)).ravel().astype(np.int64)
+    ok = (rows >= 0) & (cols >= 0)
+    key = np.unique(rows[ok] * n + cols[ok])
+    ref_rp = np.concatenate([[0], np.cumsum(np.bincount(key // n, minlength=n))])
+    d = torch.from_numpy(dofs).cuda()
+    rp = torch.full((n + 1,), -1, dtype=torch.int32, device="cuda")
+    ci = torch.full((max(len(key), 1),), -1, dtype=torch.int32, device="cuda")
+    nnz = torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    ctx.csr_pattern(d, n, rp, ci, nnz)
+    ctx.sync()
+    assert int(nnz.item()) == len(key)
+    assert np.array_equal(rp.cpu().numpy(), ref_rp)
+    assert np.array_equal(ci.cpu().numpy()[:len(key)], (key % n).astype(np.int32))
+    if len(key) > 1:
+        ctx.csr_pattern(d, n, rp, ci[:len(key) - 1], nnz)
+        with pytest.raises(RuntimeError):
+            ctx.sync()
+
+
 @pytest.mark.parametrize("p", [1, 2])
 def test_restricted_bilinear_form(X, p):
     """RestrictedBilinearForm (python/__init__.py:973-1037, utils/
