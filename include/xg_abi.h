@@ -44,7 +44,8 @@ extern "C" {
 
 /* element-matrix arithmetic */
 #define XG_PREC_FP64 0   /* FP64 MFMA (v_mfma_f64_16x16x4f64), reference mode */
-#define XG_PREC_FP32 1   /* FP32 MFMA (v_mfma_f32_16x16x4f32), FP32 accumulate */
+#define XG_PREC_FP32 1   /* FP32 result; p <= 2: FP64 MFMA and shapes, rounded once;
+                            p = 3: FP32 MFMA (v_mfma_f32_16x16x4f32), FP64 group sums */
 #define XG_PREC_BF16X3 2 /* 3-way split BF16 MFMA (6 products), FP32 accumulate */
 /* OR-ed into the precision of xg_cut_pipeline: moment form.  Per (element,
    domain type) the FP64 barycentric moments sum_i w_i lam(x_i)^alpha,

@@ -131,23 +131,21 @@ __global__ __launch_bounds__(64 * WAVES) void k_batch(int order, int ndt, int dt
   using T = float;
   using C = Cfg<D, P, T>;
   extern __shared__ char smem[];
-  __shared__ StageLds<D, T> s_stage[WAVES];
-  __shared__ double s_rule[2][PIPE_NQMAX][4];
+  __shared__ StageLds s_stage[WAVES];
+  __shared__ StageTab<D> s_tab;
+  __shared__ ElemRec s_rec[WAVES];
   __shared__ int s_vs[MAXMESH + 1];
   __shared__ int s_mesh[MAXMESH];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (C::LDS_PER_WAVE / sizeof(T));
+  using EL = ElLds<D, P, T, 0>;
+  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (EL::BYTES / sizeof(T));
   T *sW = sB + C::SB_SIZE;
-  for (int k = lane; k < C::SB_SIZE; k += 64) sB[k] = T(0);
+  for (int k = lane; k < EL::ZERO; k += 64) sB[k] = T(0);
+  GramLane gl{};
+  if constexpr (EL::GRAM) gl = gram_lane<D, P>();
   const int nq_vol = rule_cnt(D, order), nq_if = rule_cnt(D - 1, order);
-  const int off_vol = rule_off(D, order), off_if = rule_off(D - 1, order);
-  for (int k = threadIdx.x; k < nq_vol + nq_if; k += blockDim.x) {
-    const int which = k < nq_vol ? 0 : 1;
-    const int kk = which ? k - nq_vol : k;
-    const double *r = xg_rule_data_d[(which ? off_if : off_vol) + kk];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) s_rule[which][kk][c] = r[c];
-  }
+  double(*s_rule)[4] = reinterpret_cast<double(*)[4]>(smem + WAVES * EL::BYTES);
+  stage_tables<D>(s_tab, s_rule, order);
   const int nm = cls_nm[P - 1];
   for (int k = threadIdx.x; k < nm; k += blockDim.x) {
     const int m = cls_mesh[(P - 1) * nmesh + k];
@@ -184,17 +182,21 @@ __global__ __launch_bounds__(64 * WAVES) void k_batch(int order, int ndt, int dt
       }
       double V[D + 1][3], l[D + 1];
       load_geom<D>(el2v, coords, lset, e, V, l);
-      double F[D * D], Finv[D * D], absdet;
-      jacobian<D>(V, F, Finv, absdet);
+      if (lane == 0) elem_rec<D>(s_rec[wv], V, l, true);
+      wave_sync();
+      const ElemRec &R = s_rec[wv];
+      const double absdet = R.absdet;
       for (int t = 0; t < ndt; ++t) {
         const int dt = (dts >> (2 * t)) & 3;
-        int nq = 0, nv1 = 0;
         bool bad = false;
-        const int npts = build_stage<D, T>(&s_stage[wv], l, Finv, dt, nq_vol, nq_if, nq, nv1, bad);
+        StagedSrc src{&s_stage[wv], dt == IF ? s_rule + nq_vol : s_rule, 0, 0, 1.0};
+        const int npts = build_stage<D>(&s_stage[wv], s_tab, R, dt, nq_vol, nq_if, src, bad);
         if (bad && lane == 0) atomicOr(err, 1);
-        StagedSrc<D, T> src{&s_stage[wv], s_rule[dt == IF ? 1 : 0], nq, nv1};
-        elmat_one<D, P, T>(src, npts, Finv, absdet, mask, sB, sW, out + obase + (long long)t * NN);
+        T *o = out + obase + (long long)t * NN;
+        if constexpr (EL::GRAM) elmat_gram<D, P, T>(src, npts, R.g, absdet, mask, gl, reinterpret_cast<double *>(sB), o);
+        else elmat_one<D, P, T>(src, npts, R.g, absdet, mask, sB, sW, o);
       }
+      wave_sync();
     }
   }
 }
@@ -282,8 +284,7 @@ int launch_batch_mom(xg_batch *b, hipStream_t st, int32_t *err, int order, float
 
 template <int P, int W>
 int launch_batch(xg_batch *b, hipStream_t st, int32_t *err, int order, float *out, long long cap) {
-  using C = Cfg<3, P, float>;
-  const size_t lds = C::LDS_PER_WAVE * W;
+  const size_t lds = ElLds<3, P, float, 0>::BYTES * W + stage_rule_bytes(3, order);
   const int grid = b->bpc[P] * b->ncu;
   k_batch<P, W><<<grid, 64 * W, lds, st>>>(order, b->ndt, b->dts, b->mask, b->grab[P], b->el2v, b->coords, b->lset,
                                            b->d_cut, b->d_start, b->d_outoff, b->d_vstart, b->d_cls_mesh,

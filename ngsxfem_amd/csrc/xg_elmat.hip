@@ -6,20 +6,21 @@
 //   elmat += B_test^T diag(w_i |det J_i|) B_trial          (AddABt :272-287)
 // i.e. elmat = sum_i w_i |J| (phi phi^T + grad phi grad phi^T).
 //
-// Mapping on CDNA4 (one wavefront per element):
-//  * quadrature points are produced lane-parallel (lane = point, chunks of CH
-//    points); each lane evaluates the degree-P Lagrange shapes and physical
-//    gradients of its point and stores them in LDS as B[c][dof][point]
-//    (c = 0: value, 1..D: gradient components), padded to 16 dofs per block
-//    and CH+1 points per row so both the stores (lane = point) and the MFMA
-//    operand loads (lane = (c, dof)) are bank-conflict free;
-//  * the contraction over (point, component) runs on the matrix cores:
-//    v_mfma_{f32,f64}_16x16x4 with K = the 4 components of one point, so one
-//    MFMA per point per 16x16 dof block (blocks bi <= bj only; the lower
-//    blocks are mirrored at store time).  The B operand is the A operand
-//    scaled by the lane's point weight, so no second LDS read is needed.
+// Mapping on CDNA4 (one wavefront per element, a run of elements per wave: the
+// geometry of a run is computed one element per lane):
+//  * p <= 2 (FP32 and FP64 results): the Gram form of xg_elmat_core.hpp, FP64
+//    matrix instructions over 4 points at a time;
+//  * p = 3 and split BF16: quadrature points are produced lane-parallel (lane =
+//    point, chunks of CH points); each lane evaluates the degree-P Lagrange
+//    shapes and physical gradients of its point and stores them in LDS as
+//    B[c][dof][point] (c = 0: value, 1..D: gradient components), CH+1 points per
+//    row so both the stores (lane = point) and the MFMA operand loads (lane =
+//    (c, dof)) are bank-conflict free; the contraction over (point, component)
+//    runs on v_mfma_{f32,f64}_16x16x4 with K = the 4 components of one point
+//    (blocks bi <= bj only; the lower blocks are mirrored at store time).  The B
+//    operand is the A operand scaled by the point's weight.
 //  * FP64 is kept for the geometry (cut points, sub-simplex determinants,
-//    weights); the shapes are evaluated in the accumulation type T.
+//    weights).
 #include "xg_device.hpp"
 #include "xg_elmat_core.hpp"
 #include "xg_internal.hpp"
@@ -32,50 +33,59 @@ using namespace xg::ecore;
 
 // SPLIT = 1: split-BF16 products (T = float, elmat_one_bf16x3)
 template <int D, int P, typename T, int SPLIT = 0>
-__global__ __launch_bounds__(128) void k_pipeline(int nel, const int32_t *__restrict__ elems,
+__global__ __launch_bounds__(128) void k_pipeline(int nel, int run, const int32_t *__restrict__ elems,
                                                   const int32_t *__restrict__ el2v,
                                                   const double *__restrict__ coords,
                                                   const double *__restrict__ lset, int order, int ndt, int dts,
                                                   int mask, T *__restrict__ out, int32_t *err) {
   using C = Cfg<D, P, T>;
   extern __shared__ char smem[];
-  __shared__ StageLds<D, T> s_stage[C::WAVES];
-  __shared__ double s_rule[2][PIPE_NQMAX][4];  // base rules of dimension D and D-1
+  __shared__ StageLds s_stage[C::WAVES];
+  __shared__ StageTab<D> s_tab;
+  __shared__ ElemRec s_rec[C::WAVES][EL_RUN];
   const int wv = threadIdx.x >> 6;
-  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (C::LDS_PER_WAVE / sizeof(T));
+  using EL = ElLds<D, P, T, SPLIT>;
+  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (EL::BYTES / sizeof(T));
   T *sW = sB + C::SB_SIZE;
   const int lane = threadIdx.x & 63;
   // zero the padding rows once (dofs >= N never get written)
-  for (int k = lane; k < C::SB_SIZE; k += 64) sB[k] = T(0);
+  for (int k = lane; k < EL::ZERO; k += 64) sB[k] = T(0);
+  GramLane gl{};
+  if constexpr (EL::GRAM) gl = gram_lane<D, P>();
   const int nq_vol = rule_cnt(D, order), nq_if = rule_cnt(D - 1, order);
-  const int off_vol = rule_off(D, order), off_if = rule_off(D - 1, order);
-  for (int k = threadIdx.x; k < nq_vol + nq_if; k += blockDim.x) {
-    const int which = k < nq_vol ? 0 : 1;
-    const int kk = which ? k - nq_vol : k;
-    const double *r = xg_rule_data_d[(which ? off_if : off_vol) + kk];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) s_rule[which][kk][c] = r[c];
-  }
+  // base rules of dimension D, then D - 1 (sized by the order)
+  double(*s_rule)[4] = reinterpret_cast<double(*)[4]>(smem + C::WAVES * EL::BYTES);
+  stage_tables<D>(s_tab, s_rule, order);
   __syncthreads();  // the only block barrier: before the per-wave loops
   const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   constexpr int NN = C::N * C::N;
-  for (int i = wid; i < nel; i += nwaves) {
-    const int e = elems ? elems[i] : i;
-    double V[D + 1][3], l[D + 1];
-    load_geom<D>(el2v, coords, lset, e, V, l);
-    double F[D * D], Finv[D * D], absdet;
-    jacobian<D>(V, F, Finv, absdet);
-    for (int t = 0; t < ndt; ++t) {
-      const int dt = (dts >> (2 * t)) & 3;
-      int nq = 0, nv1 = 0;
-      bool bad = false;
-      const int npts = build_stage<D, T>(&s_stage[wv], l, Finv, dt, nq_vol, nq_if, nq, nv1, bad);
-      if (bad && lane == 0) atomicOr(err, 1);
-      StagedSrc<D, T> src{&s_stage[wv], s_rule[dt == IF ? 1 : 0], nq, nv1};
-      if constexpr (SPLIT) elmat_one_bf16x3<D, P>(src, npts, Finv, absdet, mask, sB, sW, out + ((size_t)i * ndt + t) * NN);
-      else elmat_one<D, P, T>(src, npts, Finv, absdet, mask, sB, sW, out + ((size_t)i * ndt + t) * NN);
+  for (long long base = (long long)wid * run; base < nel; base += (long long)nwaves * run) {
+    if (lane < run && base + lane < nel) {
+      const int e = elems ? elems[base + lane] : (int)base + lane;
+      double V[D + 1][3], l[D + 1];
+      load_geom<D>(el2v, coords, lset, e, V, l);
+      elem_rec<D>(s_rec[wv][lane], V, l, true);
     }
+    wave_sync();
+    const int m = min((long long)run, nel - base);
+    for (int j = 0; j < m; ++j) {
+      const ElemRec &R = s_rec[wv][j];
+      const double absdet = R.absdet;
+      for (int t = 0; t < ndt; ++t) {
+        const int dt = (dts >> (2 * t)) & 3;
+        bool bad = false;
+        StagedSrc src{&s_stage[wv], dt == IF ? s_rule + nq_vol : s_rule, 0, 0, 1.0};
+        const int npts = build_stage<D>(&s_stage[wv], s_tab, R, dt, nq_vol, nq_if, src, bad);
+        if (bad && lane == 0) atomicOr(err, 1);
+        T *o = out + ((size_t)(base + j) * ndt + t) * NN;
+        if constexpr (EL::GRAM)
+          elmat_gram<D, P, T>(src, npts, R.g, absdet, mask, gl, reinterpret_cast<double *>(sB), o);
+        else if constexpr (SPLIT) elmat_one_bf16x3<D, P>(src, npts, R.g, absdet, mask, sB, sW, o);
+        else elmat_one<D, P, T>(src, npts, R.g, absdet, mask, sB, sW, o);
+      }
+    }
+    wave_sync();
   }
 }
 
@@ -93,7 +103,7 @@ struct CsrSrc {
 };
 
 template <int D, int P, typename T, int SPLIT = 0>
-__global__ __launch_bounds__(128) void k_elmat_csr(int nel, const int32_t *__restrict__ elems,
+__global__ __launch_bounds__(128) void k_elmat_csr(int nel, int run, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
                                                    const double *__restrict__ coords,
                                                    const int32_t *__restrict__ offsets,
@@ -101,24 +111,71 @@ __global__ __launch_bounds__(128) void k_elmat_csr(int nel, const int32_t *__res
                                                    T *__restrict__ out) {
   using C = Cfg<D, P, T>;
   extern __shared__ char smem[];
+  __shared__ ElemRec s_rec[C::WAVES][EL_RUN];
   const int wv = threadIdx.x >> 6;
-  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (C::LDS_PER_WAVE / sizeof(T));
+  using EL = ElLds<D, P, T, SPLIT>;
+  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (EL::BYTES / sizeof(T));
   T *sW = sB + C::SB_SIZE;
   const int lane = threadIdx.x & 63;
-  for (int k = lane; k < C::SB_SIZE; k += 64) sB[k] = T(0);
+  for (int k = lane; k < EL::ZERO; k += 64) sB[k] = T(0);
+  GramLane gl{};
+  if constexpr (EL::GRAM) gl = gram_lane<D, P>();
   wave_sync();
   const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   constexpr int NN = C::N * C::N;
-  for (int i = wid; i < nel; i += nwaves) {
-    const int e = elems ? elems[i] : i;
-    double V[D + 1][3];
-    load_geom<D>(el2v, coords, nullptr, e, V, nullptr);
-    double F[D * D], Finv[D * D], absdet;
-    jacobian<D>(V, F, Finv, absdet);
-    CsrSrc<T> src{pts, offsets[i]};
-    if constexpr (SPLIT) elmat_one_bf16x3<D, P>(src, offsets[i + 1] - offsets[i], Finv, absdet, mask, sB, sW, out + (size_t)i * NN);
-    else elmat_one<D, P, T>(src, offsets[i + 1] - offsets[i], Finv, absdet, mask, sB, sW, out + (size_t)i * NN);
+  for (long long base = (long long)wid * run; base < nel; base += (long long)nwaves * run) {
+    if (lane < run && base + lane < nel) {
+      const int e = elems ? elems[base + lane] : (int)base + lane;
+      double V[D + 1][3];
+      load_geom<D>(el2v, coords, nullptr, e, V, nullptr);
+      elem_rec<D>(s_rec[wv][lane], V, nullptr, false);
+    }
+    wave_sync();
+    const int m = min((long long)run, nel - base);
+    if constexpr (EL::GRAM) {
+      // the offsets of the run, one per lane; a step's points are loaded while
+      // the step before runs, across elements too
+      const int off = offsets[base + min(lane, m)];
+      double *sL = reinterpret_cast<double *>(sB), *sW2 = sL + 4 * GRAM_PAD;
+      const int end = __builtin_amdgcn_readlane(off, m);
+      int q0 = __builtin_amdgcn_readlane(off, 0);
+      auto load = [&](int q, int q1) { return q + lane < q1 ? pts[q + lane] : make_double4(0.0, 0.0, 0.0, 0.0); };
+      int j0 = 1;  // (the run's first elements may have no points)
+      while (j0 < m && __builtin_amdgcn_readlane(off, j0) == q0) ++j0;
+      double4 nx = load(q0, __builtin_amdgcn_readlane(off, j0));
+      for (int j = 0; j < m; ++j) {
+        const int q1 = __builtin_amdgcn_readlane(off, j + 1);
+        const double absdet = s_rec[wv][j].absdet;
+        doublex4 acc{0, 0, 0, 0};
+        for (; q0 < q1; q0 += 64) {
+          const double4 p = nx;
+          if (q0 + 64 < q1) nx = load(q0 + 64, q1);
+          else if (q1 < end) {
+            // the first points of the next element that has any
+            int jn = j + 2;
+            while (__builtin_amdgcn_readlane(off, jn) == q1) ++jn;
+            nx = load(q1, __builtin_amdgcn_readlane(off, jn));
+          }
+          const double x[3] = {p.x, p.y, p.z};
+          gram_chunk<D>(x, p.w * absdet, min(64, q1 - q0), gl, sL, sW2, acc);
+        }
+        q0 = q1;
+        gram_store<D, P, T>(acc, s_rec[wv][j].g, mask, gl, sW2 + 64, out + (size_t)(base + j) * NN);
+      }
+    } else {
+      for (int j = 0; j < m; ++j) {
+        const long long i = base + j;
+        const ElemRec &R = s_rec[wv][j];
+        const double absdet = R.absdet;
+        CsrSrc<T> src{pts, offsets[i]};
+        const int npts = offsets[i + 1] - offsets[i];
+        T *o = out + (size_t)i * NN;
+        if constexpr (SPLIT) elmat_one_bf16x3<D, P>(src, npts, R.g, absdet, mask, sB, sW, o);
+        else elmat_one<D, P, T>(src, npts, R.g, absdet, mask, sB, sW, o);
+      }
+    }
+    wave_sync();
   }
 }
 
@@ -137,7 +194,7 @@ struct WeightSrc {
 };
 
 template <int P, int Q, typename T, int SPLIT = 0>
-__global__ __launch_bounds__(128) void k_elmat_weights(int nel, const int32_t *__restrict__ elems,
+__global__ __launch_bounds__(128) void k_elmat_weights(int nel, int run, const int32_t *__restrict__ elems,
                                                        const int32_t *__restrict__ el2v,
                                                        const double *__restrict__ coords,
                                                        const double *__restrict__ weights, int mask,
@@ -145,31 +202,48 @@ __global__ __launch_bounds__(128) void k_elmat_weights(int nel, const int32_t *_
   using C = Cfg<3, P, T>;
   constexpr int NQ = ndof(3, Q);
   extern __shared__ char smem[];
+  __shared__ ElemRec s_rec[C::WAVES][EL_RUN];
   const int wv = threadIdx.x >> 6;
-  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (C::LDS_PER_WAVE / sizeof(T));
+  using EL = ElLds<3, P, T, SPLIT>;
+  T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (EL::BYTES / sizeof(T));
   T *sW = sB + C::SB_SIZE;
   const int lane = threadIdx.x & 63;
-  for (int k = lane; k < C::SB_SIZE; k += 64) sB[k] = T(0);
+  for (int k = lane; k < EL::ZERO; k += 64) sB[k] = T(0);
+  GramLane gl{};
+  if constexpr (EL::GRAM) gl = gram_lane<3, P>();
   wave_sync();
   const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   constexpr int NN = C::N * C::N;
-  for (int i = wid; i < nel; i += nwaves) {
-    double Finv[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1}, absdet = 1.0;
-    if (coords) {
-      const int e = elems ? elems[i] : i;
-      double V[4][3], F[9];
-      load_geom<3>(el2v, coords, nullptr, e, V, nullptr);
-      jacobian<3>(V, F, Finv, absdet);
+  for (long long base = (long long)wid * run; base < nel; base += (long long)nwaves * run) {
+    if (lane < run && base + lane < nel) {
+      double V[4][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {0, 0, 0}};
+      if (coords) {
+        const int e = elems ? elems[base + lane] : (int)base + lane;
+        load_geom<3>(el2v, coords, nullptr, e, V, nullptr);
+      }
+      elem_rec<3>(s_rec[wv][lane], V, nullptr, false);
     }
-    WeightSrc<Q, T> src{weights + (size_t)i * NQ};
-    if constexpr (SPLIT) elmat_one_bf16x3<3, P>(src, NQ, Finv, absdet, mask, sB, sW, out + (size_t)i * NN);
-    else elmat_one<3, P, T>(src, NQ, Finv, absdet, mask, sB, sW, out + (size_t)i * NN);
+    wave_sync();
+    const int m = min((long long)run, nel - base);
+    for (int j = 0; j < m; ++j) {
+      const long long i = base + j;
+      const ElemRec &R = s_rec[wv][j];
+      const double absdet = R.absdet;
+      WeightSrc<Q, T> src{weights + (size_t)i * NQ};
+      constexpr int npts = NQ;
+      T *o = out + (size_t)i * NN;
+      if constexpr (EL::GRAM)
+        elmat_gram<3, P, T>(src, npts, R.g, absdet, mask, gl, reinterpret_cast<double *>(sB), o);
+      else elmat_one_bf16x3<3, P>(src, npts, R.g, absdet, mask, sB, sW, o);
+    }
+    wave_sync();
   }
 }
 
 int grid_waves(int nel) {
-  long long blocks = ((long long)nel + 1) / 2;
+  const int run = el_run(nel);
+  long long blocks = ((long long)nel + 2 * run - 1) / (2 * run);
   if (blocks > 16384) blocks = 16384;
   if (blocks < 1) blocks = 1;
   return (int)blocks;
@@ -179,9 +253,9 @@ template <int D, int P, typename T, int SPLIT = 0>
 int launch_pipeline(xg_ctx *ctx, int order, int nel, const int32_t *elems, const int32_t *el2v,
                     const double *coords, const double *lset, int ndt, int dts, int mask, void *out) {
   using C = Cfg<D, P, T>;
-  const size_t lds = C::LDS_PER_WAVE * C::WAVES;
+  const size_t lds = ElLds<D, P, T, SPLIT>::BYTES * C::WAVES + stage_rule_bytes(D, order);
   k_pipeline<D, P, T, SPLIT><<<grid_waves(nel), 64 * C::WAVES, lds, ctx->stream>>>(
-      nel, elems, el2v, coords, lset, order, ndt, dts, mask, (T *)out, ctx->d_err);
+      nel, el_run(nel), elems, el2v, coords, lset, order, ndt, dts, mask, (T *)out, ctx->d_err);
   XG_LAUNCH_CHECK();
   return XG_OK;
 }
@@ -190,9 +264,9 @@ template <int D, int P, typename T, int SPLIT = 0>
 int launch_csr(xg_ctx *ctx, int nel, const int32_t *elems, const int32_t *el2v, const double *coords,
                const int32_t *offsets, const double *pts, int mask, void *out) {
   using C = Cfg<D, P, T>;
-  const size_t lds = C::LDS_PER_WAVE * C::WAVES;
+  const size_t lds = ElLds<D, P, T, SPLIT>::BYTES * C::WAVES;
   k_elmat_csr<D, P, T, SPLIT><<<grid_waves(nel), 64 * C::WAVES, lds, ctx->stream>>>(
-      nel, elems, el2v, coords, offsets, reinterpret_cast<const double4 *>(pts), mask, (T *)out);
+      nel, el_run(nel), elems, el2v, coords, offsets, reinterpret_cast<const double4 *>(pts), mask, (T *)out);
   XG_LAUNCH_CHECK();
   return XG_OK;
 }
@@ -249,8 +323,8 @@ template <int P, int Q, typename T, int SPLIT = 0>
 int launch_weights(xg_ctx *ctx, int nel, const int32_t *elems, const int32_t *el2v, const double *coords,
                    const double *weights, int mask, void *out) {
   using C = Cfg<3, P, T>;
-  const size_t lds = C::LDS_PER_WAVE * C::WAVES;
-  k_elmat_weights<P, Q, T, SPLIT><<<grid_waves(nel), 64 * C::WAVES, lds, ctx->stream>>>(nel, elems, el2v, coords, weights,
+  const size_t lds = ElLds<3, P, T, SPLIT>::BYTES * C::WAVES;
+  k_elmat_weights<P, Q, T, SPLIT><<<grid_waves(nel), 64 * C::WAVES, lds, ctx->stream>>>(nel, el_run(nel), elems, el2v, coords, weights,
                                                                                 mask, (T *)out);
   XG_LAUNCH_CHECK();
   return XG_OK;

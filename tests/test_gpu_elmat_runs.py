@@ -1,0 +1,87 @@
+"""Element matrices of rules of any length and of lists of any length: the contraction takes 64 points at a time
+and 4 per matrix instruction, and a wave takes 1, 2, 4 or 8 elements in a run (more as the list grows)."""
+import numpy as np
+import pytest
+
+from ngsxfem_amd import _abi
+from ngsxfem_amd import workloads as W
+from ngsxfem_amd.meshes import Make1DMesh, MakeStructured2DMesh, MakeStructured3DMesh
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+COUNTS = [0, 0, 1, 3, 4, 5, 63, 64, 65, 0, 127, 128, 129, 200]
+
+
+def _mesh(D):
+    return Make1DMesh(5) if D == 1 else (MakeStructured2DMesh(nx=3, ny=4) if D == 2 else MakeStructured3DMesh(nx=2))
+
+
+@pytest.mark.parametrize("D", [1, 2, 3])
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("mask", [1, 2, 3])
+def test_rules_of_every_length(D, p, mask):
+    import torch
+    mesh = _mesh(D)
+    rng = np.random.default_rng(100 * D + 10 * p + mask)
+    elems = rng.integers(0, mesh.ne, len(COUNTS)).astype(np.int32)
+    off = np.concatenate([[0], np.cumsum(COUNTS)]).astype(np.int32)
+    pts = np.zeros((off[-1], 4))
+    pts[:, :D] = rng.dirichlet(np.ones(D + 1), off[-1])[:, :D]
+    pts[:, 3] = rng.uniform(-0.3, 1.0, off[-1])  # rules with negative weights too
+    ctx = _abi.Context(0)
+    up = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    nd = O.h1_ndof(D, p)
+    for prec, dtype, bar in ((_abi.XG_PREC_FP64, torch.float64, 1e-13), (_abi.XG_PREC_FP32, torch.float32, 1e-6)):
+        out = torch.full((len(COUNTS), nd, nd), float("nan"), dtype=dtype, device="cuda")
+        ctx.elmat(D, p, up(mesh.el2v), up(mesh.coords), up(off), up(pts), mask, prec, out, elems=up(elems))
+        ctx.sync()
+        g = out.cpu().numpy().astype(np.float64)
+        for i, e in enumerate(elems):
+            a, b = off[i], off[i + 1]
+            V = mesh.coords[mesh.el2v[e]]
+            ref = O.elmat(D, p, V, pts[a:b, :3], pts[a:b, 3], mask) if b > a else np.zeros((nd, nd))
+            # scale: the matrix of the absolute weights (the sums may cancel)
+            sc = np.abs(O.elmat(D, p, V, pts[a:b, :3], np.abs(pts[a:b, 3]), mask)).max() if b > a else 0.0
+            assert np.abs(g[i] - ref).max() <= bar * sc, (i, COUNTS[i])
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 32767, 32768, 65537, 131073])
+@pytest.mark.parametrize("p", [1, 2])
+def test_lists_of_every_length(n, p):
+    """a long list gives the matrices of a short one, bit for bit (the same operations per element)"""
+    import torch
+    mesh, lset = W.config2(6)
+    rng = np.random.default_rng(n)
+    pick = rng.integers(0, mesh.ne, n).astype(np.int32)
+    ctx = _abi.Context(0)
+    up = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    el, X, ls = up(mesh.el2v), up(mesh.coords), up(lset)
+    nd = O.h1_ndof(3, p)
+
+    def both(ids):
+        m = ids.numel()
+        out = torch.zeros((m, 2, nd, nd), dtype=torch.float32, device="cuda")
+        ctx.cut_pipeline(3, p, 2 * p, el, X, ls, [0, 2], 3, _abi.XG_PREC_FP32, out, elems=ids)
+        off = torch.zeros(m + 1, dtype=torch.int32, device="cuda")
+        ctx.cut_rule_count(3, el, ls, 0, 2 * p, off, elems=ids)
+        pts = torch.zeros((max(int(off[-1].item()), 1), 4), dtype=torch.float64, device="cuda")
+        ctx.cut_rule_fill(3, el, X, ls, 0, 2 * p, off, pts, elems=ids)
+        csr = torch.zeros((m, nd, nd), dtype=torch.float64, device="cuda")
+        vec = torch.zeros((m, nd), dtype=torch.float64, device="cuda")
+        ctx.elmat(3, p, el, X, off, pts, 3, _abi.XG_PREC_FP64, csr, elems=ids)
+        ctx.elvec(3, p, el, X, off, pts, vec, elems=ids)
+        ctx.sync()
+        return out, csr, vec
+
+    long = both(up(pick))
+    short = both(up(np.arange(mesh.ne, dtype=np.int32)))
+    at = up(pick).long()
+    for a, b in zip(long, short):
+        assert torch.equal(a, b[at])
+    # the short list against the oracle
+    ref = O.cut_pipeline(3, p, 2 * p, np.arange(mesh.ne, dtype=np.int32), mesh.el2v, mesh.coords, lset, [0, 2], 3)
+    g = short[0].cpu().numpy().astype(np.float64).reshape(ref.shape)
+    sc = np.abs(ref).max(axis=(-2, -1), keepdims=True)
+    assert np.all(np.abs(g - ref) <= 2e-7 * sc)
+    ctx.close()
