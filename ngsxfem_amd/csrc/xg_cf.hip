@@ -36,7 +36,9 @@ __device__ __forceinline__ void element_geometry(const int32_t *__restrict__ el2
 // w_q <- w_q * cf(x_q) for every point of every listed element; the
 // element's vertices have A coordinates (A = D, or D + 1 for boundary
 // elements given in the ambient space), x_q = sum_k lam_k X_k
-template <int D, int A>
+// DEPTH: registers of the program's stack (4, or 16 for deeper programs); MATH:
+// the program calls library functions
+template <int D, int A, int DEPTH, bool MATH>
 __global__ __launch_bounds__(256) void k_rule_scale_cf(int nel, const int32_t *__restrict__ elems,
                                                        const int32_t *__restrict__ el2v,
                                                        const double *__restrict__ coords,
@@ -74,7 +76,7 @@ __global__ __launch_bounds__(256) void k_rule_scale_cf(int nel, const int32_t *_
         for (int c = 0; c < D; ++c) a += (V[c][r] - V[D][r]) * xi[c];
         x[r] = a;
       }
-      p.w *= cf::eval<D>(P, x, lam, vv, e);
+      p.w *= cf::eval<D, DEPTH, MATH>(P, x, lam, vv, e);
       pts[q] = p;
     }
   }
@@ -82,18 +84,19 @@ __global__ __launch_bounds__(256) void k_rule_scale_cf(int nel, const int32_t *_
 
 // out[i][a] = |det F| sum_q w_q phi_a(xi_q): element vectors of the source
 // f = 1 on the rule (f is already in the weights after xg_rule_scale_cf)
+// 16 lanes per element: a wave per element added N sums over 64 lanes by six
+// shuffles each
 template <int D, int P>
 __global__ __launch_bounds__(256) void k_elvec_rule(int nel, const int32_t *__restrict__ elems,
                                                     const int32_t *__restrict__ el2v,
                                                     const double *__restrict__ coords,
                                                     const int32_t *__restrict__ offsets,
                                                     const double4 *__restrict__ pts, double *__restrict__ out) {
-  constexpr int N = ndof(D, P);
-  const int lane = threadIdx.x & 63;
-  const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int nwaves = (gridDim.x * blockDim.x) >> 6;
-  for (int i = wid; i < nel; i += nwaves) {
-    const int e = elems ? elems[i] : i;
+  constexpr int N = ndof(D, P), G = 16;
+  const int sub = threadIdx.x & (G - 1);
+  const long long ngrp = (long long)gridDim.x * (256 / G);
+  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) / G; i < nel; i += ngrp) {
+    const int e = elems ? elems[i] : (int)i;
     int32_t vv[D + 1];
     double V[D + 1][3];
     element_geometry<D>(el2v, coords, e, vv, V);
@@ -102,7 +105,8 @@ __global__ __launch_bounds__(256) void k_elvec_rule(int nel, const int32_t *__re
     double s[N];
 #pragma unroll
     for (int a = 0; a < N; ++a) s[a] = 0.0;
-    for (int q = offsets[i] + lane; q < offsets[i + 1]; q += 64) {
+    const int q1 = offsets[i + 1];
+    for (int q = offsets[i] + sub; q < q1; q += G) {
       const double4 p = pts[q];
       const double xi[3] = {p.x, p.y, p.z};
       double lam[D + 1], phi[N];
@@ -117,14 +121,16 @@ __global__ __launch_bounds__(256) void k_elvec_rule(int nel, const int32_t *__re
 #pragma unroll
       for (int a = 0; a < N; ++a) s[a] = fma(p.w, phi[a], s[a]);
     }
+    double v[(N + G - 1) / G];
 #pragma unroll
     for (int a = 0; a < N; ++a) {
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) s[a] += __shfl_xor(s[a], o, 64);
+      for (int o = G / 2; o > 0; o >>= 1) s[a] += __shfl_xor(s[a], o, G);
+      if (a % G == sub) v[a / G] = s[a];
     }
 #pragma unroll
-    for (int a = 0; a < N; ++a)
-      if (lane == a) out[(size_t)i * N + a] = absdet * s[a];
+    for (int a = 0; a < (N + G - 1) / G; ++a)
+      if (a * G + sub < N) out[(size_t)i * N + a * G + sub] = absdet * v[a];
   }
 }
 
@@ -250,7 +256,12 @@ extern "C" int xg_rule_scale_cf(xg_ctx *ctx, int D, int A, int nel, const int32_
   if (!el2v || !coords || !offsets || !pts) return set_error(XG_ERR_ARG, "xg_rule_scale_cf: null pointer");
   const int grid = cf_grid(nel);
   double4 *p = reinterpret_cast<double4 *>(pts);
-#define XG_SC(DD, AA) k_rule_scale_cf<DD, AA><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, P)
+#define XG_SC1(DD, AA, DEPTH, MATH) \
+  k_rule_scale_cf<DD, AA, DEPTH, MATH><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, P)
+#define XG_SC(DD, AA)                                    \
+  if (P.depth <= 4 && !P.math) XG_SC1(DD, AA, 4, false); \
+  else if (!P.math) XG_SC1(DD, AA, 16, false);           \
+  else XG_SC1(DD, AA, 16, true)
   switch (D * 4 + A) {
     case 5: XG_SC(1, 1); break;
     case 6: XG_SC(1, 2); break;
@@ -259,6 +270,7 @@ extern "C" int xg_rule_scale_cf(xg_ctx *ctx, int D, int A, int nel, const int32_
     default: XG_SC(3, 3); break;
   }
 #undef XG_SC
+#undef XG_SC1
   XG_LAUNCH_CHECK();
   return XG_OK;
 }
@@ -308,7 +320,8 @@ extern "C" int xg_elvec(xg_ctx *ctx, int D, int p, int nel, const int32_t *elems
   if (!ctx || D < 1 || D > 3 || p < 1 || p > 3 || nel < 0) return set_error(XG_ERR_ARG, "xg_elvec: bad argument");
   if (nel == 0) return XG_OK;
   if (!el2v || !coords || !offsets || !pts || !out) return set_error(XG_ERR_ARG, "xg_elvec: null pointer");
-  const int grid = cf_grid(nel);
+  const long long want = ((long long)nel + 15) / 16;
+  const int grid = (int)(want < 16384 ? want : 16384);
   const double4 *q = reinterpret_cast<const double4 *>(pts);
 #define XG_EV(DD, PP) \
   k_elvec_rule<DD, PP><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, q, out)

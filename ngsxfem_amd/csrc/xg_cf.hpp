@@ -64,6 +64,8 @@ constexpr int MAXSTACK = 16;  // evaluation stack depth
 // read through the scalar cache: wave-uniform)
 struct Prog {
   int32_t n;  // words of code
+  int32_t depth;  // deepest stack
+  int32_t math;   // has a function of the math library (POW .. TANH but SQRT)
   int32_t code[MAXCODE];
   double c[MAXCONST];
   const double *gf[MAXGF];
@@ -93,6 +95,8 @@ inline const char *validate(int32_t ncode, const int32_t *code, int32_t nconst, 
   if (nconst < 0 || nconst > MAXCONST || (nconst > 0 && !consts)) return "coefficient program: at most 48 constants";
   if (ngf < 0 || ngf > MAXGF || (ngf > 0 && !gf)) return "coefficient program: at most 4 grid functions";
   int depth = 0;
+  p.depth = 1;
+  p.math = 0;
   for (int pc = 0; pc < ncode;) {
     const int32_t op = code[pc];
     if (op <= END || op >= NOPS) return "coefficient program: unknown opcode";
@@ -107,6 +111,8 @@ inline const char *validate(int32_t ncode, const int32_t *code, int32_t nconst, 
     if (depth < need) return "coefficient program: stack underflow";
     depth += op_delta(op);
     if (depth > MAXSTACK) return "coefficient program: stack deeper than 16";
+    if (depth > p.depth) p.depth = depth;
+    if (op == POW || (op >= SIN && op <= TANH)) p.math = 1;
     pc += w;
   }
   if (depth != 1) return "coefficient program: must leave exactly one value";
@@ -125,59 +131,79 @@ inline bool uses_elements(const Prog &p) {
   return false;
 }
 
-// value of the program at the physical point x of element e with vertices
-// vv (D + 1 of them) and barycentrics lam (lam_k of vertex k)
-template <int D>
+// Value of the program at the physical point x of element e with vertices
+// vv (D + 1 of them) and barycentrics lam (lam_k of vertex k).  The stack is
+// DEPTH registers with the top first: a push or pop moves the others, so no
+// entry is addressed by a run-time index (an indexed private array lives in
+// scratch memory: every operation of every point went through it).  MATH =
+// false: for programs without library functions, whose registers (over 200)
+// the others would pay for with their waves.
+template <int D, int DEPTH = MAXSTACK, bool MATH = true>
 XG_CF_FN double eval(const Prog &P, const double *x, const double *lam, const int32_t *vv, int e) {
-  double st[MAXSTACK];
-  int sp = 0;
+  double st[DEPTH + 1];
+#pragma unroll
+  for (int k = 0; k <= DEPTH; ++k) st[k] = 0.0;
   for (int pc = 0; pc < P.n;) {
     const int32_t op = P.code[pc];
     const int32_t a = P.code[pc + 1 < MAXCODE ? pc + 1 : pc];
     pc += op_words(op);
-    switch (op) {
-      case CONST: st[sp++] = P.c[a]; break;
-      case COORD: st[sp++] = x[a]; break;
-      case GF1: {
+    const int delta = op_delta(op);
+    if (delta > 0) {
+      double v = 0.0;
+      if (op == CONST) v = P.c[a];
+      else if (op == COORD) v = a == 0 ? x[0] : (a == 1 ? x[1] : x[2]);
+      else if (op == GF1) {
         const double *u = P.gf[a];
-        double s = 0.0;
-        for (int k = 0; k <= D; ++k) s += lam[k] * u[vv[k]];
-        st[sp++] = s;
-        break;
-      }
-      case EL0: st[sp++] = P.gf[a][e]; break;
-      case ADD: --sp; st[sp - 1] = st[sp - 1] + st[sp]; break;
-      case SUB: --sp; st[sp - 1] = st[sp - 1] - st[sp]; break;
-      case MUL: --sp; st[sp - 1] = st[sp - 1] * st[sp]; break;
-      case DIV: --sp; st[sp - 1] = st[sp - 1] / st[sp]; break;
-      case POW: --sp; st[sp - 1] = pow(st[sp - 1], st[sp]); break;
-      case MAX: --sp; st[sp - 1] = fmax(st[sp - 1], st[sp]); break;
-      case MIN: --sp; st[sp - 1] = fmin(st[sp - 1], st[sp]); break;
-      case IFPOS: sp -= 2; st[sp - 1] = st[sp - 1] > 0.0 ? st[sp] : st[sp + 1]; break;
-      case NEG: st[sp - 1] = -st[sp - 1]; break;
+#pragma unroll
+        for (int k = 0; k <= D; ++k) v += lam[k] * u[vv[k]];
+      } else v = P.gf[a][e];
+#pragma unroll
+      for (int k = DEPTH; k > 0; --k) st[k] = st[k - 1];
+      st[0] = v;
+      continue;
+    }
+    const double t = st[0], s = st[1];  // b of "a b", or the operand; a
+    double v = t;
+    switch (op) {
+      case ADD: v = s + t; break;
+      case SUB: v = s - t; break;
+      case MUL: v = s * t; break;
+      case DIV: v = s / t; break;
+      case POW: if constexpr (MATH) v = pow(s, t); break;
+      case MAX: v = fmax(s, t); break;
+      case MIN: v = fmin(s, t); break;
+      case IFPOS: v = st[DEPTH > 1 ? 2 : 1] > 0.0 ? s : t; break;
+      case NEG: v = -t; break;
       case POWI: {
-        const double b = st[sp - 1];
         int n = a < 0 ? -a : a;
-        double r = 1.0, q = b;
+        double r = 1.0, q = t;
         while (n) {  // square and multiply
           if (n & 1) r *= q;
           q *= q;
           n >>= 1;
         }
-        st[sp - 1] = a < 0 ? 1.0 / r : r;
+        v = a < 0 ? 1.0 / r : r;
         break;
       }
-      case SQRT: st[sp - 1] = sqrt(st[sp - 1]); break;
-      case SIN: st[sp - 1] = sin(st[sp - 1]); break;
-      case COS: st[sp - 1] = cos(st[sp - 1]); break;
-      case TAN: st[sp - 1] = tan(st[sp - 1]); break;
-      case EXP: st[sp - 1] = exp(st[sp - 1]); break;
-      case LOG: st[sp - 1] = log(st[sp - 1]); break;
-      case ATAN: st[sp - 1] = atan(st[sp - 1]); break;
-      case TANH: st[sp - 1] = tanh(st[sp - 1]); break;
-      case ABS: st[sp - 1] = fabs(st[sp - 1]); break;
+      case SQRT: v = sqrt(t); break;
+      case SIN: if constexpr (MATH) v = sin(t); break;
+      case COS: if constexpr (MATH) v = cos(t); break;
+      case TAN: if constexpr (MATH) v = tan(t); break;
+      case EXP: if constexpr (MATH) v = exp(t); break;
+      case LOG: if constexpr (MATH) v = log(t); break;
+      case ATAN: if constexpr (MATH) v = atan(t); break;
+      case TANH: if constexpr (MATH) v = tanh(t); break;
+      case ABS: v = fabs(t); break;
       default: break;
     }
+    if (delta == -1) {
+#pragma unroll
+      for (int k = 1; k < DEPTH; ++k) st[k] = st[k + 1];
+    } else if (delta == -2) {
+#pragma unroll
+      for (int k = 1; k + 1 < DEPTH; ++k) st[k] = st[k + 2];
+    }
+    st[0] = v;
   }
   return st[0];
 }

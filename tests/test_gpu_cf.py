@@ -250,3 +250,53 @@ def test_set_p1_from_grid_function_expression(X):
     xc = mesh.coords
     ref = 2 * h.vec + np.sin(xc[:, 0]) - (xc[:, 1] > 0.5)
     np.testing.assert_allclose(g.vec, ref, rtol=1e-15, atol=1e-15)
+
+
+@pytest.mark.parametrize("depth", [1, 2, 4, 5, 15, 16])
+@pytest.mark.parametrize("math", [False, True])
+def test_programs_of_every_stack_depth(dev, depth, math):
+    """the evaluation stack is 4 or 16 registers, and programs that call the
+    math library have a kernel of their own: depth operands pushed, then
+    reduced by +, -, *, max, min, IfPos from the top, against numpy"""
+    torch, _abi, ctx = dev
+    rng = np.random.default_rng(depth)
+    n = 70
+    pts = np.zeros((n, 4))
+    pts[:, :3] = rng.dirichlet(np.ones(4), n)[:, :3]
+    pts[:, 3] = rng.uniform(0.5, 2.0, n)
+    V = np.array([[0.1, 0.2, 0.0], [1.3, 0.1, 0.2], [0.2, 0.9, 0.1], [0.0, 0.3, 1.1]])
+    x = V[3] + pts[:, :3] @ (V[:3] - V[3])
+    code, consts, st = [], [], []
+    for k in range(depth):
+        if k % 3 == 2:
+            consts.append(0.5 + 0.1 * k)
+            code += [1, len(consts) - 1]
+            st.append(np.full(n, consts[-1]))
+        else:
+            code += [2, k % 3]
+            st.append(x[:, k % 3].copy())
+        if math and k == 0:
+            code.append(14)  # exp
+            st[-1] = np.exp(st[-1])
+    ops = [(3, np.add), (4, np.subtract), (5, np.multiply), (21, np.maximum), (22, np.minimum)]
+    k = 0
+    while len(st) > 1:
+        if len(st) > 2 and k % 4 == 3:
+            c, b, a = st.pop(), st.pop(), st.pop()
+            code.append(20)
+            st.append(np.where(a > 0, b, c))
+        else:
+            op, f = ops[k % 5]
+            b, a = st.pop(), st.pop()
+            code.append(op)
+            st.append(f(a, b))
+        k += 1
+    d_pts = up(torch, pts)
+    ctx.rule_scale_cf(3, up(torch, np.arange(4, dtype=np.int32)[None]), up(torch, V),
+                      up(torch, np.array([0, n], np.int32)), d_pts, code, consts)
+    ctx.sync()
+    g = d_pts.cpu().numpy()
+    assert np.array_equal(g[:, :3], pts[:, :3])
+    ref = pts[:, 3] * st[0]
+    # a dozen roundings of values below 10, and one of exp
+    assert np.abs(g[:, 3] - ref).max() <= 1e-13
