@@ -17,11 +17,12 @@
 // another coordinate plays xi, or give up on the tensor product and cut the
 // 2 triangles / 6 tetrahedra of the element instead (the fallback).
 //
-// Mapping: one lane per element (the number of points varies from element
-// to element); a count pass and a fill pass produce a CSR rule like the
-// simplex rule (xg_rule.hip).  The recursion depth is fixed (hex -> slice
-// quad -> slice segment), so it is written as nested templates with small
-// functors that map a slice point back into the element and pass it on.
+// Mapping: 16 lanes per element, each with a part of its rule (a Gauss slice of
+// a piece, a sub-simplex of the fallback) in the rule's order; a count pass and
+// a fill pass produce a CSR rule like the simplex rule (xg_rule.hip).  The
+// recursion depth is fixed (hex -> slice quad -> slice segment), so it is
+// written as nested templates with small functors that map a slice point back
+// into the element and pass it on.  Marking takes one lane per element.
 #include "xg_device.hpp"
 #include "xg_internal.hpp"
 
@@ -131,9 +132,9 @@ XG_DEV int box_check(const QL &L, int D, const Box &q, double eps) {
 
 // Quadrilateral::GetVolume / GetPlainIntegrationRule, :74-78, 102-129: the
 // tensor Gauss rule (x slowest) mapped by points[0] + A ip,
-// A = (p1 - p0, p3 - p0, p4 - p0)
+// A = (p1 - p0, p3 - p0, p4 - p0); the points i0 <= i < i1 of the x rule
 template <class Sink>
-XG_DEV void box_plain(const Box &q, int D, int order, Sink &s) {
+XG_DEV void box_plain(const Box &q, int D, int order, Sink &s, int i0, int i1) {
   double p0[3], p1[3], p3[3], p4[3] = {0, 0, 0};
   box_point(q, D, 0, p0);
   box_point(q, D, 1, p1);
@@ -162,7 +163,7 @@ XG_DEV void box_plain(const Box &q, int D, int order, Sink &s) {
   if (D == 2) A[2][0] = A[2][1] = 0.0;
   const int n = rule_cnt(1, order);
   const double(*r)[4] = &xg_rule_data_d[rule_off(1, order)];
-  for (int i = 0; i < n; ++i)
+  for (int i = i0; i < i1; ++i)
     for (int j = 0; j < n; ++j)
       for (int k = 0; k < (D == 3 ? n : 1); ++k) {
         const double ip[3] = {r[i][0], r[j][0], D == 3 ? r[k][0] : 0.0};
@@ -172,6 +173,11 @@ XG_DEV void box_plain(const Box &q, int D, int order, Sink &s) {
         for (int d = 0; d < 3; ++d) x[d] = p0[d] + (A[d][0] * ip[0] + A[d][1] * ip[1] + A[d][2] * ip[2]);
         s(x, wq * tf);
       }
+}
+
+template <class Sink>
+XG_DEV void box_plain(const Box &q, int D, int order, Sink &s) {
+  box_plain(q, D, order, s, 0, rule_cnt(1, order));
 }
 
 // base rule of dimension dim on the simplex P (SimpleX::GetPlainIntegrationRule)
@@ -223,10 +229,11 @@ XG_DEV void segment_rule(const double *lv, int dt, int order, Sink &s, int &err)
 
 // GetFallbackIntegrationRule, :475-491: the 2 triangles / 6 tetrahedra of the
 // unit element, each with the clamped values of update_initial_coefs
+// (the sub-simplices s0 <= si < s1)
 template <int D, class Sink>
-XG_DEV void fallback_rule(const QL &L, int dt, int order, Sink &s, int &err) {
+XG_DEV void fallback_rule(const QL &L, int dt, int order, Sink &s, int &err, int s0 = 0, int s1 = D == 2 ? 2 : 6) {
   const Box u = unit_box();
-  for (int si = 0; si < (D == 2 ? 2 : 6); ++si) {
+  for (int si = s0; si < s1; ++si) {
     double P[4][3], l[4];
     for (int k = 0; k <= D; ++k) {
       box_point(u, D, D == 2 ? kTri[si][k] : kTet[si][k], P[k]);
@@ -282,12 +289,12 @@ struct SliceSink {
   }
 };
 
+// (the Gauss slices a <= i1 < b)
 template <int D, class Sink>
-XG_DEV void tensor_rule(const QL &L, const Box &q, int dt, int order, int pol, Sink &s, int &err) {
+XG_DEV void tensor_rule(const QL &L, const Box &q, int dt, int order, int pol, Sink &s, int &err, int a, int b) {
   const double xi0 = q.lo[D - 1], xi1 = q.hi[D - 1];
-  const int n = rule_cnt(1, order);
   const double(*r)[4] = &xg_rule_data_d[rule_off(1, order)];
-  for (int i1 = 0; i1 < n; ++i1) {
+  for (int i1 = a; i1 < b; ++i1) {
     const double xs = xi0 + r[i1][0] * (xi1 - xi0);
     SliceSink<D, Sink> ss{L, q, xs, r[i1][3], xi1 - xi0, dt, s, err};
     if constexpr (D == 2) {
@@ -332,7 +339,7 @@ XG_DEV void along_xi(const QL &L, int dt, int order, int pol, Sink &s, int &err)
     if (!dup) xs[nx++] = x;
   }
   if (!topo) {
-    tensor_rule<D>(L, u, dt, order, pol, s, err);
+    tensor_rule<D>(L, u, dt, order, pol, s, err, 0, rule_cnt(1, order));
     return;
   }
   for (int i = 1; i < nx; ++i)  // ascending, as the std::set
@@ -347,7 +354,7 @@ XG_DEV void along_xi(const QL &L, int dt, int order, int pol, Sink &s, int &err)
     sq.hi[D - 1] = xs[i + 1];
     const int ds = box_check(L, D, sq, 1e-15);
     if (ds == IF)
-      tensor_rule<D>(L, sq, dt, order, pol, s, err);
+      tensor_rule<D>(L, sq, dt, order, pol, s, err, 0, rule_cnt(1, order));
     else if (ds == dt)
       box_plain(sq, D, order, s);
   }
@@ -605,6 +612,115 @@ XG_DEV void element_rule(const double *vals, int dt, int order, int pol, Sink &s
     hex_rule(L, dt, order, pol, s, err);
 }
 
+// The parts of an element's rule in its order, for lanes that take one each:
+// element_rule above with its outermost loops cut up.
+enum { QP_NONE, QP_BOX, QP_XI, QP_FALLBACK };
+template <int D>
+struct QuadParts {
+  int kind, n;
+  int sw;
+  bool topo;
+  QL L;         // rotated for a dimension swap
+  double x[4];  // split points along xi in ascending order, 1 where there are fewer
+
+  static constexpr int PIECES = D == 2 ? 3 : 5;
+
+  XG_DEV void plan(const double *vals, int dt, int order, int pol, int &err) {
+    constexpr int NV = 1 << D;
+    const int n1 = rule_cnt(1, order);
+    kind = QP_NONE;
+    n = 0;
+    sw = SW_ID;
+    topo = false;
+    const int eldom = straight_cut(vals, NV);
+    if (eldom != IF) {
+      if (eldom == dt) {
+        kind = QP_BOX;
+        n = n1;
+      }
+      return;
+    }
+    L = D == 2 ? ql_quad(vals) : ql_hex(vals);
+    sw = dimension_swap(L, D, pol, true, err);
+    if (D == 3 && (err & ERR_BOUND)) return;
+    if (sw == SW_NONE) {
+      kind = QP_FALLBACK;
+      n = D == 2 ? 2 : 6;
+      return;
+    }
+    if (sw != SW_ID) L = transposed(L, sw);
+    const Box u = unit_box();
+    const int dq = box_check(L, D, u, 0.0);
+    if (dq != IF) {
+      if (dq == dt) {
+        kind = QP_BOX;
+        n = n1;
+      }
+      return;
+    }
+    kind = QP_XI;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      x[k] = 1.0;
+      if (k >= (D == 2 ? 2 : 4)) continue;
+      const int a = D == 2 ? kEdge2[k & 1][0] : kEdge3[k][0], b = D == 2 ? kEdge2[k & 1][1] : kEdge3[k][1];
+      double pa[3], pb[3];
+      box_point(u, D, a, pa);
+      box_point(u, D, b, pb);
+      const double v[2] = {ql_eval(L, pb), ql_eval(L, pa)};
+      if (straight_cut(v, 2) != IF) continue;
+      topo = true;
+      const double t = v[0] / (v[0] - v[1]);
+      const double c = 1.0 + t * (0.0 - 1.0);  // the cut point of the unit line from (1,0,0) to 0
+      if (!isnan(c)) x[k] = c;                   // (a NaN is never inserted into the reference's std::set)
+    }
+    // (equal split points, and those at 0 or 1, give pieces of no length,
+    // which the std::set does not have; they are skipped in run)
+    auto order2 = [](double &p, double &q) {
+      const double lo = fmin(p, q), hi = fmax(p, q);
+      p = lo;
+      q = hi;
+    };
+    order2(x[0], x[1]);
+    order2(x[2], x[3]);
+    order2(x[0], x[2]);
+    order2(x[1], x[3]);
+    order2(x[1], x[2]);
+    n = (topo ? PIECES : 1) * n1;
+  }
+
+  // part `it` of the rule
+  template <class Sink>
+  XG_DEV void run(int it, int dt, int order, int pol, Sink &s, int &err) const {
+    if (kind == QP_FALLBACK) {
+      fallback_rule<D>(L, dt, order, s, err, it, it + 1);
+      return;
+    }
+    const Box u = unit_box();
+    if (kind == QP_BOX) {
+      box_plain(u, D, order, s, it, it + 1);
+      return;
+    }
+    const int n1 = rule_cnt(1, order), pc = it / n1, i1 = it - pc * n1;
+    Box q = u;
+    if (topo) {
+      q.lo[D - 1] = pc == 0 ? 0.0 : (pc == 1 ? x[0] : (pc == 2 ? x[1] : (pc == 3 ? x[2] : x[3])));
+      q.hi[D - 1] = pc == 0 ? x[0] : (pc == 1 ? x[1] : (pc == 2 ? (D == 2 ? 1.0 : x[2]) : (pc == 3 ? x[3] : 1.0)));
+      if (q.lo[D - 1] == q.hi[D - 1]) return;
+      const int ds = box_check(L, D, q, 1e-15);
+      if (ds != IF) {
+        if (ds == dt) box_plain(q, D, order, s, i1, i1 + 1);
+        return;
+      }
+    }
+    tensor_rule<D>(L, q, dt, order, pol, s, err, i1, i1 + 1);
+  }
+};
+
+// Bound: the latency of a part (branches and FP64 chains of one lane).  With a
+// lane per element 5,300 cut hexahedra were 83 waves for 1024 SIMDs, each lane
+// going through all slices: 48^3 hexes, order 4, NEG, count and fill: 1048 -> 153 us (with the matrices 1378 -> 203).
+constexpr int QG = 16;  // lanes per element: 15 parts of a split hexahedron at order 4
 template <int D, bool FILL>
 __global__ __launch_bounds__(256) void k_quad_rule(int nel, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
@@ -613,13 +729,14 @@ __global__ __launch_bounds__(256) void k_quad_rule(int nel, const int32_t *__res
                                                    int32_t *__restrict__ offsets, double4 *__restrict__ pts,
                                                    int32_t *err_flag) {
   constexpr int NV = 1 << D;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int i = (int)(g / QG), sub = threadIdx.x & (QG - 1);
   if (i >= nel) return;
   const int e = elems ? elems[i] : i;
   double vals[NV];
   load_values<D>(el2v, lset, e, vals);
   double V[NV][3];
-  if (FILL) {
+  if (FILL && dt == IF) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int v = el2v[(size_t)e * NV + k];
@@ -627,12 +744,43 @@ __global__ __launch_bounds__(256) void k_quad_rule(int nel, const int32_t *__res
       for (int d = 0; d < 3; ++d) V[k][d] = d < D ? coords[(size_t)v * D + d] : 0.0;
     }
   }
-  const QL L = D == 2 ? ql_quad(vals) : ql_hex(vals);
-  ElemSink<D> s{L, V, FILL ? pts + offsets[i] : nullptr, dt, 0, 0.0};
   int err = 0;
-  element_rule<D>(vals, dt, order, pol, s, err);
+  QuadParts<D> parts;
+  parts.plan(vals, dt, order, pol, err);
+  const QL L = D == 2 ? ql_quad(vals) : ql_hex(vals);
+  const int base = FILL ? offsets[i] : 0;
+  int n = 0;
+  for (int it0 = 0; it0 < parts.n; it0 += QG) {
+    const int it = it0 + sub;
+    int c = 0, pre = 0;
+    // counted first; a fill then knows where its part begins
+#pragma unroll 1
+    for (int pass = 0; pass < (FILL ? 2 : 1); ++pass) {
+      ElemSink<D> s{L, V, pass ? pts + base + n + pre : nullptr, dt, 0, 0.0};
+      if (it < parts.n) {
+        if (parts.sw == SW_ID || parts.sw == SW_NONE) {
+          parts.run(it, dt, order, pol, s, err);
+        } else {
+          SwapSink<ElemSink<D>> ws{parts.sw, s};
+          parts.run(it, dt, order, pol, ws, err);
+        }
+      }
+      if (pass == 0) {
+        c = s.n;
+        int incl = c;
+#pragma unroll
+        for (int o = 1; o < QG; o <<= 1) {
+          const int y = __shfl_up(incl, o, QG);
+          if (sub >= o) incl += y;
+        }
+        pre = incl - c;
+        c = __shfl(incl, QG - 1, QG);
+      }
+    }
+    n += c;
+  }
   if (err) atomicOr(err_flag, err);
-  if (!FILL) offsets[i] = s.n;
+  if (!FILL && sub == 0) offsets[i] = n;
 }
 
 // CutInformation::Update on quads / hexes: order-0 part volumes
@@ -722,8 +870,9 @@ int waves_grid(int nel) {
 }
 
 // SymbolicCutBilinearFormIntegrator::CalcElementMatrix (xfem/symboliccutbfi.cpp:
-// 76-304) for the Q1 space of quads / hexes on a materialised cut rule: one
-// lane per element, its points in turn; out = sum_q |det F| w_q (sm phi_a
+// 76-304) for the Q1 space of quads / hexes on a materialised cut rule: 16
+// lanes per element over its points (one lane per element left most of the
+// device idle: 5,300 hexahedra were 83 waves, 327 us for them at order 4); out = sum_q |det F| w_q (sm phi_a
 // phi_b + sk grad phi_a . grad phi_b), grad phi = F^{-T} grad_ref phi, the
 // upper triangle accumulated in FP64 and mirrored (row = test dof)
 template <int D, typename T>
@@ -734,7 +883,7 @@ __global__ __launch_bounds__(256) void k_quad_elmat(int nel, const int32_t *__re
                                                     const double4 *__restrict__ pts, int mask, T *__restrict__ out) {
   constexpr int NV = 1 << D;
   constexpr int NU = NV * (NV + 1) / 2;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / QG), sub = threadIdx.x & (QG - 1);
   if (i >= nel) return;
   const int e = elems ? elems[i] : i;
   double V[NV][3];
@@ -748,7 +897,8 @@ __global__ __launch_bounds__(256) void k_quad_elmat(int nel, const int32_t *__re
   double A[NU];
 #pragma unroll
   for (int k = 0; k < NU; ++k) A[k] = 0.0;
-  for (int q = offsets[i]; q < offsets[i + 1]; ++q) {
+  const int q1 = offsets[i + 1];
+  for (int q = offsets[i] + sub; q < q1; q += QG) {
     const double4 p = pts[q];
     const double xi[3] = {p.x, p.y, p.z};
     double F[D * D], Finv[D * D], x[3];
@@ -792,21 +942,31 @@ __global__ __launch_bounds__(256) void k_quad_elmat(int nel, const int32_t *__re
         A[u++] += wq * (sm * (phi[a] * phi[b]) + sk * gg);
       }
   }
+  // the sums over the 16 lanes; lane sub keeps the entries k QG + sub
   T *o = out + (size_t)i * NV * NV;
+  constexpr int NK = (NV * NV + QG - 1) / QG;
+  double mine[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) mine[k] = 0.0;
   int u = 0;
 #pragma unroll
   for (int a = 0; a < NV; ++a)
 #pragma unroll
     for (int b = a; b < NV; ++b) {
-      o[a * NV + b] = (T)A[u];
-      o[b * NV + a] = (T)A[u];
-      ++u;
+      double v = A[u++];
+#pragma unroll
+      for (int m = QG / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, QG);
+      if ((a * NV + b) % QG == sub) mine[(a * NV + b) / QG] = v;
+      if ((b * NV + a) % QG == sub) mine[(b * NV + a) / QG] = v;
     }
+#pragma unroll
+  for (int k = 0; k < NK; ++k)
+    if (k * QG + sub < NV * NV) o[k * QG + sub] = (T)mine[k];
 }
 
 // SymbolicCutLinearFormIntegrator (xfem/symboliccutlfi.cpp:57-140) with f = 1
 // for the Q1 space on a materialised quad / hex rule: out_a = sum_q
-// |det F| w_q phi_a(xi_q), one lane per element
+// |det F| w_q phi_a(xi_q), 16 lanes per element
 template <int D>
 __global__ __launch_bounds__(256) void k_quad_elvec(int nel, const int32_t *__restrict__ elems,
                                                     const int32_t *__restrict__ el2v,
@@ -814,7 +974,7 @@ __global__ __launch_bounds__(256) void k_quad_elvec(int nel, const int32_t *__re
                                                     const int32_t *__restrict__ offsets,
                                                     const double4 *__restrict__ pts, double *__restrict__ out) {
   constexpr int NV = 1 << D;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = (int)(((long long)blockIdx.x * 256 + threadIdx.x) / QG), sub = threadIdx.x & (QG - 1);
   if (i >= nel) return;
   const int e = elems ? elems[i] : i;
   double V[NV][3];
@@ -827,7 +987,8 @@ __global__ __launch_bounds__(256) void k_quad_elvec(int nel, const int32_t *__re
   double acc[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-  for (int q = offsets[i]; q < offsets[i + 1]; ++q) {
+  const int q1 = offsets[i + 1];
+  for (int q = offsets[i] + sub; q < q1; q += QG) {
     const double4 p = pts[q];
     const double xi[3] = {p.x, p.y, p.z};
     double F[D * D], x[3];
@@ -846,8 +1007,16 @@ __global__ __launch_bounds__(256) void k_quad_elvec(int nel, const int32_t *__re
     }
   }
 #pragma unroll
-  for (int v = 0; v < NV; ++v) out[(size_t)i * NV + v] = acc[v];
+  for (int v = 0; v < NV; ++v) {
+#pragma unroll
+    for (int m = QG / 2; m > 0; m >>= 1) acc[v] += __shfl_xor(acc[v], m, QG);
+    if (v == sub) out[(size_t)i * NV + v] = acc[v];
+  }
 }
+
+// blocks of 256 for 16 lanes per element
+unsigned quad_grid(int nel) { return (unsigned)(((long long)nel * QG + 255) / 256); }
+
 
 bool quad_args_ok(int D, int dt, int order, int pol) {
   return (D == 2 || D == 3) && dt >= 0 && dt <= 2 && order >= 0 && order / 2 + 1 <= XG_RULE_NMAX && pol >= 0 &&
@@ -865,7 +1034,7 @@ extern "C" int xg_quad_rule_count(xg_ctx *ctx, int D, int nel, const int32_t *el
     XG_CHECK(hipMemsetAsync(offsets, 0, sizeof(int32_t), ctx->stream));
     return XG_OK;
   }
-  const int grid = (nel + 255) / 256;
+  const unsigned grid = quad_grid(nel);
   if (D == 2)
     k_quad_rule<2, false><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, nullptr, lset_v, dt, order, policy,
                                                          offsets, nullptr, ctx->d_err);
@@ -883,7 +1052,7 @@ extern "C" int xg_quad_rule_fill(xg_ctx *ctx, int D, int nel, const int32_t *ele
     return set_error(XG_ERR_ARG, "xg_quad_rule_fill: bad argument");
   if (nel == 0) return XG_OK;
   if (!el2v || !lset_v || !coords || !pts) return set_error(XG_ERR_ARG, "xg_quad_rule_fill: null pointer");
-  const int grid = (nel + 255) / 256;
+  const unsigned grid = quad_grid(nel);
   double4 *o = reinterpret_cast<double4 *>(pts);
   if (D == 2)
     k_quad_rule<2, true><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, policy,
@@ -949,7 +1118,7 @@ extern "C" int xg_quad_elmat(xg_ctx *ctx, int D, int nel, const int32_t *elems, 
     return set_error(XG_ERR_ARG, "xg_quad_elmat: bad argument");
   if (nel == 0) return XG_OK;
   if (!el2v || !coords || !offsets || !pts || !out) return set_error(XG_ERR_ARG, "xg_quad_elmat: null pointer");
-  const int grid = (nel + 255) / 256;
+  const unsigned grid = quad_grid(nel);
   const double4 *p = reinterpret_cast<const double4 *>(pts);
   if (precision == XG_PREC_FP64) {
     if (D == 2) k_quad_elmat<2, double><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, mask, (double *)out);
@@ -967,7 +1136,7 @@ extern "C" int xg_quad_elvec(xg_ctx *ctx, int D, int nel, const int32_t *elems, 
   if (!ctx || (D != 2 && D != 3) || nel < 0) return set_error(XG_ERR_ARG, "xg_quad_elvec: bad argument");
   if (nel == 0) return XG_OK;
   if (!el2v || !coords || !offsets || !pts || !out) return set_error(XG_ERR_ARG, "xg_quad_elvec: null pointer");
-  const int grid = (nel + 255) / 256;
+  const unsigned grid = quad_grid(nel);
   const double4 *p = reinterpret_cast<const double4 *>(pts);
   if (D == 2) k_quad_elvec<2><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, out);
   else k_quad_elvec<3><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, out);

@@ -130,6 +130,34 @@ def test_rule_parity(dev, orc, D, n, kind, pol):
         assert nbad == 0
 
 
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("order", [9, 10, 15])
+def test_rule_parity_many_parts(dev, orc, D, order):
+    """an element's rule is shared out over 16 lanes by its parts (Gauss
+    slices of up to 5 pieces): orders with more than 16, 32 and 48 of them,
+    on curved cuts and on single-cell topology changes"""
+    cases = [(warped(D, 3), None)]
+    if D == 3:
+        cases.append((MakeStructured3DMesh(hexes=True, nx=1, ny=1, nz=1),
+                      np.array([-4, 4, -1, -1, 2, -3, 5, -1], dtype=np.float64)))
+    else:
+        cases.append((MakeStructured2DMesh(quads=True, nx=1, ny=1), np.array([-1.0, 2.0, 3.0, -2.0])))
+    for mesh, lset in cases:
+        lset = level_sets(mesh, "sphere", seed=1) if lset is None else lset
+        for dt in (NEG, POS, IF):
+            rules, bad = oracle_rules(orc, mesh, lset, dt, order, OPTIMAL)
+            ok = sorted(rules)
+            off, pts = gpu_rule(dev, mesh, lset, dt, order, OPTIMAL, elems=ok)
+            for i, e in enumerate(ok):
+                r, got = rules[e], pts[off[i]:off[i + 1]]
+                if r is None:
+                    assert len(got) == 0
+                    continue
+                assert len(got) == len(r[1])
+                assert np.abs(got[:, :3] - r[0]).max() <= 1e-14
+                assert np.abs(got[:, 3] - r[1]).max() <= 1e-14 * max(1.0, np.abs(r[1]).max())
+
+
 def test_rule_parity_tpmc_all_policies(dev, orc):
     """the single-hex TPMC level set (topology change inside the element)"""
     mesh = MakeStructured3DMesh(hexes=True, nx=1, ny=1, nz=1)
