@@ -790,7 +790,8 @@ __host__ __device__ constexpr int sdx_lvl_off(int k) { return ((1 << (3 * k)) - 
 
 // vertices of every node of depth <= 5 in level-5 lattice units (root
 // (32,0,0), (0,32,0), (0,0,32), (0,0,0)), packed x | y << 8 | z << 16
-__global__ void k_sdx_node_verts(uint4 *__restrict__ out) {
+// (lat: the vertices' indices in the lattice of the node's own level, 4 x 16 bits)
+__global__ void k_sdx_node_verts(uint4 *__restrict__ out, uint2 *__restrict__ lat) {
   const int id = blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= SDX_NODES) return;
   int k = 0;
@@ -799,6 +800,13 @@ __global__ void k_sdx_node_verts(uint4 *__restrict__ out) {
   node_vertices(id - sdx_lvl_off(k), k, 1 << SDX_DMAX, W);
   out[id] = make_uint4(pack3(W[0][0], W[0][1], W[0][2]), pack3(W[1][0], W[1][1], W[1][2]),
                        pack3(W[2][0], W[2][1], W[2][2]), pack3(W[3][0], W[3][1], W[3][2]));
+  uint32_t ix[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int sh = SDX_DMAX - k;
+    ix[j] = (uint32_t)lat_index(W[j][0] >> sh, W[j][1] >> sh, W[j][2] >> sh, 1 << k);
+  }
+  lat[id] = make_uint2(ix[0] | (ix[1] << 16), ix[2] | (ix[3] << 16));
 }
 
 // exact degree-2PM moments of every node (minimal exact rule, FP64): one wave
@@ -905,8 +913,9 @@ __host__ __device__ inline size_t sdx_bytes(int L, int nq_vol, int nq_if, int NM
 // LDS of k_sdx_leaves: the vertices, sign and cut parameters of CAP cut leaves
 // (a chunk of the element's list) and the records of their pieces.  p = 3:
 // 19.4 KB, so that the 8 one-wave blocks that its registers allow (2 waves per
-// SIMD) fit in a CU's 160 KB; p <= 2: registers for 4 waves per SIMD and more,
-// so half the leaves.
+// SIMD) fit in a CU's 160 KB; p <= 2: fewer registers and smaller elements,
+// so half the leaves (p = 2: 2 waves too, 135 us of leaves at 20^3 cells, L = 3;
+// held to 3 by its registers 146 us).
 template <int PM>
 struct SdlCap {
   static constexpr int CAP = PM == 3 ? 256 : 128;  // multiples of 64
@@ -1664,8 +1673,10 @@ int launch_subdiv_exact(xg_ctx *ctx, int nel, const int32_t *elems, const double
 // node tables of the exact-rule kernel (once per context and degree)
 int ensure_sdx_tables(xg_ctx *ctx, int PM) {
   if (!ctx->sdx_verts) {
-    XG_CHECK(hipMalloc(&ctx->sdx_verts, sizeof(uint4) * SDX_NODES));
-    k_sdx_node_verts<<<(SDX_NODES + 255) / 256, 256, 0, ctx->stream>>>((uint4 *)ctx->sdx_verts);
+    // (the vertices, then their lattice indices)
+    XG_CHECK(hipMalloc(&ctx->sdx_verts, (sizeof(uint4) + sizeof(uint2)) * SDX_NODES));
+    k_sdx_node_verts<<<(SDX_NODES + 255) / 256, 256, 0, ctx->stream>>>((uint4 *)ctx->sdx_verts,
+                                                                        (uint2 *)((uint4 *)ctx->sdx_verts + SDX_NODES));
     XG_LAUNCH_CHECK();
   }
   if (!ctx->sdx_mom[PM]) {
@@ -1725,14 +1736,13 @@ int subdiv_exact_pass(xg_ctx *ctx, int nel, const int32_t *elems, const double *
 struct SdcLds {
   uint32_t *latbits;  // sign bits (v >= 0) of the finest lattice, lattice order
   uint16_t *rowst;    // (n+1)^2: lattice index of (0, b, c)
-  uint4 *nodeV;       // SDX_CH candidate vertices (level-L units)
-  uint32_t *flags;    // SDX_CH
-  uint16_t *cur, *nxt;
-  uint32_t *latq;     // lattice offsets of levels 0..3
+  uint16_t *cur;      // cut nodes of level L - 2 (paths)
+  uint32_t *latq;     // lattice offsets of levels 0..2
   double *cl;         // 20
-  uint16_t *fq;       // SDX_CH: a chunk's table rows
-  uint16_t *flq;      // SDX_CH: a chunk's leaves flagged cut by their vertex signs
+  uint16_t *fq;       // SDC_FQ: pending table rows
+  uint16_t *flq;      // 128: pending leaves flagged cut by their vertex signs
 };
+constexpr int SDC_FQ = 256;
 
 __host__ __device__ inline size_t sdc_bytes(int L, SdcLds *s, char *base) {
   size_t o = 0;
@@ -1744,23 +1754,17 @@ __host__ __device__ inline size_t sdc_bytes(int L, SdcLds *s, char *base) {
   const int n1 = (1 << L) + 1;
   const size_t a_lb = take(sizeof(uint32_t) * 2 * ((sd_nlat(L) + 63) / 64));
   const size_t a_rs = take(sizeof(uint16_t) * n1 * n1);
-  const size_t a_nv = take(sizeof(uint4) * SDX_CH);
-  const size_t a_fl = take(sizeof(uint32_t) * SDX_CH);
-  const size_t a_cur = take(sizeof(uint16_t) * sd_maxcut(L));
-  const size_t a_nxt = take(sizeof(uint16_t) * sd_maxcut(L));
+  const size_t a_cur = take(sizeof(uint16_t) * (L >= 3 ? 1 << (3 * (L - 2)) : 1));
   const size_t a_lq = take(sizeof(uint32_t) * SDX_LATQ);
   const size_t a_cl = take(sizeof(double) * 20);
-  const size_t a_fq = take(sizeof(uint16_t) * SDX_CH);
-  const size_t a_flq = take(sizeof(uint16_t) * SDX_CH);
+  const size_t a_fq = take(sizeof(uint16_t) * SDC_FQ);
+  const size_t a_flq = take(sizeof(uint16_t) * 128);
   if (s) {
     s->fq = (uint16_t *)(base + a_fq);
     s->flq = (uint16_t *)(base + a_flq);
     s->latbits = (uint32_t *)(base + a_lb);
     s->rowst = (uint16_t *)(base + a_rs);
-    s->nodeV = (uint4 *)(base + a_nv);
-    s->flags = (uint32_t *)(base + a_fl);
     s->cur = (uint16_t *)(base + a_cur);
-    s->nxt = (uint16_t *)(base + a_nxt);
     s->latq = (uint32_t *)(base + a_lq);
     s->cl = (double *)(base + a_cl);
   }
@@ -1773,21 +1777,6 @@ __device__ __forceinline__ int lat_index_rs(const uint16_t *rowst, int a, int b,
   return (int)rowst[c * (n + 1) + b] + a;
 }
 
-// q / d for 0 <= q < 2^24, d >= 1 (float estimate, one correction step)
-__device__ __forceinline__ int small_div(int q, int d, float rd, int &rem) {
-  int c = (int)((float)q * rd);
-  int t = q - c * d;
-  if (t >= d) {
-    ++c;
-    t -= d;
-  } else if (t < 0) {
-    --c;
-    t += d;
-  }
-  rem = t;
-  return c;
-}
-
 __global__ void k_zero_i32(int32_t *p) { *p = 0; }
 
 // next element of a persistent wave: lane 0 takes it from the work counter
@@ -1797,9 +1786,23 @@ __device__ __forceinline__ int next_item(int32_t *queue, int lane) {
   return __shfl(nx, 0, 64);
 }
 
-// SIDE: NEG or POS (the uncut nodes of that side: their table rows are
-// summed here, lane-parallel over the moments, and written to out), or -1
-// (cut leaves only)
+// The walk.  SIDE: NEG or POS (the uncut nodes of that side: their table rows
+// are summed here, lane-parallel over the moments, and written to out), or -1
+// (cut leaves only).
+//
+// A node's lattice check (xintegration.cpp:617-752) looks at the lattice points
+// of its subtree, which are the vertices of its leaves; so the check of a node
+// is the OR of its leaves' sign flags, and nothing but the leaves' four bits has
+// to be looked up.  The nodes of level A = L - 2 are checked one per lane on
+// their 35 points, their ancestors follow by ballots; every cut one has 64 leaves,
+// one per lane, whose parents (a byte of the ballots each) follow the same way.
+// (Checking level by level from the root, every candidate on all its lattice
+// points, took 165 + 35 + 10 + 4 lookups on the way to a leaf.)  Leaves with both
+// signs are collected and checked on their values 64 at a time, table rows are
+// collected and summed in batches.  Bound: VALU issue (969 P2 evaluations, then
+// about 22 x 64 leaves at L = 4).  128^3 cells, L = 4:
+// 6.15 -> 5.32 ms for 405,341 elements (the step 27.0 -> 24.7 ms); 20^3 cells,
+// L = 3: 71 -> 56 us (245 -> 225 us).
 template <int LO, int PM, int SIDE>
 __global__ __launch_bounds__(64) void k_sdx_tree(int nel, const int32_t *__restrict__ elems,
                                                  const double *__restrict__ lset_nodal, int L,
@@ -1813,11 +1816,15 @@ __global__ __launch_bounds__(64) void k_sdx_tree(int nel, const int32_t *__restr
   extern __shared__ char smem[];
   SdcLds S;
   sdc_bytes(L, &S, smem);
+  const uint2 *__restrict__ nlat_ix = reinterpret_cast<const uint2 *>(nverts + SDX_NODES);
   const int lane = threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
   const int n = 1 << L;
   const int nlat = sd_nlat(L);
   const int loff = xg_lat_off_d[L];
   const int shift = SDX_DMAX - L;
+  const int A = L >= 2 ? L - 2 : 0;              // level of the groups' top nodes
+  const int GL = L >= 2 ? 64 : (L == 1 ? 8 : 1);  // leaves of a group
   for (int k = lane; k < SDX_LATQ; k += 64) S.latq[k] = xg_lat_d[k];
   for (int k = lane; k < (n + 1) * (n + 1); k += 64) {
     const int c = k / (n + 1), b = k - c * (n + 1);
@@ -1850,222 +1857,164 @@ __global__ __launch_bounds__(64) void k_sdx_tree(int nel, const int32_t *__restr
         S.latbits[(q0 >> 5) + 1] = (uint32_t)(b >> 32);
       }
     }
+    wave_sync();
     uint16_t *lst = lists + (size_t)i * cap;
     // table-row sums of the kept side: moments lane and lane + 64 (16-byte
     // loads of a few rows per instruction measured slower here: registers)
     double ta = 0.0, tb = 0.0;
     int nl = 0, nf = 0, n22 = 0;
+    int nrow = 0, nflag = 0;  // pending in S.fq, S.flq
     bool ok = true, overflow = false;
-    int dom = -1;
-    int ncur = 1;
-    wave_sync();
-    for (int k = 0; k <= L && ncur > 0 && !overflow; ++k) {
-      const int r = L - k;
-      const int ncand = (k == 0) ? 1 : 8 * ncur;
-      const int np = xg_lat_cnt_d[r], poff = xg_lat_off_d[r];
-      const float rnp = 1.0f / (float)np;
-      const int koff = sdx_lvl_off(k);
-      int nnxt = 0;
-      for (int cbase = 0; cbase < ncand && !overflow; cbase += SDX_CH) {
-        const int nc = min(SDX_CH, ncand - cbase);
-        for (int c = lane; c < nc; c += 64) {
-          const int gc = cbase + c;
-          const int path = (k == 0) ? 0 : (int)S.cur[gc >> 3] * 8 + (gc & 7);
-          S.nodeV[c] = nverts[koff + path];
-          S.flags[c] = 0u;
+    const int dom = rootf == 3u ? IF : (rootf == 1u ? POS : NEG);
+    constexpr uint32_t KEEP = SIDE == POS ? 1u : 2u;  // flags of an uncut node of the kept side
+    // adds the pending rows, four per round trip
+    auto flush_rows = [&]() {
+      wave_sync();
+      int f = 0;
+      for (; f + 4 <= nrow; f += 4) {
+        const size_t r0 = (size_t)S.fq[f] * NM, r1 = (size_t)S.fq[f + 1] * NM;
+        const size_t r2 = (size_t)S.fq[f + 2] * NM, r3 = (size_t)S.fq[f + 3] * NM;
+        if (lane < NM) ta += (nmom[r0 + lane] + nmom[r1 + lane]) + (nmom[r2 + lane] + nmom[r3 + lane]);
+        if (lane + 64 < NM)
+          tb += (nmom[r0 + 64 + lane] + nmom[r1 + 64 + lane]) + (nmom[r2 + 64 + lane] + nmom[r3 + 64 + lane]);
+      }
+      for (; f < nrow; ++f) {
+        const size_t r0 = (size_t)S.fq[f] * NM;
+        if (lane < NM) ta += nmom[r0 + lane];
+        if (lane + 64 < NM) tb += nmom[r0 + 64 + lane];
+      }
+      nf += nrow;
+      nrow = 0;
+      wave_sync();
+    };
+    auto add_row = [&](bool want, int row) {
+      const unsigned long long b = __ballot(want);
+      if (want) S.fq[nrow + __popcll(b & below)] = (uint16_t)row;
+      nrow += __popcll(b);
+    };
+    // the rows of a group: lanes = nodes of level l (flags f, ballots b1 of
+    // nonnegative, b2 of negative ones) with number `node`; with 64 of them a
+    // byte is a node of level l - 1, which takes its children's place when it
+    // is uncut (the group's top node is cut)
+    auto group_rows = [&](uint32_t f, unsigned long long b1, unsigned long long b2, bool whole, bool valid, int l,
+                          int node) {
+      if constexpr (SIDE >= 0) {
+        const int sh = lane & 56;
+        const bool pcut = !whole || (((b1 >> sh) & 255ull) != 0ull && ((b2 >> sh) & 255ull) != 0ull);
+        add_row(valid && pcut && f == KEEP, sdx_lvl_off(l) + node);
+        if (whole) add_row(!pcut && (lane & 7) == 0 && f == KEEP, sdx_lvl_off(l - 1) + (node >> 3));
+        if (nrow > SDC_FQ - 144) flush_rows();
+      }
+    };
+    // Simplex::CheckIfCut on the vertex values of up to 64 pending leaves
+    auto check_leaves = [&](int m) {
+      wave_sync();
+      const bool valid = lane < m;
+      int lc = -2, path = 0;
+      bool lc22 = false;
+      if (valid) {
+        path = S.flq[lane];
+        int W[4][3];
+        unpack_uint4(nverts[sdx_lvl_off(L) + path], shift, W);
+        double vv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const double x[3] = {(double)W[j][0] * inv_n, (double)W[j][1] * inv_n, (double)W[j][2] * inv_n};
+          vv[j] = lagrange_eval3<LO>(cl, x);
         }
-        wave_sync();
-        // lattice checks above the leaves.  Up to 35 lattice points per
-        // candidate (r <= 2): one lane per candidate walks them.  More: the
-        // sign bits of every (candidate, lattice point) pair, OR-ed per
-        // candidate with ballots (the pairs of one pass cover consecutive
-        // candidates)
-        if (k == 0 && r > 0) {
-          if (lane == 0) S.flags[0] = rootf;
-          wave_sync();
-        } else if (r > 0 && r <= 2) {
-          for (int c = lane; c < nc; c += 64) {
+        lc = leaf_check(vv);
+        if (lc < 0) ok = false;
+        // two vertices on each side (zero counts POS): a 2-2 cut leaf
+        int npos = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) npos += vv[j] >= 0.0 ? 1 : 0;
+        if (lc == IF && npos == 2) lc22 = true;
+      }
+      const bool leafcut = valid && lc == IF;
+      int cl2;
+      const int sl = wave_slot(leafcut, nl, lane, cl2);
+      // room for the cut leaves and their complements
+      if (2 * (nl + cl2) > cap) {
+        overflow = true;
+        return;
+      }
+      if (leafcut) lst[sl] = (uint16_t)(sdx_lvl_off(L) + path);
+      nl += cl2;
+      n22 += __popcll(__ballot(lc22));
+      if constexpr (SIDE >= 0) add_row(valid && lc == SIDE, sdx_lvl_off(L) + path);
+      // the leaves after the first 64 move up
+      const uint16_t rest = (64 + lane < nflag) ? S.flq[64 + lane] : 0;
+      wave_sync();
+      S.flq[lane] = rest;
+      nflag = nflag > 64 ? nflag - 64 : 0;
+      wave_sync();
+    };
+    if (rootf != 3u) {
+      if constexpr (SIDE >= 0) add_row(lane == 0 && rootf == KEEP, 0);
+    } else {
+      int ncur = 1;
+      if (A == 0) {
+        if (lane == 0) S.cur[0] = 0;
+      } else {
+        ncur = 0;
+        const int na = 1 << (3 * A), np = xg_lat_cnt_d[2], poff = xg_lat_off_d[2];
+        for (int a0 = 0; a0 < na; a0 += 64) {
+          const int a = a0 + lane;
+          const bool valid = a < na;
+          uint32_t f = 0u;
+          if (valid) {
             int W[4][3];
-            unpack_uint4(S.nodeV[c], shift, W);
+            unpack_uint4(nverts[sdx_lvl_off(A) + a], shift, W);
             int E[3][3];
 #pragma unroll
             for (int m = 0; m < 3; ++m)
 #pragma unroll
               for (int d = 0; d < 3; ++d) E[m][d] = W[m + 1][d] - W[0][d];
-            uint32_t f = 0u;
             for (int t = 0; t < np; ++t) {
               const unsigned pk = S.latq[poff + t];
               const int I0 = (int)(pk & 255u), I1 = (int)((pk >> 8) & 255u), I2 = (int)(pk >> 16);
               int P[3];
 #pragma unroll
-              for (int d = 0; d < 3; ++d) P[d] = W[0][d] + ((I0 * E[0][d] + I1 * E[1][d] + I2 * E[2][d]) >> r);
-              f |= lat_bit(S.latbits, lat_index_rs(S.rowst, P[0], P[1], P[2], n)) ? 1u : 2u;
-            }
-            S.flags[c] = f;
-          }
-          wave_sync();
-        } else if (r > 0 && nc <= 8) {
-          // a few candidates with many lattice points: 8 lanes per candidate
-          const int cand = lane >> 3, sub = lane & 7;
-          uint32_t f = 0u;
-          if (cand < nc) {
-            int W[4][3];
-            unpack_uint4(S.nodeV[cand], shift, W);
-            int E[3][3];
-#pragma unroll
-            for (int m = 0; m < 3; ++m)
-#pragma unroll
-              for (int d = 0; d < 3; ++d) E[m][d] = W[m + 1][d] - W[0][d];
-            for (int t = sub; t < np; t += 8) {
-              const unsigned pk = (r <= 3) ? S.latq[poff + t] : xg_lat_d[poff + t];
-              const int I0 = (int)(pk & 255u), I1 = (int)((pk >> 8) & 255u), I2 = (int)(pk >> 16);
-              int P[3];
-#pragma unroll
-              for (int d = 0; d < 3; ++d) P[d] = W[0][d] + ((I0 * E[0][d] + I1 * E[1][d] + I2 * E[2][d]) >> r);
+              for (int d = 0; d < 3; ++d) P[d] = W[0][d] + ((I0 * E[0][d] + I1 * E[1][d] + I2 * E[2][d]) >> 2);
               f |= lat_bit(S.latbits, lat_index_rs(S.rowst, P[0], P[1], P[2], n)) ? 1u : 2u;
             }
           }
-          for (int cc = 0; cc < nc; ++cc) {
-            const unsigned long long b1 = __ballot(cand == cc && (f & 1u));
-            const unsigned long long b2 = __ballot(cand == cc && (f & 2u));
-            if (lane == 0) S.flags[cc] = (b1 ? 1u : 0u) | (b2 ? 2u : 0u);
+          const unsigned long long b1 = __ballot((f & 1u) != 0u), b2 = __ballot((f & 2u) != 0u);
+          if (A == 3 && (b1 == 0ull || b2 == 0ull)) {
+            // the level-1 node above these 64 is uncut
+            if constexpr (SIDE >= 0) add_row(lane == 0 && f == KEEP, sdx_lvl_off(1) + (a0 >> 6));
+            continue;
           }
-          wave_sync();
-        } else if (r > 0) {
-          const int npairs = nc * np;
-          for (int q0 = 0; q0 < npairs; q0 += 64) {
-            const int q = q0 + lane;
-            int c = -1;
-            uint32_t bit = 0u;
-            if (q < npairs) {
-              int t;
-              c = small_div(q, np, rnp, t);
-              const unsigned pk = (r <= 3) ? S.latq[poff + t] : xg_lat_d[poff + t];
-              const int I0 = (int)(pk & 255u), I1 = (int)((pk >> 8) & 255u), I2 = (int)(pk >> 16);
-              int W[4][3];
-              unpack_uint4(S.nodeV[c], shift, W);
-              int P[3];
-#pragma unroll
-              for (int d = 0; d < 3; ++d)
-                P[d] = W[0][d] + ((I0 * (W[1][d] - W[0][d]) + I1 * (W[2][d] - W[0][d]) + I2 * (W[3][d] - W[0][d])) >> r);
-              bit = lat_bit(S.latbits, lat_index_rs(S.rowst, P[0], P[1], P[2], n)) ? 1u : 2u;
-            }
-            int trem;
-            const int c_lo = small_div(q0, np, rnp, trem);
-            const int qhi = min(q0 + 63, npairs - 1);
-            const int c_hi = small_div(qhi, np, rnp, trem);
-            for (int cc = c_lo; cc <= c_hi; ++cc) {
-              const unsigned long long b1 = __ballot(c == cc && bit == 1u);
-              const unsigned long long b2 = __ballot(c == cc && bit == 2u);
-              if (lane == 0) S.flags[cc] |= (b1 ? 1u : 0u) | (b2 ? 2u : 0u);
-            }
-          }
-          wave_sync();
+          group_rows(f, b1, b2, A >= 2, valid, A, a);
+          int cn;
+          const int sn = wave_slot(f == 3u, ncur, lane, cn);
+          if (f == 3u) S.cur[sn] = (uint16_t)a;
+          ncur += cn;
         }
-        // classification and the lists
-        int nfc = 0;    // this chunk's table rows (S.fq)
-        int nflag = 0;  // this chunk's leaves to check on their values (S.flq)
-        for (int c0 = 0; c0 < nc; c0 += 64) {
-          const int c = c0 + lane;
-          const bool valid = c < nc;
-          int W[4][3] = {};
-          if (valid) unpack_uint4(S.nodeV[c], shift, W);
-          uint32_t f = 0u;
-          if (valid) {
-            if (r > 0) f = S.flags[c];
-            else
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                f |= lat_bit(S.latbits, lat_index_rs(S.rowst, W[j][0], W[j][1], W[j][2], n)) ? 1u : 2u;
-          }
-          const int cls = (f == 3u) ? IF : ((f == 1u) ? POS : NEG);
-          if (k == 0) dom = __shfl(cls, 0, 64);
-          // leaves whose vertex signs differ are checked on their values in a
-          // second, dense pass (flq)
-          const int path = (k == 0 || !valid) ? 0 : (int)S.cur[(cbase + c) >> 3] * 8 + ((cbase + c) & 7);
-          const bool wantfill = SIDE >= 0 && valid && cls == SIDE;
-          const bool flagged = valid && cls == IF && r == 0;
-          const bool wantnext = valid && cls == IF && r > 0;
-          int cf, cg, cn;
-          const int sf = wave_slot(wantfill, nfc, lane, cf);
-          const int sg = wave_slot(flagged, nflag, lane, cg);
-          const int sn = wave_slot(wantnext, nnxt, lane, cn);
-          if (wantfill) S.fq[sf] = (uint16_t)(koff + path);
-          if (flagged) S.flq[sg] = (uint16_t)c;
-          if (wantnext) S.nxt[sn] = (uint16_t)path;
-          nfc += cf;
-          nflag += cg;
-          nnxt += cn;
-        }
-        wave_sync();
-        // the flagged leaves: Simplex::CheckIfCut on the vertex values
-        for (int q0 = 0; q0 < nflag && !overflow; q0 += 64) {
-          const int q = q0 + lane;
-          const bool valid = q < nflag;
-          int lc = -2;
-          bool lc22 = false;
-          int path = 0;
-          if (valid) {
-            const int c = S.flq[q];
-            path = (k == 0) ? 0 : (int)S.cur[(cbase + c) >> 3] * 8 + ((cbase + c) & 7);
-            int W[4][3];
-            unpack_uint4(S.nodeV[c], shift, W);
-            double vv[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const double x[3] = {(double)W[j][0] * inv_n, (double)W[j][1] * inv_n, (double)W[j][2] * inv_n};
-              vv[j] = lagrange_eval3<LO>(cl, x);
-            }
-            lc = leaf_check(vv);
-            if (lc < 0) ok = false;
-            // two vertices on each side (zero counts POS): a 2-2 cut leaf
-            int npos = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) npos += vv[j] >= 0.0 ? 1 : 0;
-            if (lc == IF && npos == 2) lc22 = true;
-          }
-          const bool wantfill = SIDE >= 0 && valid && lc == SIDE;
-          const bool leafcut = valid && lc == IF;
-          int cf, cl2;
-          const int sf = wave_slot(wantfill, nfc, lane, cf);
-          const int sl = wave_slot(leafcut, nl, lane, cl2);
-          // room for the cut leaves and their complements
-          if (2 * (nl + cl2) > cap) {
-            overflow = true;
-            break;
-          }
-          if (wantfill) S.fq[sf] = (uint16_t)(koff + path);
-          if (leafcut) lst[sl] = (uint16_t)(koff + path);
-          nfc += cf;
-          nl += cl2;
-          n22 += __popcll(__ballot(lc22));
-        }
-        wave_sync();
-        // the chunk's table rows, four per round trip
-        if constexpr (SIDE >= 0) {
-          if (!overflow) {
-            int f = 0;
-            for (; f + 4 <= nfc; f += 4) {
-              const size_t r0 = (size_t)S.fq[f] * NM, r1 = (size_t)S.fq[f + 1] * NM;
-              const size_t r2 = (size_t)S.fq[f + 2] * NM, r3 = (size_t)S.fq[f + 3] * NM;
-              if (lane < NM) ta += (nmom[r0 + lane] + nmom[r1 + lane]) + (nmom[r2 + lane] + nmom[r3 + lane]);
-              if (lane + 64 < NM)
-                tb += (nmom[r0 + 64 + lane] + nmom[r1 + 64 + lane]) + (nmom[r2 + 64 + lane] + nmom[r3 + 64 + lane]);
-            }
-            for (; f < nfc; ++f) {
-              const size_t r0 = (size_t)S.fq[f] * NM;
-              if (lane < NM) ta += nmom[r0 + lane];
-              if (lane + 64 < NM) tb += nmom[r0 + 64 + lane];
-            }
-          }
-          wave_sync();
-        }
-        nf += nfc;
       }
-      uint16_t *tmp = S.cur;
-      S.cur = S.nxt;
-      S.nxt = tmp;
-      ncur = nnxt;
+      wave_sync();
+      for (int g = 0; g < ncur && !overflow; ++g) {
+        const int path = (int)S.cur[g] * GL + lane;
+        const bool valid = lane < GL;
+        uint32_t f = 0u;
+        if (valid) {
+          const uint2 ix = nlat_ix[sdx_lvl_off(L) + path];
+          const bool s0 = lat_bit(S.latbits, (int)(ix.x & 0xffffu)), s1 = lat_bit(S.latbits, (int)(ix.x >> 16));
+          const bool s2 = lat_bit(S.latbits, (int)(ix.y & 0xffffu)), s3 = lat_bit(S.latbits, (int)(ix.y >> 16));
+          f = ((s0 || s1 || s2 || s3) ? 1u : 0u) | ((s0 && s1 && s2 && s3) ? 0u : 2u);
+        }
+        const unsigned long long b1 = __ballot((f & 1u) != 0u), b2 = __ballot((f & 2u) != 0u);
+        group_rows(f, b1, b2, L >= 2, valid, L, path);
+        int cf;
+        const int sf = wave_slot(f == 3u, nflag, lane, cf);
+        if (f == 3u) S.flq[sf] = (uint16_t)path;
+        nflag += cf;
+        if (nflag >= 64) check_leaves(64);
+      }
+      if (nflag > 0 && !overflow) check_leaves(nflag);
+    }
+    if constexpr (SIDE >= 0) {
+      if (!overflow) flush_rows();
     }
     const bool allok = __ballot(!ok) == 0ull;
     if (lane == 0) {
@@ -2110,9 +2059,9 @@ __global__ __launch_bounds__(64) void k_sdx_tree(int nel, const int32_t *__restr
 // cut parameters; the pieces by pattern from a table), then its pieces run;
 // so the piece phase holds no sums and a piece reads its four corners only.
 // 128^3 cells, 405,341 elements, p = 3, L = 4, NEG + IF: the whole step 51.6 ->
-// 27.0 ms; 20^3, p = 2, L = 3: 400 -> 245 us.
+// 27.0 ms; 20^3, p = 2, L = 3: 400 -> 245 us (with the walk as it was).
 template <int LO, int PM, int SIDE, int WHICH>
-__global__ __launch_bounds__(64, 2) void k_sdx_leaves(int nel, const int32_t *__restrict__ elems,
+__global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, const int32_t *__restrict__ elems,
                                                      const double *__restrict__ lset_nodal,
                                                      const int32_t *__restrict__ el2v,
                                                      const double *__restrict__ coords,

@@ -122,6 +122,25 @@ def test_pipeline_leaf_chunks(orc, dev, p, dts):
         assert np.all(np.abs(got - ref) <= 1e-12 * scale), (L, dts)
 
 
+@pytest.mark.parametrize("L", [0, 1, 2, 3, 4, 5])
+def test_pipeline_walk_levels(orc, dev, L):
+    """the walk at every depth: no level above the leaf groups (L <= 2), one
+    ballot of nodes (3, 4), several (5); a small sphere keeps whole subtrees
+    uncut on either side, the quadrics cut nearly all"""
+    torch, _abi, ctx = dev
+    mesh = MakeStructured3DMesh(nx=2)
+    sphere = p2_values(mesh, np.array([[0.45, 0.52, 0.5]]), np.array([0.21]))
+    elems = np.arange(0, mesh.ne, 3, dtype=np.int32)
+    dts = [NEG, POS, IF]
+    vol = 1.0 / mesh.ne  # bounds every mass entry; the stiffness ones by their scale
+    for vals in (sphere, -sphere, W.random_quadric_p2(mesh.ne, seed=9)):
+        got = run_pipeline(dev, 1, L, elems, mesh, vals, dts, _abi.XG_PREC_FP64)
+        ref = orc.subdiv_pipeline(1, L, 2, elems, mesh.el2v, mesh.coords, vals, dts, 3, nthreads=8)
+        ref = np.asarray(ref).reshape(got.shape)
+        scale = np.maximum(np.abs(ref).max(axis=(-2, -1), keepdims=True), vol)
+        assert np.all(np.abs(got - ref) <= 1e-12 * scale), L
+
+
 def test_pipeline_zero_lattice_values(orc, dev):
     """a P2 level set that vanishes on whole lattice planes of a cut element
     (x * (y - h) with h = 2^-L on the reference tet): zero values count as
