@@ -70,13 +70,18 @@ __global__ void k_rule_count(int nel, const int32_t *__restrict__ elems, const i
 //     one, its sign mask, cut parameters and interface factor;
 //  B. the uncut elements with points: lanes over (element, base point) pairs,
 //     so every lane stores whatever the rule's length;
-//  C. the cut elements in turn: the vertices and volumes of the sub-simplices
-//     are computed by a few lanes into LDS, then lanes = points.
+//  C. the sub-simplices of all cut elements in one list, FILL_SUB at a time:
+//     lane = sub-simplex for the vertices and the volume (into LDS), then lanes
+//     over (sub-simplex, base point) pairs.
 // Bound: the stores (32 B a point).  With one wave per element every element
 // without points cost a wave its whole chain of dependent gathers, an uncut
 // one filled 27 of 64 lanes at order 4, and the decomposition's indexed
-// private arrays lived in scratch memory (rule, coefficient, matrices and
-// vectors on 40^3 cells, order 6: 856 -> 728 us).
+// private arrays lived in scratch memory (353 us at 64^3 cells, order 4); with
+// the cut elements of a run in turn, each with its own chain of table, LDS and
+// point loads, 157 us; now 101 us for 349 MB.  (Pairs of lanes writing whole
+// lines, half a point each: no fewer bytes written, 105 us.)
+constexpr int FILL_SUB = 32;
+
 template <int D>
 __global__ __launch_bounds__(256) void k_rule_fill(int nel, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
@@ -85,7 +90,10 @@ __global__ __launch_bounds__(256) void k_rule_fill(int nel, const int32_t *__res
                                                    const int32_t *__restrict__ offsets,
                                                    double4 *__restrict__ out) {
   __shared__ int32_t s_base[4][64];
-  __shared__ double s_V[4][3][4][3];  // sub-simplex vertices (mapping order)
+  __shared__ uint8_t s_item[4][192];         // sub-simplices of the run: 4 x lane of the element + number
+  __shared__ double s_V[4][FILL_SUB][13];    // vertices (mapping order; 4 x 3, one of padding)
+  __shared__ double2 s_w[4][FILL_SUB];       // volume, interface factor
+  __shared__ int2 s_out[4][FILL_SUB];        // first point, points
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const long long wid = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);
   const long long nwaves = (long long)gridDim.x * 4;
@@ -143,75 +151,156 @@ __global__ __launch_bounds__(256) void k_rule_fill(int nel, const int32_t *__res
       }
       ecore::wave_sync();
     }
-    for (unsigned long long m = mc; m; m &= m - 1) {
-      const int src = __builtin_ctzll(m);
-      const DecompEntry &E = xg_decomp_d.e[D - 1][dt][__builtin_amdgcn_readlane(msk, src)];
-      const int nv = E.nv, ns = E.ns;
-      const int cbase = __builtin_amdgcn_readlane(base, src), cnp = min(__builtin_amdgcn_readlane(npts, src), ns * nq);
-      const double t0 = __shfl(t[0], src, 64), t1 = __shfl(t[1], src, 64), t2 = __shfl(t[2], src, 64),
-                   t3 = __shfl(t[3], src, 64), cif = __shfl(ifac, src, 64);
-      if (lane < ns * nv) {
-        const int s = lane / nv, q = lane - s * nv;
-        const int code = E.v[s][q], c = code - (D + 1);
-        const int a = c >= 0 ? E.ce[c][0] : code, b = c >= 0 ? E.ce[c][1] : code;
-        const double tc = c == 1 ? t1 : (c == 2 ? t2 : (c == 3 ? t3 : t0));
+    if (mc) {
+      const DecompEntry *tab = xg_decomp_d.e[D - 1][dt];
+      const int ns = cut ? tab[msk].ns : 0;
+      const unsigned long long below = (1ull << lane) - 1ull;
+      const unsigned long long n1 = __ballot(ns > 0), n2 = __ballot(ns > 1), n3 = __ballot(ns > 2);
+      const int pos = __popcll(n1 & below) + __popcll(n2 & below) + __popcll(n3 & below);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const double pa = (d == a && a < D) ? 1.0 : 0.0, pb = (d == b && b < D) ? 1.0 : 0.0;
-          s_V[wv][s][q][d] = c >= 0 ? pa + tc * (pb - pa) : pa;
+      for (int s = 0; s < 3; ++s)
+        if (s < ns) s_item[wv][pos + s] = (uint8_t)(4 * lane + s);
+      ecore::wave_sync();
+      const int nsub = __popcll(n1) + __popcll(n2) + __popcll(n3);
+      for (int b0 = 0; b0 < nsub; b0 += FILL_SUB) {
+        const int nb = min(FILL_SUB, nsub - b0);
+        const int item = lane < nb ? s_item[wv][b0 + lane] : 0;
+        const int src = item >> 2, sub = item & 3;
+        const double t0 = __shfl(t[0], src, 64), t1 = __shfl(t[1], src, 64), t2 = __shfl(t[2], src, 64),
+                     t3 = __shfl(t[3], src, 64), cif = __shfl(ifac, src, 64);
+        const int smsk = __shfl(msk, src, 64), sbase = __shfl(base, src, 64), snp = __shfl(npts, src, 64);
+        if (lane < nb) {
+          const DecompEntry &E = tab[smsk];
+          double W[4][3];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (q > Ds) break;
+            const int code = E.v[sub][q], c = code - (D + 1);
+            const int a = c >= 0 ? E.ce[c][0] : code, b = c >= 0 ? E.ce[c][1] : code;
+            const double tc = c == 1 ? t1 : (c == 2 ? t2 : (c == 3 ? t3 : t0));
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+              const double pa = (d == a && a < D) ? 1.0 : 0.0, pb = (d == b && b < D) ? 1.0 : 0.0;
+              W[q][d] = c >= 0 ? pa + tc * (pb - pa) : pa;
+              s_V[wv][lane][3 * q + d] = W[q][d];
+            }
+          }
+          s_w[wv][lane] = make_double2(simplex_measure(Ds, W), cif);
+          s_out[wv][lane] = make_int2(sbase + sub * nq, min(snp - sub * nq, nq));
         }
+        ecore::wave_sync();
+        const int total = nb * nq;
+        for (int g = lane; g < total; g += 64) {
+          const int s = small_div(g, nq, rnq), k = g - s * nq;
+          const int2 o = s_out[wv][s];
+          if (k >= o.y) continue;
+          const double *r = xg_rule_data_d[off + k];
+          const double *W = s_V[wv][s];
+          double ow = 1.0;
+#pragma unroll
+          for (int q = 0; q < D; ++q)
+            if (q < Ds) ow -= r[q];
+          double x[3];
+#pragma unroll
+          for (int d = 0; d < 3; ++d) x[d] = ow * W[d];
+#pragma unroll
+          for (int q = 0; q < D; ++q)
+            if (q < Ds)
+#pragma unroll
+              for (int d = 0; d < 3; ++d) x[d] += r[q] * W[3 * (q + 1) + d];
+          const double2 tw = s_w[wv][s];
+          double w = r[3] * tw.x;
+          if (dt == IF) w = w * tw.y;
+          out[o.x + k] = make_double4(x[0], x[1], x[2], w);
+        }
+        ecore::wave_sync();
       }
-      ecore::wave_sync();
-      double tf[3];
-#pragma unroll
-      for (int s = 0; s < 3; ++s) tf[s] = s < ns ? simplex_measure(nv - 1, s_V[wv][s]) : 0.0;
-      for (int g = lane; g < cnp; g += 64) {
-        const int s = small_div(g, nq, rnq), k = g - s * nq;
-        const double *r = xg_rule_data_d[off + k];
-        const double(*W)[3] = s_V[wv][s];
-        double ow = 1.0;
-#pragma unroll
-        for (int q = 0; q < D; ++q)
-          if (q < Ds) ow -= r[q];
-        double x[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) x[d] = ow * W[0][d];
-#pragma unroll
-        for (int q = 0; q < D; ++q)
-          if (q < Ds)
-#pragma unroll
-            for (int d = 0; d < 3; ++d) x[d] += r[q] * W[q + 1][d];
-        double w = r[3] * (s == 0 ? tf[0] : (s == 1 ? tf[1] : tf[2]));
-        if (dt == IF) w = w * cif;
-        out[cbase + g] = make_double4(x[0], x[1], x[2], w);
-      }
-      ecore::wave_sync();
     }
   }
 }
 
-// G lanes per element.  A wave per element ran most of its lanes on nothing
-// (27 points in 64 lanes, no points at all in the elements outside), and its
-// one atomic add per wave queued up on the single address of the total:
+// adds the points q, q + G, .. (NP of them) below q1 to s, in this order.  A
+// term's coefficient and exponents are scalar loads at addresses that depend on
+// the loop, about 300 cycles each time, so a term is taken for NP points at once
+template <int D, int G, int NP>
+__device__ __forceinline__ double integrate_points(int q, int q1, const double *V, const double *F, double absdet,
+                                                   const double4 *__restrict__ pts, const Poly &f, double s) {
+  double x[NP][3], w[NP], fv[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const double4 p = q + i * G < q1 ? pts[q + i * G] : make_double4(0.0, 0.0, 0.0, 0.0);
+    const double xi[3] = {p.x, p.y, p.z};
+    w[i] = p.w;
+    fv[i] = 0.0;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) x[i][r] = 0.0;
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+      double a = V[r];
+#pragma unroll
+      for (int c = 0; c < D; ++c) a += F[r * D + c] * xi[c];
+      x[i][r] = a;
+    }
+  }
+  for (int t = 0; t < f.n; ++t) {
+    const double c = f.c[t];
+    const int ex[3] = {f.ex[t][0], f.ex[t][1], f.ex[t][2]};
+    double m[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) m[i] = c;
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      for (int j = 0; j < ex[d]; ++j)
+#pragma unroll
+        for (int i = 0; i < NP; ++i) m[i] *= x[i][d];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) fv[i] += m[i];
+  }
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (q + i * G < q1) s += absdet * w[i] * fv[i];
+  return s;
+}
+
+// A wave takes epw (a power of two, 64 / G <= epw <= INT_EPW) consecutive
+// elements: lane = element for the gathers and the map (into LDS), then G lanes
+// per element that has points.  A wave per element ran most of its lanes on
+// nothing (27 points in 64 lanes, no points at all in the elements outside),
+// and its one atomic add per wave queued up on the single address of the total:
 // 262,144 adds took 3.16 ms at 64^3 cells, order 4.  Here a block adds its
-// waves' sums in LDS and at most 1024 blocks run, so the adds are few (count,
-// fill and integral together 3547 -> 340 us).
+// waves' sums in LDS and at most 1024 blocks run, so the adds are few.  Bound:
+// the points (349 MB there, 73 us); the chain offsets, vertices, coordinates is
+// taken once for many elements (with G lanes for every element of the list,
+// empty or not, and the polynomial's terms point by point 147 us; now 116 us).
+constexpr int INT_EPW = 32;
+
 template <int D, int G>
 __global__ __launch_bounds__(512) void k_integrate(int nel, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
-                                                   const double *__restrict__ coords,
+                                                   const double *__restrict__ coords, int epw,
                                                    const int32_t *__restrict__ offsets,
                                                    const double4 *__restrict__ pts, Poly f,
                                                    double *__restrict__ per_elem, double *total) {
+  constexpr int NGEO = D + D * D + 1;
   __shared__ double s_sum[8];
-  const int sub = threadIdx.x & (G - 1);
-  const long long ngrp = (long long)gridDim.x * (512 / G);
+  __shared__ double s_geo[8][INT_EPW][NGEO];  // last vertex, F, |det F|
+  __shared__ int4 s_el[8][INT_EPW];           // first and last point, element of the list
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int sub = lane & (G - 1), grp = lane / G;
+  const long long wid = (long long)blockIdx.x * 8 + wv, nwaves = (long long)gridDim.x * 8;
   double acc_all = 0.0;
-  for (long long i = ((long long)blockIdx.x * 512 + threadIdx.x) / G; i < nel; i += ngrp) {
-    const int q0 = offsets[i], q1 = offsets[i + 1];
-    double s = 0.0;
+  for (long long i0 = wid * epw; i0 < nel; i0 += nwaves * epw) {
+    int q0 = 0, q1 = 0;
+    const bool valid = lane < epw && i0 + lane < nel;
+    if (valid) {
+      q0 = offsets[i0 + lane];
+      q1 = offsets[i0 + lane + 1];
+    }
+    const unsigned long long mp = __ballot(q1 > q0);
+    if (per_elem && valid && q1 <= q0) per_elem[i0 + lane] = 0.0;
+    if (!mp) continue;
     if (q1 > q0) {
-      const int e = elems ? elems[i] : (int)i;
+      const int e = elems ? elems[i0 + lane] : (int)i0 + lane;
       double V[D + 1][3];
 #pragma unroll
       for (int k = 0; k <= D; ++k) {
@@ -221,39 +310,49 @@ __global__ __launch_bounds__(512) void k_integrate(int nel, const int32_t *__res
       }
       double F[D * D], Finv[D * D], absdet;
       jacobian<D>(V, F, Finv, absdet);
-      for (int q = q0 + sub; q < q1; q += G) {
-        const double4 p = pts[q];
-        const double xi[3] = {p.x, p.y, p.z};
-        double x[3] = {0.0, 0.0, 0.0};
+      const int slot = __popcll(mp & ((1ull << lane) - 1ull));
+      double *geo = s_geo[wv][slot];
 #pragma unroll
-        for (int r = 0; r < D; ++r) {
-          double a = V[D][r];
+      for (int r = 0; r < D; ++r) geo[r] = V[D][r];
 #pragma unroll
-          for (int c = 0; c < D; ++c) a += F[r * D + c] * xi[c];
-          x[r] = a;
+      for (int k = 0; k < D * D; ++k) geo[D + k] = F[k];
+      geo[D + D * D] = absdet;
+      s_el[wv][slot] = make_int4(q0, q1, lane, 0);
+    }
+    ecore::wave_sync();
+    const int n = __popcll(mp);
+    for (int k = grp; k < n; k += 64 / G) {
+      const int4 el = s_el[wv][k];
+      double V[D], F[D * D];
+#pragma unroll
+      for (int r = 0; r < D; ++r) V[r] = s_geo[wv][k][r];
+#pragma unroll
+      for (int r = 0; r < D * D; ++r) F[r] = s_geo[wv][k][D + r];
+      const double absdet = s_geo[wv][k][D + D * D];
+      double s = 0.0;
+      int q = el.x + sub;
+      while (q < el.y) {
+        if (__ballot(q + G < el.y) != 0ull) {
+          s = integrate_points<D, G, 4>(q, el.y, V, F, absdet, pts, f, s);
+          q += 4 * G;
+        } else {
+          s = integrate_points<D, G, 1>(q, el.y, V, F, absdet, pts, f, s);
+          q += G;
         }
-        double fv = 0.0;
-        for (int t = 0; t < f.n; ++t) {
-          double m = f.c[t];
+      }
 #pragma unroll
-          for (int d = 0; d < 3; ++d)
-            for (int k = 0; k < f.ex[t][d]; ++k) m *= x[d];
-          fv += m;
-        }
-        s += absdet * p.w * fv;
+      for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (sub == 0) {
+        if (per_elem) per_elem[i0 + el.z] = s;
+        acc_all += s;
       }
     }
-#pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (sub == 0) {
-      if (per_elem) per_elem[i] = s;
-      acc_all += s;
-    }
+    ecore::wave_sync();
   }
   if (!total) return;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) acc_all += __shfl_xor(acc_all, o, 64);
-  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = acc_all;
+  if (lane == 0) s_sum[wv] = acc_all;
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
@@ -324,9 +423,13 @@ int fill_epw(int nel) {
 template <int D, int G>
 void launch_integrate(xg_ctx *ctx, int nel, const int32_t *elems, const int32_t *el2v, const double *coords,
                       const int32_t *offsets, const double4 *pts, const Poly &f, double *per_elem, double *total) {
-  const long long want = ((long long)nel * G + 511) / 512;
+  // elements per wave: one for each group of lanes while the waves fit on the
+  // device at once, then more
+  int epw = 64 / G;
+  while (epw < INT_EPW && nel / epw > 16384) epw *= 2;
+  const long long want = ((long long)nel + 8LL * epw - 1) / (8LL * epw);
   const int grid = (int)(want < 1024 ? want : 1024);
-  k_integrate<D, G><<<grid, 512, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, pts, f, per_elem, total);
+  k_integrate<D, G><<<grid, 512, 0, ctx->stream>>>(nel, elems, el2v, coords, epw, offsets, pts, f, per_elem, total);
 }
 
 }  // namespace
