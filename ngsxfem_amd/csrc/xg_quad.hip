@@ -719,10 +719,13 @@ struct QuadParts {
 
 // Bound: the latency of a part (branches and FP64 chains of one lane).  With a
 // lane per element 5,300 cut hexahedra were 83 waves for 1024 SIMDs, each lane
-// going through all slices: 48^3 hexes, order 4, NEG, count and fill: 1048 -> 153 us (with the matrices 1378 -> 203).
+// going through all slices: 48^3 hexes, order 4, NEG, count and fill: 1048 ->
+// 153 us (with the matrices 1378 -> 203).  Two waves per SIMD for the fill too
+// (55 spilled registers): with one the last third of the waves waited for the
+// others, 188 -> 174 us with the matrices.
 constexpr int QG = 16;  // lanes per element: 15 parts of a split hexahedron at order 4
 template <int D, bool FILL>
-__global__ __launch_bounds__(256) void k_quad_rule(int nel, const int32_t *__restrict__ elems,
+__global__ __launch_bounds__(256, 2) void k_quad_rule(int nel, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
                                                    const double *__restrict__ coords,
                                                    const double *__restrict__ lset, int dt, int order, int pol,
