@@ -363,7 +363,9 @@ int xg_assemble_csr_scaled(xg_ctx *ctx, int nel, int ndof, const int32_t *dofs, 
    matrices): every (dofs[e][a], dofs[e][b]) of the nel x ndof table (entries
    < 0 skipped), sorted and made unique.  row_ptr: int32[n + 1]; col_idx:
    int32[cap] (columns ascending per row); nnz: device int32[1].  Uses the
-   context workspace (about 32 B per coupling); nnz > cap -> XG_ERR_CAPACITY
+   context workspace (4 B per coupling, 8 B per table entry and per row; for
+   tables with more than 256 couplings per row on average about 32 B per
+   coupling); nnz > cap -> XG_ERR_CAPACITY
    and a dof >= n -> XG_ERR_ARG at xg_sync.  nel * ndof^2 < 2^31. */
 int xg_csr_pattern(xg_ctx *ctx, int nel, int ndof, const int32_t *dofs, int n, int32_t *row_ptr,
                    int32_t *col_idx, long long cap, int32_t *nnz);
@@ -426,7 +428,7 @@ int xg_subdiv_weights_mesh(xg_ctx *ctx, int L, int order, int nel, const int32_t
    107-111: the base rules are then exact for the moments, uncut tree nodes
    come from a table).  out: nel x ndt x ndof x ndof, FP32 or FP64 by
    precision.  stats (nullable): int32 nel x ndt x 4 -- table rows, volume
-   tets and interface triangles integrated point by point, cut leaves.
+   tets and interface triangles of cut leaves, cut leaves.
    Uses the context workspace (moments of up to 2^21 elements at a time).
    With order >= 2p, xg_subdiv_moments, xg_subdiv_weights and the three mesh
    entry points run in rounds of up to 2^19 elements over per-element node
@@ -437,8 +439,8 @@ int xg_subdiv_weights_mesh(xg_ctx *ctx, int L, int order, int nel, const int32_t
    be captured into a HIP graph (not tested).  Tuning knobs
    read from the environment at each call: XG_SDX_CAP (list capacity, 16 ..
    4096, default 4096), XG_SDX_QUEUE=0 (one block per element instead of
-   persistent waves), XG_SDX_NOFUSE=1 (p = 3: volume side and interface in
-   separate launches). */
+   persistent waves), XG_SDX_NOFUSE=1 (volume side and interface in separate
+   launches). */
 int xg_subdiv_pipeline(xg_ctx *ctx, int p, int L, int order, int nel, const int32_t *elems,
                        const int32_t *el2v, const double *coords, const double *lset_nodal, int ndt,
                        const int *dts, int mask, int precision, void *out, int32_t *stats);

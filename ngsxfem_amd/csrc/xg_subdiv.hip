@@ -1246,7 +1246,7 @@ __device__ __forceinline__ void aff_to_hom(double *red, int lane) {
 }
 
 // stats (nullable, int32 x 4 per element): table rows added, volume tets and
-// interface triangles integrated point by point, cut leaves
+// interface triangles of cut leaves, cut leaves
 template <int LO, int PM, int SIDE, int WHICH>
 __global__ __launch_bounds__(64, 2) void k_subdiv_exact(int nel, const int32_t *__restrict__ nel_dev,
                                                      const int32_t *__restrict__ sub,
@@ -1722,15 +1722,14 @@ int subdiv_exact_pass(xg_ctx *ctx, int nel, const int32_t *elems, const double *
 // integer and LDS work runs at two waves per SIMD.  The staged path splits
 // it into three kernels over a per-element list of uint16 node ids:
 //   1. k_sdx_tree: the walk (lattice sign checks, classification) at high
-//      occupancy; writes the cut leaves from the front of the element's list
-//      and the uncut nodes of the kept side (table rows) from the back
+//      occupancy; writes the cut leaves to the element's list and the sum of
+//      the kept side's uncut nodes (table rows) to its moments
 //   2. k_sdx_leaves: the cut leaves' pieces and their moments (the
 //      register-heavy part), the volume side and the interface in one launch
 //      where both are asked for; appends the complemented leaves after the
 //      cut leaves
-//   3. k_sdx_rows: the table rows (uncut nodes + complemented leaves),
-//      added to the moments
-// An element whose lists do not fit (2 cut leaves + rows > cap) is queued
+//   3. k_sdx_rows: the complemented leaves' table rows, added to the moments
+// An element whose list does not fit (2 x cut leaves > cap) is queued
 // and handled by the one-kernel path.
 
 struct SdcLds {
@@ -2556,34 +2555,40 @@ int subdiv_staged(xg_ctx *ctx, int nel, const int32_t *elems, const double *lset
       // host round trip is needed
       // the volume side and the interface both requested: one launch for
       // both (lane roles), then the rows, then the overflow path
+      // (a part named twice: one launch each for p <= 2)
       int u_vol = -1, u_if = -1;
+      bool twice = false;
       for (int u = 0; u < ndt; ++u) {
-        if (dts[u] == side) u_vol = u;
-        if (dts[u] == IF && !if_done) u_if = u;
-      }
-      {
-        if (u_vol >= 0 && u_if >= 0 && !getenv("XG_SDX_NOFUSE")) {
-          double *ov = o_u[u_vol], *oi = o_u[u_if];
-          int32_t *sv = s_u[u_vol], *si = s_u[u_if];
-          if (side == NEG)
-            rc = launch_sdx_leaves<LO, PM, NEG, 3>(ctx, m, el, lset, el2v, coords, fi, L, lists, cap, cnt, ov, oi,
-                                                   mstride, sv, sstride, queue, si);
-          else
-            rc = launch_sdx_leaves<LO, PM, POS, 3>(ctx, m, el, lset, el2v, coords, fi, L, lists, cap, cnt, ov, oi,
-                                                   mstride, sv, sstride, queue, si);
-          if (rc != XG_OK) return rc;
-          rc = launch_sdx_rows<PM>(ctx, m, lists, cap, cnt, ov, mstride);
-          if (rc != XG_OK) return rc;
-          rc = subdiv_exact_pass<LO, PM>(ctx, m, el, lset, el2v, coords, fi, L, side, false, ov, nullptr, mstride,
-                                         nullptr, sv, sstride, over, nover);
-          if (rc != XG_OK) return rc;
-          rc = subdiv_exact_pass<LO, PM>(ctx, m, el, lset, el2v, coords, fi, L, -1, true, nullptr, oi, mstride,
-                                         nullptr, si, sstride, over, nover);
-          if (rc != XG_OK) return rc;
-          if_done = true;
-          if (t == ndt) break;
-          continue;
+        if (dts[u] == side) {
+          twice |= u_vol >= 0;
+          u_vol = u;
         }
+        if (dts[u] == IF && !if_done) {
+          twice |= u_if >= 0;
+          u_if = u;
+        }
+      }
+      if (u_vol >= 0 && u_if >= 0 && !(PM < 3 && twice) && !getenv("XG_SDX_NOFUSE")) {
+        double *ov = o_u[u_vol], *oi = o_u[u_if];
+        int32_t *sv = s_u[u_vol], *si = s_u[u_if];
+        if (side == NEG)
+          rc = launch_sdx_leaves<LO, PM, NEG, 3>(ctx, m, el, lset, el2v, coords, fi, L, lists, cap, cnt, ov, oi,
+                                                 mstride, sv, sstride, queue, si);
+        else
+          rc = launch_sdx_leaves<LO, PM, POS, 3>(ctx, m, el, lset, el2v, coords, fi, L, lists, cap, cnt, ov, oi,
+                                                 mstride, sv, sstride, queue, si);
+        if (rc != XG_OK) return rc;
+        rc = launch_sdx_rows<PM>(ctx, m, lists, cap, cnt, ov, mstride);
+        if (rc != XG_OK) return rc;
+        rc = subdiv_exact_pass<LO, PM>(ctx, m, el, lset, el2v, coords, fi, L, side, false, ov, nullptr, mstride,
+                                       nullptr, sv, sstride, over, nover);
+        if (rc != XG_OK) return rc;
+        rc = subdiv_exact_pass<LO, PM>(ctx, m, el, lset, el2v, coords, fi, L, -1, true, nullptr, oi, mstride,
+                                       nullptr, si, sstride, over, nover);
+        if (rc != XG_OK) return rc;
+        if_done = true;
+        if (t == ndt) break;
+        continue;
       }
       for (int u = 0; u < ndt; ++u) {
         const bool vol = dts[u] == side;
