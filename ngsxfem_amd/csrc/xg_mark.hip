@@ -171,7 +171,7 @@ __device__ __forceinline__ void wave_sync_lds() {
 // (launch bounds: at most 80 VGPRs, 6 waves per SIMD; the decomposition
 // code of the queued elements otherwise sets the register count and leaves
 // 5, and 8 waves need spills -- 6 measured fastest)
-template <int D, int NB, int EPT>
+template <int D, int NB, int EPT, bool BIG>
 __global__ __launch_bounds__(NB, 6) void k_mark(int ne, const int32_t *__restrict__ el2v,
                                              const double *__restrict__ lset,
                                              uint8_t *__restrict__ dt_out,
@@ -189,19 +189,18 @@ __global__ __launch_bounds__(NB, 6) void k_mark(int ne, const int32_t *__restric
   // element rows of all EPT elements, then their level-set values.  The
   // loads are unconditional (lanes past the end read the last element
   // again): a load under a branch is waited for at the branch's end, which
-  // would serialise the EPT round trips.  Rows pass once, and
-  // the domains and cut ratios of 2^20 elements are more than the L2s hold
-  // besides the level set, so they are kept from displacing it (128^3 cells:
-  // 126.3 -> 122.3 us with the compaction; blocks mapped so that an XCD has
-  // consecutive ones: 146.8 us).
-  const bool big = ne >= (1 << 20);
+  // would serialise the EPT round trips.  BIG: rows,
+  // domains and cut ratios pass once and are kept from displacing the level set
+  // in the caches (128^3 cells: 126.3 -> 122.3 us with the compaction; blocks
+  // mapped so that an XCD has consecutive ones: 146.8 us).
   int vi[EPT][D + 1];
 #pragma unroll
   for (int k = 0; k < EPT; ++k) {
     const int ec = min(base + k * NB + tid, ne - 1);
     if constexpr (D == 3) {
       typedef int v4 __attribute__((ext_vector_type(4)));
-      const v4 v = __builtin_nontemporal_load(reinterpret_cast<const v4 *>(el2v) + ec);
+      const v4 *row = reinterpret_cast<const v4 *>(el2v) + ec;
+      const v4 v = BIG ? __builtin_nontemporal_load(row) : *row;
       vi[k][0] = v.x;
       vi[k][1] = v.y;
       vi[k][2] = v.z;
@@ -231,7 +230,7 @@ __global__ __launch_bounds__(NB, 6) void k_mark(int ne, const int32_t *__restric
         // or 0/(0+w0) = 0 (cutinfo.cpp:87-124)
         cdt[k] = eldom == NEG ? 1 : 2;
         const double cr = eldom == NEG ? 1.0 : 0.0;
-        if (big) {
+        if constexpr (BIG) {
           if (cut_ratio) __builtin_nontemporal_store(cr, cut_ratio + e);
           if (dt_out) __builtin_nontemporal_store((uint8_t)eldom, dt_out + e);
         } else {
@@ -832,16 +831,30 @@ size_t mark_scratch_ints(int ne) {
 // marking + compaction on an explicit stream with caller-owned scratch
 // (mark_scratch_ints(ne) int32); only kernel launches, so the sequence can be
 // captured into a hipGraph.  n_cut (nullable) receives the cut count.
+// rows, domains and cut ratios of 2^20 elements (25 MB on tets) are more than
+// the L2s hold; on smaller meshes the next kernel finds them there, and the
+// plain accesses are 1 us faster (60 x 60 cells: 35.4 against 36.5 us a step)
+static void launch_mark(hipStream_t st, int D, int nblk, int ne, const int32_t *el2v, const double *lset, uint8_t *dt,
+                        double *cr, uint32_t *bits, int nw, int32_t *blk, int32_t *err) {
+#define XG_MARK(DD)                                                                                              \
+  if (ne >= (1 << 20))                                                                                           \
+    k_mark<DD, MARK_BLK, MARK_EPT, true><<<nblk, MARK_BLK, 0, st>>>(ne, el2v, lset, dt, cr, bits, nw, blk, err);  \
+  else                                                                                                           \
+    k_mark<DD, MARK_BLK, MARK_EPT, false><<<nblk, MARK_BLK, 0, st>>>(ne, el2v, lset, dt, cr, bits, nw, blk, err)
+  switch (D) {
+    case 1: XG_MARK(1); break;
+    case 2: XG_MARK(2); break;
+    default: XG_MARK(3); break;
+  }
+#undef XG_MARK
+}
+
 int mark_compact(hipStream_t st, int32_t *d_err, int D, int ne, const int32_t *el2v, const double *lset,
                  uint8_t *dt, double *cr, uint32_t *bits, int32_t *scratch, int32_t *cut_list, int32_t *n_cut) {
   const int nw = (ne + 31) / 32;
   const int nblk = (ne + MARK_BLK * MARK_EPT - 1) / (MARK_BLK * MARK_EPT);
   int32_t *blk = scratch, *sums = scratch + nblk + 1;
-  switch (D) {
-    case 1: k_mark<1, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, st>>>(ne, el2v, lset, dt, cr, bits, nw, blk, d_err); break;
-    case 2: k_mark<2, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, st>>>(ne, el2v, lset, dt, cr, bits, nw, blk, d_err); break;
-    default: k_mark<3, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, st>>>(ne, el2v, lset, dt, cr, bits, nw, blk, d_err); break;
-  }
+  launch_mark(st, D, nblk, ne, el2v, lset, dt, cr, bits, nw, blk, d_err);
   XG_LAUNCH_CHECK();
   scan_block_counts(st, blk, nblk, sums, n_cut);
   k_compact<MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, st>>>(ne, bits + (size_t)4 * nw, blk, cut_list);
@@ -911,11 +924,7 @@ extern "C" int xg_mark(xg_ctx *ctx, int D, int ne, const int32_t *el2v, const do
     if (r) return r;
     blk = (int32_t *)((char *)ctx->ws + ((scan_ws + 255) / 256) * 256);
   }
-  switch (D) {
-    case 1: k_mark<1, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, ctx->stream>>>(ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err); break;
-    case 2: k_mark<2, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, ctx->stream>>>(ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err); break;
-    default: k_mark<3, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, ctx->stream>>>(ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err); break;
-  }
+  launch_mark(ctx->stream, D, nblk, ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err);
   XG_LAUNCH_CHECK();
   if (!compact) return XG_OK;
   // scan of block counts: blk[nblk] = total.  The scan scratch is the start
@@ -995,11 +1004,7 @@ extern "C" int xg_mark_noalloc(xg_ctx *ctx, int D, int ne, const int32_t *el2v, 
   const int nblk = (ne + MARK_BLK * MARK_EPT - 1) / (MARK_BLK * MARK_EPT);
   const bool compact = cut_list || n_cut;
   int32_t *blk = compact ? scr : nullptr, *sums = scr + nblk + 1;
-  switch (D) {
-    case 1: k_mark<1, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, ctx->stream>>>(ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err); break;
-    case 2: k_mark<2, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, ctx->stream>>>(ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err); break;
-    default: k_mark<3, MARK_BLK, MARK_EPT><<<nblk, MARK_BLK, 0, ctx->stream>>>(ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err); break;
-  }
+  launch_mark(ctx->stream, D, nblk, ne, el2v, lset_v, dt, cut_ratio, bits, nw, blk, ctx->d_err);
   XG_LAUNCH_CHECK();
   if (!compact) return XG_OK;
   scan_block_counts(ctx->stream, blk, nblk, sums, n_cut);
