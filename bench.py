@@ -15,6 +15,7 @@ reported under "c2".
 """
 import argparse
 import json
+import math
 import os
 import re
 import sys
@@ -26,7 +27,6 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "cut-elem/s (rule+elmat) plain vs learned/mixed at ≤1e-6 rel err; %HBM/%MFMA"
-PEAK_FP32_MFMA = 157.3e12
 PEAK_FP64_MFMA = 78.6e12
 PEAK_HBM = 8.0e12
 PEAK_FP64_VALU = 78.6e12
@@ -224,22 +224,21 @@ def c5_fp64_ops(stats, launches, p=3):
 def c5_leaf_ops(st_vol, st_if, p=3):
     """FP64 operations (FMA = 2) of the cut-leaf kernel k_sdx_leaves (volume
     side and interface in one launch) from the per-element counts of the two
-    parts (stats[..., 0..3] as c5_fp64_ops): the volume tets and interface
-    triangles point by point, the cut leaves' pieces once."""
+    parts (stats[..., 0..3] as c5_fp64_ops): every piece's moments from its
+    vertices by the truncated series, the sums over the pieces, the cut
+    leaves' geometry once."""
     nm = {1: 10, 2: 35, 3: 84}[p]
-    nq_v, nq_i = {1: (4, 3), 2: (14, 6), 3: (24, 12)}[p]
     vol = float(st_vol[..., 1].sum())
     itf = float(st_if[..., 2].sum())
     leaves = float(st_vol[..., 3].sum())
-    if p == 3:
-        # centred affine moments: per point the map (25 volume / 18 interface),
-        # 16 monomials, 19 weighted monomials, 83 FMAs + 1 add; per element the
-        # 84 x 84 map to the homogeneous moments for each of the two parts
-        nel = float(st_vol[..., 0].size)
-        return (vol * (nq_v * (25 + 16 + 19 + 167) + 17) + itf * (nq_i * (18 + 16 + 19 + 167) + 40)
-                + leaves * (48 + 4 * 42) + nel * 2 * 2 * nm * nm)
-    return (vol * (nq_v * (27 + 30 + 21 + 2 * nm) + 17) + itf * (nq_i * (18 + 30 + 21 + 2 * nm) + 40)
-            + leaves * (48 + 4 * 42))
+    nel = float(st_vol[..., 0].size)
+    # 3 products per monomial of degree < 2p and vertex (the first vertex has
+    # no addend for one product of each coefficient); a sum per coefficient
+    step = 3 * math.comb(2 * p + 2, 3)
+    first = 2 * step - (nm - 1)
+    # the 84 x 84 (p = 3) map to homogeneous moments and the scale per part
+    return (vol * (first + 3 * 2 * step + nm + 17) + itf * (first + 2 * 2 * step + nm + 40)
+            + leaves * (48 + 4 * 42) + nel * 2 * (2 * nm * nm + nm))
 
 
 def cpu_threads():
@@ -874,7 +873,7 @@ def measure_c2(args):
     paths["plain_mfma"] = {"kernel": "k_pipeline<3,2,%s>" % ("float" if prec == 1 else "double"),
                            "ms": ms_mfma, "cut_elem_per_s": n_cut / (ms_mfma * 1e-3),
                            "max_rel_err_vs_fp64": max_rel_err(out_mfma),
-                           "arith": "%s MFMA, B^T W B" % args.precision}
+                           "arith": "FP64 MFMA over the points, %s store" % args.precision}
     out_mom = torch.empty(n_cut * 2 * nd * nd, dtype=odt, device=dev)
     ms_mom, iso_mom = timed(prec | _abi.XG_METHOD_MOMENTS, out_mom)
     launch_mom = ms_mom
@@ -912,13 +911,14 @@ def measure_c2(args):
                 "kernel": "k_pipeline<3,%d,float%s>" % (pp, ",split-BF16" if name == "bf16x3" else ""),
                 "ms": msp, "cut_elem_per_s": n_cut / (msp * 1e-3),
                 "max_rel_err_vs_fp64": float((dd[nzp] / rn[nzp]).max().item()),
-                "arith": "FP32 MFMA" if name == "fp32" else "split-BF16 hi/mid/lo MFMA (6 products), FP32 sums",
-                "note": "rule order %d, FP64 sums of 8-point groups" % oo}
+                "arith": ("FP64 MFMA" if pp <= 2 else "FP32 MFMA") if name == "fp32"
+                else "split-BF16 hi/mid/lo MFMA (6 products), FP32 sums",
+                "note": "rule order %d, FP64 sums" % oo}
     best = "moments" if args.method == "moments" else "plain_mfma"
     ms_per_step = paths[best]["ms"]
     value = n_cut / (ms_per_step * 1e-3)
 
-    peak = PEAK_FP32_MFMA if prec == _abi.XG_PREC_FP32 else PEAK_FP64_MFMA
+    peak = PEAK_FP64_MFMA  # the workload's P2 matrices contract in FP64 for either store
     roof_mfma = {"bound": "mfma", "kernel": paths["plain_mfma"]["kernel"],
                  "achieved": flops / (launch_mfma * 1e-3) / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                  "frac": flops / (launch_mfma * 1e-3) / peak, "traffic": read_traffic("pipeline_c2_pmc.txt"),
