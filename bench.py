@@ -237,8 +237,9 @@ def c5_leaf_ops(st_vol, st_if, p=3):
     step = 3 * math.comb(2 * p + 2, 3)
     first = 2 * step - (nm - 1)
     # the 84 x 84 (p = 3) map to homogeneous moments and the scale per part
-    return (vol * (first + 3 * 2 * step + nm + 17) + itf * (first + 2 * 2 * step + nm + 40)
-            + leaves * (48 + 4 * 42) + nel * 2 * (2 * nm * nm + nm))
+    two = itf - leaves  # leaves with two triangles: one series over four points
+    return (vol * (first + 3 * 2 * step + nm + 17) + (leaves - two) * (first + 2 * 2 * step + nm + 40)
+            + two * (first + 3 * 2 * step + nm + 80) + leaves * (48 + 4 * 42) + nel * 2 * (2 * nm * nm + nm))
 
 
 def cpu_threads():

@@ -435,15 +435,19 @@ def gen_series(D, P, L, idx2):
     |T| k! beta! / (|beta| + k)! h_beta (Dirichlet's integral), so a piece's
     moments cost 3 FMAs per monomial of degree < 2P and vertex, whatever the
     degree's quadrature rule: multiplying by 1 / (1 - l) is the in-place
-    recursion h_beta += sum_i l_i h_(beta - e_i) in ascending degree."""
+    recursion h_beta += sum_i l_i h_(beta - e_i) in ascending degree.  Two
+    simplices that share all but one vertex (y_p of the one with weight w_1,
+    y_q of the other) are one series: w_1 / (1 - <z, y_p>) + w_2 / (1 - <z, y_q>)
+    is (w_1 + w_2 - <z, w_1 y_q + w_2 y_p>) over both factors, so aser_first
+    takes a numerator w - <z, v>."""
     n2 = 2 * P
 
     def slot(b):
         return idx2[tuple(b) + (n2 - sum(b),)]
     for first in (True, False):
         if first:
-            L.append("  // h = w / (1 - <z, y>), truncated at degree 2P")
-            L.append("  XG_DEV static void aser_first(const double *y, double w, double *h) {")
+            L.append("  // h = (w - <z, v>) / (1 - <z, y>), truncated at degree 2P")
+            L.append("  XG_DEV static void aser_first(const double *y, double w, const double *v, double *h) {")
             L.append("    h[%d] = w;" % slot([0] * D))
         else:
             L.append("  // h <- h / (1 - <z, y>), truncated at degree 2P")
@@ -452,6 +456,8 @@ def gen_series(D, P, L, idx2):
             if sum(b) == 0:
                 continue
             e = None if first else "h[%d]" % slot(b)
+            if first and sum(b) == 1:
+                e = "-v[%d]" % b.index(1)
             for i in range(D):
                 if b[i] == 0:
                     continue
@@ -461,6 +467,11 @@ def gen_series(D, P, L, idx2):
                 e = "y[%d] * %s" % (i, src) if e is None else "fma(y[%d], %s, %s)" % (i, src, e)
             L.append("    h[%d] = %s;" % (slot(b), e))
         L.append("  }")
+        if first:
+            L.append("  XG_DEV static void aser_first(const double *y, double w, double *h) {")
+            L.append("    const double v[%d] = {%s};" % (D, ", ".join(["0.0"] * D)))
+            L.append("    aser_first(y, w, v, h);")
+            L.append("  }")
 
 
 def gen_series_table(D, P):

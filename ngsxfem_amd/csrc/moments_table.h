@@ -1271,18 +1271,22 @@ struct Moments<3, 1> {
       m[7] = fma(wb, x[2], m[7]);
     }
   }
-  // h = w / (1 - <z, y>), truncated at degree 2P
-  XG_DEV static void aser_first(const double *y, double w, double *h) {
+  // h = (w - <z, v>) / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_first(const double *y, double w, const double *v, double *h) {
     h[9] = w;
-    h[3] = y[0] * h[9];
-    h[6] = y[1] * h[9];
-    h[8] = y[2] * h[9];
+    h[3] = fma(y[0], h[9], -v[0]);
+    h[6] = fma(y[1], h[9], -v[1]);
+    h[8] = fma(y[2], h[9], -v[2]);
     h[0] = y[0] * h[3];
     h[1] = fma(y[1], h[3], y[0] * h[6]);
     h[2] = fma(y[2], h[3], y[0] * h[8]);
     h[4] = y[1] * h[6];
     h[5] = fma(y[2], h[6], y[1] * h[8]);
     h[7] = y[2] * h[8];
+  }
+  XG_DEV static void aser_first(const double *y, double w, double *h) {
+    const double v[3] = {0.0, 0.0, 0.0};
+    aser_first(y, w, v, h);
   }
   // h <- h / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_step(const double *y, double *h) {
@@ -1573,12 +1577,12 @@ struct Moments<3, 2> {
       m[30] = fma(wb, t5, m[30]);
     }
   }
-  // h = w / (1 - <z, y>), truncated at degree 2P
-  XG_DEV static void aser_first(const double *y, double w, double *h) {
+  // h = (w - <z, v>) / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_first(const double *y, double w, const double *v, double *h) {
     h[34] = w;
-    h[19] = y[0] * h[34];
-    h[29] = y[1] * h[34];
-    h[33] = y[2] * h[34];
+    h[19] = fma(y[0], h[34], -v[0]);
+    h[29] = fma(y[1], h[34], -v[1]);
+    h[33] = fma(y[2], h[34], -v[2]);
     h[9] = y[0] * h[19];
     h[15] = fma(y[1], h[19], y[0] * h[29]);
     h[18] = fma(y[2], h[19], y[0] * h[33]);
@@ -1610,6 +1614,10 @@ struct Moments<3, 2> {
     h[23] = fma(y[2], h[24], y[1] * h[27]);
     h[26] = fma(y[2], h[27], y[1] * h[31]);
     h[30] = y[2] * h[31];
+  }
+  XG_DEV static void aser_first(const double *y, double w, double *h) {
+    const double v[3] = {0.0, 0.0, 0.0};
+    aser_first(y, w, v, h);
   }
   // h <- h / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_step(const double *y, double *h) {
@@ -2454,12 +2462,12 @@ struct Moments<3, 3> {
       m[77] = fma(wb, t15, m[77]);
     }
   }
-  // h = w / (1 - <z, y>), truncated at degree 2P
-  XG_DEV static void aser_first(const double *y, double w, double *h) {
+  // h = (w - <z, v>) / (1 - <z, y>), truncated at degree 2P
+  XG_DEV static void aser_first(const double *y, double w, const double *v, double *h) {
     h[83] = w;
-    h[55] = y[0] * h[83];
-    h[76] = y[1] * h[83];
-    h[82] = y[2] * h[83];
+    h[55] = fma(y[0], h[83], -v[0]);
+    h[76] = fma(y[1], h[83], -v[1]);
+    h[82] = fma(y[2], h[83], -v[2]);
     h[34] = y[0] * h[55];
     h[49] = fma(y[1], h[55], y[0] * h[76]);
     h[54] = fma(y[2], h[55], y[0] * h[82]);
@@ -2540,6 +2548,10 @@ struct Moments<3, 3> {
     h[66] = fma(y[2], h[67], y[1] * h[72]);
     h[71] = fma(y[2], h[72], y[1] * h[78]);
     h[77] = y[2] * h[78];
+  }
+  XG_DEV static void aser_first(const double *y, double w, double *h) {
+    const double v[3] = {0.0, 0.0, 0.0};
+    aser_first(y, w, v, h);
   }
   // h <- h / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_step(const double *y, double *h) {

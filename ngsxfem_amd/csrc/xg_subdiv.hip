@@ -927,8 +927,8 @@ struct SdlLds {
   uint32_t *vert;      // CAP x 4: lattice vertices (level-5 units); top byte of the first: complemented
   double *t;           // 4 x CAP: parameter of cut point c on its edge
   double *scr;         // NG * 4 x SDL_ROW (over vert and t)
-  uint32_t *vol, *itf; // 3 CAP / 2 CAP piece records: leaf | corner codes << 8
-  uint32_t *tab;       // 16 x 6 words: the pieces of every sign pattern
+  uint32_t *vol, *itf; // 3 CAP / CAP piece records: leaf | corner codes << 8
+  uint32_t *tab;       // 16 x 5 words: the pieces of every sign pattern
   double *red;         // 2 NM
   double *cl;          // 20: the element's level-set nodal values
   double *fi;          // 10: F^{-1} (row major) and |det F|
@@ -946,8 +946,8 @@ __host__ __device__ inline size_t sdl_bytes(SdlLds *s, char *base) {
   const size_t leaf = (sizeof(uint32_t) * 4 + sizeof(double) * 4) * CAP, scr = sizeof(double) * NG * 4 * SDL_ROW;
   const size_t a_leaf = take(leaf > scr ? leaf : scr);
   const size_t a_vol = take(sizeof(uint32_t) * 3 * CAP);
-  const size_t a_itf = take(sizeof(uint32_t) * 2 * CAP);
-  const size_t a_tab = take(sizeof(uint32_t) * 16 * 6);
+  const size_t a_itf = take(sizeof(uint32_t) * CAP);
+  const size_t a_tab = take(sizeof(uint32_t) * 16 * 5);
   const size_t a_red = take(sizeof(double) * 2 * NM);
   const size_t a_cl = take(sizeof(double) * 20);
   const size_t a_fi = take(sizeof(double) * 10);
@@ -969,11 +969,12 @@ __host__ __device__ inline size_t sdl_bytes(SdlLds *s, char *base) {
 // included, xintegration.cpp:1159-1164): CutSimplex<3>::MakeQuad's split
 // (xintegration.cpp:1084-1388) as leaf_pieces gives it for the kept side, the
 // corner of a piece as lv | rv << 2 | c << 4: vertex lv (lv == rv) or cut point
-// c on the edge lv < rv.  meta: volume tets | triangles << 2 | complemented << 4
+// c on the edge lv < rv; the interface as one record (corners 0 1 2, with two
+// triangles also 2 3 0).  meta: volume tets | triangles << 2 | complemented << 4
 // | cuts << 5 | edges (lv | rv << 2) << 8, 12, 16, 20; 0 where the reference
 // throws.
 struct LeafTab {
-  uint32_t w[2][16][6];  // [side][pattern]: vol[3], itf[2], meta
+  uint32_t w[2][16][5];  // [side][pattern]: vol[3], itf, meta
   static constexpr int kth(int m, int k) {
     for (int j = 0; j < 4; ++j)
       if ((m >> j) & 1) {
@@ -1012,7 +1013,7 @@ struct LeafTab {
           const bool comp = side == POS ? !minor_pos : minor_pos;
           o[0] = pk(vx(mn), cp(0), cp(1), cp(2));
           o[3] = pk(cp(0), cp(1), cp(2), 0);
-          o[5] = 1u | (1u << 2) | (comp ? 16u : 0u) | (3u << 5) | (edges << 8);
+          o[4] = 1u | (1u << 2) | (comp ? 16u : 0u) | (3u << 5) | (edges << 8);
           continue;
         }
         const int ownm = side == POS ? posm : negm, othm = side == POS ? negm : posm;
@@ -1034,9 +1035,9 @@ struct LeafTab {
         const bool f1 = c1[n0] == c1[p0] || c2[n0] == c1[p0], f2 = c1[n1] == c1[p1] || c2[n1] == c1[p1];
         const int d1 = f1 ? c1[p0] : c2[p0], e1 = f1 ? c2[p0] : c1[p0];
         const int d2 = f2 ? c1[p1] : c2[p1], e2 = f2 ? c2[p1] : c1[p1];
-        o[3] = pk(cp(d1), cp(e1), cp(d2), 0);
-        o[4] = pk(cp(d2), cp(e2), cp(d1), 0);
-        o[5] = 3u | (2u << 2) | (4u << 5) | (edges << 8);
+        // the triangles (d1, e1, d2) and (d2, e2, d1) as one record
+        o[3] = pk(cp(d1), cp(e1), cp(d2), cp(e2));
+        o[4] = 3u | (2u << 2) | (4u << 5) | (edges << 8);
       }
   }
 };
@@ -2052,13 +2053,16 @@ __global__ __launch_bounds__(64) void k_sdx_tree(int nel, const int32_t *__restr
 // x + 16, x + 32, x + 48 into accumulator row r of column x, 16 sums of every
 // coefficient in (NM + 3) / 4 registers (19 cycles each for 64 lanes, measured;
 // the probe's A index is lane % 4, its K index lane / 16).  Both parts in one
-// launch: the lanes of columns x < nc take volume pieces, the others triangles
-// (a tet with a zero fourth step).
+// launch: the lanes of columns x < nc take volume pieces, the others interface
+// pieces: a triangle (a zero fourth step), or both triangles of a 2-2 leaf as
+// one series over its four cut points, whose numerator is linear.
 // A chunk of leaves is prepared first (lane = leaf: vertex values, sign pattern,
 // cut parameters; the pieces by pattern from a table), then its pieces run;
 // so the piece phase holds no sums and a piece reads its four corners only.
 // 128^3 cells, 405,341 elements, p = 3, L = 4, NEG + IF: the whole step 51.6 ->
-// 27.0 ms; 20^3, p = 2, L = 3: 400 -> 245 us (with the walk as it was).
+// 27.0 ms; 20^3, p = 2, L = 3: 400 -> 245 us (with the walk as it was).  Two
+// triangles as one: the kernel 16.4 -> 15.0 ms and 135 -> 133 us.  (The sums by
+// permlane32 / 16 swaps and adds instead of the MFMAs: 16.3 ms, no gain.)
 template <int LO, int PM, int SIDE, int WHICH>
 __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, const int32_t *__restrict__ elems,
                                                      const double *__restrict__ lset_nodal,
@@ -2080,7 +2084,7 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
   sdl_bytes<PM>(&S, smem);
   const int lane = threadIdx.x & 63;
   const int col = lane & 15, row = lane >> 4;
-  for (int k = lane; k < 16 * 6; k += 64) S.tab[k] = (&xg_leaf_tab_d.w[SIDE == POS ? 1 : 0][0][0])[k];
+  for (int k = lane; k < 16 * 5; k += 64) S.tab[k] = (&xg_leaf_tab_d.w[SIDE == POS ? 1 : 0][0][0])[k];
   double sel[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) sel[r] = (lane & 3) == r ? 1.0 : 0.0;
@@ -2123,11 +2127,11 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
     for (int g = 0; g < NG; ++g) D[g] = 0.0;
     const int nleaf = c4.x;
     // columns of the volume role: the split with the fewest rounds (a 1-3 cut
-    // leaf has 1 tet and 1 triangle, a 2-2 one 3 and 2; c4.y: the walk's count
-    // of 2-2 leaves)
+    // leaf has 1 tet, a 2-2 one 3, and either one interface record; c4.y: the
+    // walk's count of 2-2 leaves)
     int nc = WHICH == 1 ? 16 : 0;
     if constexpr (WHICH == 3) {
-      const int nv = nleaf + 2 * c4.y, ni = nleaf + c4.y;
+      const int nv = nleaf + 2 * c4.y, ni = nleaf;
       int best = 1 << 30;
       for (int c = 6; c <= 11; ++c) {
         const int r = max((nv + 4 * c - 1) / (4 * c), (ni + 63 - 4 * c) / (64 - 4 * c));
@@ -2146,7 +2150,7 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
     const int chunk = nchunk > 0 ? ((nleaf + nchunk - 1) / nchunk + 63) & ~63 : 64;
     for (int k0 = 0; k0 < nleaf; k0 += chunk) {
       const int kend = min(nleaf, k0 + chunk);
-      int tot_vol = 0, tot_if = 0;
+      int tot_vol = 0, nquad = 0, ntri = 0;
       for (int l0 = k0; l0 < kend; l0 += 64) {
         const int l = l0 + lane, s = l - k0;
         uint32_t meta = 0u, tb = 0u;
@@ -2165,8 +2169,8 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
             vv[j] = lagrange_eval3<LO>(cl, x);
             posm |= (vv[j] < 0.0 ? 0 : 1) << j;
           }
-          tb = posm * 6;
-          meta = S.tab[tb + 5];
+          tb = posm * 5;
+          meta = S.tab[tb + 4];
           ok = ok && meta != 0u;
           if (meta & 16u) pv.x |= 0x80000000u;
           *reinterpret_cast<uint4 *>(&S.vert[4 * s]) = pv;
@@ -2202,16 +2206,19 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
           tot_vol += __popcll(b1) + 2 * __popcll(b3);
         }
         if (WHICH & 2) {
-          const unsigned long long b1 = __ballot(ni >= 1), b2 = __ballot(ni == 2), lt = (1ull << lane) - 1ull;
-          const int base = tot_if + __popcll(b1 & lt) + __popcll(b2 & lt);
-#pragma unroll
-          for (int q = 0; q < 2; ++q)
-            if (q < ni) S.itf[base + q] = (uint32_t)s | (S.tab[tb + 3 + q] << 8);
-          tot_if += __popcll(b1) + __popcll(b2);
+          // (2-2 leaves from the front, the others from the back: the rounds
+          // with a second triangle are few)
+          const unsigned long long b1 = __ballot(ni == 1), b2 = __ballot(ni == 2), lt = (1ull << lane) - 1ull;
+          const uint32_t rec = (uint32_t)s | (S.tab[tb + 3] << 8);
+          if (ni == 2) S.itf[nquad + __popcll(b2 & lt)] = rec;
+          if (ni == 1) S.itf[CAP - 1 - ntri - __popcll(b1 & lt)] = rec;
+          nquad += __popcll(b2);
+          ntri += __popcll(b1);
         }
       }
+      const int tot_if = nquad + ntri;
       st_vol += tot_vol;
-      st_if += tot_if;
+      st_if += tot_if + nquad;
       wave_sync();
       const int mine = isv ? tot_vol : tot_if;
       int rounds = 0;
@@ -2219,19 +2226,19 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
       if (WHICH & 2) rounds = max(rounds, (tot_if + 63 - 4 * nc) / (64 - 4 * nc));
       for (int rd = 0; rd < rounds; ++rd) {
         const int q = rd * wr + rank;
-        double y[4][3], wgt = 0.0;
+        double y[4][3], wgt = 0.0, num[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int m = 0; m < 4; ++m)
 #pragma unroll
           for (int d = 0; d < 3; ++d) y[m][d] = 0.0;
         if (q < mine) {
-          const uint32_t rec = isv ? S.vol[q] : S.itf[q];
+          const uint32_t rec = isv ? S.vol[q] : S.itf[q < nquad ? q : CAP - 1 - (q - nquad)];
           const int s = rec & 255u;
           const uint32_t *vx = &S.vert[4 * s];
           const bool comp = (vx[0] >> 31) != 0u;
 #pragma unroll
-          for (int m = 0; m < (WHICH == 2 ? 3 : 4); ++m) {
-            if (m == 3 && !isv) break;
+          for (int m = 0; m < 4; ++m) {
+            if (m == 3 && !isv && q >= nquad) break;  // a triangle
             const int code = (int)(rec >> (8 + 6 * m));
             const uint32_t pl = vx[code & 3], pr = vx[(code >> 2) & 3];
             const double t = S.t[((code >> 4) & 3) * CAP + s];
@@ -2242,17 +2249,14 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
 #pragma unroll
             for (int d = 0; d < 3; ++d) y[m][d] = fma(t, (double)(b[d] - a[d]) * inv, (double)a[d] * inv - 0.25);
           }
-          double a[3], b[3], cr[3];
-#pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            a[d] = y[1][d] - y[0][d];
-            b[d] = y[2][d] - y[0][d];
-          }
-          cr[0] = a[1] * b[2] - a[2] * b[1];
-          cr[1] = a[2] * b[0] - a[0] * b[2];
-          cr[2] = a[0] * b[1] - a[1] * b[0];
           if (isv) {
-            double tf = 0.0;
+            double a[3], b[3], tf = 0.0;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+              a[d] = y[1][d] - y[0][d];
+              b[d] = y[2][d] - y[0][d];
+            }
+            const double cr[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]};
 #pragma unroll
             for (int d = 0; d < 3; ++d) tf += cr[d] * (y[3][d] - y[0][d]);
             tf = fabs(tf);
@@ -2260,23 +2264,36 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
           } else {
             // |absdet F^{-T} n| / absdet times the triangle's measure; a
             // degenerate one has no normal and no weight
-            const double tf = norm3(cr), na = norm3(a), nb = norm3(b);
-            if (!(tf < 1e-14 * (na > nb ? na : nb))) {
-              wgt = tf;
-              if (have_geo) {
-                double v[3];
+            auto weight = [&](const double *p0, const double *p1, const double *p2) {
+              double a[3], b[3];
 #pragma unroll
-                for (int r = 0; r < 3; ++r) v[r] = S.fi[r] * cr[0] + S.fi[3 + r] * cr[1] + S.fi[6 + r] * cr[2];
-                wgt = norm3(v);
+              for (int d = 0; d < 3; ++d) {
+                a[d] = p1[d] - p0[d];
+                b[d] = p2[d] - p0[d];
               }
+              const double cr[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]};
+              auto sq = [](const double *x) { return x[0] * x[0] + x[1] * x[1] + x[2] * x[2]; };
+              if (sq(cr) < 1e-28 * fmax(sq(a), sq(b))) return 0.0;
+              if (!have_geo) return sqrt(sq(cr));
+              double v[3];
+#pragma unroll
+              for (int r = 0; r < 3; ++r) v[r] = S.fi[r] * cr[0] + S.fi[3 + r] * cr[1] + S.fi[6 + r] * cr[2];
+              return sqrt(sq(v));
+            };
+            wgt = weight(y[0], y[1], y[2]);
+            if (q < nquad) {
+              const double w2 = weight(y[2], y[3], y[0]);
+#pragma unroll
+              for (int d = 0; d < 3; ++d) num[d] = wgt * y[3][d] + w2 * y[1][d];
+              wgt += w2;
             }
           }
         }
         double h[NG * 4];
-        MM::aser_first(y[0], wgt, h);
+        MM::aser_first(y[0], wgt, num, h);
         MM::aser_step(y[1], h);
         MM::aser_step(y[2], h);
-        if (WHICH & 1) MM::aser_step(y[3], h);
+        MM::aser_step(y[3], h);
 #pragma unroll
         for (int k = NM; k < NG * 4; ++k) h[k] = 0.0;
 #pragma unroll

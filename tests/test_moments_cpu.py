@@ -148,14 +148,20 @@ extern "C" int mom_accum_aff(const double *pts, const double *w, int n, double *
 // the truncated series of a simplex (Moments<3, P>::aser_*) of k + 1 vertices
 // y - 1/4, scaled and mapped as the subdivision kernel does it: moments of the
 // weight w = k! |T| on the tetrahedron (k = 3) or the triangle (k = 2)
-extern "C" int mom_series(int P, const double *verts, int k, double w, double *m) {
+// (k = 2 with w2 != 0: the two triangles (0, 1, 2) and (2, 3, 0) of four vertices,
+// weights w and w2, as one series)
+extern "C" int mom_series(int P, const double *verts, int k, double w, double w2, double *m) {
 #define SCASE(PP)                                                                             \
   if (P == PP) {                                                                              \
     using M = xg::Moments<3, PP>;                                                             \
     double h[M::NM], y[4][3] = {};                                                            \
-    for (int v = 0; v <= k; ++v)                                                              \
+    const int nv = w2 != 0.0 ? 4 : k + 1;                                                     \
+    for (int v = 0; v < nv; ++v)                                                              \
       for (int d = 0; d < 3; ++d) y[v][d] = verts[3 * v + d] - 0.25;                          \
-    M::aser_first(y[0], w, h);                                                                \
+    double n[3];                                                                              \
+    for (int d = 0; d < 3; ++d) n[d] = w * y[3][d] + w2 * y[1][d];                            \
+    if (w2 != 0.0) M::aser_first(y[0], w + w2, n, h);                                         \
+    else M::aser_first(y[0], w, h);                                                           \
     for (int v = 1; v < 4; ++v) M::aser_step(y[v], h); /* a zero step changes nothing */      \
     for (int r = 0; r < M::NM; ++r) h[r] *= xg::xg_aser3##PP[r][k == 3 ? 0 : 1];              \
     for (int a = 0; a < M::NM; ++a) {                                                         \
@@ -184,7 +190,8 @@ def momlib(tmp_path_factory):
                    check=True, capture_output=True)
     lib = ctypes.CDLL(str(so))
     lib.mom_elmat.restype = ctypes.c_int
-    lib.mom_series.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_void_p]
+    lib.mom_series.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_double,
+                               ctypes.c_void_p]
     lib.mom_hsimplex.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_double,
                                  ctypes.c_void_p]
     return lib
@@ -318,8 +325,29 @@ def test_series_moments_of_simplices(momlib, P, k):
         pts = np.ascontiguousarray(b @ V)
         ref, got = np.zeros(128), np.zeros(128)
         nm = momlib.mom_accum(3, P, _p(pts), _p(w), len(w), _p(ref))
-        assert momlib.mom_series(P, _p(V), k, float(math.factorial(k)), _p(got)) == nm
+        assert momlib.mom_series(P, _p(V), k, float(math.factorial(k)), 0.0, _p(got)) == nm
         assert np.abs(got[:nm] - ref[:nm]).max() <= 1e-14 * np.abs(ref[:nm]).max(), trial
+
+
+@pytest.mark.parametrize("P", [1, 2, 3])
+def test_series_of_two_triangles(momlib, P):
+    """two triangles that share an edge as one series over their four vertices
+    (numerator w + w2 - <z, w y3 + w2 y1>): the sum of their own series, on
+    quadrilaterals of every size, with one triangle far smaller, and without
+    weight.  Bar: each series' own."""
+    rng = np.random.default_rng(P)
+    for trial in range(32):
+        V = rng.dirichlet(np.ones(4), 4)[:, :3]
+        V = V[0] + 2.0 ** -(trial % 6) * (V - V[0])
+        w, w2 = rng.uniform(0.1, 1.0, 2) * np.array([1.0, 1e-6 if trial % 5 == 1 else 1.0])
+        if trial % 5 == 2:
+            w = 0.0
+        a, b, got = np.zeros(128), np.zeros(128), np.zeros(128)
+        nm = momlib.mom_series(P, _p(np.ascontiguousarray(V[:3])), 2, w, 0.0, _p(a))
+        momlib.mom_series(P, _p(np.ascontiguousarray(V[[2, 3, 0]])), 2, w2, 0.0, _p(b))
+        momlib.mom_series(P, _p(np.ascontiguousarray(V)), 2, w, w2, _p(got))
+        ref = a[:nm] + b[:nm]
+        assert np.abs(got[:nm] - ref).max() <= 2e-14 * np.abs(ref).max(), trial
 
 
 def test_moment_table_is_current():
