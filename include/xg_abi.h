@@ -422,9 +422,10 @@ int xg_subdiv_weights_mesh(xg_ctx *ctx, int L, int order, int nel, const int32_t
    element elems[i] (required) and each dts[t] (NEG, POS or IF; host array,
    ndt <= 3) the level-L rule is contracted into FP64 degree-2p moments and
    the degree-p mass (mask 1) / stiffness (mask 2) matrix formed from them.
-   lset_nodal: ne x 10 FP64 nodal values indexed by element id (Lattice<3,2>
-   dof order); el2v / coords: the mesh (interface weights and the element
-   map).  order >= 2p (the reference's intorder = 2p, symboliccutbfi.cpp:
+   A part named more than once in dts has the same values in each of its
+   places.  lset_nodal: ne x 10 FP64 nodal values indexed by element id
+   (Lattice<3,2> dof order); el2v / coords: the mesh (interface weights and
+   the element map).  order >= 2p (the reference's intorder = 2p, symboliccutbfi.cpp:
    107-111: the base rules are then exact for the moments, uncut tree nodes
    come from a table).  out: nel x ndt x ndof x ndof, FP32 or FP64 by
    precision.  stats (nullable): int32 nel x ndt x 4 -- table rows, volume

@@ -2503,16 +2503,39 @@ int launch_sdx_rows(xg_ctx *ctx, int nel, const uint16_t *lists, int cap, const 
   return XG_OK;
 }
 
+// n values of every element's row from one part's slot to another's
+template <typename T>
+__global__ __launch_bounds__(256) void k_copy_part(long long total, int n, const T *__restrict__ src,
+                                                   T *__restrict__ dst, int stride) {
+  const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (g >= total) return;
+  const long long i = g / n;
+  const size_t at = (size_t)i * stride + (size_t)(g - i * n);
+  dst[at] = src[at];
+}
+
 // Moments of the parts dts[0..ndt) (NEG / POS / IF) of nel elements, part u
 // written at outs[u] + i * mstride (stats, nullable: stats_u[u] + i *
 // sstride), through the staged kernels; the elements whose lists overflow
-// go through the one-kernel path.  dom (nullable): each element's domain
-// type on the lattice.
+// go through the one-kernel path.  A part named more than once is computed
+// once and copied.  dom (nullable): each element's domain type on the lattice.
 template <int LO, int PM>
 int subdiv_staged(xg_ctx *ctx, int nel, const int32_t *elems, const double *lset, const int32_t *el2v,
-                  const double *coords, const double *finv, int L, int ndt, const int *dts,
+                  const double *coords, const double *finv, int L, int ndt_all, const int *dts_all,
                   double *const *outs, int mstride, int32_t *const *stats_u, int sstride, uint8_t *dom) {
   constexpr int NM = Moments<3, PM>::NM;
+  // the distinct parts: dts[0..ndt), part u first named at at[u]; list entry
+  // t is part part[t]
+  int dts[3], at[3], part[3], ndt = 0;
+  for (int t = 0; t < ndt_all; ++t) {
+    int u = 0;
+    while (u < ndt && dts[u] != dts_all[t]) ++u;
+    if (u == ndt) {
+      dts[ndt] = dts_all[t];
+      at[ndt++] = t;
+    }
+    part[t] = u;
+  }
   int rc = ensure_sdx_tables(ctx, PM);
   if (rc != XG_OK) return rc;
   // list capacity: SDC_CAP, or smaller through XG_SDX_CAP (16 and up; the
@@ -2543,8 +2566,8 @@ int subdiv_staged(xg_ctx *ctx, int nel, const int32_t *elems, const double *lset
     double *o_u[3] = {nullptr, nullptr, nullptr};
     int32_t *s_u[3] = {nullptr, nullptr, nullptr};
     for (int u = 0; u < ndt; ++u) {
-      o_u[u] = outs[u] + (size_t)off * mstride;
-      s_u[u] = (stats_u && stats_u[u]) ? stats_u[u] + (size_t)off * sstride : nullptr;
+      o_u[u] = outs[at[u]] + (size_t)off * mstride;
+      s_u[u] = (stats_u && stats_u[at[u]]) ? stats_u[at[u]] + (size_t)off * sstride : nullptr;
     }
     uint8_t *dm = dom ? dom + off : nullptr;
     // volume sides in the order requested; the interface rides on the first
@@ -2572,20 +2595,12 @@ int subdiv_staged(xg_ctx *ctx, int nel, const int32_t *elems, const double *lset
       // host round trip is needed
       // the volume side and the interface both requested: one launch for
       // both (lane roles), then the rows, then the overflow path
-      // (a part named twice: one launch each for p <= 2)
       int u_vol = -1, u_if = -1;
-      bool twice = false;
       for (int u = 0; u < ndt; ++u) {
-        if (dts[u] == side) {
-          twice |= u_vol >= 0;
-          u_vol = u;
-        }
-        if (dts[u] == IF && !if_done) {
-          twice |= u_if >= 0;
-          u_if = u;
-        }
+        if (dts[u] == side) u_vol = u;
+        if (dts[u] == IF && !if_done) u_if = u;
       }
-      if (u_vol >= 0 && u_if >= 0 && !(PM < 3 && twice) && !getenv("XG_SDX_NOFUSE")) {
+      if (u_vol >= 0 && u_if >= 0 && !getenv("XG_SDX_NOFUSE")) {
         double *ov = o_u[u_vol], *oi = o_u[u_if];
         int32_t *sv = s_u[u_vol], *si = s_u[u_if];
         if (side == NEG)
@@ -2634,6 +2649,18 @@ int subdiv_staged(xg_ctx *ctx, int nel, const int32_t *elems, const double *lset
         if (itf) if_done = true;
       }
       if (t == ndt) break;
+    }
+    for (int t = 0; t < ndt_all; ++t) {
+      const int a = at[part[t]];
+      if (a == t) continue;
+      const long long tot = (long long)m * NM;
+      k_copy_part<double><<<(unsigned)((tot + 255) / 256), 256, 0, ctx->stream>>>(
+          tot, NM, outs[a] + (size_t)off * mstride, outs[t] + (size_t)off * mstride, mstride);
+      XG_LAUNCH_CHECK();
+      if (!stats_u || !stats_u[a] || !stats_u[t]) continue;
+      k_copy_part<int32_t><<<(unsigned)((4LL * m + 255) / 256), 256, 0, ctx->stream>>>(
+          4LL * m, 4, stats_u[a] + (size_t)off * sstride, stats_u[t] + (size_t)off * sstride, sstride);
+      XG_LAUNCH_CHECK();
     }
   }
   return XG_OK;

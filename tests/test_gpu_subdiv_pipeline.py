@@ -122,6 +122,44 @@ def test_pipeline_leaf_chunks(orc, dev, p, dts):
         assert np.all(np.abs(got - ref) <= 1e-12 * scale), (L, dts)
 
 
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("dts", [[NEG, NEG], [IF, IF], [NEG, IF, IF], [NEG, NEG, IF], [POS, IF, POS], [POS, POS, POS]])
+@pytest.mark.parametrize("knobs", [{}, {"XG_SDX_CAP": "16"}, {"XG_SDX_NOFUSE": "1"}])
+def test_part_named_twice(dev, monkeypatch, p, dts, knobs):
+    """a part that a list names more than once has the same values and counts
+    in each of its places, those of the list that names it once (moments,
+    matrices and fixed-node weights; also where the node lists overflow)"""
+    torch, _abi, ctx = dev
+    for k, v in knobs.items():
+        monkeypatch.setenv(k, v)
+    mesh = MakeStructured3DMesh(nx=2)
+    vals = W.random_quadric_p2(mesh.ne, seed=8)
+    elems = np.array([1, 12, 13, 40], np.int32)
+    once = list(dict.fromkeys(dts))
+    L, n = 2, len(elems)
+    # stale values in the workspace that the matrices' moments pass through
+    run_pipeline(dev, p, L, elems, mesh, -vals, [POS, IF, NEG], _abi.XG_PREC_FP64)
+    got, st = run_pipeline(dev, p, L, elems, mesh, vals, dts, _abi.XG_PREC_FP64, stats=True)
+    ref, st1 = run_pipeline(dev, p, L, elems, mesh, vals, once, _abi.XG_PREC_FP64, stats=True)
+    at = [once.index(d) for d in dts]
+    assert np.array_equal(got, ref[:, at])
+    assert np.array_equal(st, st1[:, at])
+    d = [up(torch, a) for a in (elems, mesh.el2v, mesh.coords, vals)]
+    z = lambda k, m: torch.full((n, k, m), float("nan"), dtype=torch.float64, device="cuda")  # noqa: E731
+    nm = math.comb(2 * p + 3, 3)
+    a, b = z(len(dts), nm), z(len(once), nm)
+    ctx.subdiv_moments_mesh(p, L, 2 * p, *d, dts, a)
+    ctx.subdiv_moments_mesh(p, L, 2 * p, *d, once, b)
+    if p == 2:
+        wa, wb = z(len(dts), 35), z(len(once), 35)
+        ctx.subdiv_weights_mesh(L, 4, *d, dts, wa)
+        ctx.subdiv_weights_mesh(L, 4, *d, once, wb)
+    ctx.sync()
+    assert torch.equal(a, b[:, at])
+    if p == 2:
+        assert torch.equal(wa, wb[:, at])
+
+
 @pytest.mark.parametrize("L", [0, 1, 2, 3, 4, 5])
 def test_pipeline_walk_levels(orc, dev, L):
     """the walk at every depth: no level above the leaf groups (L <= 2), one
