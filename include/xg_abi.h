@@ -363,7 +363,7 @@ int xg_assemble_csr_scaled(xg_ctx *ctx, int nel, int ndof, const int32_t *dofs, 
    matrices): every (dofs[e][a], dofs[e][b]) of the nel x ndof table (entries
    < 0 skipped), sorted and made unique.  row_ptr: int32[n + 1]; col_idx:
    int32[cap] (columns ascending per row); nnz: device int32[1].  Uses the
-   context workspace (4 B per coupling, 8 B per table entry and per row; for
+   context workspace (about 4 B per coupling, 8 B per table entry and per row; for
    tables with more than 256 couplings per row on average about 32 B per
    coupling); nnz > cap -> XG_ERR_CAPACITY
    and a dof >= n -> XG_ERR_ARG at xg_sync.  nel * ndof^2 < 2^31. */

@@ -5,8 +5,8 @@
 // dof tables before the element matrices are added.  Here the graph is
 // built on the GPU, row by row: the elements of every dof are listed (a count
 // per dof, a scan, a fill), a wave sorts the columns of a row's elements in
-// registers and drops the repeated ones, and a scan of the row lengths places
-// the rows.  Bound: the rows' sorts (a P2 edge row of a tetrahedral mesh has
+// registers and drops the repeated ones (rows of over 1024 candidates: a block,
+// in LDS), and a scan of the row lengths places the rows.  Bound: the rows' sorts (a P2 edge row of a tetrahedral mesh has
 // about 60 candidates for 27 columns).  32^3 cells of 6 tetrahedra, P2 (19.7 M
 // couplings, 275,000 rows): graph, matrices and values 2067 -> 368 us against
 // the radix sort of all couplings as 64-bit keys (eight passes over 16 B each,
@@ -22,21 +22,40 @@ using namespace xg;
 
 namespace {
 
-__global__ void k_fill_i32(int32_t *p, long long n, int32_t v) {
+// (zero3, nullable: three more words to clear)
+__global__ void k_fill_i32(int32_t *p, long long n, int32_t v, int32_t *zero3 = nullptr) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
+  if (zero3 && threadIdx.x < 3 && blockIdx.x == 0) zero3[threadIdx.x] = 0;
 }
 
 // ---- row by row
 // elements per dof, and the place of every table entry among its dof's (in no
-// fixed order), so that the fill below needs no atomics of its own
-__global__ __launch_bounds__(256) void k_dof_count(long long m, const int32_t *__restrict__ dofs, int n,
+// fixed order), so that the fill below needs no atomics of its own.  An atomic
+// on a word that others wait for takes 11 ns, 2240 us for one dof that all
+// elements of 32^3 cells share: where the wave's elements all have the same dof
+// in a column of the table, one lane counts for them.  (step: the bits ndof, 2
+// ndof, .. below 64, so step << column are the column's lanes after the first.
+// All runs of equal dofs by one atomic each, lane = element: 4.8 -> 8.2 us on a
+// discontinuous P2 table of 20^3 cells, whose neighbours in memory were no longer
+// counters in one line.)
+__global__ __launch_bounds__(256) void k_dof_count(long long m, int ndof, unsigned long long step,
+                                                   const int32_t *__restrict__ dofs, int n,
                                                    int32_t *__restrict__ cnt, int32_t *__restrict__ pos, int32_t *err) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= m) return;
-  const int r = dofs[q];
+  const int lane = threadIdx.x & 63;
+  const int r = q < m ? dofs[q] : -1;
+  // lane = rank ndof + first (half a lane more keeps the quotient off the integers)
+  const int rank = (int)(((float)lane + 0.5f) * __builtin_amdgcn_rcpf((float)ndof)), first = lane - rank * ndof;
+  const unsigned long long after = step << first;
+  const unsigned long long same = __ballot(__shfl_up(r, ndof < 64 ? ndof : 0, 64) == r && rank > 0);
+  const bool whole = after != 0ull && (same & after) == after;
   if (r >= n) atomicOr(err, 8);
-  else if (r >= 0) pos[q] = atomicAdd(&cnt[r], 1);
+  const bool valid = r >= 0 && r < n;
+  int p = 0;
+  if (valid && (!whole || rank == 0)) p = atomicAdd(&cnt[r], whole ? 1 + __popcll(after) : 1);
+  const int base = __shfl(p, first, 64);
+  if (valid) pos[q] = whole ? base + rank : p;
 }
 
 // adj[off[r] ..] = the elements of dof r
@@ -133,20 +152,49 @@ __device__ __forceinline__ int row_unique(int c, int ndof, const int32_t *__rest
   return m;
 }
 
+// Rows by the number of their candidates (deg x ndof): up to ROW_SHORT in
+// k_row_columns, a wave each with 4 registers or fewer; up to ROW_WAVE in
+// k_long_rows, whose registers would cost the short rows their waves; up to
+// ROW_SORT, a block each that sorts them in LDS; more (a dof of nearly every
+// element: a global multiplier, the hub of a fan), a block for every window of
+// ROW_WIN columns that marks the window's columns in a bitmap in LDS.  So every
+// row costs about as much per candidate, whatever its length (log^2 in the
+// sorts): 32^3 cells of 6 tetrahedra, P2 and one dof more in every element
+// (2.2 M candidates in its row): 1446 us, 5340 by the radix sort.
+constexpr int ROW_SHORT = 256, ROW_WAVE = 1024;
+constexpr int ROW_SORT = 4096;      // (8^3 cells, P1 and one dof in every element: 157 us with the row of 15,360
+                                    // candidates sorted, 37 us by a window)
+constexpr int ROW_WIN = 1 << 20;    // 128 KB of bits
+constexpr int ROW_BLK = 1024;       // threads of a block
+constexpr int ROW_BLOCKS = 256;     // blocks of k_long_rows (one in a CU)
+
+// The rows of more than ROW_WAVE candidates: those up to ROW_SORT from the
+// front of `rows`, the others from its back; cnt their numbers, cnt[2]: there
+// are rows of more than ROW_SHORT.
+struct RowList {
+  int32_t *rows, *cnt;
+  int cap;
+};
+
 // the sorted distinct columns of every row at cols[off[r] * ndof ..], their
-// number in len[r]; a wave per row.  Rows of up to ROW_SHORT candidates here, the
-// longer ones in k_long_rows, whose registers would cost these their waves.
-constexpr int ROW_SHORT = 256;
+// number in len[r]; a wave per row
 __global__ __launch_bounds__(256) void k_row_columns(int n, int ndof, const int32_t *__restrict__ off,
                                                      const int32_t *__restrict__ adj,
                                                      const int32_t *__restrict__ dofs, int32_t *__restrict__ cols,
-                                                     int32_t *__restrict__ len) {
+                                                     int32_t *__restrict__ len, RowList L) {
   const int lane = threadIdx.x & 63;
   const long long nw = (long long)gridDim.x * 4;
   for (long long r = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); r < n; r += nw) {
     const int o = off[r], deg = off[r + 1] - o;
     const long long c = (long long)deg * ndof;
-    if (c > ROW_SHORT) continue;
+    if (c > ROW_SHORT) {
+      if (lane == 0) L.cnt[2] = 1;
+      if (c > ROW_WAVE && lane == 0) {
+        const int k = atomicAdd(&L.cnt[c > ROW_SORT], 1);
+        L.rows[c > ROW_SORT ? L.cap - 1 - k : k] = (int32_t)r;
+      }
+      continue;
+    }
     const int32_t *a = adj + o;
     int32_t *out = cols + (size_t)o * ndof;
     int m = 0;
@@ -158,59 +206,205 @@ __global__ __launch_bounds__(256) void k_row_columns(int n, int ndof, const int3
   }
 }
 
-// a wave looks through 64 rows and takes the long ones in turn
-__global__ __launch_bounds__(256) void k_long_rows(int n, int ndof, const int32_t *__restrict__ off,
-                                                   const int32_t *__restrict__ adj, const int32_t *__restrict__ dofs,
-                                                   int32_t *__restrict__ cols, int32_t *__restrict__ len) {
-  const int lane = threadIdx.x & 63;
-  const long long nw = (long long)gridDim.x * 4;
-  for (long long r0 = 64LL * __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); r0 < n;
-       r0 += 64 * nw) {
-    const long long rl = r0 + lane;
-    const bool lng = rl < n && (long long)(off[rl + 1] - off[rl]) * ndof > ROW_SHORT;
-    for (unsigned long long mk = __ballot(lng); mk; mk &= mk - 1) {
-      const long long r = r0 + __builtin_ctzll(mk);
-      const int o = off[r], deg = off[r + 1] - o;
-      const long long c = (long long)deg * ndof;
-      const int32_t *a = adj + o;
-      int32_t *out = cols + (size_t)o * ndof;
-      int m = 0;
-      if (c <= 512) m = row_unique<8>((int)c, ndof, a, dofs, n, out);
-      else if (c <= 1024) m = row_unique<16>((int)c, ndof, a, dofs, n, out);
-      else {
-        // a few very long rows: the next larger column, one at a time
-        for (int32_t last = -1;;) {
-          int32_t best = NO_COL;
-          for (long long q = lane; q < c; q += 64) {
-            const int32_t x = dofs[(size_t)a[q / ndof] * ndof + (int)(q % ndof)];
-            if (x > last && x < n && x < best) best = x;
-          }
+// sum over the ROW_BLK threads of v below this one; total: of all (part: 16 words)
+__device__ __forceinline__ int block_prefix(int v, int32_t *part, int &total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int incl = v;
 #pragma unroll
-          for (int s = 32; s > 0; s >>= 1) best = min(best, __shfl_xor(best, s, 64));
-          if (best == NO_COL) break;
-          if (lane == 0) out[m] = best;
-          ++m;
-          last = best;
+  for (int s = 1; s < 64; s <<= 1) {
+    const int y = __shfl_up(incl, s, 64);
+    if (lane >= s) incl += y;
+  }
+  __syncthreads();
+  if (lane == 63) part[w] = incl;
+  __syncthreads();
+  int before = 0;
+  total = 0;
+#pragma unroll
+  for (int k = 0; k < ROW_BLK / 64; ++k) {
+    const int p = part[k];
+    before += k < w ? p : 0;
+    total += p;
+  }
+  return before + incl - v;
+}
+
+// a block's row: its candidates sorted in LDS, equal ones dropped
+__device__ __forceinline__ void row_sorted(int c, int ndof, const int32_t *__restrict__ adj,
+                                           const int32_t *__restrict__ dofs, int n, int32_t *__restrict__ cols,
+                                           int32_t *len, int32_t *v, int32_t *part) {
+  int m = 2 * ROW_WAVE;
+  while (m < c) m <<= 1;
+  __syncthreads();  // (the row before)
+  for (int q = threadIdx.x; q < m; q += ROW_BLK) {
+    int32_t x = NO_COL;
+    if (q < c) {
+      const unsigned d = (unsigned)q / (unsigned)ndof;
+      x = dofs[(size_t)adj[d] * ndof + (q - (int)d * ndof)];
+      if (x < 0 || x >= n) x = NO_COL;
+    }
+    v[q] = x;
+  }
+  for (int size = 2; size <= m; size <<= 1)
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      __syncthreads();
+      for (int i = threadIdx.x; i < m / 2; i += ROW_BLK) {
+        const int a = 2 * i - (i & (stride - 1)), b = a + stride;
+        const int32_t x = v[a], y = v[b];
+        if ((x > y) == ((a & size) == 0)) {
+          v[a] = y;
+          v[b] = x;
         }
       }
+    }
+  __syncthreads();
+  int done = 0;
+  for (int q0 = 0; q0 < m; q0 += ROW_BLK) {
+    const int q = q0 + (int)threadIdx.x;
+    const int32_t x = v[q];
+    const bool first = x != NO_COL && (q == 0 || v[q - 1] != x);
+    int total;
+    const int at = block_prefix(first ? 1 : 0, part, total);
+    if (first) cols[done + at] = x;
+    done += total;
+  }
+  if (threadIdx.x == 0) *len = done;
+}
+
+// a block's window w of a row: marks the columns w ROW_WIN .. in a bitmap in
+// LDS and writes them (cols != nullptr) in order; returns their number
+__device__ __forceinline__ int row_window(unsigned c, int ndof, const int32_t *__restrict__ adj,
+                                          const int32_t *__restrict__ dofs, int n, int w, int32_t *__restrict__ cols,
+                                          uint32_t *bits, int32_t *part) {
+  const int base = w * ROW_WIN;
+  const int words = (min(n - base, ROW_WIN) + 31) / 32;
+  __syncthreads();  // (the window before)
+  for (int k = threadIdx.x; k < words; k += ROW_BLK) bits[k] = 0u;
+  __syncthreads();
+  constexpr int U = 8;  // candidates in flight per thread
+  for (unsigned q0 = 0; q0 < c; q0 += U * ROW_BLK) {
+    int32_t x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned q = min(q0 + u * ROW_BLK + threadIdx.x, c - 1);  // (past the end: the last one again)
+      const unsigned d = q / (unsigned)ndof;
+      x[u] = dofs[(size_t)adj[d] * ndof + (q - d * ndof)];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (x[u] >= base && x[u] < n && x[u] - base < ROW_WIN)
+        atomicOr(&bits[(x[u] - base) >> 5], 1u << (x[u] & 31));
+  }
+  __syncthreads();
+  int done = 0;
+  for (int k0 = 0; k0 < words; k0 += ROW_BLK) {
+    const int k = k0 + (int)threadIdx.x;
+    uint32_t b = k < words ? bits[k] : 0u;
+    int total;
+    int at = done + block_prefix(__popc(b), part, total);
+    if (cols)
+      for (; b; b &= b - 1) cols[at++] = base + 32 * k + __builtin_ctz(b);
+    done += total;
+  }
+  return done;
+}
+
+// The blocks take the list's rows; then a wave looks through `span` rows and takes
+// those of up to ROW_WAVE candidates in turn.  With nwin > 1 windows (of columns) the
+// list's longest rows are only counted here, in wcnt, and written by
+// k_window_rows.
+__global__ __launch_bounds__(ROW_BLK) void k_long_rows(int n, int ndof, const int32_t *__restrict__ off,
+                                                       const int32_t *__restrict__ adj,
+                                                       const int32_t *__restrict__ dofs, int32_t *__restrict__ cols,
+                                                       int32_t *__restrict__ len, RowList L, int span, int nwin,
+                                                       int32_t *__restrict__ wcnt) {
+  __shared__ int32_t row_lds[ROW_WIN / 32], part[ROW_BLK / 64];
+  if (!L.cnt[2]) return;
+  const int ns = L.cnt[0];
+  for (int k = blockIdx.x; k < ns; k += gridDim.x) {
+    const int r = L.rows[k], o = off[r];
+    row_sorted((off[r + 1] - o) * ndof, ndof, adj + o, dofs, n, cols + (size_t)o * ndof, len + r, row_lds, part);
+  }
+  const long long nt = (long long)L.cnt[1] * nwin;
+  for (long long t = blockIdx.x; t < nt; t += gridDim.x) {
+    const int k = (int)(t / nwin), w = (int)(t - (long long)k * nwin);
+    const int r = L.rows[L.cap - 1 - k], o = off[r];
+    const int m = row_window((unsigned)(off[r + 1] - o) * ndof, ndof, adj + o, dofs, n, w,
+                             nwin == 1 ? cols + (size_t)o * ndof : nullptr, (uint32_t *)row_lds, part);
+    if (threadIdx.x == 0) {
+      if (nwin == 1) len[r] = m;
+      else wcnt[t] = m;
+    }
+  }
+  const int lane = threadIdx.x & 63;
+  const long long nw = (long long)gridDim.x * (ROW_BLK / 64);
+  for (long long r0 =
+           (long long)span * __builtin_amdgcn_readfirstlane(blockIdx.x * (ROW_BLK / 64) + (threadIdx.x >> 6));
+       r0 < n; r0 += span * nw) {
+    const long long rl = r0 + lane;
+    const long long cl = lane < span && rl < n ? (long long)(off[rl + 1] - off[rl]) * ndof : 0;
+    for (unsigned long long mk = __ballot(cl > ROW_SHORT && cl <= ROW_WAVE); mk; mk &= mk - 1) {
+      const long long r = r0 + __builtin_ctzll(mk);
+      const int o = off[r], c = (off[r + 1] - o) * ndof;
+      const int32_t *a = adj + o;
+      int32_t *out = cols + (size_t)o * ndof;
+      const int m = c <= 512 ? row_unique<8>(c, ndof, a, dofs, n, out) : row_unique<16>(c, ndof, a, dofs, n, out);
       if (lane == 0) len[r] = m;
     }
   }
 }
 
-// rows to their places; 16 lanes per row
+// the windows of the list's longest rows, each behind the windows before it
+__global__ __launch_bounds__(ROW_BLK) void k_window_rows(int n, int ndof, const int32_t *__restrict__ off,
+                                                         const int32_t *__restrict__ adj,
+                                                         const int32_t *__restrict__ dofs, int32_t *__restrict__ cols,
+                                                         int32_t *__restrict__ len, RowList L, int nwin,
+                                                         const int32_t *__restrict__ wcnt) {
+  __shared__ int32_t row_lds[ROW_WIN / 32], part[ROW_BLK / 64];
+  const long long nt = (long long)L.cnt[1] * nwin;
+  for (long long t = blockIdx.x; t < nt; t += gridDim.x) {
+    const int k = (int)(t / nwin), w = (int)(t - (long long)k * nwin);
+    const int r = L.rows[L.cap - 1 - k], o = off[r];
+    int v = 0, before;
+    for (int j = threadIdx.x; j < w; j += ROW_BLK) v += wcnt[(long long)k * nwin + j];
+    block_prefix(v, part, before);
+    const int m = row_window((unsigned)(off[r + 1] - o) * ndof, ndof, adj + o, dofs, n, w,
+                             cols + (size_t)o * ndof + before, (uint32_t *)row_lds, part);
+    if (w == nwin - 1 && threadIdx.x == 0) len[r] = before + m;
+  }
+}
+
+// rows to their places; 16 lanes per row, and PLACE_BLOCKS blocks for the rows
+// of the list (one each, the longest ones all together)
+constexpr int PLACE_BLOCKS = 256;
 __global__ __launch_bounds__(256) void k_place_rows(int n, int ndof, const int32_t *__restrict__ off,
                                                     const int32_t *__restrict__ cols,
                                                     const int32_t *__restrict__ row_ptr, int32_t *__restrict__ col_idx,
-                                                    long long cap, int32_t *__restrict__ nnz, int32_t *err) {
-  const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+                                                    long long cap, RowList L, int32_t *__restrict__ nnz,
+                                                    int32_t *err) {
+  if (blockIdx.x < PLACE_BLOCKS) {
+    auto place = [&](int r, int first, int step) {
+      const int32_t *src = cols + (size_t)off[r] * ndof;
+      const int p0 = row_ptr[r], p1 = row_ptr[r + 1];
+      for (long long j = (long long)p0 + first; j < p1; j += step)
+        if (j < cap) col_idx[j] = src[j - p0];
+    };
+    const int ns = L.cnt[0], nh = L.cnt[1];
+    for (int k = blockIdx.x; k < ns; k += PLACE_BLOCKS) place(L.rows[k], threadIdx.x, 256);
+    for (int k = 0; k < nh; ++k)
+      place(L.rows[L.cap - 1 - k], blockIdx.x * 256 + threadIdx.x, PLACE_BLOCKS * 256);
+    return;
+  }
+  const long long g = (long long)(blockIdx.x - PLACE_BLOCKS) * blockDim.x + threadIdx.x;
   if (g == 0) {
     *nnz = row_ptr[n];
     if ((long long)row_ptr[n] > cap) atomicOr(err, 4);
   }
   const long long r = g >> 4;
   if (r >= n) return;
-  const int32_t *src = cols + (size_t)off[r] * ndof;
+  const int o = off[r];
+  if ((long long)(off[r + 1] - o) * ndof > ROW_WAVE) return;
+  const int32_t *src = cols + (size_t)o * ndof;
   const int p0 = row_ptr[r], p1 = row_ptr[r + 1];
   for (int j = p0 + (int)(g & 15); j < p1; j += 16)
     if (j < cap) col_idx[j] = src[j - p0];
@@ -285,29 +479,49 @@ extern "C" int xg_csr_pattern(xg_ctx *ctx, int nel, int ndof, const int32_t *dof
     const size_t b_n = align256(sizeof(int32_t) * (size_t)n1), b_m = align256(sizeof(int32_t) * (size_t)m);
     const size_t o_off = b_n, o_adj = 2 * b_n, o_pos = o_adj + b_m, o_col = o_pos + b_m;
     const size_t o_tmp = o_col + align256(sizeof(int32_t) * (size_t)nent);
-    const int rc = ensure_ws(ctx, o_tmp + t_scan);
+    // the list of long rows (the candidates of all rows are at most the
+    // couplings), its two counters, the window counts of the longest
+    RowList list{nullptr, nullptr, (int)(nent / (ROW_WAVE + 1)) + 1};
+    const int nwin = (int)(((long long)n + ROW_WIN - 1) / ROW_WIN);
+    const size_t o_list = o_tmp + align256(t_scan), o_lcnt = o_list + align256(sizeof(int32_t) * (size_t)list.cap);
+    const size_t o_wcnt = o_lcnt + 256;
+    const size_t b_wcnt = nwin > 1 ? sizeof(int32_t) * (size_t)(nent / (ROW_SORT + 1) + 1) * nwin : 0;
+    const int rc = ensure_ws(ctx, o_wcnt + b_wcnt);
     if (rc != XG_OK) return rc;
     char *ws = (char *)ctx->ws;
     int32_t *cnt = (int32_t *)ws, *off = (int32_t *)(ws + o_off), *pos = (int32_t *)(ws + o_pos);
-    int32_t *adj = (int32_t *)(ws + o_adj), *cols = (int32_t *)(ws + o_col);
+    int32_t *adj = (int32_t *)(ws + o_adj), *cols = (int32_t *)(ws + o_col), *wcnt = (int32_t *)(ws + o_wcnt);
+    list.rows = (int32_t *)(ws + o_list);
+    list.cnt = (int32_t *)(ws + o_lcnt);
     const unsigned g_n = (unsigned)((n1 + 255) / 256), g_m = (unsigned)((m + 255) / 256);
-    k_fill_i32<<<g_n, 256, 0, st>>>(cnt, n1, 0);
-    k_dof_count<<<g_m, 256, 0, st>>>(m, dofs, n, cnt, pos, ctx->d_err);
+    k_fill_i32<<<g_n, 256, 0, st>>>(cnt, n1, 0, list.cnt);
+    unsigned long long step = 0;
+    for (int k = ndof; k < 64; k += ndof) step |= 1ull << k;
+    k_dof_count<<<g_m, 256, 0, st>>>(m, ndof, step, dofs, n, cnt, pos, ctx->d_err);
     XG_LAUNCH_CHECK();
     XG_CHECK(hipcub::DeviceScan::ExclusiveSum(ws + o_tmp, t_scan, cnt, off, (int)n1, st));
     k_dof_elements<<<g_m, 256, 0, st>>>(m, ndof, dofs, n, off, pos, adj);
     XG_LAUNCH_CHECK();
     // (the counts' buffer takes the row lengths; its last entry stays 0)
-    const long long want = ((long long)n + 3) / 4, wl = ((long long)n + 255) / 256;
-    if (n > 0) {
-      k_row_columns<<<(unsigned)(want < 65536 ? want : 65536), 256, 0, st>>>(n, ndof, off, adj, dofs, cols, cnt);
-      k_long_rows<<<(unsigned)(wl < 65536 ? wl : 65536), 256, 0, st>>>(n, ndof, off, adj, dofs, cols, cnt);
-    }
+    // a wave for each row that may be long, up to ROW_BLOCKS x 16; as many rows
+    // for each to look through
+    const long long most = nent / (ROW_SHORT + 1) / (ROW_BLK / 64) + 1;
+    const unsigned g_long = (unsigned)(most < ROW_BLOCKS ? most : ROW_BLOCKS);
+    int span = 1;
+    while (span < 64 && (long long)g_long * (ROW_BLK / 64) * span < n) span *= 2;
+    const long long want = ((long long)n + 3) / 4;
+    k_row_columns<<<(unsigned)(want < 65536 ? want : 65536), 256, 0, st>>>(n, ndof, off, adj, dofs, cols, cnt, list);
     XG_LAUNCH_CHECK();
+    k_long_rows<<<g_long, ROW_BLK, 0, st>>>(n, ndof, off, adj, dofs, cols, cnt, list, span, nwin, wcnt);
+    XG_LAUNCH_CHECK();
+    if (nwin > 1) {
+      k_window_rows<<<ROW_BLOCKS, ROW_BLK, 0, st>>>(n, ndof, off, adj, dofs, cols, cnt, list, nwin, wcnt);
+      XG_LAUNCH_CHECK();
+    }
     XG_CHECK(hipcub::DeviceScan::ExclusiveSum(ws + o_tmp, t_scan, cnt, row_ptr, (int)n1, st));
-    const long long thr = (long long)(n > 0 ? n : 1) * 16;
-    k_place_rows<<<(unsigned)((thr + 255) / 256), 256, 0, st>>>(n, ndof, off, cols, row_ptr, col_idx, cap, nnz,
-                                                                ctx->d_err);
+    const long long thr = (long long)n * 16;
+    k_place_rows<<<(unsigned)(PLACE_BLOCKS + (thr + 255) / 256), 256, 0, st>>>(n, ndof, off, cols, row_ptr, col_idx,
+                                                                               cap, list, nnz, ctx->d_err);
     XG_LAUNCH_CHECK();
     return XG_OK;
   }

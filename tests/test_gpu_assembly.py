@@ -150,10 +150,9 @@ def test_csr_pattern_device_matches_numpy(dev_abi):
 @pytest.mark.parametrize("ndof,deg,n", [(1, 1, 1), (3, 21, 50), (3, 22, 50), (4, 32, 9), (8, 33, 700), (10, 25, 900),
                                         (10, 52, 40), (20, 51, 3000), (20, 52, 3000), (64, 90, 4000), (64, 300, 700)])
 def test_csr_pattern_row_lengths(dev_abi, ndof, deg, n):
-    """rows of every length that changes how they are sorted (64, 128, .. 1024
-    candidates per row, longer ones, and the radix sort of dense tables), with
-    skipped dofs, repeated dofs in an element and empty rows; a column list
-    that is too short is an error"""
+    """tables of 1 to 6390 couplings per row on average, on both sides of 256,
+    where they go to the radix sort, with skipped dofs, repeated dofs in an
+    element and empty rows; a column list that is too short is an error"""
     torch, _abi, ctx = dev_abi
     rng = np.random.default_rng(ndof * deg + n)
     nel = max(1, deg * max(n // 3, 1) // ndof)
@@ -164,6 +163,13 @@ def test_csr_pattern_row_lengths(dev_abi, ndof, deg, n):
         dofs[::5, 2] = -1
         dofs[::3, 1] = dofs[::3, 0]
     dofs[dofs == n - 1] = -1  # an empty last row
+    check_graph(dev_abi, dofs, n)
+
+
+def check_graph(dev_abi, dofs, n):
+    """xg_csr_pattern of a dof table against the sorted distinct pairs"""
+    torch, _abi, ctx = dev_abi
+    ndof = dofs.shape[1]
     rows = np.repeat(dofs, ndof, axis=1).ravel().astype(np.int64)
     cols = np.tile(dofs, (1, ndof)).ravel().astype(np.int64)
     ok = (rows >= 0) & (cols >= 0)
@@ -182,6 +188,54 @@ def test_csr_pattern_row_lengths(dev_abi, ndof, deg, n):
         ctx.csr_pattern(d, n, rp, ci[:len(key) - 1], nnz)
         with pytest.raises(RuntimeError):
             ctx.sync()
+
+
+@pytest.mark.parametrize("n", [30000, 1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("scale", [1, 64])
+def test_csr_pattern_long_rows(dev_abi, n, scale):
+    """rows of 56, 64, 72, .. 520 candidates and of 64 times as many in a table
+    that is short on average: both sides of every length at which a row goes
+    to other lanes (64, 128, 256, 512, 1024, 4096), rows of tens of thousands,
+    the rows' columns over the whole range"""
+    rng = np.random.default_rng(n + scale)
+    ndof, degs = 8, scale * np.array([7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65])
+    if scale == 64:
+        degs = np.concatenate([degs, [128, 129, 4095, 4096, 4097]])
+    nel = 9000
+    dofs = rng.integers(len(degs), n, (nel, ndof)).astype(np.int32)
+    dofs[::7, 6] = n - 1
+    dofs[::11, 5] = len(degs)
+    dofs[::9, 7] = -1
+    left = np.full(nel, 5)  # free columns of an element
+    for r, k in sorted(enumerate(degs), key=lambda t: -t[1]):
+        e = rng.permutation(np.nonzero(left > 0)[0])
+        e = e[np.argsort(-left[e], kind="stable")][:k]
+        left[e] -= 1
+        dofs[e, left[e]] = r
+    got = np.bincount(dofs[dofs >= 0], minlength=len(degs))[:len(degs)]
+    assert np.array_equal(got, degs)
+    assert nel * ndof * ndof <= 256 * n  # row by row, not the radix sort
+    check_graph(dev_abi, dofs, n)
+
+
+@pytest.mark.parametrize("nel,ndof,shared,n", [(40000, 5, 1, 9000), (20000, 4, 3, 9000), (20000, 4, 2, 2500000),
+                                               (8200, 4, 4, 4000)])
+def test_csr_pattern_dof_of_every_element(dev_abi, nel, ndof, shared, n):
+    """dofs that every element has (a global multiplier): rows of tens of
+    thousands of candidates, over one and over three windows of columns; with
+    every dof shared, all rows but those are empty"""
+    rng = np.random.default_rng(nel + shared)
+    dofs = rng.integers(0, n, (nel, ndof)).astype(np.int32)
+    for k in range(shared):
+        dofs[:, k] = k * n // shared + k  # rows in different windows
+    if shared < ndof:
+        dofs[::5, shared] = n - 1
+        dofs[1::5, shared] = 0
+        dofs[2::5, shared] = dofs[2::5, 0]  # twice in an element
+        dofs[3::5, shared] = min(n, 1 << 20) - 1
+        dofs[4::5, shared] = min(n - 1, 1 << 20)
+    assert nel * ndof * ndof <= 256 * n and nel * ndof > 4096
+    check_graph(dev_abi, dofs, n)
 
 
 @pytest.mark.parametrize("p", [1, 2])
