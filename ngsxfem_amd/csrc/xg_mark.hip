@@ -189,18 +189,19 @@ __global__ __launch_bounds__(NB, 6) void k_mark(int ne, const int32_t *__restric
   // element rows of all EPT elements, then their level-set values.  The
   // loads are unconditional (lanes past the end read the last element
   // again): a load under a branch is waited for at the branch's end, which
-  // would serialise the EPT round trips.  BIG: rows,
-  // domains and cut ratios pass once and are kept from displacing the level set
-  // in the caches (128^3 cells: 126.3 -> 122.3 us with the compaction; blocks
-  // mapped so that an XCD has consecutive ones: 146.8 us).
+  // would serialise the EPT round trips.  BIG: domains and cut ratios are
+  // stored past the caches, so that they do not displace rows and level set
+  // there.  With the compaction, us, plain / these stores / the rows past the
+  // caches too: tetrahedra 1.3 M 27.0 / 25.9 / 27.0, 6 M 56.7 / 56.4 / 63.8,
+  // 12.6 M 118.7 / 100.1 / 115.6; 4.5 M triangles 38.6 / 37.4 / 37.4, 8 M
+  // segments 51.5 / 49.1 / 49.0.  (Blocks mapped so that an XCD has consecutive
+  // ones: 146.8 at 12.6 M.)
   int vi[EPT][D + 1];
 #pragma unroll
   for (int k = 0; k < EPT; ++k) {
     const int ec = min(base + k * NB + tid, ne - 1);
     if constexpr (D == 3) {
-      typedef int v4 __attribute__((ext_vector_type(4)));
-      const v4 *row = reinterpret_cast<const v4 *>(el2v) + ec;
-      const v4 v = BIG ? __builtin_nontemporal_load(row) : *row;
+      const int4 v = reinterpret_cast<const int4 *>(el2v)[ec];
       vi[k][0] = v.x;
       vi[k][1] = v.y;
       vi[k][2] = v.z;
@@ -831,9 +832,10 @@ size_t mark_scratch_ints(int ne) {
 // marking + compaction on an explicit stream with caller-owned scratch
 // (mark_scratch_ints(ne) int32); only kernel launches, so the sequence can be
 // captured into a hipGraph.  n_cut (nullable) receives the cut count.
-// rows, domains and cut ratios of 2^20 elements (25 MB on tets) are more than
-// the L2s hold; on smaller meshes the next kernel finds them there, and the
-// plain accesses are 1 us faster (60 x 60 cells: 35.4 against 36.5 us a step)
+// domains and cut ratios of 2^20 elements (9 MB beside 16 MB of rows on tets)
+// are more than the L2s hold; on smaller meshes the next kernel finds them
+// there, and the plain stores are 1 us faster (60 x 60 cells: 35.4 against 36.5
+// us a step)
 static void launch_mark(hipStream_t st, int D, int nblk, int ne, const int32_t *el2v, const double *lset, uint8_t *dt,
                         double *cr, uint32_t *bits, int nw, int32_t *blk, int32_t *err) {
 #define XG_MARK(DD)                                                                                              \
