@@ -33,12 +33,30 @@ __device__ __forceinline__ void element_geometry(const int32_t *__restrict__ el2
   }
 }
 
+constexpr int CF_BLK = 256;
+inline size_t cf_lds(const cf::Prog &P, bool regs) {  // host
+  return regs ? 0 : sizeof(double) * CF_BLK * (size_t)(P.depth > 1 ? P.depth - 1 : 1);
+}
+inline bool cf_regs(const cf::Prog &P) { return P.depth <= 4 && !P.math; }  // host
+template <int D, bool REGS, bool MATH>
+__device__ __forceinline__ double cf_value(const cf::Prog &P, const double *x, const double *lam, const int32_t *vv,
+                                           int e) {
+  extern __shared__ double cf_stack[];
+  if constexpr (REGS) return cf::eval<D, 4, false>(P, x, lam, vv, e);
+  else return cf::eval_mem<D, MATH>(P, x, lam, vv, e, cf_stack + threadIdx.x, CF_BLK);
+}
+
 // w_q <- w_q * cf(x_q) for every point of every listed element; the
 // element's vertices have A coordinates (A = D, or D + 1 for boundary
 // elements given in the ambient space), x_q = sum_k lam_k X_k
-// DEPTH: registers of the program's stack (4, or 16 for deeper programs); MATH:
-// the program calls library functions
-template <int D, int A, int DEPTH, bool MATH>
+// REGS: the program's stack is 4 registers; else it is in LDS (cf_lds bytes);
+// MATH: the program calls library functions.  Bound: for few points the chain of
+// an operation's fetch and branches, 100 to 200 cycles each.  us, stack in scratch
+// memory / 16 registers / LDS with decoded operations, 40,000 cut tetrahedra of
+// order 4: nine operands 216 / 182 / 67, the same with an exp 232 / 335 / 171; 64
+// of order 15: 104 / 164 / 72, 112 / 179 / 82.  Four registers, before and after
+// the decoding: three operands 69 / 42, 74 / 42 for one element of order 15.
+template <int D, int A, bool REGS, bool MATH>
 __global__ __launch_bounds__(256) void k_rule_scale_cf(int nel, const int32_t *__restrict__ elems,
                                                        const int32_t *__restrict__ el2v,
                                                        const double *__restrict__ coords,
@@ -76,7 +94,7 @@ __global__ __launch_bounds__(256) void k_rule_scale_cf(int nel, const int32_t *_
         for (int c = 0; c < D; ++c) a += (V[c][r] - V[D][r]) * xi[c];
         x[r] = a;
       }
-      p.w *= cf::eval<D, DEPTH, MATH>(P, x, lam, vv, e);
+      p.w *= cf_value<D, REGS, MATH>(P, x, lam, vv, e);
       pts[q] = p;
     }
   }
@@ -137,8 +155,8 @@ __global__ __launch_bounds__(256) void k_elvec_rule(int nel, const int32_t *__re
 // InterpolateP1::Do (utils/p1interpol.cpp:27-113): the coefficient at every
 // vertex, then the perturbation |v| < eps -> eps (:104-107); one lane per
 // vertex (a grid function opcode reads the vertex's own value)
-template <int D>
-__global__ __launch_bounds__(256) void k_p1_interpolate_cf(int nv, const double *__restrict__ coords, const cf::Prog P,
+template <int D, bool REGS, bool MATH>
+__global__ __launch_bounds__(CF_BLK) void k_p1_interpolate_cf(int nv, const double *__restrict__ coords, const cf::Prog P,
                                                            double eps, double *__restrict__ out) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= nv) return;
@@ -151,7 +169,7 @@ __global__ __launch_bounds__(256) void k_p1_interpolate_cf(int nv, const double 
     lam[k] = k == 0 ? 1.0 : 0.0;
     vv[k] = v;
   }
-  double val = cf::eval<D>(P, x, lam, vv, -1);
+  double val = cf_value<D, REGS, MATH>(P, x, lam, vv, -1);
   if (fabs(val) < eps) val = eps;
   out[v] = val;
 }
@@ -256,12 +274,14 @@ extern "C" int xg_rule_scale_cf(xg_ctx *ctx, int D, int A, int nel, const int32_
   if (!el2v || !coords || !offsets || !pts) return set_error(XG_ERR_ARG, "xg_rule_scale_cf: null pointer");
   const int grid = cf_grid(nel);
   double4 *p = reinterpret_cast<double4 *>(pts);
-#define XG_SC1(DD, AA, DEPTH, MATH) \
-  k_rule_scale_cf<DD, AA, DEPTH, MATH><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, P)
-#define XG_SC(DD, AA)                                    \
-  if (P.depth <= 4 && !P.math) XG_SC1(DD, AA, 4, false); \
-  else if (!P.math) XG_SC1(DD, AA, 16, false);           \
-  else XG_SC1(DD, AA, 16, true)
+  const bool regs = cf_regs(P);
+  const size_t lds = cf_lds(P, regs);
+#define XG_SC1(DD, AA, REGS, MATH) \
+  k_rule_scale_cf<DD, AA, REGS, MATH><<<grid, CF_BLK, lds, ctx->stream>>>(nel, elems, el2v, coords, offsets, p, P)
+#define XG_SC(DD, AA)                             \
+  if (regs) XG_SC1(DD, AA, true, false);          \
+  else if (!P.math) XG_SC1(DD, AA, false, false); \
+  else XG_SC1(DD, AA, false, true)
   switch (D * 4 + A) {
     case 5: XG_SC(1, 1); break;
     case 6: XG_SC(1, 2); break;
@@ -285,12 +305,22 @@ extern "C" int xg_p1_interpolate_cf(xg_ctx *ctx, int D, int nv, const double *co
     return set_error(XG_ERR_ARG, "xg_p1_interpolate_cf: piecewise constant grid functions have no vertex values");
   if (nv == 0) return XG_OK;
   if (!coords || !out) return set_error(XG_ERR_ARG, "xg_p1_interpolate_cf: null pointer");
-  const int grid = (nv + 255) / 256;
+  const int grid = (nv + CF_BLK - 1) / CF_BLK;
+  const bool regs = cf_regs(P);
+  const size_t lds = cf_lds(P, regs);
+#define XG_IP1(DD, REGS, MATH) \
+  k_p1_interpolate_cf<DD, REGS, MATH><<<grid, CF_BLK, lds, ctx->stream>>>(nv, coords, P, eps, out)
+#define XG_IP(DD)                             \
+  if (regs) XG_IP1(DD, true, false);          \
+  else if (!P.math) XG_IP1(DD, false, false); \
+  else XG_IP1(DD, false, true)
   switch (D) {
-    case 1: k_p1_interpolate_cf<1><<<grid, 256, 0, ctx->stream>>>(nv, coords, P, eps, out); break;
-    case 2: k_p1_interpolate_cf<2><<<grid, 256, 0, ctx->stream>>>(nv, coords, P, eps, out); break;
-    default: k_p1_interpolate_cf<3><<<grid, 256, 0, ctx->stream>>>(nv, coords, P, eps, out); break;
+    case 1: XG_IP(1); break;
+    case 2: XG_IP(2); break;
+    default: XG_IP(3); break;
   }
+#undef XG_IP
+#undef XG_IP1
   XG_LAUNCH_CHECK();
   return XG_OK;
 }

@@ -34,6 +34,16 @@ extern "C" int cf_load(int ncode, const int *code, int nconst, const double *con
 extern "C" void cf_eval(int n, const double *x, const double *lam, const int *vv, double *out) {
   for (int i = 0; i < n; ++i) out[i] = eval<3>(prog, x + 3 * i, lam + 4 * i, vv, 5);
 }
+// the same with the stack in memory, its entries 3 doubles apart; -1 if one of
+// them lies past the depth that the program was found to need
+extern "C" int cf_eval_mem(int n, const double *x, const double *lam, const int *vv, double *out) {
+  double st[3 * MAXSTACK + 1];
+  for (double &v : st) v = -7.0;
+  for (int i = 0; i < n; ++i) out[i] = eval_mem<3, true>(prog, x + 3 * i, lam + 4 * i, vv, 5, st, 3);
+  for (int k = 3 * (prog.depth - 1); k <= 3 * MAXSTACK; ++k)
+    if (st[k] != -7.0) return -1;
+  return prog.depth;
+}
 """
 
 
@@ -140,3 +150,45 @@ def test_grid_function_opcode(cflib):
     got = run(cflib, 50, P, lam, vv)
     ref = (lam * u[vv]).sum(1) * P[:, 0] + 2.0
     np.testing.assert_allclose(got, ref, rtol=1e-14)
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_stack_in_memory_equals_registers(cflib, seed):
+    """random programs of every depth and operation: the evaluation with the
+    stack in memory gives the bits of the one with the stack in registers,
+    and touches no entry past the program's depth"""
+    rng = np.random.default_rng(seed)
+    gf = rng.uniform(0.5, 2.0, 6)
+    code, consts, depth, deepest = [], [], 0, 0
+    target = 1 + seed % 16
+    while len(code) < 150:
+        kind = rng.integers(0, 3) if depth else 0
+        if kind == 0 and depth < target:
+            op = int(rng.choice([1, 2, 19]))
+            if op == 1:
+                consts.append(float(rng.uniform(-2, 2)))
+                if len(consts) > 40:
+                    consts.pop()
+                    op = 2
+            code += [op, len(consts) - 1 if op == 1 else (int(rng.integers(0, 3)) if op == 2 else 0)]
+            depth += 1
+        elif kind == 1 and depth >= 3 and rng.random() < 0.2:
+            code.append(20)
+            depth -= 2
+        elif kind == 1 and depth >= 2:
+            code.append(int(rng.choice([3, 4, 5, 6, 21, 22])))
+            depth -= 1
+        elif kind == 2 and depth:
+            op = int(rng.choice([7, 8, 11, 12, 18]))
+            code += [8, int(rng.integers(-3, 4))] if op == 8 else [op]
+        deepest = max(deepest, depth)
+    code += [3] * (depth - 1)
+    r, msg = load(cflib, code, consts, [gf])
+    assert r == 0, msg
+    n = 30
+    x = np.ascontiguousarray(rng.uniform(-1, 1, (n, 3)))
+    lam = np.ascontiguousarray(rng.dirichlet(np.ones(4), n))
+    vv = np.array([0, 2, 3, 5], np.int32)
+    a, b = run(cflib, n, x, lam, vv), np.zeros(n)
+    assert cflib.cf_eval_mem(n, _p(x), _p(lam), _p(vv), _p(b)) == deepest
+    assert np.array_equal(a, b, equal_nan=True)
