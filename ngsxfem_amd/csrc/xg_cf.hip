@@ -100,20 +100,71 @@ __global__ __launch_bounds__(256) void k_rule_scale_cf(int nel, const int32_t *_
   }
 }
 
+// The sums of N values over the 64 lanes, one per lane: at every step a lane
+// gives half of its values to the lane that keeps them, so that all of them
+// take about N shuffles (6 N where every lane keeps all).  Returns the value
+// of index k; lanes with n == 0 have none.  (k = 0, n = N to begin with)
+template <int N, int M>
+__device__ __forceinline__ double wave_sums(double *s, int lane, int &k, int &n) {
+  if constexpr (M == 0) {
+    return s[0];
+  } else if constexpr (N == 1) {
+    s[0] += __shfl_xor(s[0], M, 64);
+    return wave_sums<1, M / 2>(s, lane, k, n);
+  } else {
+    constexpr int H = (N + 1) / 2;
+    const bool up = (lane & M) != 0;
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+      const double a = s[j], b = j + H < N ? s[j + H] : 0.0;
+      s[j] = (up ? b : a) + __shfl_xor(up ? a : b, M, 64);
+    }
+    if (up) k += H;
+    n = up ? max(n - H, 0) : min(n, H);
+    return wave_sums<H, M / 2>(s, lane, k, n);
+  }
+}
+
+template <int D, int P>
+__device__ __forceinline__ void elvec_point(const double4 &p, double *s) {
+  constexpr int N = ndof(D, P);
+  const double xi[3] = {p.x, p.y, p.z};
+  double lam[D + 1], phi[N];
+  double sl = 1.0;
+#pragma unroll
+  for (int c = 0; c < D; ++c) {
+    lam[c] = xi[c];
+    sl -= xi[c];
+  }
+  lam[D] = sl;
+  h1_shape<D, P, double>(lam, phi, (double(*)[D]) nullptr);
+#pragma unroll
+  for (int a = 0; a < N; ++a) s[a] = fma(p.w, phi[a], s[a]);
+}
+
 // out[i][a] = |det F| sum_q w_q phi_a(xi_q): element vectors of the source
 // f = 1 on the rule (f is already in the weights after xg_rule_scale_cf)
-// 16 lanes per element: a wave per element added N sums over 64 lanes by six
-// shuffles each
-template <int D, int P>
+// 16 lanes per element.  FEW (up to ELVEC_FEW elements, which leave waves to
+// spare): a wave per element, all of its lanes for a rule of more than LONG
+// points (so an element's vector may differ in its last bits between a short
+// and a long list; LONG is 96 points where 16 lanes take them as fast).  us, a
+// wave per element and 6 N shuffles / 16 lanes for every element / now, P3 on
+// tetrahedra: 64 elements of order 8 7.3 / 13.0 / 5.3, of order 15 13.0 / 36.9 /
+// 12.7; 2000 of order 15 21.3 / 57.1 / 24.0; 40,000 of order 2 101 / 21 / 21, of
+// order 15 313 / 318 / 318.
+constexpr int ELVEC_FEW = 4096;
+template <int D, int P, bool FEW>
 __global__ __launch_bounds__(256) void k_elvec_rule(int nel, const int32_t *__restrict__ elems,
                                                     const int32_t *__restrict__ el2v,
                                                     const double *__restrict__ coords,
                                                     const int32_t *__restrict__ offsets,
                                                     const double4 *__restrict__ pts, double *__restrict__ out) {
-  constexpr int N = ndof(D, P), G = 16;
-  const int sub = threadIdx.x & (G - 1);
-  const long long ngrp = (long long)gridDim.x * (256 / G);
-  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) / G; i < nel; i += ngrp) {
+  constexpr int N = ndof(D, P), G = 16, LONG = N > 10 ? 32 : 96, T = FEW ? 64 : G;  // lanes of an element
+  const int sub = threadIdx.x & (T - 1);
+  const long long ngrp = (long long)gridDim.x * (256 / T);
+  long long i0 = ((long long)blockIdx.x * 256 + threadIdx.x) / T;
+  if (FEW) i0 = __builtin_amdgcn_readfirstlane((int)i0);
+  for (long long i = i0; i < nel; i += ngrp) {
     const int e = elems ? elems[i] : (int)i;
     int32_t vv[D + 1];
     double V[D + 1][3];
@@ -123,32 +174,25 @@ __global__ __launch_bounds__(256) void k_elvec_rule(int nel, const int32_t *__re
     double s[N];
 #pragma unroll
     for (int a = 0; a < N; ++a) s[a] = 0.0;
-    const int q1 = offsets[i + 1];
-    for (int q = offsets[i] + sub; q < q1; q += G) {
-      const double4 p = pts[q];
-      const double xi[3] = {p.x, p.y, p.z};
-      double lam[D + 1], phi[N];
-      double sl = 1.0;
+    const int q0 = offsets[i], q1 = offsets[i + 1];
+    if (FEW && q1 - q0 > LONG) {
+      for (int q = q0 + sub; q < q1; q += 64) elvec_point<D, P>(pts[q], s);
+      int k = 0, n = N;
+      const double v = wave_sums<N, 32>(s, sub, k, n);
+      if (n > 0) out[(size_t)i * N + k] = absdet * v;
+    } else if (!FEW || sub < G) {
+      for (int q = q0 + sub; q < q1; q += G) elvec_point<D, P>(pts[q], s);
+      double v[(N + G - 1) / G];
 #pragma unroll
-      for (int c = 0; c < D; ++c) {
-        lam[c] = xi[c];
-        sl -= xi[c];
+      for (int a = 0; a < N; ++a) {
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) s[a] += __shfl_xor(s[a], o, G);
+        if (a % G == sub) v[a / G] = s[a];
       }
-      lam[D] = sl;
-      h1_shape<D, P, double>(lam, phi, (double(*)[D]) nullptr);
 #pragma unroll
-      for (int a = 0; a < N; ++a) s[a] = fma(p.w, phi[a], s[a]);
+      for (int a = 0; a < (N + G - 1) / G; ++a)
+        if (a * G + sub < N) out[(size_t)i * N + a * G + sub] = absdet * v[a];
     }
-    double v[(N + G - 1) / G];
-#pragma unroll
-    for (int a = 0; a < N; ++a) {
-#pragma unroll
-      for (int o = G / 2; o > 0; o >>= 1) s[a] += __shfl_xor(s[a], o, G);
-      if (a % G == sub) v[a / G] = s[a];
-    }
-#pragma unroll
-    for (int a = 0; a < (N + G - 1) / G; ++a)
-      if (a * G + sub < N) out[(size_t)i * N + a * G + sub] = absdet * v[a];
   }
 }
 
@@ -350,11 +394,13 @@ extern "C" int xg_elvec(xg_ctx *ctx, int D, int p, int nel, const int32_t *elems
   if (!ctx || D < 1 || D > 3 || p < 1 || p > 3 || nel < 0) return set_error(XG_ERR_ARG, "xg_elvec: bad argument");
   if (nel == 0) return XG_OK;
   if (!el2v || !coords || !offsets || !pts || !out) return set_error(XG_ERR_ARG, "xg_elvec: null pointer");
-  const long long want = ((long long)nel + 15) / 16;
+  const bool few = nel <= ELVEC_FEW;
+  const long long want = ((long long)nel + (few ? 3 : 15)) / (few ? 4 : 16);
   const int grid = (int)(want < 16384 ? want : 16384);
   const double4 *q = reinterpret_cast<const double4 *>(pts);
-#define XG_EV(DD, PP) \
-  k_elvec_rule<DD, PP><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, q, out)
+#define XG_EV(DD, PP)                                                                                       \
+  (few ? k_elvec_rule<DD, PP, true><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, q, out) \
+       : k_elvec_rule<DD, PP, false><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, offsets, q, out))
   switch (D * 4 + p) {
     case 5: XG_EV(1, 1); break;
     case 6: XG_EV(1, 2); break;

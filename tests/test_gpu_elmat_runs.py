@@ -85,3 +85,47 @@ def test_lists_of_every_length(n, p):
     sc = np.abs(ref).max(axis=(-2, -1), keepdims=True)
     assert np.all(np.abs(g - ref) <= 2e-7 * sc)
     ctx.close()
+
+
+VEC_COUNTS = [0, 1, 4, 15, 16, 17, 31, 32, 33, 64, 95, 96, 97, 129, 200, 513]
+
+
+def _long_rules(D, seed, reps):
+    """(elements, offsets, points) of a list with rules of VEC_COUNTS points, `reps` times over"""
+    mesh = _mesh(D)
+    rng = np.random.default_rng(seed)
+    n = np.tile(VEC_COUNTS, reps)
+    elems = rng.integers(0, mesh.ne, len(n)).astype(np.int32)
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    pts = np.zeros((off[-1], 4))
+    pts[:, :D] = rng.dirichlet(np.ones(D + 1), off[-1])[:, :D]
+    pts[:, 3] = rng.uniform(-0.3, 1.0, off[-1])
+    return mesh, elems, off, pts
+
+
+@pytest.mark.parametrize("D", [1, 2, 3])
+@pytest.mark.parametrize("p", [1, 2, 3])
+@pytest.mark.parametrize("reps", [1, 257])
+def test_vectors_of_rules_of_every_length(D, p, reps):
+    """an element has 16 lanes of a wave, or all of them for a long rule in a list of up to 4096 elements (16 and
+    4112 here), against the oracle's shape functions.  Bar: a rounding per point
+    of the sum and 30 of a shape function and the Jacobian"""
+    import torch
+    mesh, elems, off, pts = _long_rules(D, 10 * D + p, reps)
+    ctx = _abi.Context(0)
+    up = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    nd = O.h1_ndof(D, p)
+    out = torch.full((len(elems), nd), float("nan"), dtype=torch.float64, device="cuda")
+    ctx.elvec(D, p, up(mesh.el2v), up(mesh.coords), up(off), up(pts), out, elems=up(elems))
+    ctx.sync()
+    g = out.cpu().numpy()
+    assert len(elems) == 16 if reps == 1 else len(elems) > 4096
+    first = len(elems) - len(VEC_COUNTS)  # the last of the repetitions, and the first
+    for i in list(range(len(VEC_COUNTS))) + list(range(first, len(elems))):
+        x, w = pts[off[i]:off[i + 1], :D], pts[off[i]:off[i + 1], 3]
+        V = mesh.coords[mesh.el2v[elems[i]]]
+        det = abs(np.linalg.det((V[:D] - V[D]).T.reshape(D, D)))
+        phi = np.array([O.h1_shape(D, p, q)[0] for q in x]).reshape(-1, nd)
+        bar = 1.2e-16 * (len(w) + 30) * det * np.abs(w).sum() * max(1.0, np.abs(phi).max(initial=0.0))
+        assert np.abs(g[i] - det * (phi * w[:, None]).sum(0)).max() <= bar, (i, len(w))
+    ctx.close()
