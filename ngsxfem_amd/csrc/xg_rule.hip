@@ -498,13 +498,24 @@ extern "C" int xg_integrate(xg_ctx *ctx, int D, int nel, const int32_t *elems, c
       f.ex[t][d] = expo[3 * t + d];
     }
   }
-  // lanes per element: the fewest points that a rule of use has (order 2: 8
-  // on a tetrahedron, 4 on a triangle)
+  // lanes per element: the fewest points that a rule of use has (order 2: 8 on
+  // a tetrahedron, 4 on a triangle); a wave for each of few elements, whatever
+  // their rules, since the others would be idle.  us, a wave per element and its
+  // atomic / these lanes / a wave, tetrahedra: 64 of order 8 10.6 / 18.5 / 10.6, of
+  // order 15 19.4 / 55.5 / 12.2, there with 20 terms 80.6 / 207 / 30.8; 2000 of
+  // order 4 29.1 / 10.6 / 10.3, of order 15 40.5 / 64.4 / 17.7
+  const bool few = nel <= 4096;
   const double4 *p = reinterpret_cast<const double4 *>(pts);
   switch (D) {
     case 1: launch_integrate<1, 2>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
-    case 2: launch_integrate<2, 4>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
-    default: launch_integrate<3, 8>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total); break;
+    case 2:
+      if (few) launch_integrate<2, 64>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total);
+      else launch_integrate<2, 4>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total);
+      break;
+    default:
+      if (few) launch_integrate<3, 64>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total);
+      else launch_integrate<3, 8>(ctx, nel, elems, el2v, coords, offsets, p, f, per_elem, total);
+      break;
   }
   XG_LAUNCH_CHECK();
   return XG_OK;

@@ -129,3 +129,30 @@ def test_vectors_of_rules_of_every_length(D, p, reps):
         bar = 1.2e-16 * (len(w) + 30) * det * np.abs(w).sum() * max(1.0, np.abs(phi).max(initial=0.0))
         assert np.abs(g[i] - det * (phi * w[:, None]).sum(0)).max() <= bar, (i, len(w))
     ctx.close()
+
+
+@pytest.mark.parametrize("D", [1, 2, 3])
+@pytest.mark.parametrize("reps", [1, 257])
+def test_integrals_of_rules_of_every_length(D, reps):
+    """an element has 2, 4 or 8 lanes, or a wave in a list of up to 4096 elements, and a lane takes 4 points at once
+    while one of the wave has more, against the oracle.  Bar: a rounding per point and 30 of a term"""
+    import torch
+    mesh, elems, off, pts = _long_rules(D, 100 + D, reps)
+    ctx = _abi.Context(0)
+    up = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    terms = [(1.0 / (k + 1), (k % 4, k % 3 if D > 1 else 0, k % 2 if D > 2 else 0)) for k in range(11)]
+    per = torch.full((len(elems),), float("nan"), dtype=torch.float64, device="cuda")
+    tot = torch.full((1,), 7.0, dtype=torch.float64, device="cuda")
+    ctx.integrate(D, up(mesh.el2v), up(mesh.coords), up(off), up(pts), terms, tot, per, elems=up(elems))
+    ctx.sync()
+    g = per.cpu().numpy()
+    first = len(elems) - len(VEC_COUNTS)
+    cmax = sum(c for c, _ in terms) * max(1.0, np.abs(mesh.coords).max()) ** 6
+    for i in list(range(len(VEC_COUNTS))) + list(range(first, len(elems))):
+        x, w = pts[off[i]:off[i + 1], :3], pts[off[i]:off[i + 1], 3]
+        V = mesh.coords[mesh.el2v[elems[i]]]
+        ref = O.integrate_poly(D, V, x, w, terms) if len(w) else 0.0
+        det = abs(np.linalg.det((V[:D] - V[D]).T.reshape(D, D)))
+        assert abs(g[i] - ref) <= 1.2e-16 * (len(w) + 30) * det * np.abs(w).sum() * cmax, (i, len(w))
+    assert abs(tot.item() - g.sum()) <= 1.2e-16 * len(elems) * np.abs(g).sum()
+    ctx.close()
