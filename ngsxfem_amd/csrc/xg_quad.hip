@@ -17,12 +17,14 @@
 // another coordinate plays xi, or give up on the tensor product and cut the
 // 2 triangles / 6 tetrahedra of the element instead (the fallback).
 //
-// Mapping: 16 lanes per element, each with a part of its rule (a Gauss slice of
-// a piece, a sub-simplex of the fallback) in the rule's order; a count pass and
+// Mapping: up to 16 lanes per element, each with a part of its rule (a Gauss slice
+// of a piece, a sub-simplex of the fallback) in the rule's order; a count pass and
 // a fill pass produce a CSR rule like the simplex rule (xg_rule.hip).  The
 // recursion depth is fixed (hex -> slice quad -> slice segment), so it is
 // written as nested templates with small functors that map a slice point back
 // into the element and pass it on.  Marking takes one lane per element.
+#include <type_traits>
+
 #include "xg_device.hpp"
 #include "xg_internal.hpp"
 
@@ -135,6 +137,11 @@ XG_DEV int box_check(const QL &L, int D, const Box &q, double eps) {
 // A = (p1 - p0, p3 - p0, p4 - p0); the points i0 <= i < i1 of the x rule
 template <class Sink>
 XG_DEV void box_plain(const Box &q, int D, int order, Sink &s, int i0, int i1) {
+  if constexpr (Sink::COUNT) {
+    const int m = rule_cnt(1, order);
+    s.skip((i1 - i0) * (D == 3 ? m * m : m));
+    return;
+  }
   double p0[3], p1[3], p3[3], p4[3] = {0, 0, 0};
   box_point(q, D, 0, p0);
   box_point(q, D, 1, p1);
@@ -183,6 +190,10 @@ XG_DEV void box_plain(const Box &q, int D, int order, Sink &s) {
 // base rule of dimension dim on the simplex P (SimpleX::GetPlainIntegrationRule)
 template <class Sink>
 XG_DEV void simplex_plain(int dim, const double (*P)[3], int order, Sink &s) {
+  if constexpr (Sink::COUNT) {
+    s.skip(rule_cnt(dim, order));
+    return;
+  }
   const double vol = simplex_measure(dim, P);
   const int nq = rule_cnt(dim, order);
   const double(*r)[4] = &xg_rule_data_d[rule_off(dim, order)];
@@ -264,6 +275,8 @@ XG_DEV void quad_rule(const QL &L, int dt, int order, int pol, bool consider, Si
 // slice weights (GetTensorProductAlongXiIntegrationRule, :256-302)
 template <int D, class Sink>
 struct SliceSink {
+  static constexpr bool COUNT = Sink::COUNT;
+  XG_DEV void skip(int k) { s.skip(k); }
   const QL &L;
   const Box &q;
   double xs, w1, len;
@@ -429,6 +442,8 @@ XG_DEV int dimension_swap(const QL &L, int D, int pol, bool consider, int &err) 
 // swaps the coordinates of the rotated element's points back (:304-351)
 template <class Sink>
 struct SwapSink {
+  static constexpr bool COUNT = Sink::COUNT;
+  XG_DEV void skip(int k) { s.skip(k); }
   int sw;
   Sink &s;
   XG_DEV void operator()(const double *p, double w) {
@@ -562,6 +577,7 @@ XG_DEV double det_inv(const double *F, double *Finv) {
 // |F^{-T} n_ref| at the point (TransformQuadUntrafoToIRInterface, :558-578)
 template <int D>
 struct ElemSink {
+  static constexpr bool COUNT = false;
   const QL &L;
   const double (*V)[3];
   double4 *out;  // null: count only
@@ -594,6 +610,14 @@ struct ElemSink {
     wsum += w;
     ++n;
   }
+};
+// the number of points only (nothing of them is computed, and no error raised
+// that depends on one)
+struct CountSink {
+  static constexpr bool COUNT = true;
+  int n;
+  XG_DEV void operator()(const double *, double) { ++n; }
+  XG_DEV void skip(int k) { n += k; }
 };
 
 // StraightCutIntegrationRule (:582-677) of one element on the unit element
@@ -721,10 +745,13 @@ struct QuadParts {
 // lane per element 5,300 cut hexahedra were 83 waves for 1024 SIMDs, each lane
 // going through all slices: 48^3 hexes, order 4, NEG, count and fill: 1048 ->
 // 153 us (with the matrices 1378 -> 203).  Two waves per SIMD for the fill too
-// (55 spilled registers): with one the last third of the waves waited for the
-// others, 188 -> 174 us with the matrices.
-constexpr int QG = 16;  // lanes per element: 15 parts of a split hexahedron at order 4
-template <int D, bool FILL>
+// (19 spilled registers): with one the last third of the waves waited for the
+// others, 188 -> 174 us with the matrices.  The counting pass of a fill, and a
+// count, compute no points: 173 -> 139 us.
+// G: lanes per element (quad_lanes; 16 for the matrices and vectors below: 15
+// parts of a split hexahedron at order 4)
+constexpr int QG = 16;
+template <int D, bool FILL, int G>
 __global__ __launch_bounds__(256, 2) void k_quad_rule(int nel, const int32_t *__restrict__ elems,
                                                    const int32_t *__restrict__ el2v,
                                                    const double *__restrict__ coords,
@@ -733,7 +760,7 @@ __global__ __launch_bounds__(256, 2) void k_quad_rule(int nel, const int32_t *__
                                                    int32_t *err_flag) {
   constexpr int NV = 1 << D;
   const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
-  const int i = (int)(g / QG), sub = threadIdx.x & (QG - 1);
+  const int i = (int)(g / G), sub = threadIdx.x & (G - 1);
   if (i >= nel) return;
   const int e = elems ? elems[i] : i;
   double vals[NV];
@@ -748,39 +775,58 @@ __global__ __launch_bounds__(256, 2) void k_quad_rule(int nel, const int32_t *__
     }
   }
   int err = 0;
-  QuadParts<D> parts;
-  parts.plan(vals, dt, order, pol, err);
   const QL L = D == 2 ? ql_quad(vals) : ql_hex(vals);
   const int base = FILL ? offsets[i] : 0;
   int n = 0;
-  for (int it0 = 0; it0 < parts.n; it0 += QG) {
-    const int it = it0 + sub;
-    int c = 0, pre = 0;
-    // counted first; a fill then knows where its part begins
-#pragma unroll 1
-    for (int pass = 0; pass < (FILL ? 2 : 1); ++pass) {
-      ElemSink<D> s{L, V, pass ? pts + base + n + pre : nullptr, dt, 0, 0.0};
-      if (it < parts.n) {
-        if (parts.sw == SW_ID || parts.sw == SW_NONE) {
-          parts.run(it, dt, order, pol, s, err);
-        } else {
-          SwapSink<ElemSink<D>> ws{parts.sw, s};
-          parts.run(it, dt, order, pol, ws, err);
-        }
-      }
-      if (pass == 0) {
-        c = s.n;
-        int incl = c;
-#pragma unroll
-        for (int o = 1; o < QG; o <<= 1) {
-          const int y = __shfl_up(incl, o, QG);
-          if (sub >= o) incl += y;
-        }
-        pre = incl - c;
-        c = __shfl(incl, QG - 1, QG);
-      }
+  // (an interface point of a tensor rule without a bound on its weight is an
+  // error of the count too)
+  const bool points = FILL || (dt == IF && pol != 2);
+  if constexpr (G == 1) {
+    if (points) {
+      ElemSink<D> s{L, V, FILL ? pts + base : nullptr, dt, 0, 0.0};
+      element_rule<D>(vals, dt, order, pol, s, err);
+      n = s.n;
+    } else {
+      CountSink s{0};
+      element_rule<D>(vals, dt, order, pol, s, err);
+      n = s.n;
     }
-    n += c;
+  } else {
+    QuadParts<D> parts;
+    parts.plan(vals, dt, order, pol, err);
+    auto run = [&](int it, auto &s) {
+      if (it >= parts.n) return;
+      if (parts.sw == SW_ID || parts.sw == SW_NONE) {
+        parts.run(it, dt, order, pol, s, err);
+      } else {
+        SwapSink<std::decay_t<decltype(s)>> ws{parts.sw, s};
+        parts.run(it, dt, order, pol, ws, err);
+      }
+    };
+    for (int it0 = 0; it0 < parts.n; it0 += G) {
+      // counted first; a fill then knows where its part begins
+      int c = 0;
+      if (FILL || !points) {
+        CountSink s{0};
+        run(it0 + sub, s);
+        c = s.n;
+      } else {
+        ElemSink<D> s{L, V, nullptr, dt, 0, 0.0};
+        run(it0 + sub, s);
+        c = s.n;
+      }
+      int incl = c;
+#pragma unroll
+      for (int o = 1; o < G; o <<= 1) {
+        const int y = __shfl_up(incl, o, G);
+        if (sub >= o) incl += y;
+      }
+      if constexpr (FILL) {
+        ElemSink<D> s{L, V, pts + base + n + incl - c, dt, 0, 0.0};
+        run(it0 + sub, s);
+      }
+      n += __shfl(incl, G - 1, G);
+    }
   }
   if (err) atomicOr(err_flag, err);
   if (!FILL && sub == 0) offsets[i] = n;
@@ -1017,8 +1063,45 @@ __global__ __launch_bounds__(256) void k_quad_elvec(int nel, const int32_t *__re
   }
 }
 
-// blocks of 256 for 16 lanes per element
-unsigned quad_grid(int nel) { return (unsigned)(((long long)nel * QG + 255) / 256); }
+// blocks of 256 for g lanes per element
+unsigned quad_grid(int nel, int g = QG) { return (unsigned)(((long long)nel * g + 255) / 256); }
+
+// Lanes per element of the rule kernels: as many as an element has parts while
+// the waves fit on the device (two per SIMD), then fewer, since a part by itself
+// costs a wave the branches of all others; one lane needs no counting pass.  us
+// for a fill, order 4, NEG, 1 / 2 / 4 / 8 / 16 lanes: cut quadrilaterals 4000 38 / 29
+// / 20 / 13 / 11, 20,000 36 / 28 / 24 / 25 / 30, 100,000 38 / 56 / 58 / 79 / 118;
+// hexahedra 4000 842 / 416 / 208 / 107 / 75, 100,000 979 / 721 / 646 / 575 / 669.
+// Without tensor rules (2 triangles, 6 tetrahedra): quadrilaterals 4000 38 / 24 / 22
+// / 21 / 20, 20,000 40 / 26 / 34 / 53 / 74, 100,000 68 / 82 / 113 / 177 / 299;
+// hexahedra 20,000 475 / 311 / 266 / 274 / 340, 100,000 817 / 942 / 1043 / 964 / 1452.
+int quad_lanes(int D, int nel, int order, int pol) {
+  if (pol == 2) return D == 2 ? (nel <= 32768 ? 2 : 1) : (nel <= 49152 ? 8 : 1);
+  if (D == 2) return nel <= 4096 ? 16 : (nel <= 24576 ? 8 : (nel <= 49152 ? 4 : 1));
+  return nel <= 24576 ? 16 : (order < 4 ? 4 : 8);
+}
+
+template <bool FILL>
+void launch_quad_rule(xg_ctx *ctx, int D, int nel, const int32_t *elems, const int32_t *el2v, const double *coords,
+                      const double *lset, int dt, int order, int pol, int32_t *offsets, double4 *pts) {
+  const int g = quad_lanes(D, nel, order, pol);
+  const unsigned grid = quad_grid(nel, g);
+#define XG_QR(DD, GG)                                                                                           \
+  k_quad_rule<DD, FILL, GG><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset, dt, order, pol, offsets, \
+                                                           pts, ctx->d_err)
+#define XG_QRD(DD)                 \
+  switch (g) {                     \
+    case 1: XG_QR(DD, 1); break;   \
+    case 2: XG_QR(DD, DD == 2 ? 2 : 4); break;  /* (quadrilaterals only) */ \
+    case 4: XG_QR(DD, 4); break;   \
+    case 8: XG_QR(DD, 8); break;   \
+    default: XG_QR(DD, 16); break; \
+  }
+  if (D == 2) XG_QRD(2)
+  else XG_QRD(3)
+#undef XG_QRD
+#undef XG_QR
+}
 
 
 bool quad_args_ok(int D, int dt, int order, int pol) {
@@ -1037,13 +1120,7 @@ extern "C" int xg_quad_rule_count(xg_ctx *ctx, int D, int nel, const int32_t *el
     XG_CHECK(hipMemsetAsync(offsets, 0, sizeof(int32_t), ctx->stream));
     return XG_OK;
   }
-  const unsigned grid = quad_grid(nel);
-  if (D == 2)
-    k_quad_rule<2, false><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, nullptr, lset_v, dt, order, policy,
-                                                         offsets, nullptr, ctx->d_err);
-  else
-    k_quad_rule<3, false><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, nullptr, lset_v, dt, order, policy,
-                                                         offsets, nullptr, ctx->d_err);
+  launch_quad_rule<false>(ctx, D, nel, elems, el2v, nullptr, lset_v, dt, order, policy, offsets, nullptr);
   XG_LAUNCH_CHECK();
   return scan_exclusive_i32(ctx, offsets, nel, true);
 }
@@ -1055,14 +1132,8 @@ extern "C" int xg_quad_rule_fill(xg_ctx *ctx, int D, int nel, const int32_t *ele
     return set_error(XG_ERR_ARG, "xg_quad_rule_fill: bad argument");
   if (nel == 0) return XG_OK;
   if (!el2v || !lset_v || !coords || !pts) return set_error(XG_ERR_ARG, "xg_quad_rule_fill: null pointer");
-  const unsigned grid = quad_grid(nel);
-  double4 *o = reinterpret_cast<double4 *>(pts);
-  if (D == 2)
-    k_quad_rule<2, true><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, policy,
-                                                        const_cast<int32_t *>(offsets), o, ctx->d_err);
-  else
-    k_quad_rule<3, true><<<grid, 256, 0, ctx->stream>>>(nel, elems, el2v, coords, lset_v, dt, order, policy,
-                                                        const_cast<int32_t *>(offsets), o, ctx->d_err);
+  launch_quad_rule<true>(ctx, D, nel, elems, el2v, coords, lset_v, dt, order, policy,
+                         const_cast<int32_t *>(offsets), reinterpret_cast<double4 *>(pts));
   XG_LAUNCH_CHECK();
   return XG_OK;
 }

@@ -158,6 +158,37 @@ def test_rule_parity_many_parts(dev, orc, D, order):
                 assert np.abs(got[:, 3] - r[1]).max() <= 1e-14 * max(1.0, np.abs(r[1]).max())
 
 
+@pytest.mark.parametrize("D,n", [(2, 4097), (2, 24577), (2, 49153), (2, 32769), (3, 24577), (3, 49153)])
+@pytest.mark.parametrize("pol", [FIRST, OPTIMAL, FALLBACK])
+@pytest.mark.parametrize("order", [2, 5])
+def test_rule_lists_of_every_length(dev, D, n, pol, order):
+    """an element has 16, 8, 4, 2 lanes or one, by the length of the list and the policy: the points of a long list
+    are those of the element's own short list, bit for bit (the same operations per point, the same order)"""
+    torch, _abi, ctx = dev
+    mesh = warped(D, 9 if D == 2 else 4)
+    for kind in ("sphere", "plane"):
+        lset = level_sets(mesh, kind)
+        pick = np.random.default_rng(n).integers(0, mesh.ne, n).astype(np.int32)
+        el, xs, ls = up(torch, mesh.el2v), up(torch, mesh.coords), up(torch, lset)
+
+        def rule(dt, ids):
+            off = torch.zeros(len(ids) + 1, dtype=torch.int32, device="cuda")
+            ctx.quad_rule_count(D, el, ls, dt, order, pol, off, elems=up(torch, ids))
+            ctx.sync()
+            pts = torch.full((max(int(off[-1].item()), 1), 4), float("nan"), dtype=torch.float64, device="cuda")
+            ctx.quad_rule_fill(D, el, xs, ls, dt, order, pol, off, pts, elems=up(torch, ids))
+            ctx.sync()
+            return off.cpu().numpy(), pts.cpu().numpy()
+
+        for dt in (NEG, IF):
+            o1, p1 = rule(dt, np.arange(mesh.ne, dtype=np.int32))
+            o, p = rule(dt, pick)
+            cnt = np.diff(o1)[pick]
+            assert np.array_equal(np.diff(o), cnt)
+            src = np.repeat(o1[pick], cnt) + np.arange(int(cnt.sum())) - np.repeat(np.cumsum(cnt) - cnt, cnt)
+            assert np.array_equal(p[:len(src)], p1[src])
+
+
 def test_rule_parity_tpmc_all_policies(dev, orc):
     """the single-hex TPMC level set (topology change inside the element)"""
     mesh = MakeStructured3DMesh(hexes=True, nx=1, ny=1, nz=1)
