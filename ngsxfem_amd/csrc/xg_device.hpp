@@ -310,7 +310,7 @@ XG_DEV bool decompose(const double *l, int dt, Decomp &dc) {
 // m = sum_i [l_i >= 0] << i, so it is tabulated at compile time (same
 // construction as decompose()).  Kernels whose element is wave-uniform read
 // the entry with scalar loads instead of rebuilding it in registers.
-struct DecompEntry {
+struct alignas(8) DecompEntry {  // (copied in words of 8 bytes)
   int8_t ns, nv, nc, ok;
   int8_t v[3][4];
   int8_t ce[4][2];

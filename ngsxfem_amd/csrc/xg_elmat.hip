@@ -89,6 +89,17 @@ __global__ __launch_bounds__(128) void k_pipeline(int nel, int run, const int32_
   }
 }
 
+// gradients of the first D barycentrics (the rows of F^{-1}) and |det F|
+template <int D>
+__device__ __forceinline__ void element_gradients(const int32_t *__restrict__ el2v, const double *__restrict__ coords,
+                                                  int e, double (*g)[3], double &absdet) {
+  double V[D + 1][3], F[D * D], Finv[D * D];
+  load_geom<D>(el2v, coords, nullptr, e, V, nullptr);
+  jacobian<D>(V, F, Finv, absdet);
+#pragma unroll
+  for (int k = 0; k < D * D; ++k) g[k / D][k % D] = Finv[k];
+}
+
 template <typename T>
 struct CsrSrc {
   const double4 *pts;
@@ -111,19 +122,34 @@ __global__ __launch_bounds__(128) void k_elmat_csr(int nel, int run, const int32
                                                    T *__restrict__ out) {
   using C = Cfg<D, P, T>;
   extern __shared__ char smem[];
-  __shared__ ElemRec s_rec[C::WAVES][EL_RUN];
   const int wv = threadIdx.x >> 6;
   using EL = ElLds<D, P, T, SPLIT>;
   T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (EL::BYTES / sizeof(T));
   T *sW = sB + C::SB_SIZE;
   const int lane = threadIdx.x & 63;
   for (int k = lane; k < EL::ZERO; k += 64) sB[k] = T(0);
-  GramLane gl{};
-  if constexpr (EL::GRAM) gl = gram_lane<D, P>();
   wave_sync();
   const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   constexpr int NN = C::N * C::N;
+  if constexpr (!EL::GRAM) {
+    // an element at a time, its geometry in the wave's registers (through LDS,
+    // as below, P3 and split BF16 were 3 to 8 % slower: 40,000 tetrahedra of order 4,
+    // P3 FP32 320 -> 338 us, P2 BF16X3 139 -> 150)
+    for (int i = wid; i < nel; i += nwaves) {
+      double g[D][3], absdet;
+      element_gradients<D>(el2v, coords, elems ? elems[i] : i, g, absdet);
+      CsrSrc<T> src{pts, offsets[i]};
+      const int npts = offsets[i + 1] - offsets[i];
+      T *o = out + (size_t)i * NN;
+      if constexpr (SPLIT) elmat_one_bf16x3<D, P>(src, npts, g, absdet, mask, sB, sW, o);
+      else elmat_one<D, P, T>(src, npts, g, absdet, mask, sB, sW, o);
+    }
+    return;
+  }
+  __shared__ ElemRec s_rec[C::WAVES][EL::GRAM ? EL_RUN : 1];
+  GramLane gl{};
+  if constexpr (EL::GRAM) gl = gram_lane<D, P>();
   for (long long base = (long long)wid * run; base < nel; base += (long long)nwaves * run) {
     if (lane < run && base + lane < nel) {
       const int e = elems ? elems[base + lane] : (int)base + lane;
@@ -163,17 +189,6 @@ __global__ __launch_bounds__(128) void k_elmat_csr(int nel, int run, const int32
         q0 = q1;
         gram_store<D, P, T>(acc, s_rec[wv][j].g, mask, gl, sW2 + 64, out + (size_t)(base + j) * NN);
       }
-    } else {
-      for (int j = 0; j < m; ++j) {
-        const long long i = base + j;
-        const ElemRec &R = s_rec[wv][j];
-        const double absdet = R.absdet;
-        CsrSrc<T> src{pts, offsets[i]};
-        const int npts = offsets[i + 1] - offsets[i];
-        T *o = out + (size_t)i * NN;
-        if constexpr (SPLIT) elmat_one_bf16x3<D, P>(src, npts, R.g, absdet, mask, sB, sW, o);
-        else elmat_one<D, P, T>(src, npts, R.g, absdet, mask, sB, sW, o);
-      }
     }
     wave_sync();
   }
@@ -202,19 +217,28 @@ __global__ __launch_bounds__(128) void k_elmat_weights(int nel, int run, const i
   using C = Cfg<3, P, T>;
   constexpr int NQ = ndof(3, Q);
   extern __shared__ char smem[];
-  __shared__ ElemRec s_rec[C::WAVES][EL_RUN];
   const int wv = threadIdx.x >> 6;
   using EL = ElLds<3, P, T, SPLIT>;
   T *sB = reinterpret_cast<T *>(smem) + (size_t)wv * (EL::BYTES / sizeof(T));
   T *sW = sB + C::SB_SIZE;
   const int lane = threadIdx.x & 63;
   for (int k = lane; k < EL::ZERO; k += 64) sB[k] = T(0);
-  GramLane gl{};
-  if constexpr (EL::GRAM) gl = gram_lane<3, P>();
   wave_sync();
   const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int nwaves = (gridDim.x * blockDim.x) >> 6;
   constexpr int NN = C::N * C::N;
+  if constexpr (SPLIT) {  // (as in k_elmat_csr)
+    for (int i = wid; i < nel; i += nwaves) {
+      double g[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}}, absdet = 1.0;
+      if (coords) element_gradients<3>(el2v, coords, elems ? elems[i] : i, g, absdet);
+      WeightSrc<Q, T> src{weights + (size_t)i * NQ};
+      elmat_one_bf16x3<3, P>(src, NQ, g, absdet, mask, sB, sW, out + (size_t)i * NN);
+    }
+    return;
+  }
+  __shared__ ElemRec s_rec[C::WAVES][EL::GRAM ? EL_RUN : 1];
+  GramLane gl{};
+  if constexpr (EL::GRAM) gl = gram_lane<3, P>();
   for (long long base = (long long)wid * run; base < nel; base += (long long)nwaves * run) {
     if (lane < run && base + lane < nel) {
       double V[4][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {0, 0, 0}};
@@ -235,14 +259,12 @@ __global__ __launch_bounds__(128) void k_elmat_weights(int nel, int run, const i
       T *o = out + (size_t)i * NN;
       if constexpr (EL::GRAM)
         elmat_gram<3, P, T>(src, npts, R.g, absdet, mask, gl, reinterpret_cast<double *>(sB), o);
-      else elmat_one_bf16x3<3, P>(src, npts, R.g, absdet, mask, sB, sW, o);
     }
     wave_sync();
   }
 }
 
-int grid_waves(int nel) {
-  const int run = el_run(nel);
+int grid_waves(int nel, int run) {
   long long blocks = ((long long)nel + 2 * run - 1) / (2 * run);
   if (blocks > 16384) blocks = 16384;
   if (blocks < 1) blocks = 1;
@@ -254,8 +276,9 @@ int launch_pipeline(xg_ctx *ctx, int order, int nel, const int32_t *elems, const
                     const double *coords, const double *lset, int ndt, int dts, int mask, void *out) {
   using C = Cfg<D, P, T>;
   const size_t lds = ElLds<D, P, T, SPLIT>::BYTES * C::WAVES + stage_rule_bytes(D, order);
-  k_pipeline<D, P, T, SPLIT><<<grid_waves(nel), 64 * C::WAVES, lds, ctx->stream>>>(
-      nel, el_run(nel), elems, el2v, coords, lset, order, ndt, dts, mask, (T *)out, ctx->d_err);
+  const int run = el_run(nel);
+  k_pipeline<D, P, T, SPLIT><<<grid_waves(nel, run), 64 * C::WAVES, lds, ctx->stream>>>(
+      nel, run, elems, el2v, coords, lset, order, ndt, dts, mask, (T *)out, ctx->d_err);
   XG_LAUNCH_CHECK();
   return XG_OK;
 }
@@ -265,8 +288,9 @@ int launch_csr(xg_ctx *ctx, int nel, const int32_t *elems, const int32_t *el2v, 
                const int32_t *offsets, const double *pts, int mask, void *out) {
   using C = Cfg<D, P, T>;
   const size_t lds = ElLds<D, P, T, SPLIT>::BYTES * C::WAVES;
-  k_elmat_csr<D, P, T, SPLIT><<<grid_waves(nel), 64 * C::WAVES, lds, ctx->stream>>>(
-      nel, el_run(nel), elems, el2v, coords, offsets, reinterpret_cast<const double4 *>(pts), mask, (T *)out);
+  const int run = ElLds<D, P, T, SPLIT>::GRAM ? el_run(nel) : 1;
+  k_elmat_csr<D, P, T, SPLIT><<<grid_waves(nel, run), 64 * C::WAVES, lds, ctx->stream>>>(
+      nel, run, elems, el2v, coords, offsets, reinterpret_cast<const double4 *>(pts), mask, (T *)out);
   XG_LAUNCH_CHECK();
   return XG_OK;
 }
@@ -324,8 +348,9 @@ int launch_weights(xg_ctx *ctx, int nel, const int32_t *elems, const int32_t *el
                    const double *weights, int mask, void *out) {
   using C = Cfg<3, P, T>;
   const size_t lds = ElLds<3, P, T, SPLIT>::BYTES * C::WAVES;
-  k_elmat_weights<P, Q, T, SPLIT><<<grid_waves(nel), 64 * C::WAVES, lds, ctx->stream>>>(nel, el_run(nel), elems, el2v, coords, weights,
-                                                                                mask, (T *)out);
+  const int run = SPLIT ? 1 : el_run(nel);
+  k_elmat_weights<P, Q, T, SPLIT><<<grid_waves(nel, run), 64 * C::WAVES, lds, ctx->stream>>>(
+      nel, run, elems, el2v, coords, weights, mask, (T *)out);
   XG_LAUNCH_CHECK();
   return XG_OK;
 }
