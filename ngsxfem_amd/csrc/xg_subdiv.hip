@@ -1779,10 +1779,10 @@ __device__ __forceinline__ int lat_index_rs(const uint16_t *rowst, int a, int b,
 
 __global__ void k_zero_i32(int32_t *p) { *p = 0; }
 
-// next element of a persistent wave: lane 0 takes it from the work counter
-__device__ __forceinline__ int next_item(int32_t *queue, int lane) {
+// `grab` elements for a persistent wave: lane 0 takes them from the work counter
+__device__ __forceinline__ int next_items(int32_t *queue, int grab, int lane) {
   int nx = 0;
-  if (lane == 0) nx = atomicAdd(queue, 1);
+  if (lane == 0) nx = atomicAdd(queue, grab);
   return __shfl(nx, 0, 64);
 }
 
@@ -2074,7 +2074,8 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
                                                      int4 *__restrict__ cnt, double *__restrict__ out_vol,
                                                      double *__restrict__ out_if, int out_stride,
                                                      int32_t *__restrict__ stats, int stats_stride, int32_t *err,
-                                                     int32_t *__restrict__ queue, int32_t *__restrict__ stats_if) {
+                                                     int32_t *__restrict__ queue, int grab,
+                                                     int32_t *__restrict__ stats_if) {
   using MM = Moments<3, PM>;
   constexpr int NL = ndof(3, LO);
   constexpr int NM = MM::NM, NG = (NM + 3) / 4;
@@ -2090,9 +2091,17 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
   for (int r = 0; r < 4; ++r) sel[r] = (lane & 3) == r ? 1.0 : 0.0;
   constexpr double inv = 1.0 / (1 << SDX_DMAX);
   // elements from the work counter (persistent waves, the heavy elements do
-  // not wait behind a fixed stride) or strided by the grid
-  for (int i = queue ? next_item(queue, lane) : blockIdx.x; i < nel;
-       i = queue ? next_item(queue, lane) : i + gridDim.x) {
+  // not wait behind a fixed stride), `grab` at a time after a first one by the
+  // wave's number (grab 0: one at a time, the first too), or strided by the grid
+  int left = 1;
+  const int own = grab > 0 ? (int)gridDim.x : 0;
+  auto advance = [&](int i) {
+    if (!queue) return i + (int)gridDim.x;
+    if (--left > 0) return i + 1;
+    left = max(grab, 1);
+    return own + next_items(queue, left, lane);
+  };
+  for (int i = queue && !own ? next_items(queue, 1, lane) : blockIdx.x; i < nel; i = advance(i)) {
     const int4 c4 = cnt[i];
     if (c4.x < 0) continue;  // queued for the one-kernel path
     const int e = elems ? elems[i] : i;
@@ -2465,6 +2474,22 @@ int launch_sdx_tree(xg_ctx *ctx, int side, int nel, const int32_t *elems, const 
   return XG_OK;
 }
 
+// Elements that a wave takes from the work counter at a time.  The counter gives
+// one every 11 ns whatever the number of waves, so elements of less work than 11
+// ns times the waves (22 us of 2048) wait for it: up to level 2 four at a time, at
+// level 3 two of the lighter ones, while every wave has two such helpings.  us of
+// the kernel, one at a time / now, NEG, random quadrics: 10,368 elements P1, L 0
+// 169 / 85, P2, L 2 159 / 90, P2, L 3 169 / 120; 82,944 P1, L 2 992 / 293, P2, L 3 991
+// / 696.  The first element by the wave's number, except for the heaviest (P3, L
+// 4: 1296 elements NEG + IF 262 us, 273 so).
+template <int PM, int WHICH>
+int sdx_grab(int nel, int waves, int L) {
+  if (L >= 4) return PM == 3 ? 0 : 1;
+  const int most = (nel + 2 * waves - 1) / (2 * waves);
+  const int want = L <= 2 ? 4 : (PM == 1 || (PM == 2 && WHICH != 3) ? 2 : 1);
+  return want < most ? want : most;
+}
+
 template <int LO, int PM, int SIDE, int WHICH>
 int launch_sdx_leaves(xg_ctx *ctx, int nel, const int32_t *elems, const double *lset, const int32_t *el2v,
                       const double *coords, const double *finv, int L, uint16_t *lists, int cap, int4 *cnt,
@@ -2485,10 +2510,11 @@ int launch_sdx_leaves(xg_ctx *ctx, int nel, const int32_t *elems, const double *
     k_zero_i32<<<1, 1, 0, ctx->stream>>>(queue);
     XG_LAUNCH_CHECK();
   }
+  const int grab = sdx_grab<PM, WHICH>(nel, blocks, L);
   KernelTimer tm(ctx, WHICH == 3 ? "sdx_leaves_both" : ((WHICH & 1) ? "sdx_leaves_vol" : "sdx_leaves_if"));
   k_sdx_leaves<LO, PM, SIDE, WHICH><<<blocks, 64, lds, ctx->stream>>>(
       nel, elems, lset, el2v, coords, finv, L, (const uint4 *)ctx->sdx_verts, lists, cap, cnt, out_vol, out_if,
-      out_stride, stats, stats_stride, ctx->d_err, queue, stats_if);
+      out_stride, stats, stats_stride, ctx->d_err, queue, grab, stats_if);
   XG_LAUNCH_CHECK();
   return XG_OK;
 }
