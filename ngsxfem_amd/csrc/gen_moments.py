@@ -372,68 +372,15 @@ def gen_forms_bernstein(D, P, L):
     return nterms
 
 
-def gen_affine(D, P, L, idx2):
-    """accum_aff: the affine moments n_beta = sum_i w_i y_i^beta, |beta| <= 2P,
-    in D affine coordinates y (lam_D = 1 - sum is not formed): the monomials
-    of degree 2..P take 16 products instead of the homogeneous ones' 30
-    (D = 3, P = 3), and the constant's weighted monomial is w itself.
-    n_beta is kept in the slot of the homogeneous moment (beta, 2P - |beta|).
-    With y = lam - 1/4 (centred coordinates) the homogeneous moments follow
-    by the dense map of gen_affine_table."""
-    n2 = 2 * P
-    zero = tuple([0] * D)
-
-    def slot(b):
-        return idx2[tuple(b) + (n2 - sum(b),)]
-    L.append("  // n_beta += w y^beta, |beta| <= 2P, in the slot of the homogeneous (beta, 2P - |beta|)")
-    L.append("  XG_DEV static void accum_aff(const double *x, double w, double *m) {")
-    have = {tuple(1 if i == k else 0 for i in range(D)): "x[%d]" % k for k in range(D)}
-    cnt = 0
-    for deg in range(2, P + 1):
-        for a in monomials(D - 1, deg):
-            k = next(i for i in range(D) if a[i] > 0)
-            b = list(a)
-            b[k] -= 1
-            b = tuple(b)
-            nm = "t%d" % cnt
-            cnt += 1
-            L.append("    const double %s = %s * x[%d];" % (nm, have[b], k))
-            have[a] = nm
-    groups = {}
-    for a in affine_monomials(D, n2):
-        beta = []
-        left = P
-        for i in range(D):
-            t = min(a[i], left)
-            beta.append(t)
-            left -= t
-        beta = tuple(beta)
-        gamma = tuple(x - y for x, y in zip(a, beta))
-        groups.setdefault(beta, []).append((a, gamma))
-    for b in affine_monomials(D, P):
-        if b not in groups:
-            continue
-        L.append("    {")
-        L.append("      const double wb = %s;" % ("w" if b == zero else "w * " + have[b]))
-        for a, gamma in groups[b]:
-            s = slot(a)
-            if gamma == zero:
-                L.append("      m[%d] += wb;" % s)
-            else:
-                L.append("      m[%d] = fma(wb, %s, m[%d]);" % (s, have[gamma], s))
-        L.append("    }")
-    L.append("  }")
-
-
 def gen_series(D, P, L, idx2):
     """aser_first / aser_step: the truncated power series of
 
         prod_v 1 / (1 - <z, y_v>) = sum_beta h_beta z^beta,  |beta| <= 2P,
 
-    one vertex y_v of a simplex at a time (h in the slots of accum_aff).  The
-    integral of y^beta over a simplex of dimension k with vertices y_v is
-    |T| k! beta! / (|beta| + k)! h_beta (Dirichlet's integral), so a piece's
-    moments cost 3 FMAs per monomial of degree < 2P and vertex, whatever the
+    one vertex y_v of a simplex at a time (h_beta in the slot of the homogeneous
+    moment (beta, 2P - |beta|)).  The integral of y^beta over a simplex of
+    dimension k with vertices y_v is |T| k! beta! / (|beta| + k)! h_beta
+    (Dirichlet's integral), so a piece's moments cost 3 FMAs per monomial of degree < 2P and vertex, whatever the
     degree's quadrature rule: multiplying by 1 / (1 - l) is the in-place
     recursion h_beta += sum_i l_i h_(beta - e_i) in ascending degree.  Two
     simplices that share all but one vertex (y_p of the one with weight w_1,
@@ -467,11 +414,6 @@ def gen_series(D, P, L, idx2):
                 e = "y[%d] * %s" % (i, src) if e is None else "fma(y[%d], %s, %s)" % (i, src, e)
             L.append("    h[%d] = %s;" % (slot(b), e))
         L.append("  }")
-        if first:
-            L.append("  XG_DEV static void aser_first(const double *y, double w, double *h) {")
-            L.append("    const double v[%d] = {%s};" % (D, ", ".join(["0.0"] * D)))
-            L.append("    aser_first(y, w, v, h);")
-            L.append("  }")
 
 
 def gen_series_table(D, P):
@@ -610,7 +552,6 @@ def gen(D, P):
         L.append("    }")
     L.append("  }")
     if D == 3:
-        gen_affine(D, P, L, idx2)
         gen_series(D, P, L, idx2)
     # ---- complement: m <- (moments of the whole reference simplex) - m.
     # int_T lam^alpha = |T| D! alpha! / (|alpha| + D)! with |T| = 1/D! (the

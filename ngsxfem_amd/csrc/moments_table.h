@@ -1246,31 +1246,6 @@ struct Moments<3, 1> {
       m[9] = fma(wb, l[3], m[9]);
     }
   }
-  // n_beta += w y^beta, |beta| <= 2P, in the slot of the homogeneous (beta, 2P - |beta|)
-  XG_DEV static void accum_aff(const double *x, double w, double *m) {
-    {
-      const double wb = w;
-      m[9] += wb;
-    }
-    {
-      const double wb = w * x[0];
-      m[3] += wb;
-      m[0] = fma(wb, x[0], m[0]);
-      m[1] = fma(wb, x[1], m[1]);
-      m[2] = fma(wb, x[2], m[2]);
-    }
-    {
-      const double wb = w * x[1];
-      m[6] += wb;
-      m[4] = fma(wb, x[1], m[4]);
-      m[5] = fma(wb, x[2], m[5]);
-    }
-    {
-      const double wb = w * x[2];
-      m[8] += wb;
-      m[7] = fma(wb, x[2], m[7]);
-    }
-  }
   // h = (w - <z, v>) / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_first(const double *y, double w, const double *v, double *h) {
     h[9] = w;
@@ -1283,10 +1258,6 @@ struct Moments<3, 1> {
     h[4] = y[1] * h[6];
     h[5] = fma(y[2], h[6], y[1] * h[8]);
     h[7] = y[2] * h[8];
-  }
-  XG_DEV static void aser_first(const double *y, double w, double *h) {
-    const double v[3] = {0.0, 0.0, 0.0};
-    aser_first(y, w, v, h);
   }
   // h <- h / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_step(const double *y, double *h) {
@@ -1503,80 +1474,6 @@ struct Moments<3, 2> {
       m[34] = fma(wb, t9, m[34]);
     }
   }
-  // n_beta += w y^beta, |beta| <= 2P, in the slot of the homogeneous (beta, 2P - |beta|)
-  XG_DEV static void accum_aff(const double *x, double w, double *m) {
-    const double t0 = x[0] * x[0];
-    const double t1 = x[1] * x[0];
-    const double t2 = x[2] * x[0];
-    const double t3 = x[1] * x[1];
-    const double t4 = x[2] * x[1];
-    const double t5 = x[2] * x[2];
-    {
-      const double wb = w;
-      m[34] += wb;
-    }
-    {
-      const double wb = w * x[0];
-      m[19] += wb;
-    }
-    {
-      const double wb = w * x[1];
-      m[29] += wb;
-    }
-    {
-      const double wb = w * x[2];
-      m[33] += wb;
-    }
-    {
-      const double wb = w * t0;
-      m[9] += wb;
-      m[3] = fma(wb, x[0], m[3]);
-      m[6] = fma(wb, x[1], m[6]);
-      m[8] = fma(wb, x[2], m[8]);
-      m[0] = fma(wb, t0, m[0]);
-      m[1] = fma(wb, t1, m[1]);
-      m[2] = fma(wb, t2, m[2]);
-      m[4] = fma(wb, t3, m[4]);
-      m[5] = fma(wb, t4, m[5]);
-      m[7] = fma(wb, t5, m[7]);
-    }
-    {
-      const double wb = w * t1;
-      m[15] += wb;
-      m[12] = fma(wb, x[1], m[12]);
-      m[14] = fma(wb, x[2], m[14]);
-      m[10] = fma(wb, t3, m[10]);
-      m[11] = fma(wb, t4, m[11]);
-      m[13] = fma(wb, t5, m[13]);
-    }
-    {
-      const double wb = w * t2;
-      m[18] += wb;
-      m[17] = fma(wb, x[2], m[17]);
-      m[16] = fma(wb, t5, m[16]);
-    }
-    {
-      const double wb = w * t3;
-      m[25] += wb;
-      m[22] = fma(wb, x[1], m[22]);
-      m[24] = fma(wb, x[2], m[24]);
-      m[20] = fma(wb, t3, m[20]);
-      m[21] = fma(wb, t4, m[21]);
-      m[23] = fma(wb, t5, m[23]);
-    }
-    {
-      const double wb = w * t4;
-      m[28] += wb;
-      m[27] = fma(wb, x[2], m[27]);
-      m[26] = fma(wb, t5, m[26]);
-    }
-    {
-      const double wb = w * t5;
-      m[32] += wb;
-      m[31] = fma(wb, x[2], m[31]);
-      m[30] = fma(wb, t5, m[30]);
-    }
-  }
   // h = (w - <z, v>) / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_first(const double *y, double w, const double *v, double *h) {
     h[34] = w;
@@ -1614,10 +1511,6 @@ struct Moments<3, 2> {
     h[23] = fma(y[2], h[24], y[1] * h[27]);
     h[26] = fma(y[2], h[27], y[1] * h[31]);
     h[30] = y[2] * h[31];
-  }
-  XG_DEV static void aser_first(const double *y, double w, double *h) {
-    const double v[3] = {0.0, 0.0, 0.0};
-    aser_first(y, w, v, h);
   }
   // h <- h / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_step(const double *y, double *h) {
@@ -2299,169 +2192,6 @@ struct Moments<3, 3> {
       m[83] = fma(wb, t29, m[83]);
     }
   }
-  // n_beta += w y^beta, |beta| <= 2P, in the slot of the homogeneous (beta, 2P - |beta|)
-  XG_DEV static void accum_aff(const double *x, double w, double *m) {
-    const double t0 = x[0] * x[0];
-    const double t1 = x[1] * x[0];
-    const double t2 = x[2] * x[0];
-    const double t3 = x[1] * x[1];
-    const double t4 = x[2] * x[1];
-    const double t5 = x[2] * x[2];
-    const double t6 = t0 * x[0];
-    const double t7 = t1 * x[0];
-    const double t8 = t2 * x[0];
-    const double t9 = t3 * x[0];
-    const double t10 = t4 * x[0];
-    const double t11 = t5 * x[0];
-    const double t12 = t3 * x[1];
-    const double t13 = t4 * x[1];
-    const double t14 = t5 * x[1];
-    const double t15 = t5 * x[2];
-    {
-      const double wb = w;
-      m[83] += wb;
-    }
-    {
-      const double wb = w * x[0];
-      m[55] += wb;
-    }
-    {
-      const double wb = w * x[1];
-      m[76] += wb;
-    }
-    {
-      const double wb = w * x[2];
-      m[82] += wb;
-    }
-    {
-      const double wb = w * t0;
-      m[34] += wb;
-    }
-    {
-      const double wb = w * t1;
-      m[49] += wb;
-    }
-    {
-      const double wb = w * t2;
-      m[54] += wb;
-    }
-    {
-      const double wb = w * t3;
-      m[70] += wb;
-    }
-    {
-      const double wb = w * t4;
-      m[75] += wb;
-    }
-    {
-      const double wb = w * t5;
-      m[81] += wb;
-    }
-    {
-      const double wb = w * t6;
-      m[19] += wb;
-      m[9] = fma(wb, x[0], m[9]);
-      m[15] = fma(wb, x[1], m[15]);
-      m[18] = fma(wb, x[2], m[18]);
-      m[3] = fma(wb, t0, m[3]);
-      m[6] = fma(wb, t1, m[6]);
-      m[8] = fma(wb, t2, m[8]);
-      m[12] = fma(wb, t3, m[12]);
-      m[14] = fma(wb, t4, m[14]);
-      m[17] = fma(wb, t5, m[17]);
-      m[0] = fma(wb, t6, m[0]);
-      m[1] = fma(wb, t7, m[1]);
-      m[2] = fma(wb, t8, m[2]);
-      m[4] = fma(wb, t9, m[4]);
-      m[5] = fma(wb, t10, m[5]);
-      m[7] = fma(wb, t11, m[7]);
-      m[10] = fma(wb, t12, m[10]);
-      m[11] = fma(wb, t13, m[11]);
-      m[13] = fma(wb, t14, m[13]);
-      m[16] = fma(wb, t15, m[16]);
-    }
-    {
-      const double wb = w * t7;
-      m[29] += wb;
-      m[25] = fma(wb, x[1], m[25]);
-      m[28] = fma(wb, x[2], m[28]);
-      m[22] = fma(wb, t3, m[22]);
-      m[24] = fma(wb, t4, m[24]);
-      m[27] = fma(wb, t5, m[27]);
-      m[20] = fma(wb, t12, m[20]);
-      m[21] = fma(wb, t13, m[21]);
-      m[23] = fma(wb, t14, m[23]);
-      m[26] = fma(wb, t15, m[26]);
-    }
-    {
-      const double wb = w * t8;
-      m[33] += wb;
-      m[32] = fma(wb, x[2], m[32]);
-      m[31] = fma(wb, t5, m[31]);
-      m[30] = fma(wb, t15, m[30]);
-    }
-    {
-      const double wb = w * t9;
-      m[44] += wb;
-      m[40] = fma(wb, x[1], m[40]);
-      m[43] = fma(wb, x[2], m[43]);
-      m[37] = fma(wb, t3, m[37]);
-      m[39] = fma(wb, t4, m[39]);
-      m[42] = fma(wb, t5, m[42]);
-      m[35] = fma(wb, t12, m[35]);
-      m[36] = fma(wb, t13, m[36]);
-      m[38] = fma(wb, t14, m[38]);
-      m[41] = fma(wb, t15, m[41]);
-    }
-    {
-      const double wb = w * t10;
-      m[48] += wb;
-      m[47] = fma(wb, x[2], m[47]);
-      m[46] = fma(wb, t5, m[46]);
-      m[45] = fma(wb, t15, m[45]);
-    }
-    {
-      const double wb = w * t11;
-      m[53] += wb;
-      m[52] = fma(wb, x[2], m[52]);
-      m[51] = fma(wb, t5, m[51]);
-      m[50] = fma(wb, t15, m[50]);
-    }
-    {
-      const double wb = w * t12;
-      m[65] += wb;
-      m[61] = fma(wb, x[1], m[61]);
-      m[64] = fma(wb, x[2], m[64]);
-      m[58] = fma(wb, t3, m[58]);
-      m[60] = fma(wb, t4, m[60]);
-      m[63] = fma(wb, t5, m[63]);
-      m[56] = fma(wb, t12, m[56]);
-      m[57] = fma(wb, t13, m[57]);
-      m[59] = fma(wb, t14, m[59]);
-      m[62] = fma(wb, t15, m[62]);
-    }
-    {
-      const double wb = w * t13;
-      m[69] += wb;
-      m[68] = fma(wb, x[2], m[68]);
-      m[67] = fma(wb, t5, m[67]);
-      m[66] = fma(wb, t15, m[66]);
-    }
-    {
-      const double wb = w * t14;
-      m[74] += wb;
-      m[73] = fma(wb, x[2], m[73]);
-      m[72] = fma(wb, t5, m[72]);
-      m[71] = fma(wb, t15, m[71]);
-    }
-    {
-      const double wb = w * t15;
-      m[80] += wb;
-      m[79] = fma(wb, x[2], m[79]);
-      m[78] = fma(wb, t5, m[78]);
-      m[77] = fma(wb, t15, m[77]);
-    }
-  }
   // h = (w - <z, v>) / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_first(const double *y, double w, const double *v, double *h) {
     h[83] = w;
@@ -2548,10 +2278,6 @@ struct Moments<3, 3> {
     h[66] = fma(y[2], h[67], y[1] * h[72]);
     h[71] = fma(y[2], h[72], y[1] * h[78]);
     h[77] = y[2] * h[78];
-  }
-  XG_DEV static void aser_first(const double *y, double w, double *h) {
-    const double v[3] = {0.0, 0.0, 0.0};
-    aser_first(y, w, v, h);
   }
   // h <- h / (1 - <z, y>), truncated at degree 2P
   XG_DEV static void aser_step(const double *y, double *h) {

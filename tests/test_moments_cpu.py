@@ -129,14 +129,15 @@ extern "C" int mom_hsimplex(int D, int P, const double *lv, int nv, double s, do
   HCASE(1, 1) HCASE(1, 2) HCASE(2, 1) HCASE(2, 2) HCASE(3, 1) HCASE(3, 2)
   return -1;
 }
-// Moments<3, 3>::accum_aff over a point set in centred coordinates
-// y = x - 1/4, then the dense map xg_aff33 to the homogeneous moments
+// the affine moments sum w y^beta, |beta| <= 6, of a point set in centred
+// coordinates y = x - 1/4 (the homogeneous ones of (y, 1)), then the dense map
+// xg_aff33 to the homogeneous moments
 extern "C" int mom_accum_aff(const double *pts, const double *w, int n, double *m) {
   using M = xg::Moments<3, 3>;
   double nn[M::NM] = {0};
   for (int q = 0; q < n; ++q) {
-    const double y[3] = {pts[3 * q] - 0.25, pts[3 * q + 1] - 0.25, pts[3 * q + 2] - 0.25};
-    M::accum_aff(y, w[q], nn);
+    const double y[4] = {pts[3 * q] - 0.25, pts[3 * q + 1] - 0.25, pts[3 * q + 2] - 0.25, 1.0};
+    M::accum(y, w[q], nn);
   }
   for (int a = 0; a < M::NM; ++a) {
     double s = 0;
@@ -158,10 +159,10 @@ extern "C" int mom_series(int P, const double *verts, int k, double w, double w2
     const int nv = w2 != 0.0 ? 4 : k + 1;                                                     \
     for (int v = 0; v < nv; ++v)                                                              \
       for (int d = 0; d < 3; ++d) y[v][d] = verts[3 * v + d] - 0.25;                          \
-    double n[3];                                                                              \
-    for (int d = 0; d < 3; ++d) n[d] = w * y[3][d] + w2 * y[1][d];                            \
-    if (w2 != 0.0) M::aser_first(y[0], w + w2, n, h);                                         \
-    else M::aser_first(y[0], w, h);                                                           \
+    double n[3] = {};                                                                         \
+    for (int d = 0; d < 3; ++d)                                                               \
+      if (w2 != 0.0) n[d] = w * y[3][d] + w2 * y[1][d];                                       \
+    M::aser_first(y[0], w + w2, n, h);                                                        \
     for (int v = 1; v < 4; ++v) M::aser_step(y[v], h); /* a zero step changes nothing */      \
     for (int r = 0; r < M::NM; ++r) h[r] *= xg::xg_aser3##PP[r][k == 3 ? 0 : 1];              \
     for (int a = 0; a < M::NM; ++a) {                                                         \
@@ -266,9 +267,9 @@ def test_vertex_recursion_gives_exact_simplex_moments(momlib, D, P):
 
 
 def test_affine_accumulation_equals_homogeneous(momlib):
-    """accum_aff (monomials of three centred affine coordinates y = lam - 1/4,
-    degree <= 6, lam_3 never formed) followed by the dense map xg_aff33 gives
-    the homogeneous degree-6 moments of accum: on random points with
+    """the sums of the monomials of three centred affine coordinates
+    y = lam - 1/4, degree <= 6, through the dense map xg_aff33 are the
+    homogeneous degree-6 moments of accum: on random points with
     mixed-sign weights (complemented pieces), on points clustered at each
     vertex (where the map cancels most), and on the closed form of the whole
     reference tetrahedron (int lam^alpha = 3! alpha! / 9! |T|, a
