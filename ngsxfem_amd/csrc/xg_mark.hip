@@ -829,9 +829,6 @@ size_t mark_scratch_ints(int ne) {
   return (size_t)(nblk + 1) + (size_t)((nblk + SCAN_TILE - 1) / SCAN_TILE + 1);
 }
 
-// marking + compaction on an explicit stream with caller-owned scratch
-// (mark_scratch_ints(ne) int32); only kernel launches, so the sequence can be
-// captured into a hipGraph.  n_cut (nullable) receives the cut count.
 // domains and cut ratios of 2^20 elements (9 MB beside 16 MB of rows on tets)
 // are more than the L2s hold; on smaller meshes the next kernel finds them
 // there, and the plain stores are 1 us faster (60 x 60 cells: 35.4 against 36.5
@@ -851,6 +848,9 @@ static void launch_mark(hipStream_t st, int D, int nblk, int ne, const int32_t *
 #undef XG_MARK
 }
 
+// marking + compaction on an explicit stream with caller-owned scratch
+// (mark_scratch_ints(ne) int32); only kernel launches, so the sequence can be
+// captured into a hipGraph.  n_cut (nullable) receives the cut count.
 int mark_compact(hipStream_t st, int32_t *d_err, int D, int ne, const int32_t *el2v, const double *lset,
                  uint8_t *dt, double *cr, uint32_t *bits, int32_t *scratch, int32_t *cut_list, int32_t *n_cut) {
   const int nw = (ne + 31) / 32;

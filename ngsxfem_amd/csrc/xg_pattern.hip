@@ -6,8 +6,9 @@
 // built on the GPU, row by row: the elements of every dof are listed (a count
 // per dof, a scan, a fill), a wave sorts the columns of a row's elements in
 // registers and drops the repeated ones (rows of over 1024 candidates: a block,
-// in LDS), and a scan of the row lengths places the rows.  Bound: the rows' sorts (a P2 edge row of a tetrahedral mesh has
-// about 60 candidates for 27 columns).  32^3 cells of 6 tetrahedra, P2 (19.7 M
+// in LDS), and a scan of the row lengths places the rows.  Bound: the rows'
+// sorts (a P2 edge row of a tetrahedral mesh has about 60 candidates for 27
+// columns).  32^3 cells of 6 tetrahedra, P2 (19.7 M
 // couplings, 275,000 rows): graph, matrices and values 2067 -> 368 us against
 // the radix sort of all couplings as 64-bit keys (eight passes over 16 B each,
 // unique, an atomic count per row), which rows that are long on average

@@ -2142,6 +2142,9 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
     if constexpr (WHICH == 3) {
       const int nv = nleaf + 2 * c4.y, ni = nleaf;
       int best = 1 << 30;
+      // 6 of 16 columns: only 1-3 leaves; 11: three volume pieces a record.  Only
+      // 2-2 leaves would want 12, and mixtures do not: up to 13 columns measured
+      // 24.13 against 24.02 ms (128^3 cells, P3, L = 4)
       for (int c = 6; c <= 11; ++c) {
         const int r = max((nv + 4 * c - 1) / (4 * c), (ni + 63 - 4 * c) / (64 - 4 * c));
         if (r < best) {
@@ -2359,9 +2362,9 @@ __global__ __launch_bounds__(64, PM == 1 ? 3 : 2) void k_sdx_leaves(int nel, con
   }
 }
 
-// table rows of each listed element (uncut nodes of the kept side from the
-// back of the list, complemented leaves after the cut leaves) added to its
-// moments; one wave per element.  Rows of an even length (p = 1, 3): R =
+// table rows of each listed element's complemented leaves (after the cut leaves
+// in its list; the walk has summed the uncut nodes) added to its moments; one
+// wave per element.  Rows of an even length (p = 1, 3): R =
 // NM / 4 lanes per row, each loading 4 moments as two 16-byte loads, so a
 // wave reads 64 / R rows per instruction (3 for p = 3), four rounds of them
 // in flight; the rows' partial sums meet in LDS.  p = 2 (35 moments, rows not

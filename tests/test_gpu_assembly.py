@@ -151,7 +151,8 @@ def test_csr_pattern_device_matches_numpy(dev_abi):
                                         (10, 52, 40), (20, 51, 3000), (20, 52, 3000), (64, 90, 4000), (64, 300, 700)])
 def test_csr_pattern_row_lengths(dev_abi, ndof, deg, n):
     """tables of 1 to 6390 couplings per row on average, on both sides of 256,
-    where they go to the radix sort, with skipped dofs, repeated dofs in an
+    where they go to the radix sort (rows of 1000 candidates are the longest
+    that go row by row here), with skipped dofs, repeated dofs in an
     element and empty rows; a column list that is too short is an error"""
     torch, _abi, ctx = dev_abi
     rng = np.random.default_rng(ndof * deg + n)

@@ -254,9 +254,10 @@ def test_pipeline_queue_modes_agree(dev, monkeypatch):
 
 
 def test_pipeline_fused_and_separate_leaf_kernels(orc, dev, monkeypatch):
-    """P3 with the volume side and the interface: one leaf launch with lane
-    roles (4-point tasks) or one launch per part (XG_SDX_NOFUSE=1, 8-point
-    volume tasks); the same sums in another order: equal to 1e-13, and both
+    """P3 with the volume side and the interface: one leaf launch whose
+    lanes split into volume and interface columns, or one launch per part
+    (XG_SDX_NOFUSE=1, every lane on the part); a piece per lane in both, the
+    same sums in another order: equal to 1e-13, and both
     equal the oracle to 1e-12; the piece counts are identical"""
     torch, _abi, ctx = dev
     mesh = MakeStructured3DMesh(nx=6, ny=6, nz=6)
