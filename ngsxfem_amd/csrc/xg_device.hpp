@@ -310,7 +310,7 @@ XG_DEV bool decompose(const double *l, int dt, Decomp &dc) {
 // m = sum_i [l_i >= 0] << i, so it is tabulated at compile time (same
 // construction as decompose()).  Kernels whose element is wave-uniform read
 // the entry with scalar loads instead of rebuilding it in registers.
-struct alignas(8) DecompEntry {  // (copied in words of 8 bytes)
+struct DecompEntry {
   int8_t ns, nv, nc, ok;
   int8_t v[3][4];
   int8_t ce[4][2];
@@ -376,7 +376,7 @@ constexpr DecompEntry make_decomp_entry(int D, int dt, int mask) {
 }
 
 struct DecompTable {
-  DecompEntry e[3][3][16];  // [D-1][dt][mask]
+  alignas(8) DecompEntry e[3][3][16];  // [D-1][dt][mask]; (a dimension's 48 are also copied in 8-byte words)
   constexpr DecompTable() : e{} {
     for (int D = 1; D <= 3; ++D)
       for (int dt = 0; dt < 3; ++dt)

@@ -121,7 +121,7 @@ __device__ __forceinline__ void elem_rec(ElemRec &R, const double (*V)[3], const
 // dimension D and the base rules of dimensions D and D - 1
 template <int D>
 struct StageTab {
-  DecompEntry e[3][16];
+  alignas(8) DecompEntry e[3][16];
 };
 inline size_t stage_rule_bytes(int D, int order) {  // host
   return sizeof(double) * 4 * (size_t)(xg_rule_cnt[D][order / 2 + 1] + xg_rule_cnt[D - 1][order / 2 + 1]);
