@@ -376,7 +376,7 @@ constexpr DecompEntry make_decomp_entry(int D, int dt, int mask) {
 }
 
 struct DecompTable {
-  alignas(8) DecompEntry e[3][3][16];  // [D-1][dt][mask]; (a dimension's 48 are also copied in 8-byte words)
+  DecompEntry e[3][3][16];  // [D-1][dt][mask]
   constexpr DecompTable() : e{} {
     for (int D = 1; D <= 3; ++D)
       for (int dt = 0; dt < 3; ++dt)

@@ -130,8 +130,9 @@ inline size_t stage_rule_bytes(int D, int order) {  // host
 template <int D>
 __device__ __forceinline__ void stage_tables(StageTab<D> &tab, double (*rule)[4], int order) {
   constexpr int W = sizeof(DecompEntry) / 8 * 48;
-  const uint64_t *src = reinterpret_cast<const uint64_t *>(&xg_decomp_d.e[D - 1][0][0]);
-  for (int k = threadIdx.x; k < W; k += blockDim.x) reinterpret_cast<uint64_t *>(&tab.e[0][0])[k] = src[k];
+  const char *src = reinterpret_cast<const char *>(&xg_decomp_d.e[D - 1][0][0]);
+  for (int k = threadIdx.x; k < W; k += blockDim.x)
+    __builtin_memcpy(reinterpret_cast<uint64_t *>(&tab.e[0][0]) + k, src + 8 * k, 8);
   const int nq_vol = rule_cnt(D, order), nq_if = rule_cnt(D - 1, order);
   const int off_vol = rule_off(D, order), off_if = rule_off(D - 1, order);
   for (int k = threadIdx.x; k < nq_vol + nq_if; k += blockDim.x) {
